@@ -338,6 +338,9 @@ __device__ __forceinline__ void store_epilogue(const acc_t (&acc)[TN][TM], const
       const int lr = row_base + i * MI + (lane % MI);
       rw[i] = p.ro.row_scale[tile.row0 + (lr < tile.nrows ? lr : 0)];
     }
+    // (complete here: left pending on the paths that do not use them, they are waited for in the next tile's main loop)
+#pragma unroll
+    for (int i = 0; i < I_END; i++) asm volatile("" : "+v"(rw[i]));
   }
   // GENERAL: bias, partial sums, row factors, f32 output; otherwise bf16 results straight to memory
   auto body = [&](auto act_c, auto general_c) {
@@ -503,7 +506,11 @@ __device__ __forceinline__ TilePeek peek_tile(const TiledParams& p, int num_tile
     const int sg = logical / width, first_m = sg * GSM;
     const int gsz = min(num_tiles - first_m, GSM);
     const int m_idx = first_m + (logical % width) % gsz;
-    pk.ti = p.tiles[m_idx];
+    // (a scalar load: through the vector memory counter the record would sit in the middle of the copies in flight, and the
+    // compiler waits for everything at the first use of a register it may still be arriving in, i.e. in the main loop)
+    typedef int rec_t __attribute__((ext_vector_type(4)));
+    const rec_t rec = *(const __attribute__((address_space(4))) rec_t*)(uintptr_t)(p.tiles + m_idx);
+    pk.ti = TileInfo{rec[0], rec[1], rec[2], rec[3]};
     pk.n0 = ((logical % width) / gsz) * OUT_BN;
     pk.id = id;
     pk.valid = true;
