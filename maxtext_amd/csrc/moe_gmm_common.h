@@ -471,6 +471,10 @@ __device__ __forceinline__ void dma16_buffer(const v4i& rsrc, uint32_t voff, uin
   asm volatile("" : "+s"(soff));  // (a literal offset is not an operand the instruction takes)
   asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds_addr) : "memory", "m0");
 }
+// The same without a scalar offset (descriptors that move with the stage).
+__device__ __forceinline__ void dma16_buffer(const v4i& rsrc, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff), "s"(rsrc), "s"(lds_addr) : "memory", "m0");
+}
 // ---- the tile cursor of the persistent stream kernels -------------------------------------------------------------
 // tile id -> (m-tile, n-tile): ids congruent mod 8 run on one XCD (persistent blocks are dealt round-robin to the XCDs
 // and a block's ids advance by the grid size, a multiple of 8); each XCD owns a contiguous range of the order, which

@@ -163,467 +163,376 @@ __global__ __launch_bounds__(kTgThreads) void tgmm_kernel(const TgmmParams p) {
 
 
 // ---------------------------------------------------------------------------------------
-// 256 (n) x 256 (k) output tiles for groups of many rows, on the pipeline of the direct-to-LDS GEMM: a stage is
-// 64 contraction rows of both operands (64 x 512 bytes each), copied by global_load_lds_dwordx4 (a wave
-// instruction moves two rows of 512 bytes: whole 128-byte lines) into two buffers of 64 KB; 8 waves of
-// 64 (k) x 128 (n) on v_mfma_f32_16x16x32_bf16, two k-steps of 32 MFMAs per stage; the 4 lhs fragments of a wave
-// are double-buffered in registers, each of its 8 dout fragments is reloaded for the next k-step right after the four
-// MFMAs that use it.  Fragments come out of the row-major stage through ds_read_b64_tr_b16 as in tgmm_kernel.  LDS
-// rows are unpadded, so the 16-byte chunk q of row r is stored at slot q ^ f(r), f(r) = 4 * (r % 4) ^ 2 * ((r / 8) % 2):
-// the 4 rows x 32 bytes that 16 lanes of a transposing read address, and those of the next 16 lanes (8 rows further),
-// then fall into 8 different 32-byte bank groups.  The permutation is applied on the global side (the LDS side of
-// the copy is fixed at base + 16 * lane) and stays inside a row's 512 bytes, so every request still covers whole
-// lines.  Rows past the end of the group are copied from a row of zeros.
+// 256 (n) x 256 (k) output tiles for groups of many rows, bf16 (v_mfma_f32_16x16x32_bf16) or 1-byte operands as stored (the
+// drhs product of the fp8_full backward, kernels/megablox/ops.py:590-604: float8_e4m3fn activations x float8_e5m2 gradient,
+// v_mfma_scale_f32_16x16x128_f8f6f4).  A stage is 64 (1-byte: 128) contraction rows of both operands as they lie in memory,
+// 32 KB each, copied by buffer_load ... lds (a wave instruction moves 2 rows of 512 or 4 of 256 bytes: whole 128-byte
+// lines) into two buffers of 64 KB.  The descriptor of a stage ends at the group's last row: rows past it arrive as zeros.
+// 8 waves of 64 (k) x 128 (n).  Fragments come out of the row-major stage through ds_read_b64_tr_b16 / _b8.
+//
+// Schedule: the two waves of a SIMD take turns, as in the grouped matmul of prefill.  A stage is four phases of 256
+// matrix cycles; a phase is a fetching side (fragment reads, two requests, waits), a barrier, a multiplying side and a
+// barrier, and waves 4 .. 7 run one barrier behind waves 0 .. 3.  Phases of bf16: the two k-steps of 32 rows x the two halves
+// of the dout fragments, so a stage frees its slots by halves of 32 rows; of the 1-byte operands (one instruction spans
+// the stage): pairs of dout fragments, the pair of the third phase read a phase early so that the dout slots are free for
+// the whole fourth.  A request has five (1-byte: three) phases to land.
+// Persistent blocks, one request stream across tiles: a tile's first two stages arrive behind the previous tile's products,
+// and its stores drain behind the next tile's.  Mixtral shape, same box: 16384 rows, bf16 1.68 -> 1.55 / 1.71 -> 1.61 ms (one
+// mixed stream per wave, one barrier per stage and a block per tile before; the schedule alone 1 %, the stream across tiles
+// 6 %); 1-byte at 6000 rows 0.51 -> 0.47 / 0.53 -> 0.50 ms (six stages a tile: there the descriptors as running scalars gave
+// most).  Reading the fragments between the products instead of ahead of them is slower (1.52 -> 1.60).  What bounds bf16 now:
+// with the same stage over and over (no misses in L2) 1.40 ms, i.e. 10 % is the latency of the real stream (440 cycles at
+// 67 lines in flight per CU, against 330 for the products of the forward pass), the rest the matrix units under the power
+// limit and twice as many fragment reads as a row-major operand takes.
+//
+// bf16 swizzle: the 16-byte chunk q of row r is stored at slot q ^ f(r), f(r) = 4 * (r % 4) ^ 2 * ((r / 8) % 2): the 4 rows x
+// 32 bytes that 16 lanes of a transposing read address, and those of the next 16 lanes (8 rows further), then fall into 8
+// different 32-byte bank groups.  1-byte: 16 lanes address an 8-row x 16-byte block (lane l: row l / 2, half l % 2) and lane l
+// receives column l of the 8 rows; four such reads give the 32 contraction values of a 16 x 16 x 128 fragment.  Lane group q
+// takes stage rows 32 q .. 32 q + 31 for BOTH operands (any order of the contraction index does, as long as the fragments
+// agree); chunk c of row r sits at slot c ^ (r % 8) ^ 8 * ((r / 32) % 2): the 8 rows of a read and those of the next lane
+// group fall into 16 different 16-byte bank groups.
 // ---------------------------------------------------------------------------------------
 
-constexpr int kTdTile = 256, kTdBM = 64;       // output tile edge, contraction rows per stage
+constexpr int kTdTile = 256;                   // output tile edge
 constexpr int kTdThreads = 512, kTdWaves = 8;
-constexpr int kTdRow = kTdTile * 2;            // bytes of one operand row in a stage
-constexpr int kTdOperand = kTdBM * kTdRow;     // 32 KB
-constexpr int kTdStage = 2 * kTdOperand;       // lhs rows | dout rows
-constexpr int kTdLds = 2 * kTdStage;           // two buffers
-constexpr int kTdIpw = kTdOperand / 1024 / kTdWaves;  // requests per wave, operand and stage
-constexpr int kTdLps = 2 * kTdIpw;
 
-__device__ __attribute__((aligned(512))) uint8_t tg_zero_row[kTdRow];
-
-__global__ __launch_bounds__(kTdThreads, 2) void tgmm_dl_kernel(const TgmmParams p) {
-  extern __shared__ __attribute__((aligned(1024))) uint8_t td_smem[];
-  __shared__ int s_red[kTdWaves];
-  const int tid = threadIdx.x, lane = tid % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int wk = wave % 4, wn = wave / 4;  // wave tile: 64 k x 128 n
-  const int N = p.N, K = p.K;
-
-  // Blocks b, b + 8, .. run on one XCD: give each XCD a contiguous range of tiles, walked in patches of 8 n-tiles x
-  // 4 k-tiles of one group, so that the 32 blocks an XCD runs at a time share 8 dout and 4 lhs panels in its L2.
-  const int tiles_k = K / kTdTile, tiles_n = N / kTdTile, per_group = tiles_k * tiles_n;
-  const int total = per_group * p.G_local;
-  const int q8 = total / 8, rem = total % 8, xcd = blockIdx.x % 8, loc = blockIdx.x / 8;
-  const int logical = xcd < rem ? xcd * (q8 + 1) + loc : rem * (q8 + 1) + (xcd - rem) * q8 + loc;
-  const int g_local = logical / per_group, t = logical % per_group, g = g_local + p.group_offset;
-  constexpr int GSM = 8;
-  const int width = GSM * tiles_k, first_n = (t / width) * GSM, gsz = min(tiles_n - first_n, GSM);
-  const int n0 = (first_n + (t % width) % gsz) * kTdTile, k0 = ((t % width) / gsz) * kTdTile;
-
-  // rows of group g: [start, start + size), clipped to M
-  long long part = 0;
-  for (int i = tid; i < min(g, p.G_total); i += kTdThreads) part += max(p.group_sizes[i], 0);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
-  if (lane == 0) s_red[wave] = (int)min(part, (long long)p.M);
-  __syncthreads();
-  long long start_ll = 0;
-  for (int w = 0; w < kTdWaves; w++) start_ll += s_red[w];
-  // (uniform by construction; saying so lets the requests below use a scalar base address)
-  const int start = __builtin_amdgcn_readfirstlane((int)min(start_ll, (long long)p.M));
-  const int size = __builtin_amdgcn_readfirstlane(g < p.G_total ? min(max(p.group_sizes[g], 0), p.M - start) : 0);
-
-  const int s16 = lane % 16, gq = lane / 16;
-  if (size == 0) {  // an empty group's gradient is zero
-    for (int i = tid; i < kTdTile * (kTdTile / 4); i += kTdThreads) {
-      const size_t off = ((size_t)g_local * N + n0 + i / (kTdTile / 4)) * K + k0 + (i % (kTdTile / 4)) * 4;
-      tgmm_store4(p, off, n0 + i / (kTdTile / 4), 0.f, 0.f, 0.f, 0.f);
-    }
-    return;
-  }
-
-  // ---- sources of this wave's requests: request i of an operand covers stage rows 2 * (4 * wave + i) + {0, 1}.  A
-  // stage's first row is a scalar base, the lane adds a 32-bit offset.  Only a group's last stage can hold rows past its
-  // end: requests of full stages (FULL) need no check, the others pick the row of zeros per lane, without a branch.
-  // Requests i and i + 2 of a wave are 4 rows apart, which leaves the swizzle as it is: two per-lane offsets per operand.
-  uint32_t a_off[2], b_off[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int r = 2 * (wave * kTdIpw + i) + lane / 32;
-    const int chunk = (lane % 32) ^ tr_swz(r);
-    a_off[i] = (uint32_t)r * K * 2 + chunk * 16;
-    b_off[i] = (uint32_t)r * N * 2 + chunk * 16;
-  }
-  static_assert(kTdIpw == 4, "request i + 2 is request i four rows further down");
-  const uint8_t* const a_base = (const uint8_t*)p.lhs + ((size_t)start * K + k0) * 2;
-  const uint8_t* const b_base = (const uint8_t*)p.dout + ((size_t)start * N + n0) * 2;
-  const size_t a_step = (size_t)kTdBM * K * 2, b_step = (size_t)kTdBM * N * 2;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)td_smem;
-  auto issue_one = [&](auto full_c, int kt, int buf, int idx) {
-    constexpr bool FULL = decltype(full_c)::value;
-    const int i = idx % kTdIpw;
-    const bool is_a = idx < kTdIpw;
-    const uint8_t* src = is_a ? a_base + (kt * a_step + (size_t)(i / 2) * 8 * K) + a_off[i % 2]
-                              : b_base + (kt * b_step + (size_t)(i / 2) * 8 * N) + b_off[i % 2];
-    if constexpr (!FULL) {
-      int l = lane;
-      asm volatile("" : "+v"(l));  // keeps what follows inside the (short) loops that need it, out of the steady state's registers
-      const int r = 2 * (wave * kTdIpw + i) + l / 32;
-      const uint64_t keep = kt * kTdBM + r < size ? ~0ull : 0ull;
-      const uint64_t zero = (uint64_t)(tg_zero_row + ((l % 32) ^ tr_swz(r)) * 16);
-      src = (const uint8_t*)(((uint64_t)src & keep) | (zero & ~keep));
-    }
-    // (untracked: which buffer a copy writes and a read reads is settled by the explicit vmcnt waits and barriers below)
-    dma16_untracked(src, lds_base + buf * kTdStage + (is_a ? 0 : kTdOperand) + (wave * kTdIpw + i) * 1024);
-  };
-
-  // ---- fragments: lane (group gq, s16) addresses row 8 * gq + s16 / 4 (+ 4) of the k-step's 32 rows and the 8 bytes
-  // 8 * (s16 % 4) of the fragment's 32-byte row slice; fragment f of an operand is 32 * f bytes further along the row
-  // before the swizzle, which turns the step into an XOR of address bits 5..7.
-  const int xmask = ((s16 / 4) << 2) ^ ((gq & 1) << 1);
-  const int row_part = (gq * 8 + s16 / 4) * kTdRow, piece = s16 % 4;
-  const int k_base = row_part + ((((8 * wk + piece / 2) ^ xmask) << 4) | ((piece & 1) << 3));
-  const int n_base = row_part + ((((16 * wn + piece / 2) ^ xmask) << 4) | ((piece & 1) << 3));
-  v8bf fk[2][4], fn[8];
-  // (the two bases pass through an empty asm so that the 12 fragment addresses are formed where they are used, an XOR
-  // and an add each, instead of living in 12 registers across the loop: the kernel has none to spare)
-  auto read_k = [&](int buf, int ks, int set, int f) {
-    int base = k_base;
-    asm volatile("" : "+v"(base));
-    fk[set][f] = tr_read_frag(td_smem + buf * kTdStage + ks * 32 * kTdRow + (base ^ (32 * f)), kTdRow);
-  };
-  auto read_n = [&](int buf, int ks, int f) {
-    int base = n_base;
-    asm volatile("" : "+v"(base));
-    fn[f] = tr_read_frag(td_smem + buf * kTdStage + kTdOperand + ks * 32 * kTdRow + (base ^ (32 * f)), kTdRow);
-  };
-
-  v4f acc[4][8];  // [k fragment][n fragment]
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc[j][i][r] = 0.f;
-
-  // One k-step: 32 MFMAs on lhs fragment set SET with, slotted between them, the fragment reads of the next k-step
-  // (RD) and the requests of a stage (LD, spread over the k-step).
-  auto kstep = [&](auto set_c, auto rd_c, auto ld_c, auto full_c, int rd_buf, int rd_ks, int ld_kt, int ld_buf) {
-    constexpr int SET = decltype(set_c)::value;
-    constexpr bool RD = decltype(rd_c)::value, LD = decltype(ld_c)::value;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fk[SET][j], fn[i], acc[j][i], 0, 0, 0);
-        // (behind every fourth MFMA: one request per MFMA fills the address unit's queue and stalls the MFMAs behind it;
-        // both shapes of the Mixtral layer 1.86 -> 1.69 / 1.72 ms, every third 1.75 / 1.76 ms)
-        if (LD && (i * 4 + j) % 4 == 0 && (i * 4 + j) / 4 < kTdLps) issue_one(full_c, ld_kt, ld_buf, (i * 4 + j) / 4);
-        if (RD && j == 1 && i < 4) read_k(rd_buf, rd_ks, SET ^ 1, i);
-        if (RD && j == 3) read_n(rd_buf, rd_ks, i);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-  };
-  using T_ = std::true_type;
-  using F_ = std::false_type;
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, 1>;
-
-  // Stage kt sits in buffer kt % 2.  During a stage's first k-step the fragments of its second one are read, after
-  // which no wave needs the buffer any more: once every wave has seen its own reads return and its requests of stage
-  // kt+1 land, the block meets, and during the second k-step the fragments of stage kt+1 are read from the other
-  // buffer while stage kt+2 is requested into this one (past the last stage the last one is requested again, into a
-  // buffer nobody reads any more, which keeps the bookkeeping uniform).
-  const int nk = (size + kTdBM - 1) / kTdBM;
-#pragma unroll
-  for (int s = 0; s < 2; s++)
-#pragma unroll
-    for (int i = 0; i < kTdLps; i++) issue_one(F_{}, min(s, nk - 1), s, i);
-  wait_vmcnt<0>();
-  __syncthreads();
-#pragma unroll
-  for (int f = 0; f < 8; f++) read_n(0, 0, f);
-#pragma unroll
-  for (int f = 0; f < 4; f++) read_k(0, 0, 0, f);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  kstep(S0{}, T_{}, F_{}, F_{}, 0, 1, 0, 0);
-  int kt = 0;
-  const int nfull = size / kTdBM;  // stages 0 .. nfull-1 hold 64 rows of the group
-  for (; kt + 2 < nfull; kt++) {   // steady state: the stage requested is a full one
-    const int buf = kt % 2;
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    wait_vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-    kstep(S1{}, T_{}, T_{}, T_{}, buf ^ 1, 0, kt + 2, buf);
-    kstep(S0{}, T_{}, F_{}, F_{}, buf ^ 1, 1, 0, 0);
-  }
-  for (; kt + 1 < nk; kt++) {
-    const int buf = kt % 2;
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    wait_vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-    kstep(S1{}, T_{}, T_{}, F_{}, buf ^ 1, 0, min(kt + 2, nk - 1), buf);
-    kstep(S0{}, T_{}, F_{}, F_{}, buf ^ 1, 1, 0, 0);
-  }
-  kstep(S1{}, F_{}, F_{}, F_{}, 0, 0, 0, 0);
-  wait_vmcnt<0>();  // no request may still be writing LDS when the block ends
-
-  // D[k][n]: the lane holds n = s16 and k = 4 * gq + r of each 16 x 16 tile
-  if (!p.out_f32 && !p.existing) {
-    // plain bf16 results: neighbouring k-tiles trade halves between lanes 16 apart, so that a lane stores 16 bytes and
-    // the 64 bytes of a row n leave in one instruction
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int n = n0 + wn * 128 + i * 16 + s16;
-      const float sc = p.n_scale ? p.n_scale[n] : 1.0f;
-#pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(acc[j][i][0] * sc, acc[j][i][1] * sc),
-                                                         pack_bf16x2(acc[j + 1][i][0] * sc, acc[j + 1][i][1] * sc), false, false);
-        const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(acc[j][i][2] * sc, acc[j][i][3] * sc),
-                                                         pack_bf16x2(acc[j + 1][i][2] * sc, acc[j + 1][i][3] * sc), false, false);
-        const int k = k0 + wk * 64 + (j + (gq & 1)) * 16 + 4 * (gq & ~1);
-        *(uint4*)((uint16_t*)p.out + ((size_t)g_local * N + n) * K + k) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const int n = n0 + wn * 128 + i * 16 + s16;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int k = k0 + wk * 64 + j * 16 + 4 * gq;
-      const size_t off = ((size_t)g_local * N + n) * K + k;
-      tgmm_store4(p, off, n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
-    }
-  }
-}
-
-
-// ---------------------------------------------------------------------------------------
-// The same 256 x 256 tiles for 1-byte operands: the drhs product of the fp8_full backward (kernels/megablox/ops.py:590-604:
-// float8_e4m3fn activations x float8_e5m2 gradient, the contraction running over the rows of both) on
-// v_mfma_scale_f32_16x16x128_f8f6f4, without widening either operand.  A stage is 128 contraction rows of both operands
-// (128 x 256 bytes each, a wave instruction copies four rows), two buffers of 64 KB.  Fragments come out of the row-major
-// stage through ds_read_b64_tr_b8: 16 lanes address an 8-row x 16-byte block (lane l: row l / 2, half l % 2) and lane l
-// receives column l of the 8 rows; four such reads give a lane the 32 contraction values of its column that one
-// 16 x 16 x 128 fragment holds.  Lane group q takes stage rows 32 q .. 32 q + 31 for BOTH operands, which is all the
-// instruction needs (any order of the contraction index, as long as the two fragments agree).  A fragment is 8
-// registers, so a wave (64 k x 128 n) keeps its 4 lhs fragments and a ring of 4 of its 8 dout fragments beside the 128
-// accumulators and multiplies a stage in two halves of 16 MFMAs: dout fragments 0 .. 3 from the ring (each slot reloaded
-// with fragment + 4 after its four MFMAs), then fragments 4 .. 7, lhs fragment by lhs fragment, with the next stage's
-// fragments read behind them.  The 16-byte chunk c of stage row r sits at slot c ^ (r % 8) ^ 8 * ((r / 32) % 2): the 8 rows
-// of a read and those of the next lane group fall into 16 different 16-byte bank groups.
-// ---------------------------------------------------------------------------------------
-
-constexpr int kT8BM = 128;                            // contraction rows per stage
-constexpr int kT8Row = kTdTile;                       // bytes of one operand row in a stage
-constexpr int kT8Operand = kT8BM * kT8Row;            // 32 KB
-constexpr int kT8Stage = 2 * kT8Operand;              // lhs rows | dout rows
-constexpr int kT8Lds = 2 * kT8Stage;                  // two buffers
-constexpr int kT8Ipw = kT8Operand / 1024 / kTdWaves;  // requests per wave, operand and stage
-constexpr int kT8Lps = 2 * kT8Ipw;
-constexpr int kT8ReqStride = 2;                       // a stage's requests go out behind every second MFMA of a half
-
-__device__ __forceinline__ int t8_swz(int row) { return (row & 7) ^ (((row >> 5) & 1) << 3); }
+template <bool F8_, int DF_ = 0>
+struct TgCfg {
+  static constexpr bool F8 = F8_;
+  static constexpr int DF = DF_;               // element format of a 1-byte dout: 0 = e4m3, 1 = e5m2 (lhs is e4m3)
+  static constexpr int ESZ = F8 ? 1 : 2;
+  static constexpr int BM = F8 ? 128 : 64;     // contraction rows per stage
+  static constexpr int ROW = kTdTile * ESZ;    // bytes of one operand row in a stage
+  static constexpr int OPERAND = BM * ROW;     // 32 KB
+  static constexpr int STAGE = 2 * OPERAND;    // lhs rows | dout rows
+  static constexpr int LDS = 2 * STAGE;
+  static constexpr int RPR = 1024 / ROW;       // rows per request
+  static constexpr int IPW = OPERAND / 1024 / kTdWaves;  // requests per wave, operand and stage
+  static_assert(OPERAND == 32768 && IPW == 4, "stage shape");
+  __device__ static __forceinline__ int swz(int row) { return F8 ? (row & 7) ^ (((row >> 5) & 1) << 3) : tr_swz(row); }
+};
 
 typedef int v2i_t8 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i_t8* lds_v2i_t8;
-__device__ __forceinline__ void tr8_read_frag(v8i& f, const uint8_t* p) {
+__device__ __forceinline__ void tr8_read_frag(v8i& f, const uint8_t* p, int row_bytes) {
 #pragma unroll
   for (int t = 0; t < 4; t++) {
-    const v2i_t8 x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t8)(p + t * 8 * kT8Row));
+    const v2i_t8 x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t8)(p + t * 8 * row_bytes));
     f[2 * t] = x[0];
     f[2 * t + 1] = x[1];
   }
 }
 
-template <int DF>  // element format of dout: 0 = e4m3, 1 = e5m2 (lhs is e4m3)
-__global__ __launch_bounds__(kTdThreads, 2) void tgmm_f8_kernel(const TgmmParams p) {
-  extern __shared__ __attribute__((aligned(1024))) uint8_t t8_smem[];
-  __shared__ int s_red[kTdWaves];
+template <typename C>
+__global__ __launch_bounds__(kTdThreads, 2) void tgmm_dl_kernel(const TgmmParams p) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t td_smem[];
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wk = wave % 4, wn = wave / 4;  // wave tile: 64 k x 128 n
+  const bool late = wave >= kTdWaves / 2;  // the second wave of its SIMD
   const int N = p.N, K = p.K;
 
-  // tile of this block: the order of tgmm_dl_kernel (XCD ranges, patches of 8 n-tiles x 4 k-tiles of one group)
+  // Persistent blocks: block b works on tile ids b, b + gridDim.x, ..  Ids congruent mod 8 run on one XCD: each XCD owns a
+  // contiguous range of tiles, walked in patches of 8 n-tiles x 4 k-tiles of one group, so that the 32 blocks of an XCD
+  // share 8 dout and 4 lhs panels in its L2.
   const int tiles_k = K / kTdTile, tiles_n = N / kTdTile, per_group = tiles_k * tiles_n;
   const int total = per_group * p.G_local;
-  const int q8 = total / 8, rem = total % 8, xcd = blockIdx.x % 8, loc = blockIdx.x / 8;
-  const int logical = xcd < rem ? xcd * (q8 + 1) + loc : rem * (q8 + 1) + (xcd - rem) * q8 + loc;
-  const int g_local = logical / per_group, t = logical % per_group, g = g_local + p.group_offset;
-  constexpr int GSM = 8;
-  const int width = GSM * tiles_k, first_n = (t / width) * GSM, gsz = min(tiles_n - first_n, GSM);
-  const int n0 = (first_n + (t % width) % gsz) * kTdTile, k0 = ((t % width) / gsz) * kTdTile;
-
-  long long part = 0;
-  for (int i = tid; i < min(g, p.G_total); i += kTdThreads) part += max(p.group_sizes[i], 0);
+  struct Tile {
+    int g_local, n0, k0, start, size, nk;
+  };
+  // rows of group g: [start, start + size), clipped to M.  A block's tiles come in the order of their groups, so a new start is
+  // the old one plus the sizes of the groups in between.
+  typedef const __attribute__((address_space(4))) int32_t* const_i32_t;
+  const const_i32_t sizes = (const_i32_t)(uintptr_t)p.group_sizes;
+  int g_at = 0;          // group that `row_at` is the first row of (clipped to M)
+  long long row_at = 0;
+  auto locate = [&](int id, Tile& t) __attribute__((always_inline)) {
+    const int q8 = total / 8, rem = total % 8, xcd = id % 8, loc = id / 8;
+    const int logical = xcd < rem ? xcd * (q8 + 1) + loc : rem * (q8 + 1) + (xcd - rem) * q8 + loc;
+    const int r = logical % per_group;
+    constexpr int GSM = 8;
+    const int width = GSM * tiles_k, first_n = (r / width) * GSM, gsz = min(tiles_n - first_n, GSM);
+    t.g_local = logical / per_group;
+    t.n0 = (first_n + (r % width) % gsz) * kTdTile;
+    t.k0 = ((r % width) / gsz) * kTdTile;
+    const int g = t.g_local + p.group_offset;
+    for (; g_at < min(g, p.G_total); g_at++) row_at += max(sizes[g_at], 0);
+    t.start = (int)min(row_at, (long long)p.M);
+    t.size = g < p.G_total ? min(max(sizes[g], 0), p.M - t.start) : 0;
+    // (three stages at least: the stream looks two stages ahead, into the next tile at most; a stage past the rows is zeros)
+    t.nk = max((t.size + C::BM - 1) / C::BM, 3);
+  };
+  if (p.group_offset > 0) {  // the groups before the local ones, summed once by every wave
+    long long part = 0;
+    const int gl = min(p.group_offset, p.G_total);
+    for (int i = lane; i < gl; i += kWave) part += max(p.group_sizes[i], 0);
+    int lim = (int)min(part, (long long)p.M);  // (a sum past M is as good as M)
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
-  if (lane == 0) s_red[wave] = (int)min(part, (long long)p.M);
-  __syncthreads();
-  long long start_ll = 0;
-  for (int w = 0; w < kTdWaves; w++) start_ll += s_red[w];
-  const int start = __builtin_amdgcn_readfirstlane((int)min(start_ll, (long long)p.M));
-  const int size = __builtin_amdgcn_readfirstlane(g < p.G_total ? min(max(p.group_sizes[g], 0), p.M - start) : 0);
-
+    for (int o = 32; o > 0; o >>= 1) lim = min((int)min((long long)lim + __shfl_xor(lim, o), (long long)p.M), p.M);
+    row_at = __builtin_amdgcn_readfirstlane(lim);
+    g_at = gl;
+  }
   const int s16 = lane % 16, gq = lane / 16;
-  if (size == 0) {  // an empty group's gradient is zero
-    for (int i = tid; i < kTdTile * (kTdTile / 4); i += kTdThreads) {
-      const size_t off = ((size_t)g_local * N + n0 + i / (kTdTile / 4)) * K + k0 + (i % (kTdTile / 4)) * 4;
-      tgmm_store4(p, off, n0 + i / (kTdTile / 4), 0.f, 0.f, 0.f, 0.f);
+  // the block's first tile from `id` on whose group has rows; the gradients of empty groups are zeros, written on the way
+  auto next_tile = [&](int& id, Tile& t) __attribute__((always_inline)) -> bool {
+    for (; id < total; id += gridDim.x) {
+      locate(id, t);
+      if (t.size > 0) return true;
+      for (int i = tid; i < kTdTile * (kTdTile / 4); i += kTdThreads) {
+        const int n = t.n0 + i / (kTdTile / 4);
+        tgmm_store4(p, ((size_t)t.g_local * N + n) * K + t.k0 + (i % (kTdTile / 4)) * 4, n, 0.f, 0.f, 0.f, 0.f);
+      }
     }
-    return;
-  }
+    return false;
+  };
 
-  // ---- requests: request i of an operand covers stage rows 4 * (4 * wave + i) + {0 .. 3}, lane l the 16 bytes of LDS
-  // slot l % 16 of row l / 16.  Requests i and i + 2 of a wave are 8 rows apart inside one block of 32 rows, which leaves
-  // the swizzle as it is: two per-lane offsets per operand.  Rows past the group's end come from a row of zeros.
-  uint32_t a_off[2], b_off[2];
+  // ---- requests.  Request i of an operand and wave: half i / 2 of the stage (bf16: 32 rows each), RPR rows of it.
+  auto req_row = [&](int i) { return (i / 2) * (C::BM / 2) + (wave * 2 + i % 2) * C::RPR; };
+  uint32_t a_off[C::IPW], b_off[C::IPW];
+  const uint32_t a_pitch = (uint32_t)K * C::ESZ, b_pitch = (uint32_t)N * C::ESZ;
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int r = 4 * (wave * kT8Ipw + i) + lane / 16;
-    const int chunk = (lane % 16) ^ t8_swz(r);
-    a_off[i] = (uint32_t)r * K + chunk * 16;
-    b_off[i] = (uint32_t)r * N + chunk * 16;
+  for (int i = 0; i < C::IPW; i++) {
+    constexpr int LPR = kWave / C::RPR;  // lanes per row
+    const int r = req_row(i) + lane / LPR;
+    const uint32_t chunk = (uint32_t)((lane % LPR) ^ C::swz(r)) * 16;
+    a_off[i] = (uint32_t)r * a_pitch + chunk;
+    b_off[i] = (uint32_t)r * b_pitch + chunk;
   }
-  static_assert(kT8Ipw == 4, "request i + 2 is request i eight rows further down");
-  const uint8_t* const a_base = (const uint8_t*)p.lhs + ((size_t)start * K + k0);
-  const uint8_t* const b_base = (const uint8_t*)p.dout + ((size_t)start * N + n0);
-  const size_t a_step = (size_t)kT8BM * K, b_step = (size_t)kT8BM * N;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)t8_smem;
-  auto issue_one = [&](auto full_c, int kt, int buf, int idx) {
-    constexpr bool FULL = decltype(full_c)::value;
-    const int i = idx % kT8Ipw;
-    const bool is_a = idx < kT8Ipw;
-    const uint8_t* src = is_a ? a_base + (kt * a_step + (size_t)(i / 2) * 8 * K) + a_off[i % 2]
-                              : b_base + (kt * b_step + (size_t)(i / 2) * 8 * N) + b_off[i % 2];
-    if constexpr (!FULL) {
-      int l = lane;
-      asm volatile("" : "+v"(l));
-      const int r = 4 * (wave * kT8Ipw + i) + l / 16;
-      const uint64_t keep = kt * kT8BM + r < size ? ~0ull : 0ull;
-      const uint64_t zero = (uint64_t)(tg_zero_row + (l % 16) * 16);
-      src = (const uint8_t*)(((uint64_t)src & keep) | (zero & ~keep));
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)td_smem;
+  // The loading side: the next stage's first byte of the two panels, and the descriptors of the stage being requested.  A
+  // descriptor starts at the stage's first row and ends with the group's last one, so rows past it arrive as zeros; a stage
+  // past the end has no bytes at all and fetches nothing.  (Kept as running scalars: formed from the stage number for every
+  // request they were 18 scalar instructions in the fetching side, as long as its fragment reads.)
+  uint64_t a_next = 0, b_next = 0;
+  int a_kt = 0, b_kt = 0, src_full = 0;   // stage numbers; full stages
+  uint32_t a_part = 0, b_part = 0;        // bytes of the stage behind them
+  v4i a_desc, b_desc;
+  auto set_sources = [&](const Tile& t) __attribute__((always_inline)) {
+    a_next = (uint64_t)p.lhs + (uint64_t)t.start * a_pitch + (uint64_t)t.k0 * C::ESZ;
+    b_next = (uint64_t)p.dout + (uint64_t)t.start * b_pitch + (uint64_t)t.n0 * C::ESZ;
+    a_kt = b_kt = 0;
+    src_full = t.size / C::BM;
+    const int part = t.size % C::BM;
+    a_part = part > 0 ? (uint32_t)(part - 1) * a_pitch + C::ROW : 0u;
+    b_part = part > 0 ? (uint32_t)(part - 1) * b_pitch + C::ROW : 0u;
+  };
+  const uint32_t a_full = (uint32_t)(C::BM - 1) * a_pitch + C::ROW, b_full = (uint32_t)(C::BM - 1) * b_pitch + C::ROW;
+  auto advance = [&](bool is_a) __attribute__((always_inline)) {
+    if (is_a) {
+      a_desc = buffer_desc((const void*)a_next, a_kt < src_full ? a_full : a_kt == src_full ? a_part : 0u);
+      a_next += (uint64_t)C::BM * a_pitch;
+      a_kt++;
+    } else {
+      b_desc = buffer_desc((const void*)b_next, b_kt < src_full ? b_full : b_kt == src_full ? b_part : 0u);
+      b_next += (uint64_t)C::BM * b_pitch;
+      b_kt++;
     }
-    dma16_untracked(src, lds_base + buf * kT8Stage + (is_a ? 0 : kT8Operand) + (wave * kT8Ipw + i) * 1024);
+  };
+  // half h of an operand of the stage its descriptor stands at
+  auto issue = [&](bool is_a, int buf, int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 2 * h; i < 2 * h + 2; i++)
+      dma16_buffer(is_a ? a_desc : b_desc, is_a ? a_off[i] : b_off[i], lds_base + buf * C::STAGE + (is_a ? 0 : C::OPERAND) + req_row(i) * C::ROW);
   };
 
-  // ---- fragments: lane (group gq, s16) addresses row 32 * gq + s16 / 2 (+ 8, 16, 24) of the stage and the 8 bytes
-  // s16 % 2 of the fragment's 16-byte column block c, stored at slot c ^ (s16 / 2) ^ 8 * (gq % 2); fragment f of an operand
-  // is block c0 + f with c0 a multiple of 4 (lhs) or 8 (dout), so the step is an XOR of address bits 4 .. 6.
-  const int xmask = (s16 / 2) ^ ((gq & 1) << 3);
-  const int row_part = (32 * gq + s16 / 2) * kT8Row + (s16 % 2) * 8;
-  const int k_base = row_part + (((4 * wk) ^ xmask) << 4);
-  const int n_base = row_part + (((8 * wn) ^ xmask) << 4);
-  constexpr int RING = 4;
-  v8i fk[4], fn[RING];
-  auto read_k = [&](int buf, int f) {
-    int base = k_base;
-    asm volatile("" : "+v"(base));
-    tr8_read_frag(fk[f], t8_smem + buf * kT8Stage + (base ^ (16 * f)));
+  // ---- fragments.  bf16: lane (group gq, s16) addresses row 8 * gq + s16 / 4 (+ 4) of the k-step's 32 rows and the 8 bytes
+  // 8 * (s16 % 4) of the fragment's 32-byte row slice; fragment f of an operand is 32 * f bytes further along the row before
+  // the swizzle, which turns the step into an XOR of address bits 5 .. 7.  1-byte: row 32 * gq + s16 / 2 (+ 8, 16, 24) and the
+  // 8 bytes s16 % 2 of the fragment's 16-byte column block; the step is an XOR of address bits 4 .. 6.
+  int k_base, n_base;
+  if constexpr (C::F8) {
+    const int xmask = (s16 / 2) ^ ((gq & 1) << 3), row_part = (32 * gq + s16 / 2) * C::ROW + (s16 % 2) * 8;
+    k_base = row_part + (((4 * wk) ^ xmask) << 4);
+    n_base = row_part + (((8 * wn) ^ xmask) << 4);
+  } else {
+    const int xmask = ((s16 / 4) << 2) ^ ((gq & 1) << 1), piece = s16 % 4, row_part = (gq * 8 + s16 / 4) * C::ROW;
+    k_base = row_part + ((((8 * wk + piece / 2) ^ xmask) << 4) | ((piece & 1) << 3));
+    n_base = row_part + ((((16 * wn + piece / 2) ^ xmask) << 4) | ((piece & 1) << 3));
+  }
+  typedef typename std::conditional<C::F8, v8i, v8bf>::type frag_t;
+  constexpr int NSLOTS = C::F8 ? 6 : 4;
+  frag_t fk[4], fn[NSLOTS];
+  auto read_k = [&](int buf, int ks, int f) {
+    const uint8_t* src = td_smem + buf * C::STAGE + (k_base ^ ((C::F8 ? 16 : 32) * f));
+    if constexpr (C::F8) tr8_read_frag(fk[f], src, C::ROW);
+    else fk[f] = tr_read_frag(src + ks * 32 * C::ROW, C::ROW);
   };
-  auto read_n = [&](int buf, int f, int slot) {
-    int base = n_base;
-    asm volatile("" : "+v"(base));
-    tr8_read_frag(fn[slot], t8_smem + buf * kT8Stage + kT8Operand + (base ^ (16 * f)));
+  auto read_n = [&](int buf, int ks, int f, int slot) {
+    const uint8_t* src = td_smem + buf * C::STAGE + C::OPERAND + (n_base ^ ((C::F8 ? 16 : 32) * f));
+    if constexpr (C::F8) tr8_read_frag(fn[slot], src, C::ROW);
+    else fn[slot] = tr_read_frag(src + ks * 32 * C::ROW, C::ROW);
   };
-
   v4f acc[4][8];  // [k fragment][n fragment]
+  // n fragments f0 .. of one phase (4 of bf16, 2 of the 1-byte operands) from the slots slot0 ..
+  auto multiply = [&](auto zc_c, int f0, int slot0) __attribute__((always_inline)) {
+    constexpr bool ZC = decltype(zc_c)::value;  // a tile's first products start from zero
 #pragma unroll
-  for (int j = 0; j < 4; j++)
+    for (int i = 0; i < (C::F8 ? 2 : 4); i++)
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+      for (int j = 0; j < 4; j++) {
+        v4f& c = acc[j][f0 + i];
+        if constexpr (C::F8) c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fk[j], fn[slot0 + i], ZC ? v4f{} : c, 0, C::DF, 0, 127, 0, 127);
+        else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fk[j], fn[slot0 + i], ZC ? v4f{} : c, 0, 0, 0);
+      }
+    // (pinned to the phase: at the end the sums' only readers sit behind branches)
 #pragma unroll
-      for (int r = 0; r < 4; r++) acc[j][i][r] = 0.f;
-
-  // first half of a stage (buffer buf): dout fragments 0 .. 3 from the ring, each slot reloaded with fragment + 4
-  auto half_lo = [&](int buf) {
+    for (int i = 0; i < (C::F8 ? 2 : 4); i++)
 #pragma unroll
-    for (int t = 0; t < 16; t++) {
-      const int i = t / 4, j = t % 4;
-      acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fk[j], fn[i], acc[j][i], 0, DF, 0, 127, 0, 127);
-      if (j == 3) read_n(buf, i + RING, i);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[j][f0 + i]));
   };
-  // second half: dout fragments 4 .. 7, lhs fragment by lhs fragment.  RD: the next stage (rd_buf) is prepared behind it.
-  // LD: the requests of stage ld_kt go out into ld_buf.
-  auto half_hi = [&](auto rd_c, auto ld_c, auto full_c, int rd_buf, int ld_kt, int ld_buf) {
-    constexpr bool RD = decltype(rd_c)::value, LD = decltype(ld_c)::value;
-#pragma unroll
-    for (int t = 0; t < 16; t++) {
-      const int j = t / 4, ii = t % 4;
-      acc[j][RING + ii] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fk[j], fn[ii], acc[j][RING + ii], 0, DF, 0, 127, 0, 127);
-      if (LD && t % kT8ReqStride == 0 && t / kT8ReqStride < kT8Lps) issue_one(full_c, ld_kt, ld_buf, t / kT8ReqStride);
-      if (RD && ii == 3) read_k(rd_buf, j);
-      if (RD && j == 3) read_n(rd_buf, ii, ii);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  auto fetch_end = [&](auto wait_c) {
+    constexpr int WAIT = decltype(wait_c)::value;
+    if constexpr (WAIT >= 0) wait_vmcnt<WAIT>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+  };
+  auto multiply_end = [&]() {
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
-
-  // Stage kt sits in buffer kt % 2.  After a stage's first half every fragment of it is in registers: the block meets
-  // (own reads returned, own requests of stage kt + 1 landed), and during the second half the fragments of stage kt + 1
-  // are read from the other buffer while stage kt + 2 is requested into this one.
-  const int nk = (size + kT8BM - 1) / kT8BM;
-#pragma unroll
-  for (int s = 0; s < 2; s++)
-#pragma unroll
-    for (int i = 0; i < kT8Lps; i++) issue_one(F_{}, min(s, nk - 1), s, i);
-  wait_vmcnt<0>();
-  __syncthreads();
-#pragma unroll
-  for (int f = 0; f < RING; f++) read_n(0, f, f);
-#pragma unroll
-  for (int f = 0; f < 4; f++) read_k(0, f);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  half_lo(0);
-  int kt = 0;
-  const int nfull = size / kT8BM;  // stages 0 .. nfull-1 hold 128 rows of the group
-  for (; kt + 2 < nfull; kt++) {   // steady state: the stage requested is a full one
-    const int buf = kt % 2;
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    wait_vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-    half_hi(T_{}, T_{}, T_{}, buf ^ 1, kt + 2, buf);
-    half_lo(buf ^ 1);
-  }
-  for (; kt + 1 < nk; kt++) {
-    const int buf = kt % 2;
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    wait_vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-    half_hi(T_{}, T_{}, F_{}, buf ^ 1, min(kt + 2, nk - 1), buf);
-    half_lo(buf ^ 1);
-  }
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  half_hi(F_{}, F_{}, F_{}, 0, 0, 0);
-  wait_vmcnt<0>();  // no request may still be writing LDS when the block ends
-  // (the sums are pinned to this point: their only readers sit behind the branches below)
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-#pragma unroll
-    for (int i = 0; i < 8; i++) asm volatile("" : "+v"(acc[j][i]));
+  using NOWAIT = std::integral_constant<int, -1>;
+  using WAIT = std::integral_constant<int, C::F8 ? 6 : 10>;
 
   // D[k][n]: the lane holds n = s16 and k = 4 * gq + r of each 16 x 16 tile
-  if (!p.out_f32 && !p.existing) {
+  auto store_tile = [&](const Tile& t) __attribute__((always_inline)) {
+    float sc[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) sc[i] = p.n_scale ? p.n_scale[t.n0 + wn * 128 + i * 16 + s16] : 1.0f;
+    // everything requested so far lands here, ahead of the stores: the next tile's first stage need not count them
+    wait_vmcnt<0>();
+    if (!p.out_f32 && !p.existing) {
+      // plain bf16 results: neighbouring k-tiles trade halves between lanes 16 apart, so that a lane stores 16 bytes and
+      // the 64 bytes of a row n leave in one instruction
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int n = t.n0 + wn * 128 + i * 16 + s16;
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+          const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(acc[j][i][0] * sc[i], acc[j][i][1] * sc[i]),
+                                                           pack_bf16x2(acc[j + 1][i][0] * sc[i], acc[j + 1][i][1] * sc[i]), false, false);
+          const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(acc[j][i][2] * sc[i], acc[j][i][3] * sc[i]),
+                                                           pack_bf16x2(acc[j + 1][i][2] * sc[i], acc[j + 1][i][3] * sc[i]), false, false);
+          const int k = t.k0 + wk * 64 + (j + (gq & 1)) * 16 + 4 * (gq & ~1);
+          *(uint4*)((uint16_t*)p.out + ((size_t)t.g_local * N + n) * K + k) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const int n = n0 + wn * 128 + i * 16 + s16;
-      const float sc = p.n_scale ? p.n_scale[n] : 1.0f;
+      const int n = t.n0 + wn * 128 + i * 16 + s16;
 #pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(acc[j][i][0] * sc, acc[j][i][1] * sc),
-                                                         pack_bf16x2(acc[j + 1][i][0] * sc, acc[j + 1][i][1] * sc), false, false);
-        const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(acc[j][i][2] * sc, acc[j][i][3] * sc),
-                                                         pack_bf16x2(acc[j + 1][i][2] * sc, acc[j + 1][i][3] * sc), false, false);
-        const int k = k0 + wk * 64 + (j + (gq & 1)) * 16 + 4 * (gq & ~1);
-        *(uint4*)((uint16_t*)p.out + ((size_t)g_local * N + n) * K + k) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+      for (int j = 0; j < 4; j++) {
+        const size_t off = ((size_t)t.g_local * N + n) * K + t.k0 + wk * 64 + j * 16 + 4 * gq;
+        tgmm_store4(p, off, n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
       }
     }
-    return;
-  }
+  };
+
+  Tile cur, nxt;
+  int id = blockIdx.x;
+  if (!next_tile(id, cur)) return;
+  // ---- head: stage 0, and stage 1 up to the half that the first phase requests ----
+  set_sources(cur);
+  advance(true); advance(false);
+  issue(true, 0, 0); issue(false, 0, 0); issue(true, 0, 1); issue(false, 0, 1);
+  advance(true); advance(false);
+  issue(true, 1, 0); issue(false, 1, 0);
+  issue(true, 1, 1);
+  wait_vmcnt<0>();
+  asm volatile("s_barrier" ::: "memory");
+
+  int cb = 0;  // buffer of the current stage
+  while (true) {
+    bool have_n = false;
+    const int nk = cur.nk;
+    // the first phase of stage kt: it requests the last half of the next stage; the rest requests stage kt + 2.
+    // FIRST: what these phases start with landed before the tile began (no waits)
+    auto stage_head = [&](auto first_c) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const int n = n0 + wn * 128 + i * 16 + s16;
+      for (int f = 0; f < 4; f++) read_k(cb, 0, f);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int k = k0 + wk * 64 + j * 16 + 4 * gq;
-      const size_t off = ((size_t)g_local * N + n) * K + k;
-      tgmm_store4(p, off, n, acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
+      for (int f = 0; f < (C::F8 ? 2 : 4); f++) read_n(cb, 0, f, f);
+      issue(false, cb ^ 1, 1);
+      fetch_end(NOWAIT{});
+      multiply(first_c, 0, 0);
+      multiply_end();
+    };
+    auto stage_rest = [&](auto first_c) __attribute__((always_inline)) {
+      using W = typename std::conditional<decltype(first_c)::value, NOWAIT, WAIT>::type;
+      if constexpr (C::F8) {
+        // lhs slots are free behind phase 1 (requested in 2 and 3), dout slots behind phase 3 (4 and the next stage's 1)
+#pragma unroll
+        for (int f = 2; f < 6; f++) read_n(cb, 0, f, f);
+        advance(true);
+        issue(true, cb, 0);
+        fetch_end(NOWAIT{});
+        multiply(first_c, 2, 2);
+        multiply_end();
+        read_n(cb, 0, 6, 0);
+        read_n(cb, 0, 7, 1);
+        issue(true, cb, 1);
+        fetch_end(NOWAIT{});
+        multiply(first_c, 4, 4);
+        multiply_end();
+        advance(false);
+        issue(false, cb, 0);
+        fetch_end(WAIT{});  // (the next stage's last half is this stage's first request: waited for in every stage)
+        multiply(first_c, 6, 0);
+        multiply_end();
+      } else {
+#pragma unroll
+        for (int f = 0; f < 4; f++) read_n(cb, 0, 4 + f, f);
+        advance(true);
+        issue(true, cb, 0);
+        fetch_end(W{});
+        multiply(first_c, 4, 0);
+        multiply_end();
+#pragma unroll
+        for (int f = 0; f < 4; f++) read_k(cb, 1, f);
+#pragma unroll
+        for (int f = 0; f < 4; f++) read_n(cb, 1, f, f);
+        advance(false);
+        issue(false, cb, 0);
+        fetch_end(NOWAIT{});
+        multiply(F_{}, 0, 0);
+        multiply_end();
+#pragma unroll
+        for (int f = 0; f < 4; f++) read_n(cb, 1, 4 + f, f);
+        issue(true, cb, 1);
+        fetch_end(W{});
+        multiply(F_{}, 4, 0);
+        multiply_end();
+      }
+      cb ^= 1;
+    };
+    if (late) asm volatile("s_barrier" ::: "memory");
+    stage_head(T_{});
+    stage_rest(T_{});
+    for (int kt = 1; kt < nk - 2; kt++) {
+      stage_head(F_{});
+      stage_rest(F_{});
     }
+    stage_head(F_{});
+    // the stream crosses into the next tile
+    id += gridDim.x;
+    have_n = next_tile(id, nxt);
+    if (have_n) set_sources(nxt);
+    stage_rest(F_{});
+    stage_head(F_{});
+    stage_rest(F_{});
+    if (!late) asm volatile("s_barrier" ::: "memory");
+    store_tile(cur);
+    if (!have_n) break;
+    cur = nxt;
   }
+  wait_vmcnt<0>();  // no request may still be writing LDS when the block ends
 }
 
 }  // namespace moe
@@ -631,11 +540,24 @@ __global__ __launch_bounds__(kTdThreads, 2) void tgmm_f8_kernel(const TgmmParams
 using namespace moe;
 
 namespace moe {
-int prepare_tgmm() { return reserve_lds(tgmm_dl_kernel, kTdLds, lds_flags<TgmmParams>()); }
-struct TgmmF8Tag0 {};
-struct TgmmF8Tag1 {};
-static int prepare_tgmm_f8(int df) {
-  return df ? reserve_lds(tgmm_f8_kernel<1>, kT8Lds, lds_flags<TgmmF8Tag1>()) : reserve_lds(tgmm_f8_kernel<0>, kT8Lds, lds_flags<TgmmF8Tag0>());
+template <typename C>
+static int launch_tgmm_dl(const TgmmParams& p, hipStream_t s) {
+  if (int st = reserve_lds(tgmm_dl_kernel<C>, C::LDS, lds_flags<C>())) return st;
+  // one persistent block per CU (the LDS footprint allows no more); a multiple of 8 keeps "tile id mod 8" equal to the XCD
+  // a block runs on
+  int blocks = 0;
+  if (int st = device_cu_count(&blocks)) return st;
+  const long long tiles = (long long)(p.K / kTdTile) * (p.N / kTdTile) * p.G_local;
+  if (tiles < blocks) blocks = (int)tiles;
+  if (blocks >= 8) blocks -= blocks % 8;
+  tgmm_dl_kernel<C><<<(unsigned)blocks, kTdThreads, C::LDS, s>>>(p);
+  return check_launch("tgmm_dl_kernel");
+}
+int prepare_tgmm() {
+  int st = reserve_lds(tgmm_dl_kernel<TgCfg<false>>, TgCfg<false>::LDS, lds_flags<TgCfg<false>>());
+  if (!st) st = reserve_lds(tgmm_dl_kernel<TgCfg<true, 0>>, TgCfg<true, 0>::LDS, lds_flags<TgCfg<true, 0>>());
+  if (!st) st = reserve_lds(tgmm_dl_kernel<TgCfg<true, 1>>, TgCfg<true, 1>::LDS, lds_flags<TgCfg<true, 1>>());
+  return st;
 }
 }  // namespace moe
 
@@ -668,12 +590,7 @@ extern "C" int moe_tgmm_fp8(const void* lhs, const void* dout, int dout_dtype, c
   p.out_f32 = out_dtype == MOE_F32;
   p.existing = existing_out; p.existing_f32 = existing_dtype == MOE_F32;
   p.n_scale = out_row_scale;
-  const int df = dout_dtype == MOE_FP8_E5M2;
-  if (int st = prepare_tgmm_f8(df)) return st;
-  const unsigned tiles = (unsigned)((K / kTdTile) * (N / kTdTile) * num_groups_local);
-  if (df) tgmm_f8_kernel<1><<<tiles, kTdThreads, kT8Lds, (hipStream_t)stream>>>(p);
-  else tgmm_f8_kernel<0><<<tiles, kTdThreads, kT8Lds, (hipStream_t)stream>>>(p);
-  return check_launch("tgmm_f8_kernel");
+  return dout_dtype == MOE_FP8_E5M2 ? launch_tgmm_dl<TgCfg<true, 1>>(p, (hipStream_t)stream) : launch_tgmm_dl<TgCfg<true, 0>>(p, (hipStream_t)stream);
 }
 
 extern "C" int moe_tgmm_scaled(const void* lhs, const void* dout, const int32_t* group_sizes, int M, int K, int N,
@@ -699,11 +616,8 @@ extern "C" int moe_tgmm_scaled(const void* lhs, const void* dout, const int32_t*
   p.n_scale = out_row_scale;
   // groups of 128 rows and more on average take the 256 x 256 tiles when the shape allows it
   const long long tiles = (long long)(K / kTdTile) * (N / kTdTile) * num_groups_local;
-  if (K % kTdTile == 0 && N % kTdTile == 0 && K < (1 << 24) && N < (1 << 24) && (long long)M >= 128LL * num_groups_total && tiles >= 128 && tiles <= 0x7fffffffLL) {
-    if (int st = prepare_tgmm()) return st;
-    tgmm_dl_kernel<<<(unsigned)tiles, kTdThreads, kTdLds, (hipStream_t)stream>>>(p);
-    return check_launch("tgmm_dl_kernel");
-  }
+  if (K % kTdTile == 0 && N % kTdTile == 0 && K < (1 << 24) && N < (1 << 24) && (long long)M >= 128LL * num_groups_total && tiles >= 128 && tiles <= 0x7fffffffLL)
+    return launch_tgmm_dl<TgCfg<false>>(p, (hipStream_t)stream);
   dim3 grid(cdiv(K, kTgBK), cdiv(N, kTgBN), num_groups_local);
   tgmm_kernel<<<grid, kTgThreads, 0, (hipStream_t)stream>>>(p);
   return check_launch("tgmm_kernel");

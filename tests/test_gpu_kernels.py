@@ -912,6 +912,27 @@ def test_tgmm_big_tiles_exact_on_small_integers_and_group_window(K):
   assert torch.equal(got16.cpu(), want.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("offset,g_local", [(0, 12), (3, 6)])
+def test_tgmm_stream_across_tiles_at_stage_edges(K, fp8, offset, g_local):
+  """Persistent 256 x 256 blocks with several tiles each, groups of none, one, less than a stage, exactly whole stages and one
+  row more (stages of 64 rows, 128 of 1-byte operands): the request stream crosses from each kind into each other."""
+  rng = np.random.default_rng(9)
+  gs = np.array([1, 0, 64, 700, 63, 128, 129, 0, 192, 65, 300, 127], np.int32)
+  m, k, n = int(gs.sum()) + 31, 2048, 1536
+  lhs = torch.from_numpy(rng.integers(-3, 4, (m, k)).astype(np.float32)).to(torch.bfloat16)
+  dout = torch.from_numpy(rng.integers(-3, 4, (m, n)).astype(np.float32)).to(torch.bfloat16)
+  want = O.tgmm(lhs, dout, gs, out_dtype=torch.float32).transpose(1, 2)[offset:offset + g_local]
+  kw = dict(num_groups_local=g_local, group_offset=offset, out_dtype=torch.float32)
+  if fp8:
+    assert K.tgmm_fp8_supported(m, k, n, 12, g_local)
+    got = K.tgmm_fp8(cuda(lhs).to(torch.float8_e4m3fn), cuda(dout).to(torch.float8_e5m2), cuda(gs), **kw)
+  else:
+    got = K.tgmm(cuda(lhs), cuda(dout), cuda(gs), **kw)
+  assert torch.equal(got.cpu(), want)  # sums of at most 700 products of magnitude <= 9 are exact in f32
+
+
+
 @pytest.mark.parametrize("m,k,n,gs", [(333, 136, 264, [40, 0, 100, 93, 100]), (700, 1024, 3072, [140, 0, 199, 193, 100])])
 @pytest.mark.parametrize("existing_dtype,out_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
 def test_tgmm_existing_out_is_added_before_rounding(K, m, k, n, gs, existing_dtype, out_dtype):
