@@ -646,6 +646,7 @@ int launch_dl(int op, bool glu, int stage_bytes, bool rhs_kn, const TiledParams&
 // (fp8 x fp8 with epilogue scales too; lhs_e5m2: the activations are float8_e5m2, the weights e4m3)
 int launch_dls(int op, bool glu, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2 = 0, int rhs_kn = 0);
 bool dls_takes(int op, int K, int N, long long indexed_lhs_rows);
+bool dls_kn_takes(int op, int K, int N, long long indexed_lhs_rows);  // the same for [G, K, N] weights (bf16, fp8)
 // moe_gmm_f8s.hip: the same stream for block-scaled fp8 (1 x 128 activation scales, 128 x 128 weight scales)
 struct Fp8TiledParams;
 int launch_f8s(bool glu, const Fp8TiledParams& P, int M, int G_total, hipStream_t s);

@@ -43,9 +43,9 @@ struct DlsCfg {
   static constexpr int OP = OP_;
   static constexpr bool GLU = GLU_;
   static constexpr int LF = LF_;  // fp8 activations: 0 = e4m3, 1 = e5m2 (format selector of the MFMA's second operand)
-  // fp8 weights given as [G, K, N] (the contraction index as the row: dlhs of a layer whose weights are [G, N, K], read as
-  // they are).  The weight half of a stage then holds 128 contraction rows x 256 output channels (128 x 256 B, four rows per
-  // wave instruction) and the weight fragments come out of it through ds_read_b64_tr_b8.
+  // weights given as [G, K, N] (the contraction index as the row: dlhs of a layer whose weights are [G, N, K], read as they
+  // are).  The weight half of a stage then holds 128 (bf16: 64) contraction rows x 256 output channels (four rows of 256 or two
+  // of 512 bytes per wave instruction) and the weight fragments come out of it through ds_read_b64_tr_b8 / _b16.
   static constexpr bool KN = KN_;
   static constexpr int BM = 256, BN = 256, BKB = 128, MI = 16;
   static constexpr int ESZ = OP == OP_BF16 ? 2 : 1, BK = BKB / ESZ;
@@ -56,10 +56,12 @@ struct DlsCfg {
   static constexpr int OUT_BN = GLU ? BN / 2 : BN;
   static_assert(OP == OP_I8 || OP == OP_BF16 || OP == OP_F8, "operands");
   static_assert(LF == 0 || OP == OP_F8, "only fp8 activations come in two formats");
-  static_assert(!KN || (OP == OP_F8 && !GLU), "[G, K, N] weights: fp8 without rhs_up");
+  static_assert(!KN || (OP != OP_I8 && !GLU), "[G, K, N] weights: fp8 or bf16 without rhs_up");
   // slot of the 16-byte chunk c of contraction row r in a [G, K, N] weight stage: c ^ kn_swz(r); the 8 rows of a transposing
-  // read and those of the next lane group (16 rows further) then fall into 16 different 16-byte bank groups
-  __device__ static __forceinline__ int kn_swz(int row) { return (row & 7) ^ (((row >> 4) & 1) << 3); }
+  // 1-byte read and those of the next lane group (16 rows further) then fall into 16 different 16-byte bank groups (bf16: see
+  // tr_swz)
+  __device__ static __forceinline__ int kn_swz(int row) { return OP == OP_BF16 ? tr_swz(row) : (row & 7) ^ (((row >> 4) & 1) << 3); }
+  static constexpr int KN_ROW = BN * ESZ, KN_RPR = 1024 / KN_ROW;  // bytes of a contraction row, rows per request
   __device__ static __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 };
 
@@ -116,9 +118,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
 #pragma unroll
   for (int i = 0; i < C::B_IPW; i++) {
     if constexpr (C::KN) {
-      // request i covers contraction rows (wave * 4 + i) * 4 + lane / 16 of the stage, the lane LDS slot lane % 16 of its row
-      const int r = (wave * C::B_IPW + i) * 4 + lane / 16;
-      b_voff[i] = (uint32_t)r * (uint32_t)N + (uint32_t)(((lane % 16) ^ C::kn_swz(r)) << 4);
+      // request i covers KN_RPR contraction rows of the stage, the lane one 16-byte LDS slot of its row
+      constexpr int LPR = kWave / C::KN_RPR;
+      const int r = (wave * C::B_IPW + i) * C::KN_RPR + lane / LPR;
+      b_voff[i] = (uint32_t)r * (uint32_t)(N * C::ESZ) + (uint32_t)(((lane % LPR) ^ C::kn_swz(r)) << 4);
     } else {
       b_voff[i] = lane_off(b_req_row(i), (uint32_t)((C::GLU ? b_req_row(i) % 128 : b_req_row(i)) + lane / 8));
     }
@@ -126,7 +129,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   auto set_b_sources = [&](const Tile& t) {
     b_desc[0] = buffer_desc(p.rhs + (size_t)t.info.group * N * row_bytes, clamp_u32((size_t)N * row_bytes));
     if constexpr (C::GLU) b_desc[1] = buffer_desc(p.rhs_up + (size_t)t.info.group * N * row_bytes, clamp_u32((size_t)N * row_bytes));
-    b_soff = C::KN ? (uint32_t)t.n0 : (uint32_t)t.n0 * row_bytes;  // (KN: a byte offset inside every contraction row)
+    b_soff = C::KN ? (uint32_t)t.n0 * C::ESZ : (uint32_t)t.n0 * row_bytes;  // (KN: a byte offset inside every contraction row)
   };
   auto issue_a = [&](int kt, int buf, int h) {
 #pragma unroll
@@ -151,9 +154,14 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   auto b_tile = [&](int j) { return (C::GLU ? (j / HN) * (C::BN / 2) + (j % HN) * C::MI : j * C::MI) * C::BKB; };
   // fragment of a 64-byte k-step ks: row (lane % 16), chunk q = 4 * ks + lane / 16, stored at slot q ^ swz(row)
   const int frag_lane = (lane % 16) * C::BKB + (((lane / 16) ^ C::swz(lane % 16)) << 4);
-  // [G, K, N] weights: lane (s, q) addresses row 16 q + s / 2 (+ 8, 64, 72) of the stage's 128 contraction rows, i.e. the K
-  // bytes 16 q .. and 64 + 16 q .. its activation fragment holds, and the 8 bytes s % 2 of the fragment's 16-byte channel block
-  const int kn_base = C::A_STAGE + (16 * (lane / 16) + (lane % 16) / 2) * C::BN + ((((wn * C::TN) ^ ((lane % 16) / 2) ^ (((lane / 16) & 1) << 3))) << 4) + (lane % 2) * 8;
+  // [G, K, N] weights.  fp8: lane (s, q) addresses row 16 q + s / 2 (+ 8, 64, 72) of the stage's 128 contraction rows, i.e. the
+  // K bytes 16 q .. and 64 + 16 q .. its activation fragment holds, and the 8 bytes s % 2 of the fragment's 16-byte channel
+  // block.  bf16: row 8 q + s / 4 (+ 4) of the k-step's 32 rows and the 8 bytes s % 4 of the fragment's 32-byte slice.  Channel
+  // tile j is 16 * ESZ * j bytes further along the row before the swizzle: an XOR.
+  const int kn_s = lane % 16, kn_q = lane / 16;
+  const int kn_base = C::A_STAGE + (OP == OP_BF16
+      ? (8 * kn_q + kn_s / 4) * C::KN_ROW + ((((8 * wn + (kn_s % 4) / 2) ^ C::kn_swz(8 * kn_q + kn_s / 4)) << 4) | ((kn_s & 1) << 3))
+      : (16 * kn_q + kn_s / 2) * C::KN_ROW + (((wn * C::TN) ^ C::kn_swz(16 * kn_q + kn_s / 2)) << 4) + (kn_s % 2) * 8);
 
   typedef typename std::conditional<OP == OP_I8, v4i, v4f>::type acc_t;
   acc_t acc[C::TN][C::TM];
@@ -173,13 +181,17 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
 #pragma unroll
     for (int jj = 0; jj < HN; jj++) {
       const int j = g * HN + jj;
-      if constexpr (C::KN) {
+      if constexpr (C::KN && OP == OP_BF16) {
+        const uint8_t* src = smem + buf * C::STAGE + (kn_base ^ (j << 5));
+        const v4i lo = __builtin_bit_cast(v4i, tr_read_frag(src, C::KN_ROW)), hi = __builtin_bit_cast(v4i, tr_read_frag(src + 32 * C::KN_ROW, C::KN_ROW));
+        fb[g][jj] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      } else if constexpr (C::KN) {
         typedef int v2i_kn __attribute__((ext_vector_type(2)));
         typedef __attribute__((address_space(3))) v2i_kn* lds_v2i_kn;
         const uint8_t* src = smem + buf * C::STAGE + (kn_base ^ (j << 4));
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-          const v2i_kn x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_kn)(src + ((t & 1) * 8 + (t >> 1) * 64) * C::BN));
+          const v2i_kn x = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_kn)(src + ((t & 1) * 8 + (t >> 1) * 64) * C::KN_ROW));
           fb[g][jj][2 * t] = x[0];
           fb[g][jj][2 * t + 1] = x[1];
         }
@@ -344,6 +356,7 @@ int prepare_dls() {
   if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false>>();
   if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, true>>();
   if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false, 1>>();
+  if (!st) st = prepare_dls_cfg<DlsCfg<OP_BF16, false, 0, true>>();
   if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false, 0, true>>();
   if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false, 1, true>>();
   return st;
@@ -379,16 +392,23 @@ bool dls_takes(int op, int K, int N, long long indexed_lhs_rows) {
          (indexed_lhs_rows + 256) * pitch < (1LL << 32);
 }
 
+bool dls_kn_takes(int op, int K, int N, long long indexed_lhs_rows) {
+  // [G, K, N] weights: whole 256-channel tiles, a contraction row's offset inside the expert's matrix in 32 bits
+  return op != OP_I8 && dls_takes(op, K, N, indexed_lhs_rows) && N % 256 == 0 && ((long long)K + 128) * N * (op == OP_BF16 ? 2 : 1) < (1LL << 32);
+}
+
 int launch_dls(int op, bool glu, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2, int rhs_kn) {
   if (!dls_takes(op, p.K, p.N, p.ro.row_idx ? p.ro.lhs_rows : 0))
     return fail(MOE_ERR_UNSUPPORTED, "gmm: the stream kernel needs int8, bf16 or fp8 operands, whole 128-byte stages (three or more) and 32-bit byte offsets");
   if (lhs_e5m2 && (op != OP_F8 || glu)) return fail(MOE_ERR_UNSUPPORTED, "gmm: e5m2 activations run against e4m3 weights without rhs_up");
-  if (rhs_kn && (op != OP_F8 || glu || p.N % 256 != 0)) return fail(MOE_ERR_UNSUPPORTED, "gmm: [G, K, N] weights on the stream kernel need fp8 operands, no rhs_up and N %% 256 == 0");
+  if (rhs_kn && (glu || !dls_kn_takes(op, p.K, p.N, p.ro.row_idx ? p.ro.lhs_rows : 0)))
+    return fail(MOE_ERR_UNSUPPORTED, "gmm: [G, K, N] weights on the stream kernel need bf16 or fp8 operands, no rhs_up, N %% 256 == 0 and 32-bit byte offsets");
   if (op == OP_F8) {
     if (rhs_kn) return lhs_e5m2 ? launch_dls_cfg<DlsCfg<OP_F8, false, 1, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_F8, false, 0, true>>(p, M, G_total, s);
     if (lhs_e5m2) return launch_dls_cfg<DlsCfg<OP_F8, false, 1>>(p, M, G_total, s);
     return glu ? launch_dls_cfg<DlsCfg<OP_F8, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_F8, false>>(p, M, G_total, s);
   }
+  if (rhs_kn) return launch_dls_cfg<DlsCfg<OP_BF16, false, 0, true>>(p, M, G_total, s);
   if (op == OP_I8) return glu ? launch_dls_cfg<DlsCfg<OP_I8, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_I8, false>>(p, M, G_total, s);
   return glu ? launch_dls_cfg<DlsCfg<OP_BF16, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_BF16, false>>(p, M, G_total, s);
 }
