@@ -28,6 +28,8 @@
 //                     with K split over the waves of a block.
 
 
+#include <math.h>
+
 #include "moe_gmm_common.h"
 #include "moe_gmm_wqs.h"
 #include "moe_gmm_f8d.h"
@@ -193,9 +195,40 @@ static int scratch_of(void** ptr) {
   return MOE_OK;
 }
 
+// Height of the persistent stream kernels' tiles (256, 192 or 160 rows) for M rows routed to G groups and tiles_n columns of
+// tiles: the one whose rounds of tiles over the chip's blocks cost least, a tile counted as its rows plus what it costs
+// whatever its height (its weight panel, its fetching sides: 96 rows' worth by the Mixtral shape at 128 to 400 rows per
+// expert).  Routed groups scatter around their mean: a group of n ~ N(a, sqrt(a)) rows takes sum_j P(n > j * BM) tiles, so at
+// 128 rows per expert nearly all groups fit 160 rows (int8 first projection 0.283 -> 0.217 ms, on 256-row tiles 0.268), at
+// 160 they need 192 (0.280 -> 0.236), at 320 two of 192 (0.441 -> 0.361); a whole round more than another height needs can
+// decide the other way (Qwen3 shape at 128 rows: three rounds of 256-row tiles, 0.182 ms, against four of 160-row ones, 0.209).
+static int stream_tile_rows(int M, int G, int tiles_n) {
+  int cus = 0;
+  if (device_cu_count(&cus) != MOE_OK) cus = 256;
+  const double a = (double)M / G, sd = sqrt(a > 1.0 ? a : 1.0);
+  int best = 256;
+  double best_cost = 0.0;
+  for (int bm : {256, 192, 160}) {
+    double tiles = 0.0;
+    for (int j = 0; j * bm < a + 4.0 * sd; j++) tiles += 0.5 * erfc((j * (double)bm - a) / (sd * 1.41421356));
+    const double cost = ceil(tiles * G * tiles_n / cus - 1e-3) * (bm + 96.0);
+    if (bm == 256 || cost < best_cost) { best = bm; best_cost = cost; }
+  }
+  return best;
+}
+// Rows per expert on average from which the stream kernel takes operands that need no conversion: 32 for bf16 (level with the
+// 64-row tiles there, 0.365 / 0.361 ms on the Mixtral shape, 5 % ahead on the Qwen3 one); past the LDS-streamed decode
+// kernel's range for 8-bit operands (at 56 rows fp8 0.212 -> 0.199 ms against the 128 x 128 kernel, int8 at 64 level with the
+// 128-row tiles and ahead from 128 on).
+constexpr long long STREAM_ROWS_LO_BF16 = 32, STREAM_ROWS_LO_8BIT = 49;
+// enough tiles for at least half of the chip's CUs
+static bool stream_fills_chip(int M, int G, int N, bool glu) {
+  return (long long)max_tiles_for(M, G, 256) * cdiv(N, glu ? 128 : 256) >= 128;
+}
+
 // Which kernel family takes a shape (rows per expert on average decide the m-tile) and its m-tile: one decision for the
 // tile map and for the launch.
-enum TiledKind { K_T64, K_T128, K_T256, K_DL128, K_DL64, K_DLW, K_DLW128 };
+enum TiledKind { K_T64, K_T128, K_T256, K_DLS, K_DL128, K_DL64, K_DLW, K_DLW128 };
 
 static TiledKind pick_tiled_kind(int op, int bsrc, bool glu, int M, int K, int N, int G_total, bool wq_kmajor = false, long long indexed_lhs_rows = 0) {
   // full 256-row tiles for prefill, 64 otherwise; a problem with fewer 256 x 256 tiles than half the CUs of the chip also
@@ -223,6 +256,7 @@ static TiledKind pick_tiled_kind(int op, int bsrc, bool glu, int M, int K, int N
   if (dlw_ok && !big && (long long)M >= 16LL * G_total && (long long)M < 128LL * G_total &&
       (long long)max_tiles_for(M, G_total, 128) * cdiv(N, glu ? 128 : 256) >= 128)
     return K_DLW128;
+  if (bsrc == BSRC_SAME && (long long)M >= (op == OP_BF16 ? STREAM_ROWS_LO_BF16 : STREAM_ROWS_LO_8BIT) * G_total && dls_takes(op, K, N, indexed_lhs_rows) && stream_fills_chip(M, G_total, N, glu)) return K_DLS;
   if (mid) return K_T128;
   if (big && dlw_ok) return K_DLW;
   // operands that need no conversion stream straight into LDS when every stage is a full row slice
@@ -232,17 +266,14 @@ static TiledKind pick_tiled_kind(int op, int bsrc, bool glu, int M, int K, int N
   return K_T64;
 }
 
-static int tiled_kind_bm(TiledKind k) { return k == K_T64 ? 64 : k == K_T128 || k == K_DLW128 ? 128 : 256; }  // (every direct-to-LDS kernel: 256)
+static int tiled_kind_bm(TiledKind k, int stream_bm) { return k == K_T64 ? 64 : k == K_T128 || k == K_DLW128 ? 128 : k == K_DLS ? stream_bm : 256; }
 
 static int launch_tiled_kind(TiledKind kind, int op, int bsrc, bool glu, const TiledParams& p, int M, int G_total, hipStream_t s) {
-  if (kind == K_DL128) {
-    // the stream kernel where its 32-bit offsets reach and K has three stages; the kernel that drains between tiles otherwise
-    if (dls_takes(op, p.K, p.N, p.ro.row_idx ? p.ro.lhs_rows : 0)) return launch_dls(op, glu, p, M, G_total, s);
-    return launch_dl(op, glu, 128, false, p, M, G_total, s);
-  }
+  if (kind == K_DLS) return launch_dls(op, glu, stream_tile_rows(M, G_total, cdiv(p.N, glu ? 128 : 256)), p, M, G_total, s);
+  if (kind == K_DL128) return launch_dl(op, glu, 128, false, p, M, G_total, s);
   if (kind == K_DL64) return launch_dl(op, glu, 64, false, p, M, G_total, s);
   if (kind == K_DLW || kind == K_DLW128) return launch_dlw(bsrc, glu, kind == K_DLW128, p, M, G_total, s);
-  return launch_tiled_bm(op, bsrc, glu, tiled_kind_bm(kind), false, p, M, G_total, s);
+  return launch_tiled_bm(op, bsrc, glu, tiled_kind_bm(kind, 0), false, p, M, G_total, s);
 }
 
 }  // namespace moe
@@ -349,6 +380,12 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       tile_map_split_kernel<<<1, kMapThreads, 0, s>>>(a->group_sizes, G, a->group_offset, a->group_offset_dev, a->num_groups_local, M, bm, tail_rows,
                                                       tail_base, zero_fill, header, tiles);
   };
+  // MOE_GMM_KERNEL_TILED: the register-staged kernel on the tiles it would have without the direct-to-LDS kernels
+  auto tiled_only = [&](TiledKind k) {
+    if (k == K_DL128 || k == K_DL64 || k == K_DLW) return K_T256;
+    if (k == K_DLS) return (long long)M >= 128LL * G ? K_T256 : (long long)M >= 32LL * G ? K_T128 : K_T64;
+    return k == K_DLW128 ? K_T128 : k;
+  };
   RowOpts ro;
   ro.row_idx = a->lhs_row_idx; ro.idx_div = a->lhs_row_idx_div < 1 ? 1 : a->lhs_row_idx_div;
   ro.lhs_rows = a->lhs_row_idx ? a->lhs_rows : M; ro.out_f32 = a->out_dtype == MOE_F32; ro.row_scale = a->out_row_scale;
@@ -420,8 +457,7 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
                                                      : kernel != MOE_GMM_KERNEL_STREAM;
     if (kernel > MOE_GMM_KERNEL_BIG) return fail(MOE_ERR_UNSUPPORTED, "gmm: kernel family %d does not take fp8 operands", kernel);
     // prefill-sized groups: the persistent 256 x 256 stream, where it takes the shape
-    const bool chip_full = (long long)max_tiles_for(M, G, 256) * cdiv(N, glu ? 128 : 256) >= 128;
-    const bool prefill = kernel == MOE_GMM_KERNEL_BIG || (kernel == MOE_GMM_KERNEL_AUTO && (long long)M >= 128LL * G && chip_full);
+    const bool prefill = kernel == MOE_GMM_KERNEL_BIG || (kernel == MOE_GMM_KERNEL_AUTO && (long long)M >= (fp8_blocks ? 128LL : STREAM_ROWS_LO_8BIT) * G && stream_fills_chip(M, G, N, glu));
     // scales in the epilogue only (per row / per tensor x per channel / per tensor): the int8 x int8 problem on another MFMA
     const bool stream_epi = !fp8_blocks && prefill && dls_takes(OP_F8, K, N, ro.row_idx ? ro.lhs_rows : 0);
     if (kn_fp8 && !stream_epi) return fail(MOE_ERR_UNSUPPORTED, "gmm: [G, K, N] fp8 weights run on the persistent 256 x 256 kernel only (no K-block scales)");
@@ -430,7 +466,7 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
                   "K %% 128 == 0, K >= 384, no rhs_up, no K-block scales); widen them to bf16 for other shapes");
     if (stream_epi) {
       if (lhs_e5m2 && glu) return fail(MOE_ERR_UNSUPPORTED, "gmm: float8_e5m2 activations take no rhs_up");
-      map_tiles(256);
+      map_tiles(stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256)));
       TiledParams q = {};
       q.lhs = (const uint8_t*)a->lhs; q.rhs = (const uint8_t*)a->rhs; q.rhs_up = (const uint8_t*)a->rhs_up;
       q.rhs_bias = a->rhs_bias; q.rhs_up_bias = a->rhs_up_bias;
@@ -440,7 +476,7 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       q.lhs_scale = sp.lhs_epi; q.lhs_scale_stride = sp.lhs_epi_stride;
       q.rhs_scale = a->rhs_scale; q.rhs_up_scale = a->rhs_up_scale;
       q.rhs_scale_gstride = sp.rhs_gstride; q.rhs_scale_nstride = sp.rhs_nstride;
-      return launch_dls(OP_F8, glu, q, M, G, s, lhs_e5m2 ? 1 : 0, kn_fp8 ? 1 : 0);
+      return launch_dls(OP_F8, glu, stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256)), q, M, G, s, lhs_e5m2 ? 1 : 0, kn_fp8 ? 1 : 0);
     }
     if (tiled) {
       const bool big = kernel == MOE_GMM_KERNEL_BIG;
@@ -544,8 +580,8 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       return launch_f8l(q, glu, true, bm, a->num_groups_local, s);
     }
     TiledKind kind = pick_tiled_kind(op, BSRC_SAME, glu, M, K, N, G);
-    if (kernel == MOE_GMM_KERNEL_TILED && (kind == K_DL128 || kind == K_DL64)) kind = K_T256;
-    map_tiles(tiled_kind_bm(kind));
+    if (kernel == MOE_GMM_KERNEL_TILED) kind = tiled_only(kind);
+    map_tiles(tiled_kind_bm(kind, stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256))));
     return launch_tiled_kind(kind, op, BSRC_SAME, glu, p, M, G, s);
   }
 
@@ -591,10 +627,11 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
   if (a->flags & MOE_GMM_RHS_KN) {
     if (variant != V_BF16 || glu || !moe_gmm_rhs_kn_supported(M, K, N, G))
       return fail(MOE_ERR_UNSUPPORTED, "gmm: [G, K, N] weights need bf16 x bf16 without rhs_up and a shape moe_gmm_rhs_kn_supported accepts");
-    map_tiles(256);
+    const bool kn_stream = dls_kn_takes(OP_BF16, K, N, ro.row_idx ? ro.lhs_rows : 0);
+    map_tiles(kn_stream ? stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256)) : 256);
     // the stream kernel where its 32-bit offsets reach and K has three stages (dlhs of the Mixtral shape 1.65 -> 1.47 and
     // 1.79 -> 1.59 ms), the kernel that drains between tiles otherwise
-    if (dls_kn_takes(OP_BF16, K, N, ro.row_idx ? ro.lhs_rows : 0)) return launch_dls(OP_BF16, false, p, M, G, s, 0, 1);
+    if (kn_stream) return launch_dls(OP_BF16, false, stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256)), p, M, G, s, 0, 1);
     return launch_dl(OP_BF16, false, 128, true, p, M, G, s);
   }
   const int bsrc = variant == V_BF16 ? BSRC_SAME : variant == V_W8 ? BSRC_I8 : variant == V_W4 ? BSRC_I4 : BSRC_MX4;
@@ -649,13 +686,13 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
     return launch_dl(op, glu, 64, false, p, M, G, s);
   }
   TiledKind kind = kernel == MOE_GMM_KERNEL_BIG ? K_T256 : pick_tiled_kind(op, bsrc, glu, M, K, N, G, wq_kmajor, a->lhs_row_idx ? ro.lhs_rows : 0);
-  if (kernel == MOE_GMM_KERNEL_TILED && (kind == K_DL128 || kind == K_DL64 || kind == K_DLW || kind == K_DLW128)) kind = kind == K_DLW128 ? K_T128 : K_T256;
+  if (kernel == MOE_GMM_KERNEL_TILED) kind = tiled_only(kind);
   // 4-bit weights on the persistent kernel: a group's last rows, when they are few, go to the decode kernel in a second
   // launch (16-row tiles of a second list) instead of filling a corner of one more 128- or 256-row tile
   const bool split_tails = (kind == K_DLW || kind == K_DLW128) && kernel == MOE_GMM_KERNEL_AUTO && (bsrc == BSRC_I4 || bsrc == BSRC_MX4) && !wq_kmajor &&
                            wqs_takes(wq_fmt, K, N, a->num_groups_local, glu);
   if (split_tails) {
-    const int bm = tiled_kind_bm(kind);
+    const int bm = tiled_kind_bm(kind, 0);
     const int tail_base = max_tiles_for(M, G, bm);  // past every record the first list can hold
     if ((size_t)16 + ((size_t)tail_base + (size_t)G * cdiv(kTailRows, kTailTile)) * sizeof(TileInfo) <= workspace_bytes) {
       map_tiles_split(bm, kTailRows, tail_base);
@@ -670,7 +707,7 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       return launch_wqs(wq_fmt, q, glu, a->num_groups_local, s);
     }
   }
-  map_tiles(tiled_kind_bm(kind));
+  map_tiles(tiled_kind_bm(kind, stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256))));
   return launch_tiled_kind(kind, op, bsrc, glu, p, M, G, s);
 }
 

@@ -265,7 +265,8 @@ struct EpilogueScales {
   float4 sg[NT_OUT][4], su[NT_OUT][4];
 };
 
-template <int TM, int NT_OUT, bool GLU, bool CHANNEL_SCALES, int MI = 32>
+// (RS: rows from one row tile of the wave to its next)
+template <int TM, int NT_OUT, bool GLU, bool CHANNEL_SCALES, int MI = 32, int RS = MI>
 __device__ __forceinline__ void load_epilogue_scales(EpilogueScales<TM, NT_OUT, GLU>& e, const TiledParams& p, const TileInfo& tile,
                                                      int row_base, int n_base, int lane) {
   // every decision is uniform and taken once, so that the loads of a kind go out back to back
@@ -276,7 +277,7 @@ __device__ __forceinline__ void load_epilogue_scales(EpilogueScales<TM, NT_OUT, 
     int rows[TM];
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-      const int lr = row_base + i * MI + (lane % MI);
+      const int lr = row_base + i * RS + (lane % MI);
       rows[i] = tile.row0 + (lr < tile.nrows ? lr : 0);
     }
     lhs_rows_of<TM>(p.ro, rows);
@@ -320,10 +321,11 @@ __device__ __forceinline__ void load_epilogue_scales(EpilogueScales<TM, NT_OUT, 
 // lanes in different rows; the plain bf16 case pairs tiles and stores 16 bytes per lane (below).  (Passing each row tile
 // through LDS so that consecutive lanes store consecutive 16 bytes was measured and is slower.)
 // (I_END < TM: only the wave's first I_END row tiles hold rows of this tile.)
-template <int TM, int TN, int NT_OUT, bool GLU, int I_END = TM, typename acc_t>
+template <int TM, int TN, int NT_OUT, bool GLU, int I_END = TM, int ROW_STRIDE = 0, typename acc_t>
 __device__ __forceinline__ void store_epilogue(const acc_t (&acc)[TN][TM], const EpilogueScales<TM, NT_OUT, GLU>& e,
                                                const TiledParams& p, const TileInfo& tile, int row_base, int n_base, int lane) {
   constexpr int MI = sizeof(acc_t) == 16 ? 16 : 32;  // 4 accumulator registers per tile: the 16 x 16 instructions
+  constexpr int RS = ROW_STRIDE ? ROW_STRIDE : MI;   // rows from one row tile of the wave to its next
   // Everything that needs a load is decided and loaded up front, by uniform branches, and the variants of the body are
   // separate straight-line instantiations: a branch or a load between two stores makes the compiler wait for ALL memory
   // operations in flight, the stores included, i.e. one memory round trip per store (measured on 256 x 256 tiles: 18 us
@@ -335,7 +337,7 @@ __device__ __forceinline__ void store_epilogue(const acc_t (&acc)[TN][TM], const
   if (p.ro.row_scale) {
 #pragma unroll
     for (int i = 0; i < I_END; i++) {
-      const int lr = row_base + i * MI + (lane % MI);
+      const int lr = row_base + i * RS + (lane % MI);
       rw[i] = p.ro.row_scale[tile.row0 + (lr < tile.nrows ? lr : 0)];
     }
     // (complete here: left pending on the paths that do not use them, they are waited for in the next tile's main loop)
@@ -353,7 +355,7 @@ __device__ __forceinline__ void store_epilogue(const acc_t (&acc)[TN][TM], const
       // (256 x 256 int8 tiles, 14336-long K: 0.929 against 0.947 ms).
 #pragma unroll
       for (int i = 0; i < I_END; i++) {
-        const int lr = row_base + i * MI + (lane % MI);
+        const int lr = row_base + i * RS + (lane % MI);
         const bool row_ok = lr < tile.nrows;
 #pragma unroll
         for (int j = 0; j < NT_OUT; j += 2) {
@@ -383,7 +385,7 @@ __device__ __forceinline__ void store_epilogue(const acc_t (&acc)[TN][TM], const
     }
 #pragma unroll
     for (int i = 0; i < I_END; i++) {
-      const int lr = row_base + i * MI + (lane % MI);
+      const int lr = row_base + i * RS + (lane % MI);
       const bool row_ok = lr < tile.nrows;
 #pragma unroll
       for (int j = 0; j < NT_OUT; j++)
@@ -642,9 +644,9 @@ int launch_tiled_bm(int op, int bsrc, bool glu, int bm, bool block_scaled, const
 // moe_gmm_dl.hip: direct-to-LDS persistent kernel, 256 x 256 tiles; stage_bytes 128 or 64; rhs_kn: [G, K, N] bf16 weights
 int launch_dl(int op, bool glu, int stage_bytes, bool rhs_kn, const TiledParams& p, int M, int G_total, hipStream_t s);
 // moe_gmm_dlw.hip: the same pipeline for bf16 activations x int8 / int4 / mxfp4 weights (K % 64 == 0, default scale layouts)
-// moe_gmm_dls.hip: the persistent 256 x 256 kernel for int8 x int8 / bf16 x bf16 with one request stream across tiles
+// moe_gmm_dls.hip: the persistent kernel (tiles of bm = 256, 192 or 160 rows x 256 channels) for int8 x int8 / bf16 x bf16 with one request stream across tiles
 // (fp8 x fp8 with epilogue scales too; lhs_e5m2: the activations are float8_e5m2, the weights e4m3)
-int launch_dls(int op, bool glu, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2 = 0, int rhs_kn = 0);
+int launch_dls(int op, bool glu, int bm, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2 = 0, int rhs_kn = 0);
 bool dls_takes(int op, int K, int N, long long indexed_lhs_rows);
 bool dls_kn_takes(int op, int K, int N, long long indexed_lhs_rows);  // the same for [G, K, N] weights (bf16, fp8)
 // moe_gmm_f8s.hip: the same stream for block-scaled fp8 (1 x 128 activation scales, 128 x 128 weight scales)

@@ -1,10 +1,10 @@
-// Grouped matmul: the persistent 256 x 256 kernel for operands that need no conversion (int8 x int8, bf16 x bf16 and
+// Grouped matmul: the persistent kernel on tiles of 256, 192 or 160 rows x 256 channels for operands that need no conversion (int8 x int8, bf16 x bf16 and
 // fp8 x fp8 with per-row x per-channel scales, prefill) with the stages of a block's consecutive tiles as ONE request
 // stream.
 //
 // Both operands go global -> LDS without passing through registers (buffer_load ... lds, 1 KB = 8 rows of 128 bytes per
-// wave instruction; XOR-swizzled unpadded rows; two buffers of 64 KB).  8 waves as 2 x 4, each 128 x 64 of the tile in
-// 16 x 16 MFMAs (16x16x64 i8 / 16x16x32 bf16 / 16x16x128 f8f6f4).
+// wave instruction; XOR-swizzled unpadded rows; two buffers of 64 KB, 56 KB for lower tiles).  8 waves as 2 x 4, each 128 (96,
+// 80) x 64 of the tile in 16 x 16 MFMAs (16x16x64 i8 / 16x16x32 bf16 / 16x16x128 f8f6f4).
 //
 // Schedule: the two waves of a SIMD take turns.  A stage (128 bytes of K) is four phases, one 64 x 32 quadrant of the
 // wave's tile each (16 MFMAs, 8 of fp8: 256 cycles); a phase is a fetching side (fragment reads, two requests, waits), a
@@ -38,7 +38,7 @@
 
 namespace moe {
 
-template <int OP_, bool GLU_, int LF_ = 0, bool KN_ = false>
+template <int OP_, bool GLU_, int LF_ = 0, bool KN_ = false, int TM_ = 8>
 struct DlsCfg {
   static constexpr int OP = OP_;
   static constexpr bool GLU = GLU_;
@@ -47,12 +47,18 @@ struct DlsCfg {
   // are).  The weight half of a stage then holds 128 (bf16: 64) contraction rows x 256 output channels (four rows of 256 or two
   // of 512 bytes per wave instruction) and the weight fragments come out of it through ds_read_b64_tr_b8 / _b16.
   static constexpr bool KN = KN_;
-  static constexpr int BM = 256, BN = 256, BKB = 128, MI = 16;
+  // Row tiles of a wave: 8, 6 or 5, i.e. 256, 192 or 160 rows to a tile.  Row tile i of wave row wm holds the tile's rows
+  // 32 i + 16 wm .. + 15; the first four are half h = 0 of the activations (128 rows), the others half h = 1.
+  static constexpr int TM = TM_, H1 = TM - 4;
+  static constexpr int BM = TM * 32, BN = 256, BKB = 128, MI = 16;
   static constexpr int ESZ = OP == OP_BF16 ? 2 : 1, BK = BKB / ESZ;
   static constexpr int WAVES_M = 2, WAVES_N = 4, NWAVES = 8, THREADS = NWAVES * kWave;
-  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / MI, TN = WN / MI;
-  static constexpr int A_STAGE = BM * BKB, STAGE = (BM + BN) * BKB, LDS_BYTES = 2 * STAGE;
-  static constexpr int A_IPW = BM / 8 / NWAVES, B_IPW = BN / 8 / NWAVES;  // requests per wave and stage: 4 + 4
+  static constexpr int WN = BN / WAVES_N, TN = WN / MI;
+  // requests per wave and stage: 2 for the first activation half, NA1 for the second (64 rows' worth at least: rows past the
+  // tile's are past its descriptor and fetch nothing), 4 for the weights
+  static constexpr int NA1 = H1 > 2 ? 2 : 1, A_IPW = 2 + NA1, B_IPW = BN / 8 / NWAVES;
+  static constexpr int A_ROWS = 128 + NA1 * 64, A_STAGE = A_ROWS * BKB, STAGE = A_STAGE + BN * BKB, LDS_BYTES = 2 * STAGE;
+  static_assert(TM == 8 || TM == 6 || TM == 5, "row tiles");
   static constexpr int OUT_BN = GLU ? BN / 2 : BN;
   static_assert(OP == OP_I8 || OP == OP_BF16 || OP == OP_F8, "operands");
   static_assert(LF == 0 || OP == OP_F8, "only fp8 activations come in two formats");
@@ -85,13 +91,17 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   auto resolve = [&](Peek pk, Tile& t) { return resolve_tile<C::OUT_BN, C::THREADS>(p, num_tiles, pk, t, tid); };
 
   // ---- the loading side of the stream ---------------------------------------------------------------------------
-  // A stage arrives in four halves of two requests per wave (1 KB = 8 rows x 128 bytes each): the activation rows of row
-  // tiles 0 .. 3 (h = 0) and 4 .. 7 (h = 1) of both wave rows, and the weight rows of channel tiles 0, 1 (g = 0) and 2, 3
+  // A stage arrives in four halves of two requests per wave (1 KB = 8 rows x 128 bytes each; the second half of a lower tile:
+  // one request): activation rows 0 .. 127 and 128 .. of the tile, and the weight rows of channel tiles 0, 1 (g = 0) and 2, 3
   // (g = 1) of the four wave columns (with GLU: the first and the second projection).  The lane's 16 bytes: global chunk =
   // LDS slot ^ swizzle of the row.
-  auto a_req_row = [&](int i) { return (wave / 4) * 128 + (i / 2) * 64 + (wave % 4) * 16 + (i % 2) * 8; };
-  auto b_req_row = [&](int i) {
-    return C::GLU ? (i / 2) * 128 + wave * 16 + (i % 2) * 8 : (wave / 2) * 64 + (i / 2) * 32 + (wave % 2) * 16 + (i % 2) * 8;
+  // (w: the wave as a scalar for LDS addresses, wave_v for lane offsets: a value the compiler shares between the two ends up in
+  // a vector register, which the copy's scalar operand then cannot take)
+  int wave_v = wave;
+  asm volatile("" : "+v"(wave_v));
+  auto a_req_row = [&](int i, int w) { return i < 2 ? w * 16 + i * 8 : 128 + w * 8 * C::NA1 + (i - 2) * 8; };
+  auto b_req_row = [&](int i, int w) {
+    return C::GLU ? (i / 2) * 128 + w * 16 + (i % 2) * 8 : (w / 2) * 64 + (i / 2) * 32 + (w % 2) * 16 + (i % 2) * 8;
   };
   auto lane_off = [&](int req_row, uint32_t row) {
     return row * row_bytes + (uint32_t)(((lane % 8) ^ C::swz(req_row + lane / 8)) << 4);
@@ -103,27 +113,28 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
       a_desc = buffer_desc(p.lhs, clamp_u32((size_t)p.ro.lhs_rows * row_bytes));
       int rows[C::A_IPW];
 #pragma unroll
-      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + a_req_row(i) + lane / 8, p.M - 1);
+      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + a_req_row(i, wave_v) + lane / 8, p.M - 1);
       lhs_rows_of<C::A_IPW>(p.ro, rows);
+      // (rows past the tile's end: one row past the descriptor's, i.e. zeros without a request to memory)
 #pragma unroll
-      for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i), (uint32_t)rows[i]);
+      for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i, wave_v), (uint32_t)(a_req_row(i, wave_v) + lane / 8 < t.info.nrows ? rows[i] : p.ro.lhs_rows));
     } else {
       a_desc = buffer_desc(p.lhs + (size_t)t.info.row0 * row_bytes, clamp_u32((size_t)t.info.nrows * row_bytes));
     }
   };
   if (!p.ro.row_idx) {
 #pragma unroll
-    for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i), (uint32_t)(a_req_row(i) + lane / 8));
+    for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i, wave_v), (uint32_t)(a_req_row(i, wave_v) + lane / 8));
   }
 #pragma unroll
   for (int i = 0; i < C::B_IPW; i++) {
     if constexpr (C::KN) {
       // request i covers KN_RPR contraction rows of the stage, the lane one 16-byte LDS slot of its row
       constexpr int LPR = kWave / C::KN_RPR;
-      const int r = (wave * C::B_IPW + i) * C::KN_RPR + lane / LPR;
+      const int r = (wave_v * C::B_IPW + i) * C::KN_RPR + lane / LPR;
       b_voff[i] = (uint32_t)r * (uint32_t)(N * C::ESZ) + (uint32_t)(((lane % LPR) ^ C::kn_swz(r)) << 4);
     } else {
-      b_voff[i] = lane_off(b_req_row(i), (uint32_t)((C::GLU ? b_req_row(i) % 128 : b_req_row(i)) + lane / 8));
+      b_voff[i] = lane_off(b_req_row(i, wave_v), (uint32_t)((C::GLU ? b_req_row(i, wave_v) % 128 : b_req_row(i, wave_v)) + lane / 8));
     }
   }
   auto set_b_sources = [&](const Tile& t) {
@@ -133,13 +144,13 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   };
   auto issue_a = [&](int kt, int buf, int h) {
 #pragma unroll
-    for (int i = 2 * h; i < 2 * h + 2; i++)
-      dma16_buffer(a_desc, a_voff[i], (uint32_t)kt * C::BKB, lds_base + buf * C::STAGE + a_req_row(i) * C::BKB);
+    for (int i = 2 * h; i < (h ? C::A_IPW : 2); i++)
+      dma16_buffer(a_desc, a_voff[i], (uint32_t)kt * C::BKB, lds_base + buf * C::STAGE + a_req_row(i, wave) * C::BKB);
   };
   auto issue_b = [&](int kt, int buf, int g) {
 #pragma unroll
     for (int i = 2 * g; i < 2 * g + 2; i++) {
-      const uint32_t dst = lds_base + buf * C::STAGE + C::A_STAGE + (C::KN ? (wave * C::B_IPW + i) * 1024 : b_req_row(i) * C::BKB);
+      const uint32_t dst = lds_base + buf * C::STAGE + C::A_STAGE + (C::KN ? (wave * C::B_IPW + i) * 1024 : b_req_row(i, wave) * C::BKB);
       dma16_buffer(b_desc[C::GLU ? g : 0], b_voff[i], b_soff + (uint32_t)kt * C::BKB * (C::KN ? (uint32_t)N : 1u), dst);
     }
   };
@@ -148,7 +159,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   using T_ = std::true_type;
   using F_ = std::false_type;
   constexpr int NT_OUT = C::GLU ? C::TN / 2 : C::TN;
-  constexpr int HM = C::TM / 2, HN = C::TN / 2;  // row tiles and channel tiles of a quadrant: 4 x 2
+  constexpr int HN = C::TN / 2;  // channel tiles of a quadrant
+  auto row_tiles = [](int h) { return h ? C::H1 : 4; };
   // first LDS row of channel tile j
   const int b_base = C::A_STAGE + (C::GLU ? wn * (C::WN / 2) : wn * C::WN) * C::BKB;
   auto b_tile = [&](int j) { return (C::GLU ? (j / HN) * (C::BN / 2) + (j % HN) * C::MI : j * C::MI) * C::BKB; };
@@ -167,7 +179,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   acc_t acc[C::TN][C::TM];
   // fragments: 8 registers per tile and stage, the two 64-byte k-steps of int8 / bf16 or the one 128-byte operand of fp8
   // (K bytes 16 q .. and 64 + 16 q ..: both operands alike, so the order of K inside the instruction does not matter)
-  v8i fa[HM], fb[2][HN];
+  v8i fa[4], fb[2][HN];
   auto read_frag = [&](v8i& f, const uint8_t* src) {
     const v4i lo = *(const v4i*)(src + frag_lane), hi = *(const v4i*)(src + (frag_lane ^ 64));
     f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   };
   auto read_a = [&](int buf, int h) {
 #pragma unroll
-    for (int i = 0; i < HM; i++) read_frag(fa[i], smem + buf * C::STAGE + (wm * C::WM + (h * HM + i) * 16) * C::BKB);
+    for (int i = 0; i < row_tiles(h); i++) read_frag(fa[i], smem + buf * C::STAGE + ((h * 4 + i) * 32 + wm * 16) * C::BKB);
   };
   auto read_b = [&](int buf, int g) {
 #pragma unroll
@@ -202,25 +214,25 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   };
   auto lo4 = [](const v8i& v) { return __builtin_shufflevector(v, v, 0, 1, 2, 3); };
   auto hi4 = [](const v8i& v) { return __builtin_shufflevector(v, v, 4, 5, 6, 7); };
-  // One quadrant: row tiles 4h .. 4h + 3 x channel tiles 2g, 2g + 1.  ZC: a tile's first stage starts from zero.
+  // One quadrant: row tiles 4h .. x channel tiles 2g, 2g + 1.  ZC: a tile's first stage starts from zero.
   auto quadrant = [&](auto zc_c, int h, int g) __attribute__((always_inline)) {
     constexpr bool ZC = decltype(zc_c)::value;
     if constexpr (OP == OP_F8) {
 #pragma unroll
-      for (int i = 0; i < HM; i++)
+      for (int i = 0; i < row_tiles(h); i++)
 #pragma unroll
         for (int jj = 0; jj < HN; jj++) {
-          acc_t& c = acc[g * HN + jj][h * HM + i];
+          acc_t& c = acc[g * HN + jj][h * 4 + i];
           c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[g][jj], fa[i], ZC ? acc_t{} : c, 0, C::LF, 0, 127, 0, 127);
         }
     } else {
 #pragma unroll
       for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-        for (int i = 0; i < HM; i++)
+        for (int i = 0; i < row_tiles(h); i++)
 #pragma unroll
           for (int jj = 0; jj < HN; jj++) {
-            acc_t& c = acc[g * HN + jj][h * HM + i];
+            acc_t& c = acc[g * HN + jj][h * 4 + i];
             const v4i b = ks ? hi4(fb[g][jj]) : lo4(fb[g][jj]), a = ks ? hi4(fa[i]) : lo4(fa[i]);
             if constexpr (OP == OP_I8) c = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a, ZC && ks == 0 ? acc_t{} : c, 0, 0, 0);
             else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, b), __builtin_bit_cast(v8bf, a), ZC && ks == 0 ? acc_t{} : c, 0, 0, 0);
@@ -244,14 +256,16 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
 #pragma unroll
     for (int jj = 0; jj < HN; jj++)
 #pragma unroll
-      for (int i = 0; i < HM; i++) asm volatile("" : "+v"(acc[g * HN + jj][h * HM + i]));
+      for (int i = 0; i < row_tiles(h); i++) asm volatile("" : "+v"(acc[g * HN + jj][h * 4 + i]));
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_barrier" ::: "memory");
   };
   using NOWAIT = std::integral_constant<int, -1>;
-  using W10 = std::integral_constant<int, 10>;
-  using W8 = std::integral_constant<int, 8>;
+  // requests that may be outstanding where a phase ends ahead of new data: those behind the last half that the next phase reads
+  using W1 = std::integral_constant<int, 6 + 2 * C::NA1>;                // ahead of phase 2 (weights, g = 1)
+  using W2 = std::integral_constant<int, 8 + C::NA1>;                    // ahead of phase 3 (activations, h = 1)
+  using W4 = std::integral_constant<int, (C::KN ? 6 : 8) + C::NA1>;      // ahead of phase 1 ([G, K, N]: both weight halves)
 
   Tile cur, nxt;
   if (!resolve(peek_from(blockIdx.x), cur)) return;
@@ -274,7 +288,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
     // Stage `it`, in four phases.  first: the stage's data and what the next one starts with landed before the tile began
     // (no waits).  cross: the stream moves on to the next tile after the first phase.
     auto stage_head = [&](int it, auto first_c) __attribute__((always_inline)) {
-      using WA = typename std::conditional<decltype(first_c)::value, NOWAIT, W10>::type;
+      using WA = typename std::conditional<decltype(first_c)::value, NOWAIT, W1>::type;
       // 1: both first halves; requests the last half of the next stage (its slot was read two phases ago)
       read_b(cb, 0);
       read_a(cb, 0);
@@ -285,8 +299,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
     };
     auto stage_rest = [&](int it, auto first_c) __attribute__((always_inline)) {
       constexpr bool FIRST = decltype(first_c)::value;
-      using WA = typename std::conditional<FIRST, NOWAIT, W10>::type;
-      using WB = typename std::conditional<FIRST, NOWAIT, typename std::conditional<C::KN, W8, W10>::type>::type;
+      using WA = typename std::conditional<FIRST, NOWAIT, W2>::type;
+      using WB = typename std::conditional<FIRST, NOWAIT, W4>::type;
       // 2
       const int kt2 = stream_kt(it + 2);
       read_b(cb, 1);
@@ -326,10 +340,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
     if (!late) asm volatile("s_barrier" ::: "memory");
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
-    load_epilogue_scales<C::TM, NT_OUT, C::GLU, true, C::MI>(esc, p, cur.info, wm * C::WM, n_out0, lane_e);
+    load_epilogue_scales<C::TM, NT_OUT, C::GLU, true, C::MI, 32>(esc, p, cur.info, wm * C::MI, n_out0, lane_e);
     // everything requested so far lands here, ahead of the stores: the next tile's first stage need not count them
     wait_vmcnt<0>();
-    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU>(acc, esc, p, cur.info, wm * C::WM, n_out0, lane_e);
+    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, C::TM, 32>(acc, esc, p, cur.info, wm * C::MI, n_out0, lane_e);
     if (!have_n) break;
     cur = nxt;
   }
@@ -347,19 +361,33 @@ static int prepare_dls_cfg() {
   return reserve_lds(gmm_dls_kernel<C>, C::LDS_BYTES, lds_flags<C>());
 }
 
+// Calls f with the configuration of a call: operand, GLU, e5m2 activations, [G, K, N] weights, row tiles.
+template <typename F>
+static int with_dls_cfg(int op, bool glu, int lhs_e5m2, int rhs_kn, int tm, F&& f) {
+  auto rows = [&](auto tm_c) {
+    constexpr int TM = decltype(tm_c)::value;
+    if (op == OP_F8) {
+      if (rhs_kn) return lhs_e5m2 ? f(DlsCfg<OP_F8, false, 1, true, TM>{}) : f(DlsCfg<OP_F8, false, 0, true, TM>{});
+      if (lhs_e5m2) return f(DlsCfg<OP_F8, false, 1, false, TM>{});
+      return glu ? f(DlsCfg<OP_F8, true, 0, false, TM>{}) : f(DlsCfg<OP_F8, false, 0, false, TM>{});
+    }
+    if (op == OP_I8) return glu ? f(DlsCfg<OP_I8, true, 0, false, TM>{}) : f(DlsCfg<OP_I8, false, 0, false, TM>{});
+    if (rhs_kn) return f(DlsCfg<OP_BF16, false, 0, true, TM>{});
+    return glu ? f(DlsCfg<OP_BF16, true, 0, false, TM>{}) : f(DlsCfg<OP_BF16, false, 0, false, TM>{});
+  };
+  return tm == 5 ? rows(std::integral_constant<int, 5>{}) : tm == 6 ? rows(std::integral_constant<int, 6>{}) : rows(std::integral_constant<int, 8>{});
+}
+
 int prepare_dls() {
-  int st = MOE_OK;
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_I8, false>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_I8, true>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_BF16, false>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_BF16, true>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, true>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false, 1>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_BF16, false, 0, true>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false, 0, true>>();
-  if (!st) st = prepare_dls_cfg<DlsCfg<OP_F8, false, 1, true>>();
-  return st;
+  auto prep = [](auto cfg) { return prepare_dls_cfg<decltype(cfg)>(); };
+  for (int tm : {5, 6, 8})
+    for (int op : {OP_I8, OP_BF16, OP_F8})
+      for (int v = 0; v < 5; v++) {  // plain, GLU, e5m2, [G, K, N], both
+        const bool glu = v == 1, e5m2 = v == 2 || v == 4, kn = v >= 3;
+        if ((e5m2 && op != OP_F8) || (kn && op == OP_I8)) continue;
+        if (int st = with_dls_cfg(op, glu, e5m2, kn, tm, prep)) return st;
+      }
+  return MOE_OK;
 }
 
 template <typename C>
@@ -397,20 +425,14 @@ bool dls_kn_takes(int op, int K, int N, long long indexed_lhs_rows) {
   return op != OP_I8 && dls_takes(op, K, N, indexed_lhs_rows) && N % 256 == 0 && ((long long)K + 128) * N * (op == OP_BF16 ? 2 : 1) < (1LL << 32);
 }
 
-int launch_dls(int op, bool glu, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2, int rhs_kn) {
+int launch_dls(int op, bool glu, int bm, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2, int rhs_kn) {
   if (!dls_takes(op, p.K, p.N, p.ro.row_idx ? p.ro.lhs_rows : 0))
     return fail(MOE_ERR_UNSUPPORTED, "gmm: the stream kernel needs int8, bf16 or fp8 operands, whole 128-byte stages (three or more) and 32-bit byte offsets");
   if (lhs_e5m2 && (op != OP_F8 || glu)) return fail(MOE_ERR_UNSUPPORTED, "gmm: e5m2 activations run against e4m3 weights without rhs_up");
   if (rhs_kn && (glu || !dls_kn_takes(op, p.K, p.N, p.ro.row_idx ? p.ro.lhs_rows : 0)))
     return fail(MOE_ERR_UNSUPPORTED, "gmm: [G, K, N] weights on the stream kernel need bf16 or fp8 operands, no rhs_up, N %% 256 == 0 and 32-bit byte offsets");
-  if (op == OP_F8) {
-    if (rhs_kn) return lhs_e5m2 ? launch_dls_cfg<DlsCfg<OP_F8, false, 1, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_F8, false, 0, true>>(p, M, G_total, s);
-    if (lhs_e5m2) return launch_dls_cfg<DlsCfg<OP_F8, false, 1>>(p, M, G_total, s);
-    return glu ? launch_dls_cfg<DlsCfg<OP_F8, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_F8, false>>(p, M, G_total, s);
-  }
-  if (rhs_kn) return launch_dls_cfg<DlsCfg<OP_BF16, false, 0, true>>(p, M, G_total, s);
-  if (op == OP_I8) return glu ? launch_dls_cfg<DlsCfg<OP_I8, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_I8, false>>(p, M, G_total, s);
-  return glu ? launch_dls_cfg<DlsCfg<OP_BF16, true>>(p, M, G_total, s) : launch_dls_cfg<DlsCfg<OP_BF16, false>>(p, M, G_total, s);
+  if (bm != 256 && bm != 192 && bm != 160) return fail(MOE_ERR_INVALID_ARG, "gmm: the stream kernel has no tiles of %d rows", bm);
+  return with_dls_cfg(op, glu, lhs_e5m2, rhs_kn, bm / 32, [&](auto cfg) { return launch_dls_cfg<decltype(cfg)>(p, M, G_total, s); });
 }
 
 }  // namespace moe

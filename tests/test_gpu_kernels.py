@@ -417,6 +417,47 @@ def test_gmm_bf16(K, m, k, n, gs):
   assert relerr(got, want) <= TOL
 
 
+# groups around the heights of the stream kernel's tiles (160 rows at 128 rows per expert on average, 192 at 170 with these many
+# columns), the wave rows' 32-row stripes and the 128 rows of a stage's first half
+STREAM_TILE_GROUPS = {
+    160: [160, 161, 159, 128, 129, 127, 1, 0, 96, 97, 320, 33, 150, 144, 200, 130],
+    192: [192, 193, 191, 160, 161, 128, 129, 1, 384, 0, 170, 225, 180, 190, 200, 210],
+}
+
+
+@pytest.mark.parametrize("height,n", [(160, 1032), (192, 8200)])
+@pytest.mark.parametrize("kind", ["int8", "bf16", "fp8"])
+@pytest.mark.parametrize("glu", [False, True])
+def test_gmm_stream_tile_heights(K, height, n, kind, glu):
+  """The persistent stream kernel on its lower tiles: against the register-staged kernel (int8: the sums are integers, so bit
+  for bit) with rows read through an index, a bias and rows that belong to no group."""
+  gs = np.array(STREAM_TILE_GROUPS[height], np.int32)
+  m, k = int(gs.sum()) + 40, 384
+  g = torch.Generator().manual_seed(height)
+  idx = torch.randperm(m, generator=g).to(torch.int32)
+  kw = dict(lhs_row_idx=cuda(idx), rhs_bias=cuda(torch.randn(16, n, generator=g)))
+  if kind == "bf16":
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+  elif kind == "int8":
+    mk = lambda *s: torch.randint(-127, 128, s, generator=g).to(torch.int8)
+  else:
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.float8_e4m3fn)
+  lhs, w = mk(m, k), mk(16, n, k)
+  if kind != "bf16":
+    kw.update(lhs_scale=cuda(torch.rand(m, generator=g) * 0.02), rhs_scale=cuda(torch.rand(16, n, generator=g) * 0.02))
+  if glu:
+    kw.update(rhs_up=cuda(mk(16, n, k)), act="silu")
+    if kind != "bf16":
+      kw["rhs_up_scale"] = cuda(torch.rand(16, n, generator=g) * 0.02)
+  got = K.gmm_raw(cuda(lhs), cuda(w), cuda(gs), **kw)
+  want = K.gmm_raw(cuda(lhs), cuda(w), cuda(gs), kernel="tiled", **kw)
+  assert torch.all(got[int(gs.sum()):] == 0)
+  if kind == "int8":
+    assert torch.equal(got, want)
+  else:
+    assert relerr(got, want) <= TOL
+
+
 RHS_KN_SHAPES = [
     (1065, 192, 3328, [300, 0, 700, 65]),  # three k stages, an empty group, ragged m-tiles
     (2100, 1024, 2560, [1000, 500, 436, 64]),  # 100 rows belong to no group
