@@ -196,12 +196,15 @@ static int scratch_of(void** ptr) {
 }
 
 // Height of the persistent stream kernels' tiles (256, 192 or 160 rows) for M rows routed to G groups and tiles_n columns of
-// tiles: the one whose rounds of tiles over the chip's blocks cost least, a tile counted as its rows plus what it costs
-// whatever its height (its weight panel, its fetching sides: 96 rows' worth by the Mixtral shape at 128 to 400 rows per
-// expert).  Routed groups scatter around their mean: a group of n ~ N(a, sqrt(a)) rows takes sum_j P(n > j * BM) tiles, so at
-// 128 rows per expert nearly all groups fit 160 rows (int8 first projection 0.283 -> 0.217 ms, on 256-row tiles 0.268), at
-// 160 they need 192 (0.280 -> 0.236), at 320 two of 192 (0.441 -> 0.361); a whole round more than another height needs can
-// decide the other way (Qwen3 shape at 128 rows: three rounds of 256-row tiles, 0.182 ms, against four of 160-row ones, 0.209).
+// tiles: the one whose rounds of tiles over the chip's blocks cost least.  Routed groups scatter around their mean: a group of
+// n ~ N(a, sqrt(a)) rows takes sum_j P(n > j * BM) tiles.  A tile costs its rows plus 96 (its weight panel, its fetching sides
+// and its stores, by the Mixtral shape at 2048 rows per expert: 54.7 / 44.7 / 40.0 us a round); where a group is about one
+// tile it is bound by its weights and costs no less than one of 200 rows.  A last round that is not full counts half of what
+// it leaves idle (the other blocks run at a higher clock then), in full where weights are the bound.
+// At 128 rows per expert nearly all groups fit 160 rows (int8 first projection 0.283 -> 0.217 ms; on 256-row tiles 0.268), at
+// 160 they need 192 (0.280 -> 0.236), at 320 two of 192 (0.441 -> 0.361); at 2048 the second projection takes 4.25 rounds of
+// 256-row tiles (0.862 ms) rather than 5.6 of 192 (0.905); the Qwen3 shape at 128 rows three rounds of 256 (0.182 ms), not
+// four of 160 (0.209).
 static int stream_tile_rows(int M, int G, int tiles_n) {
   int cus = 0;
   if (device_cu_count(&cus) != MOE_OK) cus = 256;
@@ -211,7 +214,10 @@ static int stream_tile_rows(int M, int G, int tiles_n) {
   for (int bm : {256, 192, 160}) {
     double tiles = 0.0;
     for (int j = 0; j * bm < a + 4.0 * sd; j++) tiles += 0.5 * erfc((j * (double)bm - a) / (sd * 1.41421356));
-    const double cost = ceil(tiles * G * tiles_n / cus - 1e-3) * (bm + 96.0);
+    const double rounds = tiles * G * tiles_n / cus, whole = ceil(rounds - 1e-3);
+    const bool weight_bound = tiles < 1.5;
+    // (the lower one of two that weights bind)
+    const double cost = weight_bound ? whole * ((bm > 200 ? bm : 200 + 0.01 * bm) + 96.0) : 0.5 * (rounds + whole) * (bm + 96.0);
     if (bm == 256 || cost < best_cost) { best = bm; best_cost = cost; }
   }
   return best;
@@ -220,7 +226,9 @@ static int stream_tile_rows(int M, int G, int tiles_n) {
 // 64-row tiles there, 0.365 / 0.361 ms on the Mixtral shape, 5 % ahead on the Qwen3 one); past the LDS-streamed decode
 // kernel's range for 8-bit operands (at 56 rows fp8 0.212 -> 0.199 ms against the 128 x 128 kernel, int8 at 64 level with the
 // 128-row tiles and ahead from 128 on).
-constexpr long long STREAM_ROWS_LO_BF16 = 32, STREAM_ROWS_LO_8BIT = 49;
+// Block-scaled fp8: past the decode kernel's 14 rows (DeepSeek-V3 shape at 16 / 64 / 128 rows 1.46 -> 1.38, 1.58 -> 1.50, 2.14 ->
+// 1.68 ms against the 128 x 128 kernel).
+constexpr long long STREAM_ROWS_LO_BF16 = 32, STREAM_ROWS_LO_8BIT = 49, STREAM_ROWS_LO_F8B = 15;
 // enough tiles for at least half of the chip's CUs
 static bool stream_fills_chip(int M, int G, int N, bool glu) {
   return (long long)max_tiles_for(M, G, 256) * cdiv(N, glu ? 128 : 256) >= 128;
@@ -428,13 +436,9 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       return fail(MOE_ERR_INVALID_ARG, "gmm: fp8 block scales missing");
     if (K % 128 != 0) return fail(MOE_ERR_UNSUPPORTED, "gmm: fp8 needs K %% 128 == 0 (K=%d)", K);
     if ((long long)N * K >= (1LL << 31)) return fail(MOE_ERR_UNSUPPORTED, "gmm: fp8 needs N * K < 2^31");
-    // Up to 14 rows per expert on average (decode): the streaming kernel with 16-row tiles, one MFMA row tile per
-    // wave; a group with more rows simply gets several tiles, which are adjacent in the grid, run at the same time
-    // and share the group's weights through L2.  Beyond that the LDS-tiled kernel with 128 x 128 tiles (measured on
-    // 256 experts of 7168 x 2048: at 12 rows per expert 1.26 against 1.44 ms, at 16, where half of the experts need a
-    // second 16-row tile, 1.66 against 1.43 ms), and from 128 rows per expert on the persistent 256 x 256 stream (with
-    // groups of exactly 128 rows 1.94 against 1.70 ms, at 160 rows 2.05 against 2.54 ms; routed groups scatter around
-    // their mean, and those over 128 rows cost the 128 x 128 kernel a second tile).
+    // Up to 14 rows per expert on average (decode): the streaming kernels with 16-row tiles; a group with more rows simply gets
+    // several tiles, which run at the same time and share the group's weights through L2.  Beyond that the persistent stream
+    // where it takes the shape and fills the chip, the LDS-tiled kernel with 128 x 128 tiles otherwise.
     const bool few_rows = (long long)M <= 16LL * G;
     // decode sizes: the LDS-streamed persistent kernels where they take the shape, one for block-scaled operands, one for
     // per-row x per-channel scales (MOE_GMM_KERNEL_STREAM keeps the register-staged kernel)
@@ -457,7 +461,7 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
                                                      : kernel != MOE_GMM_KERNEL_STREAM;
     if (kernel > MOE_GMM_KERNEL_BIG) return fail(MOE_ERR_UNSUPPORTED, "gmm: kernel family %d does not take fp8 operands", kernel);
     // prefill-sized groups: the persistent 256 x 256 stream, where it takes the shape
-    const bool prefill = kernel == MOE_GMM_KERNEL_BIG || (kernel == MOE_GMM_KERNEL_AUTO && (long long)M >= (fp8_blocks ? 128LL : STREAM_ROWS_LO_8BIT) * G && stream_fills_chip(M, G, N, glu));
+    const bool prefill = kernel == MOE_GMM_KERNEL_BIG || (kernel == MOE_GMM_KERNEL_AUTO && (long long)M >= (fp8_blocks ? STREAM_ROWS_LO_F8B : STREAM_ROWS_LO_8BIT) * G && stream_fills_chip(M, G, N, glu));
     // scales in the epilogue only (per row / per tensor x per channel / per tensor): the int8 x int8 problem on another MFMA
     const bool stream_epi = !fp8_blocks && prefill && dls_takes(OP_F8, K, N, ro.row_idx ? ro.lhs_rows : 0);
     if (kn_fp8 && !stream_epi) return fail(MOE_ERR_UNSUPPORTED, "gmm: [G, K, N] fp8 weights run on the persistent 256 x 256 kernel only (no K-block scales)");
@@ -482,7 +486,8 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       const bool big = kernel == MOE_GMM_KERNEL_BIG;
       if (big && !fp8_blocks) return fail(MOE_ERR_UNSUPPORTED, "gmm: the 256 x 256 fp8 kernel takes block-scaled operands only");
       const bool stream = fp8_blocks && f8s_takes(K, N, M, ro.row_idx ? ro.lhs_rows : 0) && prefill;
-      map_tiles(big || stream ? 256 : 128);
+      const int stream_bm = stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256));
+      map_tiles(stream ? stream_bm : big ? 256 : 128);
       Fp8TiledParams P = {};
       TiledParams& q = P.base;
       q.lhs = (const uint8_t*)a->lhs; q.rhs = (const uint8_t*)a->rhs; q.rhs_up = (const uint8_t*)a->rhs_up;
@@ -497,7 +502,7 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
         q.rhs_scale = a->rhs_scale; q.rhs_up_scale = a->rhs_up_scale;
         q.rhs_scale_gstride = sp.rhs_gstride; q.rhs_scale_nstride = sp.rhs_nstride;
       }
-      if (stream) return launch_f8s(glu, P, M, G, s);
+      if (stream) return launch_f8s(glu, stream_bm, P, M, G, s);
       const bool vec4 = fp8_blocks && (K / 128) % 4 == 0 && ((uintptr_t)a->lhs_scale & 15) == 0;
       return launch_fp8_tiled(big, glu, vec4, P, M, G, s);
     }

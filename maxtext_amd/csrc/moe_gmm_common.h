@@ -651,7 +651,7 @@ bool dls_takes(int op, int K, int N, long long indexed_lhs_rows);
 bool dls_kn_takes(int op, int K, int N, long long indexed_lhs_rows);  // the same for [G, K, N] weights (bf16, fp8)
 // moe_gmm_f8s.hip: the same stream for block-scaled fp8 (1 x 128 activation scales, 128 x 128 weight scales)
 struct Fp8TiledParams;
-int launch_f8s(bool glu, const Fp8TiledParams& P, int M, int G_total, hipStream_t s);
+int launch_f8s(bool glu, int bm, const Fp8TiledParams& P, int M, int G_total, hipStream_t s);
 bool f8s_takes(int K, int N, long long M, long long indexed_lhs_rows);
 int prepare_f8s();
 int launch_dlw(int bsrc, bool glu, bool half, const TiledParams& p, int M, int G_total, hipStream_t s);

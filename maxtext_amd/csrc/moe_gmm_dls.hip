@@ -285,8 +285,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
     const int n_out0 = cur.n0 + (C::GLU ? wn * (C::WN / 2) : wn * C::WN);
     EpilogueScales<C::TM, NT_OUT, C::GLU> esc;
     auto stream_kt = [&](int s) { return s < nk ? s : (have_n ? s - nk : nk - 1); };
-    // Stage `it`, in four phases.  first: the stage's data and what the next one starts with landed before the tile began
-    // (no waits).  cross: the stream moves on to the next tile after the first phase.
+    // Stage `it`, in four phases.  first: the stage's data landed before the tile began.  cross: the stream moves on to the next tile after the first phase.
     auto stage_head = [&](int it, auto first_c) __attribute__((always_inline)) {
       using WA = typename std::conditional<decltype(first_c)::value, NOWAIT, W1>::type;
       // 1: both first halves; requests the last half of the next stage (its slot was read two phases ago)
@@ -300,7 +299,6 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
     auto stage_rest = [&](int it, auto first_c) __attribute__((always_inline)) {
       constexpr bool FIRST = decltype(first_c)::value;
       using WA = typename std::conditional<FIRST, NOWAIT, W2>::type;
-      using WB = typename std::conditional<FIRST, NOWAIT, W4>::type;
       // 2
       const int kt2 = stream_kt(it + 2);
       read_b(cb, 1);
@@ -316,7 +314,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
       multiply_end(1, 1);
       // 4
       issue_b(kt2, cb, 1);
-      fetch_end(WB{});
+      fetch_end(W4{});
       quadrant(first_c, 1, 0);
       multiply_end(1, 0);
       cb ^= 1;
@@ -341,8 +339,9 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     load_epilogue_scales<C::TM, NT_OUT, C::GLU, true, C::MI, 32>(esc, p, cur.info, wm * C::MI, n_out0, lane_e);
-    // everything requested so far lands here, ahead of the stores: the next tile's first stage need not count them
-    wait_vmcnt<0>();
+    // the next tile's stage 0 lands ahead of the stores, so that its phases need not count them (stage 1's three halves are
+    // waited for in that stage's last phase, the stores with them)
+    wait_vmcnt<6>();
     store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, C::TM, 32>(acc, esc, p, cur.info, wm * C::MI, n_out0, lane_e);
     if (!have_n) break;
     cur = nxt;

@@ -1,43 +1,43 @@
 // Grouped matmul: block-scaled fp8 (1 x 128 activation scales, 128 x 128 weight scales; the DeepSeek-V3 recipe) for many
-// rows per expert, on the persistent 256 x 256 stream of the int8 / bf16 prefill kernel.
+// rows per expert, on the persistent stream of the int8 / bf16 / fp8 prefill kernel (moe_gmm_dls.hip): tiles of 256, 192 or
+// 160 rows x 256 channels, operands global -> LDS by halves requested across tile boundaries, the two waves of a SIMD taking
+// turns fetching and multiplying.
 //
-// A stage is one 128-wide scale block: 128 bytes of K for 256 activation rows and 256 weight rows, global -> LDS without
-// passing through registers (buffer_load ... lds, 8 rows x 128 bytes per wave instruction, XOR-swizzled unpadded rows, two
-// buffers of 64 KB), requested two stages ahead of the MFMAs across tile boundaries.  8 waves as 2 x 4, each 128 rows x
-// 64 channels in 8 x 4 tiles of v_mfma_f32_16x16x128_f8f6f4: ONE instruction per tile and stage gives the block's
-// partial sum, which is multiplied by a_scale[row, kb] * w_scale[n / 128, kb] and added to the f32 result, exactly as the
-// reference's block-scaled product is defined.  With weights as the first MFMA operand a lane holds 4 channels of ONE row
-// per tile, so the factor is one register per row tile (two with GLU: gate and up have their own weight scales).
+// A stage is one 128-wide scale block.  ONE v_mfma_f32_16x16x128_f8f6f4 per 16 x 16 tile and stage gives the block's partial
+// sum, which is multiplied by a_scale[row, kb] * w_scale[n / 128, kb] and added to the f32 result, exactly as the reference's
+// block-scaled product is defined.  With weights as the first MFMA operand a lane holds 4 channels of ONE row per tile, so the
+// factor is one register per row tile.  Of a quadrant's partial sums the last four stay in registers past the multiplying
+// side and are added in the next fetching side: behind an MFMA of its own wave an addition would wait for it, behind the
+// neighbour's it costs nothing.
 //
-// Registers decide the schedule: a 16x16x128 operand fragment is 8 registers, so only 4 of a wave's 8 activation
-// fragments and its 4 weight fragments are live (64 registers beside the 128 accumulators).  A stage is multiplied in two
-// halves of 16 MFMAs: row tiles 0 .. 3 fragment by fragment (each reloaded with row tile + 4 right after its four MFMAs),
-// then row tiles 4 .. 7 weight fragment by weight fragment (each weight fragment reloaded with the next stage's right
-// after its four MFMAs, the activation fragments during the last four).  The stage barrier sits between the halves: by
-// then every fragment of the stage is in registers and its buffer takes the stage after next.
+// The activation scales of four stages (16 bytes a row) and the two weight-scale rows the tile needs travel like the
+// operands, into two small LDS buffers, ahead of every fourth stage's requests.
 //
-// The activation scales of four stages (256 rows x 16 bytes) and the two weight-scale rows the tile needs travel the same
-// way, into two small LDS buffers, so that nothing but LDS reads and the stream's own requests is ever waited for inside
-// the loop.
+// DeepSeek-V3 shape, 256 experts: at 128 rows each first projection 2.14 -> 1.68 ms, second 1.00 -> 0.90 (160-row tiles; one
+// mixed stream on 256-row tiles before), at 288 rows 3.79 -> 3.18 and 1.99 -> 1.64, at 574 rows 6.05 -> 5.45 and 2.88 -> 2.92
+// (sixteen stages a tile: the second projection is bound by what lies between its tiles).  Up to 128 rows the weights are the
+// bound: 7.5 GB of the first projection at 4.5 TB/s.
 
 #include "moe_gmm_common.h"
 
 namespace moe {
 
-template <bool GLU_>
+template <bool GLU_, int TM_>
 struct F8sCfg {
   static constexpr bool GLU = GLU_;
-  static constexpr int BM = 256, BN = 256, BKB = 128, MI = 16;
+  // row tile i of wave row wm: the tile's rows 32 i + 16 wm .. + 15 (moe_gmm_dls.hip)
+  static constexpr int TM = TM_, H1 = TM - 4;
+  static constexpr int BM = TM * 32, BN = 256, BKB = 128, MI = 16;
   static constexpr int WAVES_M = 2, WAVES_N = 4, NWAVES = 8, THREADS = NWAVES * kWave;
-  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / MI, TN = WN / MI, RING = 4;
-  static constexpr int A_STAGE = BM * BKB, STAGE = (BM + BN) * BKB;
-  static constexpr int A_IPW = BM / 8 / NWAVES, B_IPW = BN / 8 / NWAVES;  // requests per wave and stage: 4 + 4
-  // scales of four stages: 256 rows x 4 f32, then the two weight-scale rows (each lane of the request writes the same
-  // 16 bytes: 1 KB per row)
-  static constexpr int SC_A = BM * 16, SC_BYTES = SC_A + 2 * 1024, SC_OFF = 2 * STAGE;
+  static constexpr int WN = BN / WAVES_N, TN = WN / MI;
+  static constexpr int NA1 = H1 > 2 ? 2 : 1, A_IPW = 2 + NA1, B_IPW = BN / 8 / NWAVES;  // requests per wave and stage
+  static constexpr int A_ROWS = 128 + NA1 * 64, A_STAGE = A_ROWS * BKB, STAGE = A_STAGE + BN * BKB;
+  // scales of four stages: one row's four f32 per activation row, then the two weight-scale rows (each lane of the request
+  // writes the same 16 bytes: 1 KB per row)
+  static constexpr int SC_A = A_ROWS * 16, SC_BYTES = SC_A + 2 * 1024, SC_OFF = 2 * STAGE;
   static constexpr int LDS_BYTES = 2 * STAGE + 2 * SC_BYTES;
   static constexpr int OUT_BN = GLU ? BN / 2 : BN;
-  static_assert(TM == 8 && TN == 4 && 2 * RING == TM, "the two halves of a stage");
+  static_assert(TM == 8 || TM == 6 || TM == 5, "row tiles");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
   __device__ static __forceinline__ int swz(int row) { return (row >> 1) & 7; }
 };
@@ -49,6 +49,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_f8s_kernel(const Fp8TiledPa
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave % C::WAVES_M, wn = wave / C::WAVES_M;
+  const bool late = wave >= C::NWAVES / 2;  // the second wave of its SIMD
   const int N = p.N, K = p.K;
   const uint32_t row_bytes = (uint32_t)K;
   const int num_tiles = p.header[0];
@@ -61,31 +62,32 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_f8s_kernel(const Fp8TiledPa
   auto peek_from = [&](int id0) { return peek_tile<C::OUT_BN>(p, num_tiles, id0); };
   auto resolve = [&](Peek pk, Tile& t) { return resolve_tile<C::OUT_BN, C::THREADS>(p, num_tiles, pk, t, tid); };
 
-  // ---- the loading side of the stream ---------------------------------------------------------------------------
-  // request i of this wave covers rows (wave * 4 + i) * 8 .. + 7 of the tile's 256 activation (weight) rows, 128 bytes
-  // of each; the lane's 16 bytes: global chunk = LDS slot ^ swizzle of the row
-  auto lane_off = [&](int i, uint32_t row) {
-    const int r = (wave * C::A_IPW + i) * 8 + lane / 8;
-    return row * row_bytes + (uint32_t)(((lane % 8) ^ C::swz(r)) << 4);
+  // ---- the loading side of the stream: halves, rows and swizzle of moe_gmm_dls.hip ---------------------------------
+  // (wave_v: the wave number for lane offsets, in a vector register; the scalar one is for LDS addresses)
+  int wave_v = wave;
+  asm volatile("" : "+v"(wave_v));
+  auto a_req_row = [&](int i, int w) { return i < 2 ? w * 16 + i * 8 : 128 + w * 8 * C::NA1 + (i - 2) * 8; };
+  auto b_req_row = [&](int i, int w) {
+    return C::GLU ? (i / 2) * 128 + w * 16 + (i % 2) * 8 : (w / 2) * 64 + (i / 2) * 32 + (w % 2) * 16 + (i % 2) * 8;
   };
-  v4i a_desc, b_desc, s_desc, w_desc = {0, 0, 0, 0};
+  auto lane_off = [&](int req_row, uint32_t row) { return row * row_bytes + (uint32_t)(((lane % 8) ^ C::swz(req_row + lane / 8)) << 4); };
+  v4i a_desc, b_desc[C::GLU ? 2 : 1], s_desc, w_desc = {0, 0, 0, 0};
   uint32_t a_voff[C::A_IPW], b_voff[C::B_IPW], b_soff = 0, s_voff = 0, w_soff = 0;
   const uint32_t scale_row_bytes = (uint32_t)nk * 4;
+  constexpr int S_WAVES = (C::A_ROWS + 63) / 64;  // waves that request activation scales, 64 rows each
   auto set_a_sources = [&](const Tile& t) {
     if (p.ro.row_idx) {
       a_desc = buffer_desc(p.lhs, clamp_u32((size_t)p.ro.lhs_rows * row_bytes));
       s_desc = buffer_desc(P.a_scale, clamp_u32((size_t)p.ro.lhs_rows * scale_row_bytes));
-      int rows[C::A_IPW];
+      int rows[C::A_IPW + 1];
 #pragma unroll
-      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + (wave * C::A_IPW + i) * 8 + lane / 8, p.M - 1);
-      lhs_rows_of<C::A_IPW>(p.ro, rows);
+      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + a_req_row(i, wave_v) + lane / 8, p.M - 1);
+      rows[C::A_IPW] = min(t.info.row0 + wave_v * 64 + lane, p.M - 1);
+      lhs_rows_of<C::A_IPW + 1>(p.ro, rows);
+      // (rows past the tile's end: one row past the descriptor's, i.e. zeros without a request to memory)
 #pragma unroll
-      for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(i, (uint32_t)rows[i]);
-      if (wave < 4) {  // the scale rows of tile rows wave * 64 + lane
-        int srow[1] = {min(t.info.row0 + wave * 64 + lane, p.M - 1)};
-        lhs_rows_of<1>(p.ro, srow);
-        s_voff = (uint32_t)srow[0] * scale_row_bytes;
-      }
+      for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i, wave_v), (uint32_t)(a_req_row(i, wave_v) + lane / 8 < t.info.nrows ? rows[i] : p.ro.lhs_rows));
+      s_voff = (uint32_t)(wave_v * 64 + lane < t.info.nrows ? rows[C::A_IPW] : p.ro.lhs_rows) * scale_row_bytes;
     } else {
       a_desc = buffer_desc(p.lhs + (size_t)t.info.row0 * row_bytes, clamp_u32((size_t)t.info.nrows * row_bytes));
       s_desc = buffer_desc(P.a_scale + (size_t)t.info.row0 * nk, clamp_u32((size_t)t.info.nrows * scale_row_bytes));
@@ -93,37 +95,34 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_f8s_kernel(const Fp8TiledPa
   };
   if (!p.ro.row_idx) {
 #pragma unroll
-    for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(i, (uint32_t)((wave * C::A_IPW + i) * 8 + lane / 8));
-    s_voff = (uint32_t)(wave * 64 + lane) * scale_row_bytes;
+    for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i, wave_v), (uint32_t)(a_req_row(i, wave_v) + lane / 8));
+    s_voff = (uint32_t)(wave_v * 64 + lane) * scale_row_bytes;
   }
-  // weights: with GLU the upper 128 of the tile's 256 rows are the second projection's, whose requests come from waves 4 .. 7
-  const bool load_up = C::GLU && wave >= C::NWAVES / 2;
 #pragma unroll
-  for (int i = 0; i < C::B_IPW; i++) {
-    const int r = (wave * C::B_IPW + i) * 8 + lane / 8;
-    b_voff[i] = lane_off(i, (uint32_t)(C::GLU ? r % (C::BN / 2) : r));
-  }
+  for (int i = 0; i < C::B_IPW; i++) b_voff[i] = lane_off(b_req_row(i, wave_v), (uint32_t)((C::GLU ? b_req_row(i, wave_v) % 128 : b_req_row(i, wave_v)) + lane / 8));
   auto set_b_sources = [&](const Tile& t) {
-    b_desc = buffer_desc((load_up ? p.rhs_up : p.rhs) + (size_t)t.info.group * N * row_bytes, clamp_u32((size_t)N * row_bytes));
+    b_desc[0] = buffer_desc(p.rhs + (size_t)t.info.group * N * row_bytes, clamp_u32((size_t)N * row_bytes));
+    if constexpr (C::GLU) b_desc[1] = buffer_desc(p.rhs_up + (size_t)t.info.group * N * row_bytes, clamp_u32((size_t)N * row_bytes));
     b_soff = (uint32_t)t.n0 * row_bytes;
     // the tile's two weight-scale rows: gate and up of its 128 channels, or its two blocks of 128 channels; waves 4 and 5
     // request one each
-    if (wave == 4 || wave == 5) {
-      const int sel = wave - 4;
-      const float* base = C::GLU && sel ? P.u_scale : P.w_scale;
-      const int nb = C::GLU ? t.n0 / 128 : min(t.n0 / 128 + sel, nnb - 1);
-      w_desc = buffer_desc(base, 0xffffffffu);
-      w_soff = (uint32_t)(((size_t)t.info.group * nnb + nb) * scale_row_bytes);
-    }
+    const int sel = wave == 5 ? 1 : 0;
+    const int nb = C::GLU ? t.n0 / 128 : min(t.n0 / 128 + sel, nnb - 1);
+    w_desc = buffer_desc(C::GLU && sel ? P.u_scale : P.w_scale, 0xffffffffu);
+    w_soff = (uint32_t)(((size_t)t.info.group * nnb + nb) * scale_row_bytes);
   };
-  // request idx of the stage: 0 .. 3 activations, 4 .. 7 weights
-  auto issue_one = [&](int kt, int buf, int idx) {
-    if (idx < C::A_IPW) dma16_buffer(a_desc, a_voff[idx], (uint32_t)kt * C::BKB, lds_base + buf * C::STAGE + (wave * C::A_IPW + idx) * 1024);
-    else dma16_buffer(b_desc, b_voff[idx - C::A_IPW], b_soff + (uint32_t)kt * C::BKB, lds_base + buf * C::STAGE + C::A_STAGE + (wave * C::B_IPW + idx - C::A_IPW) * 1024);
+  auto issue_a = [&](int kt, int buf, int h) {
+#pragma unroll
+    for (int i = 2 * h; i < (h ? C::A_IPW : 2); i++)
+      dma16_buffer(a_desc, a_voff[i], (uint32_t)kt * C::BKB, lds_base + buf * C::STAGE + a_req_row(i, wave) * C::BKB);
+  };
+  auto issue_b = [&](int kt, int buf, int g) {
+#pragma unroll
+    for (int i = 2 * g; i < 2 * g + 2; i++)
+      dma16_buffer(b_desc[C::GLU ? g : 0], b_voff[i], b_soff + (uint32_t)kt * C::BKB, lds_base + buf * C::STAGE + C::A_STAGE + b_req_row(i, wave) * C::BKB);
   };
   // the scales of stages 4 * chunk .. + 3 into scale buffer sb
   auto issue_scales = [&](int chunk, int sb) {
-    const uint32_t dst = lds_base + C::SC_OFF + sb * C::SC_BYTES;
     // one request with operands chosen per wave (two requests in the arms of a branch get merged by the compiler into
     // one whose scalar operands it can no longer keep in scalar registers)
     const bool is_w = wave >= 4;
@@ -131,149 +130,108 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_f8s_kernel(const Fp8TiledPa
 #pragma unroll
     for (int c = 0; c < 4; c++) d[c] = __builtin_amdgcn_readfirstlane(is_w ? w_desc[c] : s_desc[c]);
     const uint32_t so = (uint32_t)__builtin_amdgcn_readfirstlane((int)((is_w ? w_soff : 0u) + (uint32_t)chunk * 16));
+    const uint32_t dst = lds_base + C::SC_OFF + sb * C::SC_BYTES;
     const uint32_t la = (uint32_t)__builtin_amdgcn_readfirstlane((int)(dst + (is_w ? C::SC_A + (wave - 4) * 1024 : wave * 1024)));
-    if (wave < 6) dma16_buffer(d, is_w ? 0u : s_voff, so, la);
+    if (wave < S_WAVES || wave == 4 || wave == 5) dma16_buffer(d, is_w ? 0u : s_voff, so, la);
   };
 
   // ---- the multiplying side ----------------------------------------------------------------------------------------
-  v4f acc[C::TN][C::TM];
-  int b_row[C::TN];
-#pragma unroll
-  for (int j = 0; j < C::TN; j++) {
-    if (C::GLU) {
-      constexpr int H = C::TN / 2;
-      b_row[j] = (j < H ? 0 : C::BN / 2) + wn * (C::WN / 2) + (j < H ? j : j - H) * C::MI;
-    } else {
-      b_row[j] = wn * C::WN + j * C::MI;
-    }
-  }
-  // which of the two weight-scale rows a weight fragment takes
-  constexpr int NSEL = C::GLU ? 2 : 1;
-  auto sel_of = [&](int j) { return C::GLU ? (j >= C::TN / 2 ? 1 : 0) : 0; };
-  const int w_row_off = C::GLU ? 0 : (wn >= 2 ? 1024 : 0);
+  using T_ = std::true_type;
+  using F_ = std::false_type;
+  constexpr int NT_OUT = C::GLU ? C::TN / 2 : C::TN, HN = C::TN / 2;
+  auto row_tiles = [](int h) { return h ? C::H1 : 4; };
+  const int b_base = C::A_STAGE + (C::GLU ? wn * (C::WN / 2) : wn * C::WN) * C::BKB;
+  auto b_tile = [&](int j) { return (C::GLU ? (j / HN) * (C::BN / 2) + (j % HN) * C::MI : j * C::MI) * C::BKB; };
   // fragment: row (lane % 16), K bytes 16 q .. and 64 + 16 q .. with q = lane / 16 (both operands alike), i.e. the 16-byte
   // chunks q and 4 + q of the row, stored at slot chunk ^ swz(row)
   const int frag_lane = (lane % 16) * C::BKB + (((lane / 16) ^ C::swz(lane % 16)) << 4);
-  v8i ga[C::RING], gb[C::TN];
-  auto read_frag = [&](v8i& f, const uint8_t* base) {
-    const v4i lo = *(const v4i*)(base + frag_lane), hi = *(const v4i*)(base + (frag_lane ^ 64));
+  v4f acc[C::TN][C::TM];
+  v8i fa[4], fb[2][HN];
+  auto read_frag = [&](v8i& f, const uint8_t* src) {
+    const v4i lo = *(const v4i*)(src + frag_lane), hi = *(const v4i*)(src + (frag_lane ^ 64));
     f[0] = lo[0]; f[1] = lo[1]; f[2] = lo[2]; f[3] = lo[3];
     f[4] = hi[0]; f[5] = hi[1]; f[6] = hi[2]; f[7] = hi[3];
   };
-  auto read_a = [&](int buf, int i, int slot) { read_frag(ga[slot], smem + buf * C::STAGE + (wm * C::WM + i * 16) * C::BKB); };
-  auto read_b = [&](int buf, int j) { read_frag(gb[j], smem + buf * C::STAGE + C::A_STAGE + b_row[j] * C::BKB); };
-  // factors of the current stage per row tile: s_lo for row tiles 0 .. 3, s_hi for 4 .. 7
-  float s_lo[NSEL][C::RING], s_hi[NSEL][C::RING];
-  float a_raw[C::RING], w_raw[NSEL];
-  const int scale_lane = (wm * C::WM + lane % 16) * 16;
-  auto read_scales = [&](int sb, int col, int half) {
-    const uint8_t* base = smem + C::SC_OFF + sb * C::SC_BYTES;
+  auto read_a = [&](int buf, int h) {
 #pragma unroll
-    for (int ii = 0; ii < C::RING; ii++) a_raw[ii] = *(const float*)(base + scale_lane + (half * C::RING + ii) * 256 + col * 4);
-#pragma unroll
-    for (int s = 0; s < NSEL; s++) w_raw[s] = *(const float*)(base + C::SC_A + w_row_off + s * 1024 + col * 4);
+    for (int i = 0; i < row_tiles(h); i++) read_frag(fa[i], smem + buf * C::STAGE + ((h * 4 + i) * 32 + wm * 16) * C::BKB);
   };
-  auto set_factors = [&](float (&dst)[NSEL][C::RING]) {
+  auto read_b = [&](int buf, int g) {
 #pragma unroll
-    for (int s = 0; s < NSEL; s++)
-#pragma unroll
-      for (int ii = 0; ii < C::RING; ii++) dst[s][ii] = a_raw[ii] * w_raw[s];
+    for (int jj = 0; jj < HN; jj++) read_frag(fb[g][jj], smem + buf * C::STAGE + b_base + b_tile(g * HN + jj));
   };
-  v4f pq[2];  // partial sums of the last two MFMAs
-  const v4f zero = {0.f, 0.f, 0.f, 0.f};
-  // (the empty asm statements pin a result to its place in the instruction stream: an MFMA whose sum is only used a slot
-  // later and the FMAs that use it are otherwise placed wherever the instruction selector likes, which is not between
-  // the requests and reads they are meant to overlap)
-  auto add_scaled = [&](v4f& a, const v4f& part, float f) {
+  // scales: the row tiles' of half h in a_sc, the weights' in w_sc (GLU: one per projection); the factors of a quadrant
+  constexpr int NSEL = C::GLU ? 2 : 1;
+  float a_sc[4], w_sc[NSEL], f[4];
+  const int scale_lane = (wm * C::MI + lane % 16) * 16;
+  const int w_row_off = C::GLU ? 0 : (wn >= 2 ? 1024 : 0);
+  auto read_a_scales = [&](int sb, int col, int h) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) a[r] = fmaf(part[r], f, a[r]);
+    for (int i = 0; i < row_tiles(h); i++) a_sc[i] = *(const float*)(smem + C::SC_OFF + sb * C::SC_BYTES + scale_lane + (h * 4 + i) * 512 + col * 4);
+  };
+  auto read_w_scales = [&](int sb, int col) {
+#pragma unroll
+    for (int x = 0; x < NSEL; x++) w_sc[x] = *(const float*)(smem + C::SC_OFF + sb * C::SC_BYTES + C::SC_A + w_row_off + x * 1024 + col * 4);
+  };
+  auto set_factors = [&](int h, int g) {
+#pragma unroll
+    for (int i = 0; i < row_tiles(h); i++) f[i] = a_sc[i] * w_sc[C::GLU ? g : 0];
+  };
+  v4f pq[4];  // partial sums on their way into acc
+  auto add = [&](auto zc_c, int h, int g, int t) __attribute__((always_inline)) {
+    v4f& a = acc[g * HN + t % HN][h * 4 + t / HN];
+#pragma unroll
+    for (int r = 0; r < 4; r++) a[r] = decltype(zc_c)::value ? pq[t % 4][r] * f[t / HN] : fmaf(pq[t % 4][r], f[t / HN], a[r]);
     asm volatile("" : "+v"(a));
   };
-  // slot t: the MFMA goes out first, then the FMAs of the slot before it
-  auto mfma = [&](int t, const v8i& w, const v8i& x) {
-    pq[t % 2] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, zero, 0, 0, 0, 127, 0, 127);
-    asm volatile("" : "+v"(pq[0]), "+v"(pq[1]));
-  };
-  using T_ = std::true_type;
-  using F_ = std::false_type;
-
-  // First half of a stage (in buffer buf): row tiles 0 .. 3 from the ring, each slot reloaded with row tile + 4; the
-  // factors of row tiles 4 .. 7 are read (scale buffer sb, column col).  PEND: the partial sum of the MFMA before this
-  // half (weight fragment 3, row tile 7) is still to be added.
-  auto half_lo = [&](auto pend_c, int buf, int sb, int col) {
-    constexpr bool PEND = decltype(pend_c)::value;
+  // products of quadrant (h, g): row tiles 4h .. x channel tiles 2g, 2g + 1; the last four partial sums are left to drain()
+  auto quadrant = [&](auto zc_c, int h, int g) __attribute__((always_inline)) {
+    const int nt = row_tiles(h) * HN;
 #pragma unroll
-    for (int t = 0; t < 16; t++) {
-      const int i = t / 4, j = t % 4;
-      mfma(t, gb[j], ga[i]);
-      if (t == 0) {
-        if (PEND) add_scaled(acc[3][7], pq[1], s_hi[sel_of(3)][3]);
-        read_scales(sb, col, 1);
-      } else {
-        add_scaled(acc[(t - 1) % 4][(t - 1) / 4], pq[(t - 1) % 2], s_lo[sel_of((t - 1) % 4)][(t - 1) / 4]);
-      }
-      if (t == 2) set_factors(s_hi);
-      if (j == 3) read_a(buf, i + C::RING, i);
+    for (int t = 0; t < nt; t++) {
+      if (t >= 4) add(zc_c, h, g, t - 4);
+      pq[t % 4] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[g][t % HN], fa[t / HN], v4f{}, 0, 0, 0, 127, 0, 127);
+      asm volatile("" : "+v"(pq[t % 4]));
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // Second half of a stage: row tiles 4 .. 7 (in the ring), weight fragment by weight fragment.  RD: the next stage
-  // (buffer rd_buf) is prepared behind it: its weight fragments, its row tiles 0 .. 3 and the factors of those (scale
-  // buffer sb, column col).  LD: the eight requests of stage ld_kt go out into ld_buf, then the scales of chunk
-  // sc_chunk into scale buffer sc_sb (sc_chunk < 0: none).
-  auto half_hi = [&](auto rd_c, int rd_buf, int sb, int col, int ld_kt, int ld_buf, int sc_chunk, int sc_sb) {
-    constexpr bool RD = decltype(rd_c)::value;
+  auto drain = [&](auto zc_c, int h, int g) __attribute__((always_inline)) {
+    const int nt = row_tiles(h) * HN;
 #pragma unroll
-    for (int t = 0; t < 16; t++) {
-      const int j = t / 4, i = C::RING + t % 4;
-      mfma(t, gb[j], ga[t % 4]);
-      if (t == 0) {
-        add_scaled(acc[3][3], pq[1], s_lo[sel_of(3)][3]);
-        if (RD) read_scales(sb, col, 0);
-      } else {
-        add_scaled(acc[(t - 1) / 4][C::RING + (t - 1) % 4], pq[(t - 1) % 2], s_hi[sel_of((t - 1) / 4)][(t - 1) % 4]);
-      }
-      if (RD && t == 2) set_factors(s_lo);
-      if (t < C::A_IPW + C::B_IPW) issue_one(ld_kt, ld_buf, t);
-      if (t == C::A_IPW + C::B_IPW && sc_chunk >= 0) issue_scales(sc_chunk, sc_sb);
-      if (RD && t % 4 == 3) read_b(rd_buf, j);
-      if (RD && j == 3) read_a(rd_buf, t % 4, t % 4);
-      (void)i;
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int t = nt > 4 ? nt - 4 : 0; t < nt; t++) add(zc_c, h, g, t);
   };
-  constexpr int NT_OUT = C::GLU ? C::TN / 2 : C::TN;
-
-  // What a tile's first half stage needs, with nothing to hide behind: zeroed sums, row tiles 0 .. 3 and the weight
-  // fragments of stage 0 (buffer buf), the factors of row tiles 0 .. 3 (scale buffer sb, column 0).
-  auto first_fragments = [&](int buf, int sb) {
-#pragma unroll
-    for (int j = 0; j < C::TN; j++)
-#pragma unroll
-      for (int i = 0; i < C::TM; i++) acc[j][i] = zero;
-    read_scales(sb, 0, 0);
-#pragma unroll
-    for (int i = 0; i < C::RING; i++) read_a(buf, i, i);
-#pragma unroll
-    for (int j = 0; j < C::TN; j++) read_b(buf, j);
-    set_factors(s_lo);
+  auto fetch_end = [&](auto wait_c, int h, int g) __attribute__((always_inline)) {
+    constexpr int WAIT = decltype(wait_c)::value;
+    if constexpr (WAIT >= 0) wait_vmcnt<WAIT>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    set_factors(h, g);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
   };
+  auto multiply_end = [&]() {
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+  };
+  using NOWAIT = std::integral_constant<int, -1>;
+  // requests that may be outstanding where a phase ends ahead of new data (moe_gmm_dls.hip; a scale request among them only
+  // makes a wait stricter)
+  using W1 = std::integral_constant<int, 6 + 2 * C::NA1>;
+  using W2 = std::integral_constant<int, 8 + C::NA1>;
 
   Tile cur, nxt;
   if (!resolve(peek_from(blockIdx.x), cur)) return;
-  // ---- head of the stream: the first tile's stages 0 and 1 and its first scales ----
+  // ---- head of the stream: the first tile's stage 0, stage 1 up to the half that its first phase requests, its first scales
   set_a_sources(cur);
   set_b_sources(cur);
-#pragma unroll
-  for (int s = 0; s < 2; s++)
-#pragma unroll
-    for (int i = 0; i < C::A_IPW + C::B_IPW; i++) issue_one(s, s, i);
   issue_scales(0, 0);
+  issue_a(0, 0, 0); issue_b(0, 0, 0); issue_b(0, 0, 1); issue_a(0, 0, 1);
+  issue_a(1, 1, 0); issue_b(1, 1, 0); issue_b(1, 1, 1);
   wait_vmcnt<0>();
   asm volatile("s_barrier" ::: "memory");
-  first_fragments(0, 0);
 
-  int base = 0;   // the buffer that holds stage 0 of the current tile
+  int cb = 0;     // buffer of the current stage
   int sbase = 0;  // the scale buffer that holds the current tile's stages 0 .. 3
   const int nchunk = nk / 4;
   while (true) {
@@ -281,57 +239,83 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_f8s_kernel(const Fp8TiledPa
     Peek pk = peek_from(cur.id + gridDim.x);
     bool have_n = false;
     const int n_out0 = cur.n0 + (C::GLU ? wn * (C::WN / 2) : wn * C::WN);
-    // first half of stage 0
-    half_lo(F_{}, base, sbase, 0);
-    // Iteration `it`: the second half of stage it, then the first half of stage it + 1.  Every fragment of stage it is in
-    // registers before the barrier, and stage it + 1 has landed at it: the buffer of stage it takes stage it + 2 of the
-    // stream (from nk on: the next tile's); every fourth iteration the scales of the four stages from it + 2 on follow.
     auto stream_kt = [&](int s) { return s < nk ? s : (have_n ? s - nk : nk - 1); };
-    int cb = base;  // buffer of stage `it`
-    auto iteration = [&](int it, auto last_c) {
-      constexpr bool LAST = decltype(last_c)::value;  // the tile's last half stage: nothing is prepared behind it
-      // own fragment reads done, own requests landed: then everybody's
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-      wait_vmcnt<0>();
-      asm volatile("s_barrier" ::: "memory");
-      const int s2 = it + 2;
-      int sc_chunk = -1, sc_sb = 0;
-      if (s2 % 4 == 0) {
-        if (s2 < nk) {
-          sc_chunk = s2 / 4;
-          sc_sb = (sbase + sc_chunk) & 1;
-        } else if (have_n) {
-          sc_chunk = 0;
-          sc_sb = (sbase + nchunk) & 1;
-        }
+    // The phases of moe_gmm_dls.hip; each begins with what the phase before it left in pq.  pend: whether that one belongs to
+    // this tile, and to its first stage.
+    auto stage_head = [&](int it, auto first_c, auto pend_c, auto pend_first_c) __attribute__((always_inline)) {
+      using WA = typename std::conditional<decltype(first_c)::value, NOWAIT, W1>::type;
+      const int sb = (sbase + it / 4) & 1, col = it % 4;
+      read_b(cb, 0);
+      read_a(cb, 0);
+      if constexpr (decltype(pend_c)::value) drain(pend_first_c, 1, 0);
+      read_a_scales(sb, col, 0);
+      read_w_scales(sb, col);
+      issue_a(stream_kt(it + 1), cb ^ 1, 1);
+      fetch_end(WA{}, 0, 0);
+      quadrant(first_c, 0, 0);
+      multiply_end();
+    };
+    auto stage_rest = [&](int it, auto first_c) __attribute__((always_inline)) {
+      constexpr bool FIRST = decltype(first_c)::value;
+      using WA = typename std::conditional<FIRST, NOWAIT, W2>::type;
+      const int kt2 = stream_kt(it + 2), sb = (sbase + it / 4) & 1, col = it % 4;
+      // 2
+      read_b(cb, 1);
+      drain(first_c, 0, 0);
+      if ((it + 2) % 4 == 0) {  // the scales of the four stages from it + 2 on, or of the next tile's first four
+        if (it + 2 < nk) issue_scales((it + 2) / 4, (sbase + (it + 2) / 4) & 1);
+        else if (have_n) issue_scales(0, (sbase + nchunk) & 1);
       }
-      const int s1 = it + 1;  // the stage prepared behind this half
-      if (LAST) {
-        half_hi(F_{}, 0, 0, 0, stream_kt(s2), cb, sc_chunk, sc_sb);
-      } else {
-        half_hi(T_{}, cb ^ 1, (sbase + s1 / 4) & 1, s1 % 4, stream_kt(s2), cb, sc_chunk, sc_sb);
-        half_lo(T_{}, cb ^ 1, (sbase + s1 / 4) & 1, s1 % 4);
-      }
+      issue_a(kt2, cb, 0);
+      fetch_end(WA{}, 0, 1);
+      quadrant(first_c, 0, 1);
+      multiply_end();
+      // 3
+      read_a(cb, 1);
+      drain(first_c, 0, 1);
+      read_a_scales(sb, col, 1);
+      issue_b(kt2, cb, 0);
+      fetch_end(NOWAIT{}, 1, 1);
+      quadrant(first_c, 1, 1);
+      multiply_end();
+      // 4
+      drain(first_c, 1, 1);
+      issue_b(kt2, cb, 1);
+      fetch_end(W2{}, 1, 0);
+      quadrant(first_c, 1, 0);
+      multiply_end();
       cb ^= 1;
     };
-    for (int it = 0; it < nk - 2; it++) iteration(it, F_{});
+    if (late) asm volatile("s_barrier" ::: "memory");
+    stage_head(0, T_{}, F_{}, F_{});
+    stage_rest(0, T_{});
+    stage_head(1, F_{}, T_{}, T_{});
+    stage_rest(1, F_{});
+    for (int it = 2; it < nk - 2; it++) {
+      stage_head(it, F_{}, T_{}, F_{});
+      stage_rest(it, F_{});
+    }
+    stage_head(nk - 2, F_{}, T_{}, F_{});
     // the stream crosses into the next tile
     have_n = resolve(pk, nxt);
     if (have_n) {
       set_a_sources(nxt);
       set_b_sources(nxt);
     }
-    iteration(nk - 2, F_{});
-    iteration(nk - 1, T_{});
-    add_scaled(acc[3][7], pq[1], s_hi[sel_of(3)][3]);
+    stage_rest(nk - 2, F_{});
+    stage_head(nk - 1, F_{}, T_{}, F_{});
+    stage_rest(nk - 1, F_{});
+    if (!late) asm volatile("s_barrier" ::: "memory");
+    drain(F_{}, 1, 0);
     EpilogueScales<C::TM, NT_OUT, C::GLU> esc;
-    load_epilogue_scales<C::TM, NT_OUT, C::GLU, false, C::MI>(esc, p, cur.info, wm * C::WM, n_out0, lane);
-    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU>(acc, esc, p, cur.info, wm * C::WM, n_out0, lane);
+    load_epilogue_scales<C::TM, NT_OUT, C::GLU, false, C::MI, 32>(esc, p, cur.info, wm * C::MI, n_out0, lane);
+    // the next tile's stage 0 lands ahead of the stores, so that its phases need not count them (stage 1's three halves are
+    // waited for in that stage's last phase, the stores with them)
+    wait_vmcnt<6>();
+    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, C::TM, 32>(acc, esc, p, cur.info, wm * C::MI, n_out0, lane);
     if (!have_n) break;
     cur = nxt;
-    base = cb;  // the buffer of stage nk = the next tile's stage 0, landed before the last barrier
     sbase = (sbase + nchunk) & 1;
-    first_fragments(base, sbase);
   }
   // nothing may still be writing LDS when the block ends
   __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -348,8 +332,12 @@ static int prepare_f8s_cfg() {
 }
 
 int prepare_f8s() {
-  int st = prepare_f8s_cfg<F8sCfg<false>>();
-  if (!st) st = prepare_f8s_cfg<F8sCfg<true>>();
+  int st = prepare_f8s_cfg<F8sCfg<false, 5>>();
+  if (!st) st = prepare_f8s_cfg<F8sCfg<true, 5>>();
+  if (!st) st = prepare_f8s_cfg<F8sCfg<false, 6>>();
+  if (!st) st = prepare_f8s_cfg<F8sCfg<true, 6>>();
+  if (!st) st = prepare_f8s_cfg<F8sCfg<false, 8>>();
+  if (!st) st = prepare_f8s_cfg<F8sCfg<true, 8>>();
   return st;
 }
 
@@ -385,11 +373,14 @@ bool f8s_takes(int K, int N, long long M, long long indexed_lhs_rows) {
   return K % 512 == 0 && K >= 512 && ((long long)N + 256) * K < (1LL << 32) && (rows + 256) * K < (1LL << 32);
 }
 
-int launch_f8s(bool glu, const Fp8TiledParams& P, int M, int G_total, hipStream_t s) {
+int launch_f8s(bool glu, int bm, const Fp8TiledParams& P, int M, int G_total, hipStream_t s) {
   const TiledParams& p = P.base;
   if (!P.a_scale || !P.w_scale || !f8s_takes(p.K, p.N, M, p.ro.row_idx ? p.ro.lhs_rows : 0))
     return fail(MOE_ERR_UNSUPPORTED, "gmm: the fp8 stream kernel needs block scales, K a multiple of 512 and 32-bit byte offsets");
-  return glu ? launch_f8s_cfg<F8sCfg<true>>(P, M, G_total, s) : launch_f8s_cfg<F8sCfg<false>>(P, M, G_total, s);
+  if (bm == 160) return glu ? launch_f8s_cfg<F8sCfg<true, 5>>(P, M, G_total, s) : launch_f8s_cfg<F8sCfg<false, 5>>(P, M, G_total, s);
+  if (bm == 192) return glu ? launch_f8s_cfg<F8sCfg<true, 6>>(P, M, G_total, s) : launch_f8s_cfg<F8sCfg<false, 6>>(P, M, G_total, s);
+  if (bm != 256) return fail(MOE_ERR_INVALID_ARG, "gmm: the fp8 stream kernel has no tiles of %d rows", bm);
+  return glu ? launch_f8s_cfg<F8sCfg<true, 8>>(P, M, G_total, s) : launch_f8s_cfg<F8sCfg<false, 8>>(P, M, G_total, s);
 }
 
 }  // namespace moe

@@ -404,8 +404,9 @@ __global__ __launch_bounds__(kTdThreads, 2) void tgmm_dl_kernel(const TgmmParams
     float sc[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) sc[i] = p.n_scale ? p.n_scale[t.n0 + wn * 128 + i * 16 + s16] : 1.0f;
-    // everything requested so far lands here, ahead of the stores: the next tile's first stage need not count them
-    wait_vmcnt<0>();
+    // the next tile's stage 0 lands ahead of the stores, so that its phases need not count them (stage 1's three halves are
+    // waited for in that stage's last phase, the stores with them)
+    wait_vmcnt<6>();
     if (!p.out_f32 && !p.existing) {
       // plain bf16 results: neighbouring k-tiles trade halves between lanes 16 apart, so that a lane stores 16 bytes and
       // the 64 bytes of a row n leave in one instruction
@@ -506,7 +507,7 @@ __global__ __launch_bounds__(kTdThreads, 2) void tgmm_dl_kernel(const TgmmParams
 #pragma unroll
         for (int f = 0; f < 4; f++) read_n(cb, 1, 4 + f, f);
         issue(true, cb, 1);
-        fetch_end(W{});
+        fetch_end(WAIT{});
         multiply(F_{}, 4, 0);
         multiply_end();
       }

@@ -426,13 +426,13 @@ STREAM_TILE_GROUPS = {
 
 
 @pytest.mark.parametrize("height,n", [(160, 1032), (192, 8200)])
-@pytest.mark.parametrize("kind", ["int8", "bf16", "fp8"])
+@pytest.mark.parametrize("kind", ["int8", "bf16", "fp8", "fp8_blocks"])
 @pytest.mark.parametrize("glu", [False, True])
 def test_gmm_stream_tile_heights(K, height, n, kind, glu):
   """The persistent stream kernel on its lower tiles: against the register-staged kernel (int8: the sums are integers, so bit
   for bit) with rows read through an index, a bias and rows that belong to no group."""
   gs = np.array(STREAM_TILE_GROUPS[height], np.int32)
-  m, k = int(gs.sum()) + 40, 384
+  m, k = int(gs.sum()) + 40, 512 if kind == "fp8_blocks" else 384
   g = torch.Generator().manual_seed(height)
   idx = torch.randperm(m, generator=g).to(torch.int32)
   kw = dict(lhs_row_idx=cuda(idx), rhs_bias=cuda(torch.randn(16, n, generator=g)))
@@ -443,12 +443,16 @@ def test_gmm_stream_tile_heights(K, height, n, kind, glu):
   else:
     mk = lambda *s: torch.randn(*s, generator=g).to(torch.float8_e4m3fn)
   lhs, w = mk(m, k), mk(16, n, k)
+  scales = lambda *s: cuda(torch.rand(*s, generator=g) * 0.02)
+  rhs_scales = (lambda: scales(16, -(-n // 128), k // 128)) if kind == "fp8_blocks" else lambda: scales(16, n)
   if kind != "bf16":
-    kw.update(lhs_scale=cuda(torch.rand(m, generator=g) * 0.02), rhs_scale=cuda(torch.rand(16, n, generator=g) * 0.02))
+    kw.update(lhs_scale=scales(m, k // 128) if kind == "fp8_blocks" else scales(m), rhs_scale=rhs_scales())
+  if kind == "fp8_blocks":
+    kw.update(lhs_scale_block_k=128, rhs_scale_block_n=128, rhs_scale_block_k=128)
   if glu:
     kw.update(rhs_up=cuda(mk(16, n, k)), act="silu")
     if kind != "bf16":
-      kw["rhs_up_scale"] = cuda(torch.rand(16, n, generator=g) * 0.02)
+      kw["rhs_up_scale"] = rhs_scales()
   got = K.gmm_raw(cuda(lhs), cuda(w), cuda(gs), **kw)
   want = K.gmm_raw(cuda(lhs), cuda(w), cuda(gs), kernel="tiled", **kw)
   assert torch.all(got[int(gs.sum()):] == 0)
