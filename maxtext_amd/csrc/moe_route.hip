@@ -619,7 +619,7 @@ __global__ void invert_perm_kernel(const int32_t* __restrict__ perm, int M,
 // ---------------------------------------------------------------------------------------
 
 constexpr int kGqThreads = 256;
-constexpr int kGqMaxChunks = 8;  // 16-byte chunks per thread -> d <= 256*8*8
+constexpr int kGqMaxChunks = 8;  // 16-byte chunks per thread -> d <= 256*8*8; the kernels hold 1, 2, 4 or 8
 
 enum { GQ_COPY = 0, GQ_INT8 = 1, GQ_FP8 = 2 };
 
@@ -689,11 +689,39 @@ __device__ __forceinline__ float quant_value(float f, float sc, float inv, int r
     if (fabsf(__builtin_amdgcn_fractf(q) - 0.5f) < 1e-4f || !(fabsf(q) < 200.0f)) q = sc == 0.f ? 0.f : f / sc;
     return fminf(fmaxf(rintf(q), -qmax), qmax);
   }
-  const float q = sc == 0.f ? 0.f : f / sc;
+  // The correctly rounded quotient in five operations instead of a division's dozen: inv is the rounded reciprocal, the
+  // first correction brings the estimate within an ulp, and from there one exact residual and one fma round correctly
+  // (Markstein's theorem).  Nothing in it may overflow, or lose bits below the normal range that e4m3 could see; scales
+  // outside [2^-80, 2^80] (0 and infinity among them) divide.
+  float q;
+  if (sc >= 0x1p-80f && sc <= 0x1p80f) {
+    const float est = f * inv;
+    q = fmaf(fmaf(-est, sc, f), inv, est);
+    q = fmaf(fmaf(-q, sc, f), inv, q);
+    q = fabsf(est) < 1024.0f ? q : est;  // (beyond the range by far: a static scale; the residual may overflow there)
+  } else {
+    q = sc == 0.f ? 0.f : f / sc;
+  }
   return fminf(fmaxf(q, -qmax), qmax);
 }
 
-template <int MODE>
+// Largest of the lane's value and those of the lanes that share its K block (16, 32 or 64 consecutive lanes).
+__device__ __forceinline__ float block_max(float m, int lanes) {
+  const auto step = [&](auto ctrl) {
+    m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), decltype(ctrl)::value, 0xf, 0xf, false)));
+  };
+  step(std::integral_constant<int, 0xb1>{});   // lane ^ 1
+  step(std::integral_constant<int, 0x4e>{});   // lane ^ 2
+  step(std::integral_constant<int, 0x141>{});  // 7 - lane of each 8
+  step(std::integral_constant<int, 0x140>{});  // 15 - lane of each 16
+  for (int o = 16; o < lanes; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+  return m;
+}
+
+// CH: 16-byte chunks per thread, the least of 1, 2, 4, 8 that covers the row.  Bound by HBM; the work per value counts too:
+// with eight chunks' worth of block maxima, divisions and predicates for every row, the e4m3 blocks of a 36891 x 2048
+// activation took 174 us, 50 (4.6 TB/s) with what the row needs and the division above.
+template <int MODE, int CH>
 __global__ __launch_bounds__(kGqThreads) void gather_rows_kernel(
     const uint4* __restrict__ x, const int32_t* __restrict__ row_idx, int idx_div, int R_in, int d,
     void* __restrict__ out, float* __restrict__ scale, const QuantCfg qc) {
@@ -706,16 +734,16 @@ __global__ __launch_bounds__(kGqThreads) void gather_rows_kernel(
   bool in_range = src >= 0 && src < R_in;
   if (qc.row_range) in_range = in_range && r >= qc.row_range[0] && r < qc.row_range[1];
   const uint4* xrow = x + (size_t)(in_range ? src : 0) * nch;
-  uint4 regs[kGqMaxChunks];
+  uint4 regs[CH];
 #pragma unroll
-  for (int c = 0; c < kGqMaxChunks; c++) {
+  for (int c = 0; c < CH; c++) {
     int ci = threadIdx.x + c * kGqThreads;
     regs[c] = ci < nch && in_range ? xrow[ci] : make_uint4(0, 0, 0, 0);
   }
   if (qc.row_weight) {  // x[indices] * weights[:, None] (ragged_gather.py:316-319), product rounded to bf16
     const float w = qc.row_weight[r];
 #pragma unroll
-    for (int c = 0; c < kGqMaxChunks; c++) {
+    for (int c = 0; c < CH; c++) {
       float f[8];
       unpack8(regs[c], f);
       regs[c] = make_uint4(pack_bf16x2(f[0] * w, f[1] * w), pack_bf16x2(f[2] * w, f[3] * w), pack_bf16x2(f[4] * w, f[5] * w),
@@ -726,7 +754,7 @@ __global__ __launch_bounds__(kGqThreads) void gather_rows_kernel(
   if (MODE == GQ_COPY) {
     uint4* orow = (uint4*)out + (size_t)r * nch;
 #pragma unroll
-    for (int c = 0; c < kGqMaxChunks; c++) {
+    for (int c = 0; c < CH; c++) {
       int ci = threadIdx.x + c * kGqThreads;
       if (ci < nch) orow[ci] = regs[c];
     }
@@ -743,7 +771,7 @@ __global__ __launch_bounds__(kGqThreads) void gather_rows_kernel(
   } else if (qc.block_lanes == 0) {
     float m = 0.f;
 #pragma unroll
-    for (int c = 0; c < kGqMaxChunks; c++) m = fmaxf(m, absmax8(regs[c]));
+    for (int c = 0; c < CH; c++) m = fmaxf(m, absmax8(regs[c]));
     m = wave_max(m);
     if (threadIdx.x % kWave == 0) s_red[threadIdx.x / kWave] = m;
     __syncthreads();
@@ -753,13 +781,12 @@ __global__ __launch_bounds__(kGqThreads) void gather_rows_kernel(
   }
   uint2* orow = (uint2*)out + (size_t)r * nch;
 #pragma unroll
-  for (int c = 0; c < kGqMaxChunks; c++) {
+  for (int c = 0; c < CH; c++) {
     int ci = threadIdx.x + c * kGqThreads;
     float sc = row_sc, inv = row_inv;
     if (!is_static && qc.block_lanes != 0) {
       // a K block is block_lanes consecutive 16-byte chunks == consecutive lanes of one wave
-      float m = absmax8(regs[c]);
-      for (int o = qc.block_lanes / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+      const float m = block_max(absmax8(regs[c]), qc.block_lanes);
       quant_scale<MODE>(m, qc.rule, sc, inv);
       if (ci < nch && (threadIdx.x & (qc.block_lanes - 1)) == 0) scale[(size_t)r * qc.nkb + ci / qc.block_lanes] = sc;
     }
@@ -955,6 +982,19 @@ __global__ __launch_bounds__(256) void transpose_kernel(const T* __restrict__ in
   }
   __syncthreads();
   for (int i = ty; i < 64; i += 4) {
+template <int MODE>
+static void launch_gather_rows(const uint4* x, const int32_t* row_idx, int idx_div, int R_in, int R_out, int d, void* out, float* scale, const QuantCfg& qc,
+                               hipStream_t s) {
+  const auto go = [&](auto ch) {
+    gather_rows_kernel<MODE, decltype(ch)::value><<<R_out, kGqThreads, 0, s>>>(x, row_idx, idx_div, R_in, d, out, scale, qc);
+  };
+  const int ch = cdiv(d / 8, kGqThreads);
+  if (ch <= 1) go(std::integral_constant<int, 1>{});
+  else if (ch <= 2) go(std::integral_constant<int, 2>{});
+  else if (ch <= 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, kGqMaxChunks>{});
+}
+
     int nn = n0 + i, kk = k0 + tx;
     if (kk < K && nn < N) out[(g * N + nn) * K + kk] = tile[tx][i];
   }
@@ -1256,7 +1296,7 @@ int moe_gather_rows(const void* x, const int32_t* row_idx, int idx_div, int R_in
   QuantCfg qc;
   qc.rule = rule; qc.block_lanes = 0; qc.nkb = 1; qc.static_scale = nullptr; qc.row_weight = row_weight; qc.row_range = row_range;
   if (out_dtype == MOE_BF16) {
-    gather_rows_kernel<GQ_COPY><<<R_out, kGqThreads, 0, s>>>(xs, row_idx, idx_div, R_in, d, out, scale, qc);
+    launch_gather_rows<GQ_COPY>(xs, row_idx, idx_div, R_in, R_out, d, out, scale, qc, s);
     return check_launch("gather_rows_kernel");
   }
   if (out_dtype != MOE_INT8 && out_dtype != MOE_FP8_E4M3) return fail(MOE_ERR_UNSUPPORTED, "gather: out_dtype %d", out_dtype);
@@ -1270,9 +1310,9 @@ int moe_gather_rows(const void* x, const int32_t* row_idx, int idx_div, int R_in
     qc.nkb = block_k ? cdiv(d, block_k) : 1;
   }
   if (out_dtype == MOE_INT8)
-    gather_rows_kernel<GQ_INT8><<<R_out, kGqThreads, 0, s>>>(xs, row_idx, idx_div, R_in, d, out, scale, qc);
+    launch_gather_rows<GQ_INT8>(xs, row_idx, idx_div, R_in, R_out, d, out, scale, qc, s);
   else
-    gather_rows_kernel<GQ_FP8><<<R_out, kGqThreads, 0, s>>>(xs, row_idx, idx_div, R_in, d, out, scale, qc);
+    launch_gather_rows<GQ_FP8>(xs, row_idx, idx_div, R_in, R_out, d, out, scale, qc, s);
   return check_launch("gather_rows_kernel");
 }
 

@@ -212,6 +212,21 @@ def _v2_inputs(d, seed):
     x[4] = 0
     x[4, :4] = torch.tensor([1.0, 0.703125, 0.99609375, -0.99609375])
     x[6] = 0
+@pytest.mark.parametrize("d", [2040, 2048, 2056, 4096, 4104, 8192, 8200])
+@pytest.mark.parametrize("block_k", [0, 128, 256, 512])
+def test_gather_rows_fp8_at_chunk_edges_and_extreme_scales(K, d, block_k):
+  """Rows just within and just past what 1, 2, 4 and 8 chunks per thread hold; magnitudes from subnormal to the largest."""
+  g = torch.Generator().manual_seed(d + block_k)
+  x = (torch.randn(24, d, generator=g) * torch.logspace(-38, 37, 24)[:, None]).to(torch.bfloat16)
+  x[7] = 0
+  q, s = K.gather_rows(cuda(x), None, 1, out_dtype=torch.float8_e4m3fn, block_k=block_k)
+  width = block_k or d
+  pad = torch.nn.functional.pad(x, (0, -d % width))
+  oq, os_ = O.quantize_fp8_blocks(pad, 1, width)
+  assert torch.equal(s.cpu().reshape(os_.shape), os_)
+  assert torch.equal(q.cpu().view(torch.uint8), oq[:, :d].contiguous().view(torch.uint8))
+
+
     x[6, :3] = torch.tensor([1.5, 1.4921875, 0.75])
   return x
 
