@@ -8,6 +8,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
+
 #include "moe_gmm_common.h"
 
 namespace moe {
@@ -369,6 +371,125 @@ __global__ __launch_bounds__(kSortWaves* kWave) void sort_scan_kernel(int32_t* _
                                                                      int32_t* __restrict__ group_sizes) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int e = blockIdx.x * kSortWaves + wave;
+// The same product for calls whose 32 x 32 tiles alone fill the chip.  There the kernel above is bound by its loads: x is
+// read once per 32 experts, and a wave's load instruction touches 64 rows for 16 bytes each.  Here a block owns TT tokens
+// and NE experts, stages of 64 values of K arrive as whole 128-byte lines by LDS copies, two stages ahead (72 or 96 KB of
+// LDS), and TT / 32 x 2 waves hold 32 tokens x NE / 2 experts each.  The 16-byte slot of row r is stored at
+// slot ^ (r / 2 % 8): 16 rows read at one slot cover all banks.  K is summed in the four quarters that the four waves
+// above take, and these are added in the same order, so the logits are bit for bit the same; with gridDim.z == 4 a block
+// sums one quarter and the routing kernel adds the four.  Bound by the latency of what a CU has in flight.
+// With the routing kernel, T x d x E: 4099 x 7168 x 256 178 -> 54 us, 1024 x 7168 x 256 49 -> 25 us, 16384 x 2048 x 128
+// 106 -> 48 us, 1100 x 2048 x 128 21 -> 14 us.
+template <int S, int NE, int TT_>
+struct GateWide {
+  static constexpr int TT = TT_;                     // tokens
+  static constexpr int NW = TT / 16;                 // waves
+  static constexpr int ROWS = TT + S * NE;           // staged rows of 128 bytes
+  static constexpr int STAGE = ROWS * 128;           // bytes
+  static constexpr int NST = 3;
+  static constexpr int ND = ROWS / (8 * NW);         // copies per wave and stage (8 rows each)
+  static constexpr int NT = NE / 64;                 // 32-expert tiles per wave
+  static constexpr int LDS = NST * STAGE;
+};
+
+template <int S, int NE, int TT>
+__global__ __launch_bounds__(TT * 4) void gate_gemm_wide_kernel(const GateGemmParams p) {
+  using C = GateWide<S, NE, TT>;
+  __shared__ __attribute__((aligned(128))) uint8_t lds[C::LDS];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int r = lane % 32, g = lane / 32;
+  const int wt = wave / 2, we = wave % 2;
+  const int t0 = blockIdx.x * C::TT, e0 = blockIdx.y * NE;
+  const int nchunks = p.d / 64;
+  const int quarter = (nchunks + 3) / 4;
+  const int c_begin = min(nchunks, (int)blockIdx.z * quarter);
+  const int c_end = gridDim.z == 1 ? nchunks : min(nchunks, c_begin + quarter);
+  const int n = c_end - c_begin;
+
+  // copy i of this wave fetches rows (i * NW + wave) * 8 .. + 7 of the stage: the tokens, then the terms' experts
+  const uint8_t* src[C::ND];
+#pragma unroll
+  for (int i = 0; i < C::ND; i++) {
+    const int row = (i * C::NW + wave) * 8 + lane / 8;
+    const int slot = (lane % 8) ^ ((row >> 1) & 7);
+    const int er = row - C::TT;
+    const uint16_t* base = row < C::TT ? p.x + (size_t)min(t0 + row, p.T - 1) * p.d
+                                       : p.wg + ((size_t)(er / NE) * p.E + min(e0 + er % NE, p.E - 1)) * p.d;
+    src[i] = (const uint8_t*)base + (size_t)c_begin * 128 + slot * 16;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
+  auto issue = [&](int c) {  // stage c of the block's range
+    const uint32_t dst = lds0 + (c % C::NST) * C::STAGE + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < C::ND; i++) dma16_untracked(src[i] + (size_t)c * 128, dst + i * (C::NW * 1024));
+  };
+
+  v16f acc[S][C::NT], sum[C::NT];
+#pragma unroll
+  for (int j = 0; j < C::NT; j++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      sum[j][i] = 0.f;
+#pragma unroll
+      for (int s = 0; s < S; s++) acc[s][j][i] = 0.f;
+    }
+
+  for (int c = 0; c < C::NST - 1 && c < n; c++) issue(c);
+  const int swz = (r >> 1) & 7;  // (every fragment's rows start at a multiple of 16)
+  int until = quarter;           // stages left of this quarter
+  for (int c = 0; c < n; c++) {
+    // stage c has landed when only the requests of the stages behind it are outstanding
+    if (c + C::NST - 2 < n) wait_vmcnt<(C::NST - 2) * C::ND>();
+    else wait_vmcnt<0>();
+    __syncthreads();  // everyone's part of stage c is there, and stage c - 1's buffer has been read by all
+    if (c + C::NST - 1 < n) issue(c + C::NST - 1);
+    const uint8_t* st = lds + (c % C::NST) * C::STAGE;
+    const uint8_t* xs = st + (wt * 32 + r) * 128;
+    const uint8_t* ws = st + (C::TT + we * (NE / 2) + r) * 128;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int off = ((g * 4 + q) ^ swz) * 16;
+      const v8bf xv = *(const v8bf*)(xs + off);
+#pragma unroll
+      for (int s = 0; s < S; s++)
+#pragma unroll
+        for (int j = 0; j < C::NT; j++)
+          acc[s][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const v8bf*)(ws + (s * NE + j * 32) * 128 + off), xv, acc[s][j], 0, 0, 0);
+    }
+    if (--until == 0 || c + 1 == n) {
+      until = quarter;
+#pragma unroll
+      for (int j = 0; j < C::NT; j++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          float v = acc[S - 1][j][i];  // smallest term first
+#pragma unroll
+          for (int s = S - 2; s >= 0; s--) v += acc[s][j][i];
+          sum[j][i] += v;
+#pragma unroll
+          for (int s = 0; s < S; s++) acc[s][j][i] = 0.f;
+        }
+    }
+  }
+
+  const int t = t0 + wt * 32 + r;
+  if (t >= p.T) return;
+  float* out = p.partial + ((size_t)blockIdx.z * p.T + t) * p.E;
+#pragma unroll
+  for (int j = 0; j < C::NT; j++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int e = e0 + we * (NE / 2) + j * 32 + 8 * q + 4 * g;
+      if (e < p.E) *(float4*)(out + e) = make_float4(sum[j][4 * q], sum[j][4 * q + 1], sum[j][4 * q + 2], sum[j][4 * q + 3]);
+    }
+}
+
+template <int S, int NE, int TT>
+static void launch_gate_wide(const GateGemmParams& p, int ks, hipStream_t s) {
+  gate_gemm_wide_kernel<S, NE, TT><<<dim3(cdiv(p.T, TT), cdiv(p.E, NE), ks), TT * 4, 0, s>>>(p);
+}
+
   if (e >= E) return;
   int running = 0;
   for (int s0 = 0; s0 < nseg; s0 += kWave) {
@@ -1105,18 +1226,25 @@ int moe_route_topk(const float* gate_logits, const float* pre_bias_logits, int T
   return check_launch("route_topk_kernel");
 }
 
-static int gate_k_splits(int T, int d, int E) {
+// How the gate product is cut.  Below 129 tiles of 32 tokens x 32 experts the chip is filled by splitting K (at least 8
+// chunks of 64, 2 per wave, in a block).  From there on, with more than 32 experts, the wide kernel: with up to 32 the
+// narrow one reads x once as well and is bound by that.
+struct GatePlan {
+  int ks;      // partial sums per logit
+  int tt, ne;  // tile of the wide kernel, 0: the narrow one
+};
+static GatePlan gate_plan(int T, int d, int E, int S) {
   const int tiles = cdiv(T, 32) * cdiv(E, 32), nchunks = d / 64;
   int ks = 256 / tiles;
   ks = ks < 1 ? 1 : ks;
-  const int cap = nchunks / 8 < 1 ? 1 : nchunks / 8;  // at least 8 chunks (2 per wave) per block
+  const int cap = nchunks / 8 < 1 ? 1 : nchunks / 8;
   ks = ks > cap ? cap : ks;
-  return ks > 16 ? 16 : ks;
+  return {ks > 16 ? 16 : ks, 0, 0};
 }
 
 size_t moe_gate_route_workspace_bytes(int T, int d, int E) {
   if (T < 0 || d <= 0 || E <= 0) return 0;
-  return (size_t)gate_k_splits(T, d, E) * T * E * sizeof(float) + 16;
+  return (size_t)std::max(gate_plan(T, d, E, 1).ks, gate_plan(T, d, E, 3).ks) * T * E * sizeof(float) + 16;
 }
 
 int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, const float* gate_bias, int T, int d,
@@ -1141,15 +1269,23 @@ int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, 
   if (((uintptr_t)x | (uintptr_t)gate_kernel_terms | (uintptr_t)workspace) & 15) return fail(MOE_ERR_UNSUPPORTED, "gate_route: pointers must be 16-byte aligned");
   if (T == 0) return MOE_OK;
   hipStream_t s = (hipStream_t)stream;
-  const int ks = gate_k_splits(T, d, E);
+  const GatePlan plan = gate_plan(T, d, E, num_terms);
+  const int ks = plan.ks;
   GateGemmParams gp;
   gp.x = (const uint16_t*)x; gp.wg = (const uint16_t*)gate_kernel_terms; gp.partial = (float*)workspace;
   gp.T = T; gp.d = d; gp.E = E; gp.S = num_terms; gp.chunks_per_block = cdiv(d / 64, ks);
-  dim3 grid(cdiv(T, 32), cdiv(E, 32), ks);
-  if (num_terms == 3)
-    gate_gemm_kernel<3><<<grid, 256, 0, s>>>(gp);
-  else
-    gate_gemm_kernel<1><<<grid, 256, 0, s>>>(gp);
+  if (plan.tt) {
+    if (num_terms == 3) launch_gate_wide<3, 64, 64>(gp, ks, s);
+    else if (plan.tt == 128) launch_gate_wide<1, 128, 128>(gp, ks, s);
+    else if (plan.ne == 128) launch_gate_wide<1, 128, 64>(gp, ks, s);
+    else launch_gate_wide<1, 64, 64>(gp, ks, s);
+  } else {
+    const dim3 grid(cdiv(T, 32), cdiv(E, 32), ks);
+    if (num_terms == 3)
+      gate_gemm_kernel<3><<<grid, 256, 0, s>>>(gp);
+    else
+      gate_gemm_kernel<1><<<grid, 256, 0, s>>>(gp);
+  }
   GateEpilogue ge;
   ge.partials = (const float*)workspace; ge.bias = gate_bias; ge.logits_out = gate_logits_out; ge.pre_bias_out = pre_bias_logits_out;
   ge.num_partials = ks; ge.score_func = score_func; ge.round_bf16 = gate_round_bf16;
@@ -1159,6 +1295,14 @@ int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, 
   return check_launch("gate_route");
 }
 
+  if (ks <= 1 && E > 32) {
+    // Large tiles load less, small ones and a quarter of K per block load from more CUs at once; a CU takes in no more
+    // than what it can have in flight.  Whole-K blocks once there is one for every CU.
+    if (S == 3) return {cdiv(T, 64) * cdiv(E, 64) < 256 ? 4 : 1, 64, 64};
+    if (cdiv(T, 64) * cdiv(E, 128) >= 256) return {1, 64, 128};
+    if (cdiv(T, 128) * cdiv(E, 128) * 4 >= 192) return {4, 128, 128};
+    return {4, 64, 64};
+  }
 size_t moe_sort_workspace_bytes(int T, int k, int E) {
   if (T < 0 || k <= 0 || E <= 0) return 0;
   size_t M = (size_t)T * k;

@@ -1250,6 +1250,22 @@ def test_gate_route_exact_on_integers(K):
   t, d, e, k = 513, 1024, 64, 6
   x = torch.from_numpy(rng.integers(-4, 5, (t, d)).astype(np.float32)).to(torch.bfloat16)
   wg = torch.from_numpy(rng.integers(-8, 9, (d, e)).astype(np.float32)) / 16.0
+# one shape for each tile of the wide kernel, with ragged tokens, experts and K quarters (empty ones too), and the last
+# shape that still takes the narrow kernel; k and E cover one to eight scores per lane of the top-k
+@pytest.mark.parametrize("t,d,e,k,terms", [(1100, 320, 132, 8, 1), (3073, 64, 260, 5, 1), (8200, 448, 132, 3, 1), (2049, 192, 68, 2, 3),
+                                           (4099, 128, 252, 8, 3), (2048, 320, 64, 16, 1), (4099, 704, 36, 4, 1)])
+def test_gate_route_tiles_exact_on_integers(K, t, d, e, k, terms):
+  from maxtext_amd.quantizations import split_gate_kernel
+
+  rng = np.random.default_rng(t + e)
+  x = torch.from_numpy(rng.integers(-4, 5, (t, d)).astype(np.float32)).to(torch.bfloat16)
+  wg = torch.from_numpy(rng.integers(-8, 9, (d, e)).astype(np.float32)) / 16.0
+  _, idx, logits, _ = K.gate_route(cuda(x), cuda(split_gate_kernel(wg, terms)), k=k, return_logits=True)
+  want = x.float().numpy() @ wg.numpy()  # every partial sum is exact
+  np.testing.assert_array_equal(logits.cpu().numpy(), want)
+  np.testing.assert_array_equal(idx.cpu().numpy(), O.get_topk(want, k=k)[1])
+
+
   terms = split_gate_kernel(wg)
   assert torch.all(terms[1] == 0) and torch.all(terms[2] == 0)
   w, idx, logits, _ = K.gate_route(cuda(x), cuda(terms), k=k, norm_topk_prob=True, return_logits=True)
