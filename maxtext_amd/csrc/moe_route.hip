@@ -35,24 +35,53 @@ int check_launch(const char* what) {
 // ---------------------------------------------------------------------------------------
 
 constexpr int kRouteMaxE = 512;
-constexpr int kRouteVpl = kRouteMaxE / kWave;  // values per lane
 constexpr int kRouteWaves = 4;
 
-// (value, index) order of lax.top_k as adopted here: larger value first, lower index first.
-__device__ __forceinline__ bool better(float av, int ai, float bv, int bi) {
-  return av > bv || (av == bv && ai < bi);
+// Order of lax.top_k as adopted here: larger value first, lower index first.  Scores are compared as unsigned keys that
+// grow with the float (-0 as +0; NaN and scores already taken are 0, below every number).
+__device__ __forceinline__ uint32_t score_key(float v) {
+  const uint32_t b = __float_as_uint(v + 0.0f);  // -0 + 0 = +0
+  if ((b & 0x7fffffffu) > 0x7f800000u) return 0;
+  return b & 0x80000000u ? ~b : b | 0x80000000u;
+}
+__device__ __forceinline__ float key_score(uint32_t key) { return __uint_as_float(key & 0x80000000u ? key & 0x7fffffffu : ~key); }
+
+// Largest key of the wave, as a scalar: four steps inside rows of 16 lanes and two across them, all on the vector unit
+// (a shuffle through LDS costs ten times a step, and a top-8 is a chain of 8 x 6 of them).
+__device__ __forceinline__ uint32_t wave_max_key(uint32_t k) {
+  const auto step = [&](auto ctrl, auto rows) {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)k, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    k = k > o ? k : o;
+  };
+  using std::integral_constant;
+  step(integral_constant<int, 0xb1>{}, integral_constant<int, 0xf>{});   // lane ^ 1
+  step(integral_constant<int, 0x4e>{}, integral_constant<int, 0xf>{});   // lane ^ 2
+  step(integral_constant<int, 0x141>{}, integral_constant<int, 0xf>{});  // 7 - lane of each 8
+  step(integral_constant<int, 0x140>{}, integral_constant<int, 0xf>{});  // 15 - lane of each 16
+  step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // rows 0, 2 into rows 1, 3
+  step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row 1 into rows 2, 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)k, kWave - 1);
 }
 
-__device__ __forceinline__ void wave_argmax(float& bv, int& bi) {
+// Takes the best of the wave's scores away (key = 0) and returns its index, lane + 64 * j; -1 when only NaN is left.
+template <int N>
+__device__ __forceinline__ int take_best(uint32_t (&key)[N], int lane, uint32_t& best) {
+  uint32_t m = key[0];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o);
-    int oi = __shfl_xor(bi, o);
-    if (better(ov, oi, bv, bi)) {
-      bv = ov;
-      bi = oi;
+  for (int j = 1; j < N; j++) m = m > key[j] ? m : key[j];
+  best = wave_max_key(m);
+  if (best == 0) return -1;
+  int at = -1;
+#pragma unroll
+  for (int j = 0; j < N; j++) {
+    const unsigned long long hit = __ballot(key[j] == best);
+    if (at < 0 && hit) {
+      const int l = __builtin_ctzll(hit);
+      at = l + kWave * j;
+      if (lane == l) key[j] = 0;
     }
   }
+  return at;
 }
 
 // With GATE the scores are built here from the partial sums of the gate matmul (GateLogit.__call__,
@@ -70,8 +99,9 @@ struct GateEpilogue {
 };
 
 // One token per wave: token t_raw of T (a wave past the end repeats the last token and writes nothing; every wave of the
-// block must make the call, there is a block barrier inside).  s_row_w / s_pre_w: this wave's kRouteMaxE floats of LDS.
-template <bool GATE>
+// block must make the call, there is a block barrier inside).  s_row_w / s_pre_w: this wave's 64 * VPL floats of LDS.
+// VPL: scores per lane, at least E / 64.
+template <bool GATE, int VPL>
 __device__ __forceinline__ void route_token(
     const float* __restrict__ logits, const float* __restrict__ pre_bias, int T, int E, int k,
     int mode, int norm, int round_bf16, float scaling, int n_groups, int topk_groups,
@@ -80,16 +110,35 @@ __device__ __forceinline__ void route_token(
   const int t = active ? t_raw : T - 1;
   const float* row = logits + (size_t)t * E;
 
-  float v[kRouteVpl];
-  unsigned taken = 0;
+  float v[VPL];
+  if (GATE) {
+    // the partials are added in order, but fetched four at a time: one after the other they are a chain of memory latencies
 #pragma unroll
-  for (int j = 0; j < kRouteVpl; j++) {
+    for (int j = 0; j < VPL; j++) v[j] = 0.f;
+    for (int s0 = 0; s0 < g.num_partials; s0 += 4) {
+      float part[4][VPL];
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int j = 0; j < VPL; j++) {
+          const int e = lane + kWave * j;
+          part[s][j] = s0 + s < g.num_partials && e < E ? g.partials[((size_t)(s0 + s) * T + t) * E + e] : 0.f;
+        }
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        if (s0 + s < g.num_partials) {
+#pragma unroll
+          for (int j = 0; j < VPL; j++) v[j] += part[s][j];
+        }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < VPL; j++) {
     int e = lane + kWave * j;
     if (GATE) {
       float x = -INFINITY;
       if (e < E) {
-        x = 0.f;
-        for (int s = 0; s < g.num_partials; s++) x += g.partials[((size_t)s * T + t) * E + e];
+        x = v[j];
         if (g.round_bf16) x = round_bf16_fn(x);
         if (g.score_func == 1) x = 1.0f / (1.0f + expf(-x));
         // sqrt(softplus(x)), softplus as logaddexp(x, 0) = max(x, 0) + log1p(exp(-|x|)) (linears.py:51-53)
@@ -103,7 +152,6 @@ __device__ __forceinline__ void route_token(
     } else {
       v[j] = e < E ? row[e] : -INFINITY;
     }
-    if (e >= E) taken |= 1u << j;
   }
 
   if (n_groups > 0) {
@@ -111,17 +159,18 @@ __device__ __forceinline__ void route_token(
     // topk_groups groups, everything else becomes -inf (still selectable, as in jnp.where).
     const int gs = E / n_groups;
 #pragma unroll
-    for (int j = 0; j < kRouteVpl; j++) {
+    for (int j = 0; j < VPL; j++) {
       int e = lane + kWave * j;
       if (e < E) s_row_w[e] = v[j];
     }
     __syncthreads();
-    float score = -INFINITY;
-    int gi = INT_MAX;
-    if (lane < n_groups) {
-      float b1 = -INFINITY, b2 = -INFINITY;
-      for (int i = 0; i < gs; i++) {
-        float x = s_row_w[lane * gs + i];
+    // 2^share_bits lanes share a group, as many as fit the wave, each with every 2^share_bits-th score
+    const int share_bits = 31 - __builtin_clz(kWave / n_groups), share = 1 << share_bits;
+    const int grp = lane >> share_bits;
+    float b1 = -INFINITY, b2 = -INFINITY;
+    if (grp < n_groups) {
+      for (int i = lane & (share - 1); i < gs; i += share) {
+        float x = s_row_w[grp * gs + i];
         if (x > b1) {
           b2 = b1;
           b1 = x;
@@ -129,47 +178,38 @@ __device__ __forceinline__ void route_token(
           b2 = x;
         }
       }
-      score = b1 + b2;
-      gi = lane;
     }
+    for (int o = 1; o < share; o <<= 1) {
+      const float o1 = __shfl_xor(b1, o), o2 = __shfl_xor(b2, o);
+      b2 = fmaxf(fminf(b1, o1), fmaxf(b2, o2));
+      b1 = fmaxf(b1, o1);
+    }
+    uint32_t gkey[1] = {grp < n_groups && (lane & (share - 1)) == 0 ? score_key(b1 + b2) : 0u};
     unsigned long long sel = 0;
-    bool mine_taken = lane >= n_groups;
     for (int r = 0; r < topk_groups; r++) {
-      float bv = mine_taken ? -INFINITY : score;
-      int bi = mine_taken ? INT_MAX : gi;
-      wave_argmax(bv, bi);
-      if (bi < n_groups) sel |= 1ull << bi;
-      if (bi == lane) mine_taken = true;
+      uint32_t best;
+      const int l = take_best(gkey, lane, best);
+      if (l >= 0) sel |= 1ull << (l >> share_bits);
     }
 #pragma unroll
-    for (int j = 0; j < kRouteVpl; j++) {
+    for (int j = 0; j < VPL; j++) {
       int e = lane + kWave * j;
       if (e < E && !((sel >> (e / gs)) & 1ull)) v[j] = -INFINITY;
     }
   }
 
+  uint32_t key[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; j++) key[j] = lane + kWave * j < E ? score_key(v[j]) : 0u;
   float myv = 0.f;
   int myi = 0;
   for (int r = 0; r < k; r++) {
-    float bv = -INFINITY;
-    int bi = INT_MAX;
-#pragma unroll
-    for (int j = 0; j < kRouteVpl; j++) {
-      if (!((taken >> j) & 1u)) {
-        int e = lane + kWave * j;
-        if (better(v[j], e, bv, bi)) {
-          bv = v[j];
-          bi = e;
-        }
-      }
-    }
-    wave_argmax(bv, bi);
-    if (bi == INT_MAX) bi = 0;  // only reachable with NaN scores
+    uint32_t best;
+    const int at = take_best(key, lane, best);
     if (lane == r) {
-      myv = bv;
-      myi = bi;
+      myv = at < 0 ? -INFINITY : key_score(best);
+      myi = at < 0 ? 0 : at;  // (none left: only with NaN scores)
     }
-    if ((bi & (kWave - 1)) == lane) taken |= 1u << (bi >> 6);
   }
 
   float w;
@@ -191,7 +231,7 @@ __device__ __forceinline__ void route_token(
       // softmax over every expert (the best score is the first selected one), read at the selected experts
       float part = 0.f;
 #pragma unroll
-      for (int j = 0; j < kRouteVpl; j++)
+      for (int j = 0; j < VPL; j++)
         if (lane + kWave * j < E) part += expf(v[j] - mx);
       const float s = wave_sum(part);
       w = lane < k ? expf(myv - mx) / s : 0.f;
@@ -214,16 +254,25 @@ __device__ __forceinline__ void route_token(
   }
 }
 
-template <bool GATE>
+template <bool GATE, int VPL>
 __global__ __launch_bounds__(kRouteWaves* kWave) void route_topk_kernel(
     const float* __restrict__ logits, const float* __restrict__ pre_bias, int T, int E, int k,
     int mode, int norm, int round_bf16, float scaling, int n_groups, int topk_groups,
     float* __restrict__ w_out, int32_t* __restrict__ idx_out, const GateEpilogue g) {
-  __shared__ float s_row[kRouteWaves][kRouteMaxE];
-  __shared__ float s_pre[GATE ? kRouteWaves : 1][GATE ? kRouteMaxE : 1];
+  __shared__ float s_row[kRouteWaves][VPL * kWave];
+  __shared__ float s_pre[GATE ? kRouteWaves : 1][GATE ? VPL * kWave : 1];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  route_token<GATE>(logits, pre_bias, T, E, k, mode, norm, round_bf16, scaling, n_groups, topk_groups, w_out, idx_out, g,
-                    blockIdx.x * kRouteWaves + wave, lane, s_row[wave], s_pre[GATE ? wave : 0]);
+  route_token<GATE, VPL>(logits, pre_bias, T, E, k, mode, norm, round_bf16, scaling, n_groups, topk_groups, w_out, idx_out, g,
+                         blockIdx.x * kRouteWaves + wave, lane, s_row[wave], s_pre[GATE ? wave : 0]);
+}
+
+// Calls f(std::integral_constant<int, scores per lane>) for E experts.
+template <typename F>
+static void dispatch_vpl(int E, F&& f) {
+  if (E <= kWave) f(std::integral_constant<int, 1>{});
+  else if (E <= 2 * kWave) f(std::integral_constant<int, 2>{});
+  else if (E <= 4 * kWave) f(std::integral_constant<int, 4>{});
+  else f(std::integral_constant<int, kRouteMaxE / kWave>{});
 }
 
 // ---------------------------------------------------------------------------------------
@@ -322,55 +371,6 @@ __global__ __launch_bounds__(256) void gate_gemm_kernel(const GateGemmParams p) 
   }
 }
 
-// ---------------------------------------------------------------------------------------
-// Stable counting sort of the flattened expert ids.
-//   pass 1: per-wave-segment histograms; pass 2: exclusive scan over segments (one wave per expert);
-//   pass 3: each wave re-reads its segment and ranks equal ids with ballots, in index order.
-// ---------------------------------------------------------------------------------------
-
-constexpr int kSortWaves = 4;
-constexpr int kSortRounds = 4;
-constexpr int kSortSeg = kSortRounds * kWave;    // entries per wave
-constexpr int kSortChunk = kSortSeg * kSortWaves;  // entries per block
-constexpr int kSortMaxE = 512;
-
-__device__ __forceinline__ int clamp_expert(int e, int E) { return e < 0 ? 0 : (e >= E ? E - 1 : e); }
-// sort key of expert id e: (e - roll) mod E (permute's roll_to_expert_id, moe.py:953-954; roll = 0: the id itself)
-// the roll as given, or read from the device and taken mod E
-__device__ __forceinline__ int resolve_roll(int roll, const int32_t* roll_dev, int E) {
-  if (!roll_dev) return roll;
-  const int r = *roll_dev % E;
-  return r < 0 ? r + E : r;
-}
-__device__ __forceinline__ int sort_key(int e, int E, int roll) {
-  e = clamp_expert(e, E) - roll;
-  return e < 0 ? e + E : e;
-}
-
-__global__ __launch_bounds__(kSortWaves* kWave) void sort_hist_kernel(
-    const int32_t* __restrict__ flat, int M, int E, int roll, const int32_t* __restrict__ roll_dev, int32_t* __restrict__ seg_hist) {
-  roll = resolve_roll(roll, roll_dev, E);
-  __shared__ int cnt[kSortWaves][kSortMaxE];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  for (int e = lane; e < E; e += kWave) cnt[wave][e] = 0;
-  __syncthreads();
-  const int base = blockIdx.x * kSortChunk + wave * kSortSeg;
-#pragma unroll
-  for (int r = 0; r < kSortRounds; r++) {
-    int i = base + r * kWave + lane;
-    if (i < M) atomicAdd(&cnt[wave][sort_key(flat[i], E, roll)], 1);
-  }
-  __syncthreads();
-  int32_t* dst = seg_hist + (size_t)(blockIdx.x * kSortWaves + wave) * E;
-  for (int e = lane; e < E; e += kWave) dst[e] = cnt[wave][e];
-}
-
-// pass 2: one wave per expert turns its column of segment counts into exclusive prefixes (64 segments per step,
-// a shuffle scan inside the wave) and writes the expert's total to group_sizes.
-__global__ __launch_bounds__(kSortWaves* kWave) void sort_scan_kernel(int32_t* __restrict__ seg_hist, int nseg, int E,
-                                                                     int32_t* __restrict__ group_sizes) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int e = blockIdx.x * kSortWaves + wave;
 // The same product for calls whose 32 x 32 tiles alone fill the chip.  There the kernel above is bound by its loads: x is
 // read once per 32 experts, and a wave's load instruction touches 64 rows for 16 bytes each.  Here a block owns TT tokens
 // and NE experts, stages of 64 values of K arrive as whole 128-byte lines by LDS copies, two stages ahead (72 or 96 KB of
@@ -490,6 +490,55 @@ static void launch_gate_wide(const GateGemmParams& p, int ks, hipStream_t s) {
   gate_gemm_wide_kernel<S, NE, TT><<<dim3(cdiv(p.T, TT), cdiv(p.E, NE), ks), TT * 4, 0, s>>>(p);
 }
 
+// ---------------------------------------------------------------------------------------
+// Stable counting sort of the flattened expert ids.
+//   pass 1: per-wave-segment histograms; pass 2: exclusive scan over segments (one wave per expert);
+//   pass 3: each wave re-reads its segment and ranks equal ids with ballots, in index order.
+// ---------------------------------------------------------------------------------------
+
+constexpr int kSortWaves = 4;
+constexpr int kSortRounds = 4;
+constexpr int kSortSeg = kSortRounds * kWave;    // entries per wave
+constexpr int kSortChunk = kSortSeg * kSortWaves;  // entries per block
+constexpr int kSortMaxE = 512;
+
+__device__ __forceinline__ int clamp_expert(int e, int E) { return e < 0 ? 0 : (e >= E ? E - 1 : e); }
+// sort key of expert id e: (e - roll) mod E (permute's roll_to_expert_id, moe.py:953-954; roll = 0: the id itself)
+// the roll as given, or read from the device and taken mod E
+__device__ __forceinline__ int resolve_roll(int roll, const int32_t* roll_dev, int E) {
+  if (!roll_dev) return roll;
+  const int r = *roll_dev % E;
+  return r < 0 ? r + E : r;
+}
+__device__ __forceinline__ int sort_key(int e, int E, int roll) {
+  e = clamp_expert(e, E) - roll;
+  return e < 0 ? e + E : e;
+}
+
+__global__ __launch_bounds__(kSortWaves* kWave) void sort_hist_kernel(
+    const int32_t* __restrict__ flat, int M, int E, int roll, const int32_t* __restrict__ roll_dev, int32_t* __restrict__ seg_hist) {
+  roll = resolve_roll(roll, roll_dev, E);
+  __shared__ int cnt[kSortWaves][kSortMaxE];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  for (int e = lane; e < E; e += kWave) cnt[wave][e] = 0;
+  __syncthreads();
+  const int base = blockIdx.x * kSortChunk + wave * kSortSeg;
+#pragma unroll
+  for (int r = 0; r < kSortRounds; r++) {
+    int i = base + r * kWave + lane;
+    if (i < M) atomicAdd(&cnt[wave][sort_key(flat[i], E, roll)], 1);
+  }
+  __syncthreads();
+  int32_t* dst = seg_hist + (size_t)(blockIdx.x * kSortWaves + wave) * E;
+  for (int e = lane; e < E; e += kWave) dst[e] = cnt[wave][e];
+}
+
+// pass 2: one wave per expert turns its column of segment counts into exclusive prefixes (64 segments per step,
+// a shuffle scan inside the wave) and writes the expert's total to group_sizes.
+__global__ __launch_bounds__(kSortWaves* kWave) void sort_scan_kernel(int32_t* __restrict__ seg_hist, int nseg, int E,
+                                                                     int32_t* __restrict__ group_sizes) {
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int e = blockIdx.x * kSortWaves + wave;
   if (e >= E) return;
   int running = 0;
   for (int s0 = 0; s0 < nseg; s0 += kWave) {
@@ -713,13 +762,13 @@ struct RouteArgs {
   int32_t* idx_out;
 };
 
-template <int NW>
+template <int NW, int VPL>
 __global__ __launch_bounds__(NW* kWave) void route_sort_small_kernel(
     const RouteArgs r, int roll, int ebits, int32_t* __restrict__ group_sizes, int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm,
     int32_t* __restrict__ sorted_experts, const SortMapArgs mp) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   // (one token per wave, all at once: r.T <= NW, no routing groups)
-  route_token<false>(r.logits, r.pre_bias, r.T, r.E, r.k, r.mode, r.norm, r.round_bf16, r.scaling, 0, 0, r.w_out, r.idx_out, GateEpilogue{}, wave, lane,
+  route_token<false, VPL>(r.logits, r.pre_bias, r.T, r.E, r.k, r.mode, r.norm, r.round_bf16, r.scaling, 0, 0, r.w_out, r.idx_out, GateEpilogue{}, wave, lane,
                      nullptr, nullptr);
   __syncthreads();  // the indices, written above by this block, are read back from memory
   sort_small_block<NW>(r.idx_out, r.T * r.k, r.E, roll, nullptr, ebits, group_sizes, perm, inv_perm, sorted_experts, mp);
@@ -933,6 +982,19 @@ __global__ __launch_bounds__(kGqThreads) void gather_rows_kernel(
   }
 }
 
+template <int MODE>
+static void launch_gather_rows(const uint4* x, const int32_t* row_idx, int idx_div, int R_in, int R_out, int d, void* out, float* scale, const QuantCfg& qc,
+                               hipStream_t s) {
+  const auto go = [&](auto ch) {
+    gather_rows_kernel<MODE, decltype(ch)::value><<<R_out, kGqThreads, 0, s>>>(x, row_idx, idx_div, R_in, d, out, scale, qc);
+  };
+  const int ch = cdiv(d / 8, kGqThreads);
+  if (ch <= 1) go(std::integral_constant<int, 1>{});
+  else if (ch <= 2) go(std::integral_constant<int, 2>{});
+  else if (ch <= 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, kGqMaxChunks>{});
+}
+
 // ---------------------------------------------------------------------------------------
 // Unpermute + weighted combine: one block per token, f32 accumulation over the k rows.
 // ---------------------------------------------------------------------------------------
@@ -1103,19 +1165,6 @@ __global__ __launch_bounds__(256) void transpose_kernel(const T* __restrict__ in
   }
   __syncthreads();
   for (int i = ty; i < 64; i += 4) {
-template <int MODE>
-static void launch_gather_rows(const uint4* x, const int32_t* row_idx, int idx_div, int R_in, int R_out, int d, void* out, float* scale, const QuantCfg& qc,
-                               hipStream_t s) {
-  const auto go = [&](auto ch) {
-    gather_rows_kernel<MODE, decltype(ch)::value><<<R_out, kGqThreads, 0, s>>>(x, row_idx, idx_div, R_in, d, out, scale, qc);
-  };
-  const int ch = cdiv(d / 8, kGqThreads);
-  if (ch <= 1) go(std::integral_constant<int, 1>{});
-  else if (ch <= 2) go(std::integral_constant<int, 2>{});
-  else if (ch <= 4) go(std::integral_constant<int, 4>{});
-  else go(std::integral_constant<int, kGqMaxChunks>{});
-}
-
     int nn = n0 + i, kk = k0 + tx;
     if (kk < K && nn < N) out[(g * N + nn) * K + kk] = tile[tx][i];
   }
@@ -1220,9 +1269,11 @@ int moe_route_topk(const float* gate_logits, const float* pre_bias_logits, int T
       return fail(MOE_ERR_UNSUPPORTED, "route: bad routing groups %d/%d for E=%d", ng, topk_routing_group, E);
   }
   if (T == 0) return MOE_OK;
-  route_topk_kernel<false><<<cdiv(T, kRouteWaves), kRouteWaves * kWave, 0, (hipStream_t)stream>>>(
-      gate_logits, pre_bias_logits, T, E, k, mode, norm_topk_prob, weights_round_bf16,
-      routed_scaling_factor, ng, topk_routing_group, topk_weights, topk_idx, GateEpilogue{});
+  dispatch_vpl(E, [&](auto vpl) {
+    route_topk_kernel<false, decltype(vpl)::value><<<cdiv(T, kRouteWaves), kRouteWaves * kWave, 0, (hipStream_t)stream>>>(
+        gate_logits, pre_bias_logits, T, E, k, mode, norm_topk_prob, weights_round_bf16,
+        routed_scaling_factor, ng, topk_routing_group, topk_weights, topk_idx, GateEpilogue{});
+  });
   return check_launch("route_topk_kernel");
 }
 
@@ -1236,6 +1287,14 @@ struct GatePlan {
 static GatePlan gate_plan(int T, int d, int E, int S) {
   const int tiles = cdiv(T, 32) * cdiv(E, 32), nchunks = d / 64;
   int ks = 256 / tiles;
+  if (ks <= 1 && E > 32) {
+    // Large tiles load less, small ones and a quarter of K per block load from more CUs at once; a CU takes in no more
+    // than what it can have in flight.  Whole-K blocks once there is one for every CU.
+    if (S == 3) return {cdiv(T, 64) * cdiv(E, 64) < 256 ? 4 : 1, 64, 64};
+    if (cdiv(T, 64) * cdiv(E, 128) >= 256) return {1, 64, 128};
+    if (cdiv(T, 128) * cdiv(E, 128) * 4 >= 192) return {4, 128, 128};
+    return {4, 64, 64};
+  }
   ks = ks < 1 ? 1 : ks;
   const int cap = nchunks / 8 < 1 ? 1 : nchunks / 8;
   ks = ks > cap ? cap : ks;
@@ -1289,20 +1348,14 @@ int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, 
   GateEpilogue ge;
   ge.partials = (const float*)workspace; ge.bias = gate_bias; ge.logits_out = gate_logits_out; ge.pre_bias_out = pre_bias_logits_out;
   ge.num_partials = ks; ge.score_func = score_func; ge.round_bf16 = gate_round_bf16;
-  route_topk_kernel<true><<<cdiv(T, kRouteWaves), kRouteWaves * kWave, 0, s>>>(
-      nullptr, nullptr, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, ng, topk_routing_group,
-      topk_weights, topk_idx, ge);
+  dispatch_vpl(E, [&](auto vpl) {
+    route_topk_kernel<true, decltype(vpl)::value><<<cdiv(T, kRouteWaves), kRouteWaves * kWave, 0, s>>>(
+        nullptr, nullptr, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, ng, topk_routing_group,
+        topk_weights, topk_idx, ge);
+  });
   return check_launch("gate_route");
 }
 
-  if (ks <= 1 && E > 32) {
-    // Large tiles load less, small ones and a quarter of K per block load from more CUs at once; a CU takes in no more
-    // than what it can have in flight.  Whole-K blocks once there is one for every CU.
-    if (S == 3) return {cdiv(T, 64) * cdiv(E, 64) < 256 ? 4 : 1, 64, 64};
-    if (cdiv(T, 64) * cdiv(E, 128) >= 256) return {1, 64, 128};
-    if (cdiv(T, 128) * cdiv(E, 128) * 4 >= 192) return {4, 128, 128};
-    return {4, 64, 64};
-  }
 size_t moe_sort_workspace_bytes(int T, int k, int E) {
   if (T < 0 || k <= 0 || E <= 0) return 0;
   size_t M = (size_t)T * k;
@@ -1409,12 +1462,15 @@ int moe_route_sort_mapped(const float* gate_logits, const float* pre_bias_logits
   const int zero_fill = keep_other_rows ? 0 : 1;
   const SortMapArgs mp = {(TileInfo*)((uint8_t*)gmm_workspace + 16), (int32_t*)gmm_workspace, num_groups_local, group_offset, tile_rows, zero_fill};
   const RouteArgs r = {gate_logits, pre_bias_logits, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, 0, 0, topk_weights, topk_idx};
-  if (T <= kSortWaves)
-    route_sort_small_kernel<kSortWaves><<<1, kSortWaves * kWave, 0, (hipStream_t)stream>>>(r, roll_to_expert_id, ebits, group_sizes, perm, inv_perm,
-                                                                                            sorted_experts, mp);
-  else
-    route_sort_small_kernel<4 * kSortWaves><<<1, 4 * kSortWaves * kWave, 0, (hipStream_t)stream>>>(r, roll_to_expert_id, ebits, group_sizes, perm,
-                                                                                                    inv_perm, sorted_experts, mp);
+  dispatch_vpl(E, [&](auto vpl) {
+    constexpr int V = decltype(vpl)::value;
+    const hipStream_t st = (hipStream_t)stream;
+    if (T <= kSortWaves)
+      route_sort_small_kernel<kSortWaves, V><<<1, kSortWaves * kWave, 0, st>>>(r, roll_to_expert_id, ebits, group_sizes, perm, inv_perm, sorted_experts, mp);
+    else
+      route_sort_small_kernel<4 * kSortWaves, V><<<1, 4 * kSortWaves * kWave, 0, st>>>(r, roll_to_expert_id, ebits, group_sizes, perm, inv_perm,
+                                                                                        sorted_experts, mp);
+  });
   if (int st = check_launch("route_sort_small_kernel")) return st;
   note_tile_map_built(gmm_workspace, group_sizes, (int)M, E, group_offset, num_groups_local, tile_rows, zero_fill);
   return MOE_OK;

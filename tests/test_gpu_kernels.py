@@ -84,6 +84,15 @@ def test_route_deepseek(K, t, e, k, groups, topg):
   np.testing.assert_allclose(w.cpu().numpy(), ow, rtol=1e-5)
 
 
+@pytest.mark.parametrize("e,k,groups,topg", [(60, 6, 3, 2), (128, 4, 64, 5), (66, 9, 33, 8), (130, 16, 5, 5), (512, 8, 2, 1)])
+def test_route_deepseek_group_shapes_with_ties(K, e, k, groups, topg):
+  rng = np.random.default_rng(e)
+  gate = (np.round(rng.standard_normal((37, e)) * 4) / 4).astype(np.float32)
+  gate[0] = 0.0
+  _, idx = K.route_topk(cuda(gate), cuda(gate), k=k, mode="deepseek", n_routing_groups=groups, topk_routing_group=topg)
+  np.testing.assert_array_equal(idx.cpu().numpy(), O.get_topk(gate, gate, k=k, mode="deepseek", n_routing_groups=groups, topk_routing_group=topg)[1])
+
+
 def test_route_deepseek_reference_known_answer(K):
   # tests/unit/moe_test.py:293-326
   gate = np.array(
@@ -203,15 +212,6 @@ def test_gather_rows_fp8_block_quant(K, d):
   assert torch.equal(q.cpu().view(torch.uint8), oq.view(torch.uint8))
 
 
-def _v2_inputs(d, seed):
-  g = torch.Generator().manual_seed(seed)
-  x = (torch.randn(41, d, generator=g) * torch.logspace(-3, 2, 41)[:, None]).to(torch.bfloat16)
-  x[3] = 0
-  if d >= 8:
-    # the hand cases of tests/test_oracle_golden.py (truncation, x * (1/scale) against x / scale) in two rows
-    x[4] = 0
-    x[4, :4] = torch.tensor([1.0, 0.703125, 0.99609375, -0.99609375])
-    x[6] = 0
 @pytest.mark.parametrize("d", [2040, 2048, 2056, 4096, 4104, 8192, 8200])
 @pytest.mark.parametrize("block_k", [0, 128, 256, 512])
 def test_gather_rows_fp8_at_chunk_edges_and_extreme_scales(K, d, block_k):
@@ -227,6 +227,15 @@ def test_gather_rows_fp8_at_chunk_edges_and_extreme_scales(K, d, block_k):
   assert torch.equal(q.cpu().view(torch.uint8), oq[:, :d].contiguous().view(torch.uint8))
 
 
+def _v2_inputs(d, seed):
+  g = torch.Generator().manual_seed(seed)
+  x = (torch.randn(41, d, generator=g) * torch.logspace(-3, 2, 41)[:, None]).to(torch.bfloat16)
+  x[3] = 0
+  if d >= 8:
+    # the hand cases of tests/test_oracle_golden.py (truncation, x * (1/scale) against x / scale) in two rows
+    x[4] = 0
+    x[4, :4] = torch.tensor([1.0, 0.703125, 0.99609375, -0.99609375])
+    x[6] = 0
     x[6, :3] = torch.tensor([1.5, 1.4921875, 0.75])
   return x
 
@@ -1241,15 +1250,6 @@ def test_gate_route_softmax_f32(K, t, d, e, k):
   np.testing.assert_array_equal(w.cpu().numpy(), ow2)
 
 
-def test_gate_route_exact_on_integers(K):
-  """Small-integer activations and gate weights make every partial sum exact in f32, so logits and indices
-  must match the oracle bit for bit whatever the summation order (and the mid / lo terms are zero)."""
-  from maxtext_amd.quantizations import split_gate_kernel
-
-  rng = np.random.default_rng(7)
-  t, d, e, k = 513, 1024, 64, 6
-  x = torch.from_numpy(rng.integers(-4, 5, (t, d)).astype(np.float32)).to(torch.bfloat16)
-  wg = torch.from_numpy(rng.integers(-8, 9, (d, e)).astype(np.float32)) / 16.0
 # one shape for each tile of the wide kernel, with ragged tokens, experts and K quarters (empty ones too), and the last
 # shape that still takes the narrow kernel; k and E cover one to eight scores per lane of the top-k
 @pytest.mark.parametrize("t,d,e,k,terms", [(1100, 320, 132, 8, 1), (3073, 64, 260, 5, 1), (8200, 448, 132, 3, 1), (2049, 192, 68, 2, 3),
@@ -1266,6 +1266,15 @@ def test_gate_route_tiles_exact_on_integers(K, t, d, e, k, terms):
   np.testing.assert_array_equal(idx.cpu().numpy(), O.get_topk(want, k=k)[1])
 
 
+def test_gate_route_exact_on_integers(K):
+  """Small-integer activations and gate weights make every partial sum exact in f32, so logits and indices
+  must match the oracle bit for bit whatever the summation order (and the mid / lo terms are zero)."""
+  from maxtext_amd.quantizations import split_gate_kernel
+
+  rng = np.random.default_rng(7)
+  t, d, e, k = 513, 1024, 64, 6
+  x = torch.from_numpy(rng.integers(-4, 5, (t, d)).astype(np.float32)).to(torch.bfloat16)
+  wg = torch.from_numpy(rng.integers(-8, 9, (d, e)).astype(np.float32)) / 16.0
   terms = split_gate_kernel(wg)
   assert torch.all(terms[1] == 0) and torch.all(terms[2] == 0)
   w, idx, logits, _ = K.gate_route(cuda(x), cuda(terms), k=k, norm_topk_prob=True, return_logits=True)
