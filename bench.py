@@ -33,8 +33,8 @@ PROFILE_OF = {
     "c2": ("profiles/gmm_dls_kernel_int8_mixtral_prefill_c2.md", ["moe_gmm_dls.hip", "moe_gmm_common.h", "moe_common.h"]),
     "c2f8": ("profiles/gmm_dls_kernel_fp8_mixtral_shape_prefill_c2f8.md", ["moe_gmm_dls.hip", "moe_gmm_common.h", "moe_common.h"]),
     "c3": ("profiles/gmm_f8d_kernel_deepseek_decode_c3.md", ["moe_gmm_f8d.hip", "moe_gmm_f8d.h", "moe_gmm_common.h", "moe_common.h"]),
-    "c4": ("profiles/gmm_dlw_kernel_int8w_qwen3_prefill_c4.md", ["moe_gmm_dlw.hip", "moe_gmm_common.h", "moe_common.h"]),
-    "c5": ("profiles/gmm_dlw_kernel_int4w_gptoss_prefill_c5_t4096.md", ["moe_gmm_dlw.hip", "moe_gmm_common.h", "moe_common.h"]),
+    "c4": ("profiles/gmm_dlt_kernel_int8w_qwen3_prefill_c4.md", ["moe_gmm_dlt.hip", "moe_gmm_common.h", "moe_common.h"]),
+    "c5": ("profiles/gmm_dlt_kernel_int4w_gptoss_prefill_c5_t4096.md", ["moe_gmm_dlt.hip", "moe_gmm_common.h", "moe_common.h"]),
     "c2_t16": ("profiles/gmm_f8l_kernel_int8_mixtral_decode_c2_t16.md", ["moe_gmm_f8l.hip", "moe_gmm_f8d.h", "moe_gmm_common.h", "moe_common.h"]),
     "c2_t128": ("profiles/gmm_f8l_kernel_int8_mixtral_decode_c2_t128.md", ["moe_gmm_f8l.hip", "moe_gmm_f8d.h", "moe_gmm_common.h", "moe_common.h"]),
     "c2_train": ("profiles/tgmm_dl_kernel_bf16_mixtral_shape_train.md", ["moe_tgmm.hip", "moe_common.h"]),
@@ -145,8 +145,8 @@ def dominant_kernel_model(wl, group_sizes):
   if cfg.act_quant in ("int8", "fp8_row") or wl.weight_quant in (None, "bf16"):
     kernel = "gmm_dls_kernel" if rows >= 128 * len(group_sizes) else "gmm_tiled_kernel"
   else:
-    # (from 16 rows per expert on: on 128-row tiles up to 112, on 256-row tiles above)
-    kernel = "gmm_dlw_kernel" if rows >= 16 * len(group_sizes) and d % 64 == 0 else "gmm_tiled_kernel"
+    # (from 16 rows per expert on)
+    kernel = "gmm_dlt_kernel" if rows >= 16 * len(group_sizes) and d % 64 == 0 else "gmm_tiled_kernel"
   return dict(bound="mfma", work=flops, unit="TFLOP/s", peak=PEAK_TFLOPS[op], scale=1e12,
               name=kernel + " (wi_0|wi_1 + SwiGLU)", dtype=op)
 

@@ -13,9 +13,9 @@
 //                     tiles, operands copied global -> LDS without passing through registers, the requests of a block's
 //                     consecutive tiles as one stream.  gmm_dl_kernel (moe_gmm_dl.hip) is its predecessor, kept for the
 //                     shapes the stream kernel does not take and for [G, K, N] weights.
-//   gmm_dlw_kernel    the same stream for bf16 activations x int8 / int4 / mxfp4 weights (moe_gmm_dlw.hip): raw weight
-//                     bytes through LDS, widened by the wave that multiplies them; on 128-row tiles (half of the row tiles
-//                     multiplied) for int8 / int4 between the streaming kernel's range and prefill-sized groups.
+//   gmm_dlt_kernel    the same stream for bf16 activations x int8 / int4 / mxfp4 weights (moe_gmm_dlt.hip): raw weight
+//                     bytes through LDS, widened by the wave that multiplies them, on tiles of 256 or 192 rows.
+//                     gmm_dlw_kernel (moe_gmm_dlw.hip) is its predecessor, kept for 4-bit weights whose scales do not fit LDS.
 //   gmm_f8s_kernel    the same stream for block-scaled fp8 (moe_gmm_f8s.hip): scales staged through LDS.
 //   gmm_fp8_skinny_kernel  block-scaled fp8 for few rows per expert (decode): no LDS, every wave
 //                     streams 16 weight rows through v_mfma_f32_16x16x128_f8f6f4 and applies the
@@ -222,6 +222,31 @@ static int stream_tile_rows(int M, int G, int tiles_n) {
   }
   return best;
 }
+// The same choice for the weight-only stream kernel, 256 or 192 rows: the height whose tiles cost least for groups of
+// n ~ N(a, sqrt(a)) rows.  tail_rows: a group's last rows, up to so many, run on the decode kernel.  Costs in us a round, from the
+// GPT-OSS int4 layer at 52 to 512 rows per expert: 62 on 192-row tiles however full they are (the widening of the weights bounds
+// them; 160- and 128-row tiles were level, 331 / 333 / 326 us for the layer at 104 rows, and are not built), 68 to 84 on 256-row
+// ones by the rows they hold, 26 for a tail.  Layer on 192 / 256 rows: 336 / 379 us at 128 rows per expert, 356 / 397 at 160,
+// 457 / 411 at 200, 614 / 517 at 256, 688 / 704 at 375, 919 / 888 at 512; MXFP4 517 / 611 at 325; Qwen3 int8 249 / 269 at 156,
+// 1281 / 1187 at 1024.
+static int dlt_tile_rows(int M, int G, int tiles_n, int tail_rows) {
+  int cus = 0;
+  if (device_cu_count(&cus) != MOE_OK) cus = 256;
+  const double a = (double)M / G, sd = sqrt(a > 1.0 ? a : 1.0);
+  auto above = [&](double rows) { return 0.5 * erfc((rows - a) / (sd * 1.41421356)); };  // P(n > rows)
+  auto cost_of = [&](int bm) {
+    double tiles = 0.0, tails = 0.0;
+    for (int j = 0; j * bm < a + 4.0 * sd; j++) {
+      tiles += above(j * (double)bm + tail_rows);
+      tails += above(j * (double)bm) - above(j * (double)bm + tail_rows);
+    }
+    const double held = a / (tiles > 0.01 ? tiles : 0.01);
+    const double tile = bm == 192 ? 62.0 : held <= 190.0 ? 68.0 : 68.0 + (held < 256.0 ? held - 190.0 : 66.0) * 16.0 / 66.0;
+    const double rounds = tiles * G * tiles_n / cus;
+    return 0.5 * (rounds + ceil(rounds - 0.1)) * tile + tails * G * tiles_n / cus * 26.0;
+  };
+  return cost_of(192) < cost_of(256) ? 192 : 256;
+}
 // Rows per expert on average from which the stream kernel takes operands that need no conversion: 32 for bf16 (level with the
 // 64-row tiles there, 0.365 / 0.361 ms on the Mixtral shape, 5 % ahead on the Qwen3 one); past the LDS-streamed decode
 // kernel's range for 8-bit operands (at 56 rows fp8 0.212 -> 0.199 ms against the 128 x 128 kernel, int8 at 64 level with the
@@ -244,9 +269,9 @@ static TiledKind pick_tiled_kind(int op, int bsrc, bool glu, int M, int K, int N
   const long long tiles_big = (long long)max_tiles_for(M, G_total, 256) * cdiv(N, glu ? 128 : 256);
   const bool dlw_ok = bsrc != BSRC_SAME && dlw_takes(K, N, indexed_lhs_rows, wq_kmajor);
   // 256-row tiles from 128 rows per expert on average, where half of the routed groups no longer fit a 128-row tile (int8
-  // x int8 on the Qwen3 shape: 0.106 against 0.126 ms at 112 rows, 0.133 against 0.131 at 128); the weight-only stream
-  // kernel from 112: below, the same kernel runs on 128-row tiles (GPT-OSS int4 layer at 104 / 112 rows per expert 0.38 /
-  // 0.45 ms on those, 0.44 / 0.44 on 256-row tiles)
+  // x int8 on the Qwen3 shape: 0.106 against 0.126 ms at 112 rows, 0.133 against 0.131 at 128); gmm_dlw_kernel from 112:
+  // below, the same kernel runs on 128-row tiles (GPT-OSS int4 layer at 104 / 112 rows per expert 0.38 / 0.45 ms on those,
+  // 0.44 / 0.44 on 256-row tiles)
   const bool big = (long long)M >= (dlw_ok ? 112LL : 128LL) * G_total && tiles_big >= 128;
   // 32 to 128 rows per expert on average: 128-row tiles; below 32, 64-row tiles.  With routed groups of near-equal size
   // the 64-row tiles are 5-10 % ahead up to 56 rows per expert (GPT-OSS shape, 384 tokens: 0.38 against 0.41 ms for the
@@ -256,11 +281,10 @@ static TiledKind pick_tiled_kind(int op, int bsrc, bool glu, int M, int K, int N
   // their 256-row register-staged tiles pass the 128-row ones at 128 rows per expert as well.
   const bool mid = !big && (long long)M >= 32LL * G_total && (long long)M < 128LL * G_total;
   const int esz = op == OP_I8 ? 1 : 2;
-  // weight-only formats between the streaming kernel's range and the 256-row tiles: the stream kernel on 128-row tiles
-  // (half of its row tiles multiplied, nothing requested for the other half) is 10-15 % ahead of the register-staged
-  // 128-row tiles for int8 and int4 (GPT-OSS int4 layer at 40 to 96 rows per expert 0.34-0.35 against 0.40-0.42 ms, Qwen3
-  // int8 with Zipf routing at 20 to 80 rows 0.14-0.20 against 0.15-0.25 ms), 1-2 % for MXFP4 (0.338-0.352 against
-  // 0.344-0.358 ms), and level with the 64-row tiles at 16 to 32 rows
+  // weight-only formats between the streaming kernel's range and prefill: the stream kernels are ahead of the register-staged
+  // 128-row tiles (GPT-OSS int4 layer at 52 to 104 rows per expert 0.32-0.35 against 0.40-0.42 ms, Qwen3 int8 with Zipf
+  // routing at 20 to 94 rows 0.11-0.18 against 0.15-0.25 ms, MXFP4 0.285-0.295 against 0.344-0.358 ms), and level with the
+  // 64-row tiles at 16 to 32 rows
   if (dlw_ok && !big && (long long)M >= 16LL * G_total && (long long)M < 128LL * G_total &&
       (long long)max_tiles_for(M, G_total, 128) * cdiv(N, glu ? 128 : 256) >= 128)
     return K_DLW128;
@@ -274,14 +298,25 @@ static TiledKind pick_tiled_kind(int op, int bsrc, bool glu, int M, int K, int N
   return K_T64;
 }
 
-static int tiled_kind_bm(TiledKind k, int stream_bm) { return k == K_T64 ? 64 : k == K_T128 || k == K_DLW128 ? 128 : k == K_DLS ? stream_bm : 256; }
+static bool on_dlt(TiledKind k, int bsrc, const TiledParams& p) {
+  return (k == K_DLW || k == K_DLW128) && dlt_takes(bsrc, p.K, p.N, p.i4_group, p.ro.row_idx ? p.ro.lhs_rows : 0, p.wq_kmajor != 0);
+}
+// Rows of a tile.  tail_rows: a group's last rows, up to so many, go elsewhere.
+static int tiled_kind_bm(TiledKind k, int bsrc, bool glu, const TiledParams& p, int M, int G, int tail_rows) {
+  if (k == K_T64) return 64;
+  if (k == K_T128) return 128;
+  if (k == K_DLS) return stream_tile_rows(M, G, cdiv(p.N, glu ? 128 : 256));
+  if (on_dlt(k, bsrc, p)) return dlt_tile_rows(M, G, cdiv(p.N, glu ? 128 : 256), tail_rows);
+  return k == K_DLW128 ? 128 : 256;
+}
 
-static int launch_tiled_kind(TiledKind kind, int op, int bsrc, bool glu, const TiledParams& p, int M, int G_total, hipStream_t s) {
-  if (kind == K_DLS) return launch_dls(op, glu, stream_tile_rows(M, G_total, cdiv(p.N, glu ? 128 : 256)), p, M, G_total, s);
+static int launch_tiled_kind(TiledKind kind, int op, int bsrc, bool glu, int bm, const TiledParams& p, int M, int G_total, hipStream_t s) {
+  if (kind == K_DLS) return launch_dls(op, glu, bm, p, M, G_total, s);
   if (kind == K_DL128) return launch_dl(op, glu, 128, false, p, M, G_total, s);
   if (kind == K_DL64) return launch_dl(op, glu, 64, false, p, M, G_total, s);
+  if (on_dlt(kind, bsrc, p)) return launch_dlt(bsrc, glu, bm, p, M, G_total, s);
   if (kind == K_DLW || kind == K_DLW128) return launch_dlw(bsrc, glu, kind == K_DLW128, p, M, G_total, s);
-  return launch_tiled_bm(op, bsrc, glu, tiled_kind_bm(kind, 0), false, p, M, G_total, s);
+  return launch_tiled_bm(op, bsrc, glu, bm, false, p, M, G_total, s);
 }
 
 }  // namespace moe
@@ -586,8 +621,9 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
     }
     TiledKind kind = pick_tiled_kind(op, BSRC_SAME, glu, M, K, N, G);
     if (kernel == MOE_GMM_KERNEL_TILED) kind = tiled_only(kind);
-    map_tiles(tiled_kind_bm(kind, stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256))));
-    return launch_tiled_kind(kind, op, BSRC_SAME, glu, p, M, G, s);
+    const int bm = tiled_kind_bm(kind, BSRC_SAME, glu, p, M, G, 0);
+    map_tiles(bm);
+    return launch_tiled_kind(kind, op, BSRC_SAME, glu, bm, p, M, G, s);
   }
 
   enum { V_NONE, V_BF16, V_W8, V_W4, V_MX4 } variant = V_NONE;
@@ -697,11 +733,11 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
   const bool split_tails = (kind == K_DLW || kind == K_DLW128) && kernel == MOE_GMM_KERNEL_AUTO && (bsrc == BSRC_I4 || bsrc == BSRC_MX4) && !wq_kmajor &&
                            wqs_takes(wq_fmt, K, N, a->num_groups_local, glu);
   if (split_tails) {
-    const int bm = tiled_kind_bm(kind, 0);
+    const int bm = tiled_kind_bm(kind, bsrc, glu, p, M, G, kTailRows);
     const int tail_base = max_tiles_for(M, G, bm);  // past every record the first list can hold
     if ((size_t)16 + ((size_t)tail_base + (size_t)G * cdiv(kTailRows, kTailTile)) * sizeof(TileInfo) <= workspace_bytes) {
       map_tiles_split(bm, kTailRows, tail_base);
-      if (int st = launch_tiled_kind(kind, op, bsrc, glu, p, M, G, s)) return st;
+      if (int st = launch_tiled_kind(kind, op, bsrc, glu, bm, p, M, G, s)) return st;
       WqSkinnyParams q = {};
       q.lhs = (const uint8_t*)a->lhs; q.rhs = (const uint8_t*)a->rhs; q.rhs_up = (const uint8_t*)a->rhs_up;
       q.rhs_scale = a->rhs_scale; q.rhs_up_scale = a->rhs_up_scale;
@@ -712,8 +748,9 @@ static int gmm_impl(const moe_gmm_args* a, void* workspace, size_t workspace_byt
       return launch_wqs(wq_fmt, q, glu, a->num_groups_local, s);
     }
   }
-  map_tiles(tiled_kind_bm(kind, stream_tile_rows(M, G, cdiv(N, glu ? 128 : 256))));
-  return launch_tiled_kind(kind, op, bsrc, glu, p, M, G, s);
+  const int bm = tiled_kind_bm(kind, bsrc, glu, p, M, G, 0);
+  map_tiles(bm);
+  return launch_tiled_kind(kind, op, bsrc, glu, bm, p, M, G, s);
 }
 
 int moe_gmm(const moe_gmm_args* a, void* stream) {
@@ -741,6 +778,7 @@ int moe_init(void) {
   if (int st = prepare_tiled()) return st;
   if (int st = prepare_dl()) return st;
   if (int st = prepare_dlw()) return st;
+  if (int st = prepare_dlt()) return st;
   if (int st = prepare_dls()) return st;
   if (int st = prepare_wqs()) return st;
   if (int st = prepare_f8d()) return st;

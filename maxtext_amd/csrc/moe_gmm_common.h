@@ -634,6 +634,7 @@ int prepare_tiled();
 int prepare_dl();
 int prepare_fp8();
 int prepare_dlw();
+int prepare_dlt();
 int prepare_dls();
 int prepare_tgmm();
 
@@ -643,7 +644,6 @@ int prepare_tgmm();
 int launch_tiled_bm(int op, int bsrc, bool glu, int bm, bool block_scaled, const TiledParams& p, int M, int G_total, hipStream_t s);
 // moe_gmm_dl.hip: direct-to-LDS persistent kernel, 256 x 256 tiles; stage_bytes 128 or 64; rhs_kn: [G, K, N] bf16 weights
 int launch_dl(int op, bool glu, int stage_bytes, bool rhs_kn, const TiledParams& p, int M, int G_total, hipStream_t s);
-// moe_gmm_dlw.hip: the same pipeline for bf16 activations x int8 / int4 / mxfp4 weights (K % 64 == 0, default scale layouts)
 // moe_gmm_dls.hip: the persistent kernel (tiles of bm = 256, 192 or 160 rows x 256 channels) for int8 x int8 / bf16 x bf16 with one request stream across tiles
 // (fp8 x fp8 with epilogue scales too; lhs_e5m2: the activations are float8_e5m2, the weights e4m3)
 int launch_dls(int op, bool glu, int bm, const TiledParams& p, int M, int G_total, hipStream_t s, int lhs_e5m2 = 0, int rhs_kn = 0);
@@ -654,9 +654,13 @@ struct Fp8TiledParams;
 int launch_f8s(bool glu, int bm, const Fp8TiledParams& P, int M, int G_total, hipStream_t s);
 bool f8s_takes(int K, int N, long long M, long long indexed_lhs_rows);
 int prepare_f8s();
+// moe_gmm_dlw.hip: bf16 activations x int4 / mxfp4 weights whose scales do not fit beside the stages of gmm_dlt_kernel
 int launch_dlw(int bsrc, bool glu, bool half, const TiledParams& p, int M, int G_total, hipStream_t s);
-// whether that kernel takes the shape (indexed_lhs_rows: rows of lhs when a row index is used, else 0)
+// whether one of the two weight-only stream kernels takes the shape (indexed_lhs_rows: rows of lhs when a row index is used, else 0)
 bool dlw_takes(int K, int N, long long indexed_lhs_rows, bool wq_kmajor);
+// moe_gmm_dlt.hip: bf16 activations x int8 / int4 / mxfp4 weights (K % 64 == 0, default scale layouts), the waves of a SIMD taking turns, tiles of bm = 256 or 192 rows
+int launch_dlt(int bsrc, bool glu, int bm, const TiledParams& p, int M, int G_total, hipStream_t s);
+bool dlt_takes(int bsrc, int K, int N, int i4_group, long long indexed_lhs_rows, bool wq_kmajor);
 // moe_gmm_fp8.hip
 int launch_fp8_tiled(bool big, bool glu, bool vec4, const Fp8TiledParams& P, int M, int G_total, hipStream_t s);
 int launch_fp8_skinny(bool few_rows, const SkinnyParams& p, bool glu, int max_tiles, hipStream_t s);

@@ -1,0 +1,447 @@
+// Grouped matmul: the persistent kernel for bf16 activations x int8 / int4 / mxfp4 weights (prefill), the two waves of a
+// SIMD taking turns.
+//
+// Tiles of 256 or 192 rows x 256 channels, 8 waves as 2 x 4, each 128 (96) x 64 of the tile in 16x16x32
+// MFMAs.  Both operands go global -> LDS without passing through registers (buffer_load ... lds, 1 KB per wave
+// instruction): the activations as XOR-swizzled rows of 128 bytes (64 bf16 values of K: a stage), the weights as the raw
+// bytes of the checkpoint format (64 or 32 bytes per row and stage), for the 4-bit formats with a tile's block scales as one
+// panel beside them.  The stages of a block's consecutive tiles form one request stream, as in gmm_dls_kernel.
+//
+// What bounds it.  A wave of 256 x 32 (gmm_dlw_kernel) widens every weight once per block but reads all of the tile's
+// activation rows out of LDS: 256 + 16 KB a stage and block, 2176 cycles at 128 bytes a cycle against 2048 of MFMAs.  128 x 64
+// reads 128 + 32 KB and widens every weight twice, which is vector work in the shadow of the other wave's MFMAs.
+//
+// Schedule.  A stage is four phases, (32 values of K) x (half of the wave's row tiles) each: up to 16 MFMAs, 256 cycles.  A
+// phase is a fetching side, a barrier, a multiplying side and a barrier; waves 4 .. 7 run one barrier behind waves 0 .. 3, so
+// that one wave of a SIMD fetches while its neighbour multiplies.  A fetching side reads the phase's activation fragments and
+// the raw bytes of two weight fragments and sends its share of requests; a multiplying side widens those two behind its own
+// products.  The widened fragments are two sets, one per 32 values of K: phases 1 and 2 multiply set 0 and complete set 1, phases 3
+// and 4 multiply set 1 and build set 0 of the next stage.
+//
+// Measured against gmm_dlw_kernel, same box, us of the first (with SwiGLU) and second projection: MXFP4 GPT-OSS shape at 4096 tokens
+// 503 -> 450 and 327 -> 289, int4 at 1023 tokens 289 -> 263 and 174 -> 167 on the same 256-row tiles and less on 192-row ones
+// (layer 404 -> 341), int8 Qwen3 shape at 16384 tokens 739 -> 721 and 446 -> 440.  What is left is the widening: with its vector
+// instructions on the fetching side (28 a phase for int8, 60 for int4) the same kernel took 792 and 475 us for int8 and 328 and
+// 210 for int4, and int8 through halves and mixed multiply-adds (36 a phase, exact as well) 860.
+
+#include "moe_gmm_common.h"
+
+namespace moe {
+
+template <int BSRC_, bool GLU_, int TM_>
+struct DltCfg {
+  static constexpr int BSRC = BSRC_;
+  static constexpr bool GLU = GLU_;
+  // row tile i of wave row wm holds the tile's rows 32 i + 16 wm .. + 15; the first H0 are half h = 0
+  static constexpr int TM = TM_, H0 = TM / 2, H1 = TM - H0;
+  static constexpr int BM = TM * 32, BN = 256, BKB = 128, BK = 64, MI = 16;
+  static constexpr int WAVES_M = 2, WAVES_N = 4, NWAVES = 8, THREADS = NWAVES * kWave;
+  static constexpr int WN = BN / WAVES_N, TN = WN / MI;
+  static constexpr bool NIBBLES = BSRC == BSRC_I4 || BSRC == BSRC_MX4;
+  static constexpr int W_ROW = NIBBLES ? BK / 2 : BK;  // raw bytes of a weight row per stage
+  // activation requests per wave and stage (64 rows of all waves each): NA0 hold half h = 0, NA1 the rest
+  static constexpr int A_IPW = (BM + 63) / 64, NA0 = (H0 + 1) / 2, NA1 = A_IPW - NA0;
+  static constexpr int B_IPW = BN * W_ROW / 1024 / NWAVES;  // weight requests per wave and stage: 2 (int8) or 1
+  static constexpr int B_RPI = 1024 / W_ROW;                // weight rows per request
+  // three stages of activations; weights three, for the 4-bit formats two (the scale panels take the room)
+  static constexpr int NA = 3, NB = NIBBLES ? 2 : 3;
+  static constexpr int A_STAGE = A_IPW * 64 * BKB, B_STAGE = BN * W_ROW, B_BASE = NA * A_STAGE, S_BASE = B_BASE + NB * B_STAGE;
+  static constexpr int OUT_BN = GLU ? BN / 2 : BN;
+  static_assert(BSRC != BSRC_SAME && (TM == 8 || TM == 6), "shape");
+  __device__ static __forceinline__ int swz_a(int row) { return (row >> 1) & 7; }
+  __device__ static __forceinline__ int swz_b(int row) { return NIBBLES ? (row >> 3) & 1 : (row >> 2) & 3; }
+};
+
+constexpr int kDltLds = 160 * 1024;
+
+// Scale bytes of a weight row (4-bit formats), and of one panel: the 256 rows of a tile, with GLU the 128 of each projection
+// in whole KBs.
+static __host__ __device__ inline uint32_t dlt_scale_row_bytes(int bsrc, int K, int i4_group) {
+  return bsrc == BSRC_I4 ? (uint32_t)((K + i4_group - 1) / i4_group) * 2 : (uint32_t)(K / 32);
+}
+static __host__ __device__ inline uint32_t dlt_scale_part(bool glu, uint32_t row_bytes) { return ((glu ? 128 : 256) * row_bytes + 1023) / 1024 * 1024; }
+
+template <typename C>
+__global__ __launch_bounds__(C::THREADS, 2) void gmm_dlt_kernel(const TiledParams p0) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  // (bf16 activations carry no scale: saying so here lets the epilogue fold the per-row factor away)
+  TiledParams p = p0;
+  p.lhs_scale = nullptr;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave % C::WAVES_M, wn = wave / C::WAVES_M;
+  const bool late = wave >= C::NWAVES / 2;  // the second wave of its SIMD
+  const int N = p.N, K = p.K;
+  const uint32_t row_bytes = (uint32_t)K * 2;
+  const uint32_t w_row_bytes = C::NIBBLES ? (uint32_t)K / 2 : (uint32_t)K;
+  const int num_tiles = p.header[0];
+  const int nk = K / C::BK;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
+
+  using Tile = StreamTile;
+  using Peek = TilePeek;
+  auto peek_from = [&](int id0) { return peek_tile<C::OUT_BN>(p, num_tiles, id0); };
+  auto resolve = [&](Peek pk, Tile& t) { return resolve_tile<C::OUT_BN, C::THREADS>(p, num_tiles, pk, t, tid); };
+
+  // ---- the loading side of the stream ---------------------------------------------------------------------------
+  // activations: request i covers rows 64 i + 8 wave .. + 7 of the tile, 128 bytes of each; the lane's 16 bytes: global
+  // chunk = LDS slot ^ swizzle of the row.  (wave_v: see gmm_dls_kernel)
+  int wave_v = wave;
+  asm volatile("" : "+v"(wave_v));
+  auto a_lane_off = [&](int i, uint32_t row) { return row * row_bytes + (uint32_t)(((lane % 8) ^ C::swz_a(i * 64 + wave_v * 8 + lane / 8)) << 4); };
+  v4i a_desc;
+  uint32_t a_voff[C::A_IPW];
+  auto set_a_sources = [&](const Tile& t) {
+    if (p.ro.row_idx) {
+      a_desc = buffer_desc(p.lhs, clamp_u32((size_t)p.ro.lhs_rows * row_bytes));
+      int rows[C::A_IPW];
+#pragma unroll
+      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + i * 64 + wave_v * 8 + lane / 8, p.M - 1);
+      lhs_rows_of<C::A_IPW>(p.ro, rows);
+      // (rows past the tile's end: one row past the descriptor's, i.e. zeros without a request to memory)
+#pragma unroll
+      for (int i = 0; i < C::A_IPW; i++) a_voff[i] = a_lane_off(i, (uint32_t)(i * 64 + wave_v * 8 + lane / 8 < t.info.nrows ? rows[i] : p.ro.lhs_rows));
+    } else {
+      a_desc = buffer_desc(p.lhs + (size_t)t.info.row0 * row_bytes, clamp_u32((size_t)t.info.nrows * row_bytes));
+    }
+  };
+  if (!p.ro.row_idx) {
+#pragma unroll
+    for (int i = 0; i < C::A_IPW; i++) a_voff[i] = a_lane_off(i, (uint32_t)(i * 64 + wave_v * 8 + lane / 8));
+  }
+  // weights: request i covers the tile's weight rows (wave * B_IPW + i) * B_RPI .. + B_RPI - 1; with GLU the upper 128 of the
+  // 256 rows are the second projection's, whose requests come from waves 4 .. 7
+  const bool load_up = C::GLU && late;
+  v4i b_desc, s_desc;
+  uint32_t b_soff = 0, s_soff = 0;
+  uint32_t b_voff[C::B_IPW];
+#pragma unroll
+  for (int i = 0; i < C::B_IPW; i++) {
+    const int r = (wave_v * C::B_IPW + i) * C::B_RPI + lane / (C::W_ROW / 16);
+    const int pr = C::GLU ? r % (C::BN / 2) : r;
+    b_voff[i] = (uint32_t)pr * w_row_bytes + (uint32_t)(((lane % (C::W_ROW / 16)) ^ C::swz_b(r)) << 4);
+  }
+  // the scale panel of a tile: contiguous in memory, 1 KB requests dealt to the waves (with GLU: of the projection's half)
+  const uint32_t s_row_bytes = C::NIBBLES ? dlt_scale_row_bytes(C::BSRC, K, p.i4_group) : 0;
+  const uint32_t s_part = dlt_scale_part(C::GLU, s_row_bytes), s_panel = C::GLU ? 2 * s_part : s_part;
+  int load_panel = 0;  // panel the loading side fills next
+  auto set_b_sources = [&](const Tile& t) {
+    b_desc = buffer_desc((load_up ? p.rhs_up : p.rhs) + (size_t)t.info.group * N * w_row_bytes, clamp_u32((size_t)N * w_row_bytes));
+    b_soff = (uint32_t)t.n0 * w_row_bytes;
+    if (C::NIBBLES) {
+      s_desc = buffer_desc((const uint8_t*)(load_up ? p.rhs_up_scale : p.rhs_scale) + (size_t)t.info.group * N * s_row_bytes, clamp_u32((size_t)N * s_row_bytes));
+      s_soff = (uint32_t)t.n0 * s_row_bytes;
+    }
+  };
+  auto issue_scales = [&]() {
+    if (!C::NIBBLES) return;
+    constexpr int STEP = C::GLU ? C::NWAVES / 2 : C::NWAVES;
+    for (uint32_t o = (uint32_t)(wave % STEP) * 1024; o < s_part; o += STEP * 1024)
+      dma16_buffer(s_desc, o + (uint32_t)lane * 16, s_soff, lds_base + C::S_BASE + load_panel * s_panel + (load_up ? s_part : 0) + o);
+    load_panel ^= 1;
+  };
+  auto issue_a = [&](int kt, int buf, int h) {
+#pragma unroll
+    for (int i = h ? C::NA0 : 0; i < (h ? C::A_IPW : C::NA0); i++)
+      dma16_buffer(a_desc, a_voff[i], (uint32_t)kt * C::BKB, lds_base + buf * C::A_STAGE + (i * 64 + wave * 8) * C::BKB);
+  };
+  auto issue_b = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < C::B_IPW; i++)
+      dma16_buffer(b_desc, b_voff[i], b_soff + (uint32_t)kt * C::W_ROW, lds_base + C::B_BASE + buf * C::B_STAGE + (wave * C::B_IPW + i) * 1024);
+  };
+
+  // ---- the multiplying side --------------------------------------------------------------------------------------
+  using T_ = std::true_type;
+  using F_ = std::false_type;
+  constexpr int NT_OUT = C::GLU ? C::TN / 2 : C::TN;
+  // weight fragment j of this wave: rows frag_row(j) .. + 15 of the tile; the lane widens row + lane % 16
+  auto frag_row = [&](int j) { return C::GLU ? (j / 2) * (C::BN / 2) + wn * 32 + (j % 2) * 16 : wn * C::WN + j * 16; };
+  typedef v4f acc_t;
+  acc_t acc[C::TN][C::TM];
+  v4i fa[C::H0], fb[2][C::TN];
+  // activation fragment of row tile i, k-step ks: row 32 i + 16 wm + lane % 16, chunk q = 4 ks + lane / 16, at slot q ^ swz_a(row)
+  const int a_lane = (wm * 16 + lane % 16) * C::BKB + (((lane / 16) ^ C::swz_a(lane % 16)) << 4);
+  auto read_a = [&](int buf, int ks, int h) {
+#pragma unroll
+    for (int i = 0; i < (h ? C::H1 : C::H0); i++)
+      fa[i] = *(const v4i*)(smem + buf * C::A_STAGE + (h * C::H0 + i) * 32 * C::BKB + (a_lane ^ (ks * 64)));
+  };
+  // raw weight fragments (two): row frag_row(j) + lane % 16, the 8 values of K from 32 ks + 8 (lane / 16) on
+  const int b_lane = C::NIBBLES ? (lane % 16) * C::W_ROW + (lane / 16) * 4 : (lane % 16) * C::W_ROW + ((lane / 16) & 1) * 8;
+  const int b_sw = C::swz_b(lane % 16);
+  typedef typename std::conditional<C::NIBBLES, uint32_t, uint2>::type raw_t;
+  raw_t braw[2];
+  uint32_t sraw[2] = {0, 0};
+  // pair: fragments 2 pair, 2 pair + 1 of the stage kt in buffer buf; their scale bits with them
+  auto read_raw = [&](int buf, int kt, int panel, int ks, int pair) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int j = 2 * pair + t;
+      const int slot = C::NIBBLES ? ks : 2 * ks + (lane / 32);  // 16-byte slot of the row that holds the lane's bytes
+      braw[t] = *(const raw_t*)(smem + C::B_BASE + buf * C::B_STAGE + frag_row(j) * C::W_ROW + b_lane + ((slot ^ b_sw) << 4));
+      if (C::NIBBLES) {
+        const int row = C::GLU ? wn * 32 + (j % 2) * 16 + lane % 16 : frag_row(j) + lane % 16;
+        const uint8_t* sp = smem + C::S_BASE + panel * s_panel + (C::GLU && j >= 2 ? s_part : 0) + row * s_row_bytes;
+        if (C::BSRC == BSRC_MX4) sraw[t] = sp[2 * kt + ks];
+        else sraw[t] = *(const uint16_t*)(sp + (p.i4_group == 32 ? 2 * kt + ks : kt >> 1) * 2);
+      }
+    }
+  };
+  typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+  uint32_t half_1024 = 0x64006400u, nib_mask = 0x000f000fu;  // (opaque: one and-or with registers, two instructions with literals)
+  if constexpr (C::BSRC == BSRC_I4) asm volatile("" : "+v"(half_1024), "+s"(nib_mask));
+  // Piece q (0 .. 7) of the two fragments just read: two of a fragment's eight values -> one register of fb[ks][2 pair + q / 4].
+  uint32_t nib[2];
+  float sc = 1.0f, sc_off = 0.0f;
+  auto widen_piece = [&](int ks, int pair, int q) __attribute__((always_inline)) {
+    const int t = q / 4;
+    v4i& o = fb[ks][2 * pair + t];
+    const raw_t raw = braw[t];
+    if constexpr (C::BSRC == BSRC_I8) {
+      const int pc = q % 4, sh = (pc & 1) * 16, w = (int)(pc < 2 ? raw.x : raw.y);
+      o[pc] = (int)pack_bf16x2((float)((w << (24 - sh)) >> 24), (float)((w << (16 - sh)) >> 24));
+    } else if constexpr (C::BSRC == BSRC_MX4) {
+      if (q % 4 == 0) sc = __uint_as_float(sraw[t] << 23);
+      // (the byte selector is an immediate)
+      o[q % 4] = q % 4 == 0   ? __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, sc, 0))
+                 : q % 4 == 1 ? __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, sc, 1))
+                 : q % 4 == 2 ? __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, sc, 2))
+                              : __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw, sc, 3));
+    } else {
+      // (nibble - 8) * scale rounded to bf16, as the reference dequantises.  A nibble is the low mantissa of a half 1024, two
+      // of them to a word (values i and i + 4); (1024 + nibble) * scale - 1032 * scale is exact in f32 (19 significant bits ahead
+      // of the sum, 12 behind it), so the mixed multiply-add gives it bit for bit in one instruction per value
+      if (q % 4 == 0) {
+        sc = __uint_as_float(sraw[t] << 16);
+        sc_off = -1032.0f * sc;
+      }
+      const int half = q % 2, pc = (q % 4) / 2 + 2 * half;  // registers 0, 2 (values 0, 1 and 4, 5), then 1, 3
+      if (!half) {
+        nib[0] = ((raw >> (4 * 2 * pc)) & nib_mask) | half_1024;
+        nib[1] = ((raw >> (4 * (2 * pc + 1))) & nib_mask) | half_1024;
+      }
+      o[pc] = (int)pack_bf16x2(fmaf((float)__builtin_bit_cast(v2h, nib[0])[half], sc, sc_off), fmaf((float)__builtin_bit_cast(v2h, nib[1])[half], sc, sc_off));
+    }
+  };
+  auto widen = [&](int ks, int pair) {
+#pragma unroll
+    for (int q = 0; q < 8; q++) widen_piece(ks, pair, q);
+  };
+  // The two sides of a phase.  fetch_end: this wave's fragment reads have landed and so have its requests up to the ones
+  // that may still be outstanding (WAIT), then the hand-over barrier.
+  auto fetch_end = [&](auto wait_c) {
+    constexpr int WAIT = decltype(wait_c)::value;
+    if constexpr (WAIT >= 0) wait_vmcnt<WAIT>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+  };
+  // Half h of the row tiles x values ks of K, with the widening of pair wp of set wks in the shadow of the products.
+  auto multiply = [&](auto zc_c, int ks, int h, int wks, int wp) __attribute__((always_inline)) {
+    constexpr bool ZC = decltype(zc_c)::value;
+    const int slots = (h ? C::H1 : C::H0) * C::TN;  // products of the phase
+#pragma unroll
+    for (int i = 0; i < (h ? C::H1 : C::H0); i++)
+#pragma unroll
+      for (int j = 0; j < C::TN; j++) {
+        acc_t& c = acc[j][h * C::H0 + i];
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, fb[ks][j]), __builtin_bit_cast(v8bf, fa[i]), ZC ? acc_t{} : c, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+          if (q * slots / 8 == i * C::TN + j) widen_piece(wks, wp, q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    // (sums and fragments are pinned: left alone the compiler moves the last products past a tile's branches, and the
+    // widening to where its result is multiplied)
+#pragma unroll
+    for (int i = 0; i < (h ? C::H1 : C::H0); i++)
+#pragma unroll
+      for (int j = 0; j < C::TN; j++) asm volatile("" : "+v"(acc[j][h * C::H0 + i]));
+#pragma unroll
+    for (int t = 0; t < 2; t++) asm volatile("" : "+v"(fb[wks][2 * wp + t]));
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+  };
+  using NOWAIT = std::integral_constant<int, -1>;
+  // Requests of stage t + 2 go out in stage t: with three weight buffers weights, activations h = 0 and h = 1 in phases 1, 2 and
+  // 3; with two, whose slot is last read in phase 2, activations h = 0, weights and activations h = 1 in phases 2, 3 and 4.
+  // What may be outstanding where a phase ends ahead of new data:
+  constexpr bool B3 = C::NB == 3;
+  using W1 = std::integral_constant<int, B3 ? 2 * C::B_IPW + C::A_IPW : C::A_IPW + C::B_IPW>;                              // ahead of phase 2 (activations h = 1)
+  using W2 = std::integral_constant<int, B3 ? C::A_IPW + C::B_IPW + C::NA0 : C::A_IPW>;                                    // ahead of phase 3 (the next stage's weights)
+  using W4 = std::integral_constant<int, B3 ? C::NA1 + C::B_IPW + C::A_IPW : C::NA1 + 2 * C::B_IPW + C::A_IPW>;            // ahead of phase 1 (activations h = 0)
+
+  Tile cur, nxt;
+  if (!resolve(peek_from(blockIdx.x), cur)) return;
+  // ---- head of the stream: the first tile's stages 0 and 1, the first stage's fragments of phases 1 and 2 ----
+  set_a_sources(cur);
+  set_b_sources(cur);
+  issue_scales();
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    issue_b(s, s);
+    issue_a(s, s, 0);
+    issue_a(s, s, 1);
+  }
+  wait_vmcnt<0>();
+  asm volatile("s_barrier" ::: "memory");
+  int panel = 0;            // scale panel of the current tile
+  int ab = 0, bb = 0;       // buffers of the current stage
+  read_raw(0, 0, 0, 0, 0);
+  widen(0, 0);
+  read_raw(0, 0, 0, 0, 1);
+  widen(0, 1);
+
+  while (true) {
+    // the record of the block's next tile is requested now and looked at two stages before this tile ends
+    Peek pk = peek_from(cur.id + gridDim.x);
+    bool have_n = false;
+    const int n_out0 = cur.n0 + (C::GLU ? wn * (C::WN / 2) : wn * C::WN);
+    EpilogueScales<C::TM, NT_OUT, C::GLU> esc;
+    auto stream_kt = [&](int s) { return s < nk ? s : (have_n ? s - nk : nk - 1); };
+    // Stage `it`.  first: its data and the next stage's weights landed before the tile began.  cross: the stream has just
+    // moved on to the next tile, whose scales are requested ahead of its weights.
+    auto stage = [&](int it, auto first_c, auto cross_c) __attribute__((always_inline)) {
+      constexpr bool FIRST = decltype(first_c)::value, CROSS = decltype(cross_c)::value;
+      using WA = typename std::conditional<FIRST, NOWAIT, W1>::type;
+      using WB = typename std::conditional<FIRST, NOWAIT, W2>::type;
+      const int kt2 = stream_kt(it + 2);
+      const int ab2 = ab == 0 ? C::NA - 1 : ab - 1;                                      // the buffer of stage it - 1 takes stage it + 2
+      const int bb1 = bb == C::NB - 1 ? 0 : bb + 1, bb2 = !B3 ? bb : bb1 == C::NB - 1 ? 0 : bb1 + 1;
+      // the stage whose weights are widened ahead, and its tile's panel
+      const int kt1 = it + 1 < nk ? it + 1 : 0;
+      const int panel1 = it + 1 < nk ? panel : panel ^ 1;
+      auto request_b = [&]() {
+        if (CROSS) issue_scales();
+        issue_b(kt2, bb2);
+      };
+      // 1
+      read_a(ab, 0, 0);
+      read_raw(bb, it, panel, 1, 0);
+      if (B3) request_b();
+      fetch_end(WA{});
+      multiply(first_c, 0, 0, 1, 0);
+      // 2
+      read_a(ab, 0, 1);
+      read_raw(bb, it, panel, 1, 1);
+      issue_a(kt2, ab2, 0);
+      fetch_end(WB{});
+      multiply(first_c, 0, 1, 1, 1);
+      // 3
+      read_a(ab, 1, 1);
+      read_raw(bb1, kt1, panel1, 0, 0);
+      if (B3) issue_a(kt2, ab2, 1);
+      else request_b();
+      fetch_end(NOWAIT{});
+      multiply(F_{}, 1, 1, 0, 0);
+      // 4
+      read_a(ab, 1, 0);
+      read_raw(bb1, kt1, panel1, 0, 1);
+      if (!B3) issue_a(kt2, ab2, 1);
+      fetch_end(W4{});
+      multiply(F_{}, 1, 0, 0, 1);
+      ab = ab == C::NA - 1 ? 0 : ab + 1;
+      bb = bb1;
+    };
+    if (late) asm volatile("s_barrier" ::: "memory");
+    stage(0, T_{}, F_{});
+    for (int it = 1; it < nk - 2; it++) stage(it, F_{}, F_{});
+    have_n = resolve(pk, nxt);
+    if (have_n) {
+      set_a_sources(nxt);
+      set_b_sources(nxt);
+    }
+    stage(nk - 2, F_{}, T_{});
+    stage(nk - 1, F_{}, F_{});
+    if (!late) asm volatile("s_barrier" ::: "memory");
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));
+    load_epilogue_scales<C::TM, NT_OUT, C::GLU, C::BSRC == BSRC_I8, C::MI, 32>(esc, p, cur.info, wm * C::MI, n_out0, lane_e);
+    // the next tile's stage 0 and the weights of its stage 1 land ahead of the stores, so that the first phases need not count them
+    wait_vmcnt<B3 ? C::A_IPW : C::NA1>();
+    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, C::TM, 32>(acc, esc, p, cur.info, wm * C::MI, n_out0, lane_e);
+    if (!have_n) break;
+    cur = nxt;
+    panel ^= 1;
+  }
+  // nothing may still be writing LDS when the block ends
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  wait_vmcnt<0>();
+}
+
+// ---------------------------------------------------------------------------------------
+// Host side
+// ---------------------------------------------------------------------------------------
+
+// Calls f with the configuration of a call: weight format, GLU, row tiles.
+template <typename F>
+static int with_dlt_cfg(int bsrc, bool glu, int tm, F&& f) {
+  auto fmt = [&](auto tm_c, auto glu_c) {
+    constexpr int TM = decltype(tm_c)::value;
+    constexpr bool GLU = decltype(glu_c)::value;
+    if (bsrc == BSRC_I8) return f(DltCfg<BSRC_I8, GLU, TM>{});
+    if (bsrc == BSRC_I4) return f(DltCfg<BSRC_I4, GLU, TM>{});
+    return f(DltCfg<BSRC_MX4, GLU, TM>{});
+  };
+  auto rows = [&](auto tm_c) { return glu ? fmt(tm_c, std::true_type{}) : fmt(tm_c, std::false_type{}); };
+  return tm == 6 ? rows(std::integral_constant<int, 6>{}) : rows(std::integral_constant<int, 8>{});
+}
+
+template <typename C>
+static int prepare_dlt_cfg() {
+  return reserve_lds(gmm_dlt_kernel<C>, kDltLds, lds_flags<C>());
+}
+
+int prepare_dlt() {
+  for (int tm : {6, 8})
+    for (int bsrc : {BSRC_I8, BSRC_I4, BSRC_MX4})
+      for (bool glu : {false, true})
+        if (int st = with_dlt_cfg(bsrc, glu, tm, [](auto cfg) { return prepare_dlt_cfg<decltype(cfg)>(); })) return st;
+  return MOE_OK;
+}
+
+// LDS of a launch: the stages, and two scale panels of the 4-bit formats
+template <typename C>
+static int dlt_lds_bytes(int K, int i4_group) {
+  const int part = C::NIBBLES ? (int)dlt_scale_part(C::GLU, dlt_scale_row_bytes(C::BSRC, K, i4_group)) : 0;
+  return C::S_BASE + 2 * (C::GLU ? 2 * part : part);
+}
+
+template <typename C>
+static int launch_dlt_cfg(const TiledParams& p0, int M, int G_total, hipStream_t s) {
+  if (int st = prepare_dlt_cfg<C>()) return st;
+  TiledParams p = p0;
+  p.max_m_tiles = max_tiles_for(M, G_total, C::BM);
+  p.tiles_n = cdiv(p.N, C::OUT_BN);
+  const long long tiles = (long long)p.max_m_tiles * p.tiles_n;
+  if (tiles > 0x7fffffffLL) return fail(MOE_ERR_UNSUPPORTED, "gmm: grid too large");
+  if (p.tune <= 0) p.tune = default_super_row(M, G_total, C::BM);
+  // one persistent block per CU; a multiple of 8 keeps "tile id mod 8" equal to the XCD a block runs on
+  int num_cus = 0;
+  if (int st = device_cu_count(&num_cus)) return st;
+  long long blocks = tiles < num_cus ? tiles : num_cus;
+  if (blocks >= 8) blocks -= blocks % 8;
+  gmm_dlt_kernel<C><<<(unsigned)blocks, C::THREADS, dlt_lds_bytes<C>(p.K, p.i4_group), s>>>(p);
+  return check_launch("gmm_dlt_kernel");
+}
+
+bool dlt_takes(int bsrc, int K, int N, int i4_group, long long indexed_lhs_rows, bool wq_kmajor) {
+  // whole 64-value stages, three or more, 32-bit byte offsets (see dls_takes), and a tile's scales twice beside its stages:
+  // MXFP4 to K = 3072, int4 of group 128 to K = 6144 (the lower tiles leave more room, but a format's range is the same on all)
+  if (K % 64 != 0 || K < 192 || wq_kmajor || ((long long)N + 256) * K >= (1LL << 32) || (indexed_lhs_rows + 256) * K * 2 >= (1LL << 32)) return false;
+  if (bsrc == BSRC_I8) return true;
+  if (bsrc == BSRC_I4) return dlt_lds_bytes<DltCfg<BSRC_I4, true, 8>>(K, i4_group) <= kDltLds;
+  return bsrc == BSRC_MX4 && dlt_lds_bytes<DltCfg<BSRC_MX4, true, 8>>(K, 32) <= kDltLds;
+}
+
+int launch_dlt(int bsrc, bool glu, int bm, const TiledParams& p, int M, int G_total, hipStream_t s) {
+  if (!dlt_takes(bsrc, p.K, p.N, p.i4_group, p.ro.row_idx ? p.ro.lhs_rows : 0, p.wq_kmajor != 0))
+    return fail(MOE_ERR_UNSUPPORTED, "gmm: the weight-only stream kernel needs K %% 64 == 0, K >= 192, scales in the default layout and 32-bit byte offsets");
+  if (bm != 256 && bm != 192) return fail(MOE_ERR_INVALID_ARG, "gmm: the weight-only stream kernel has no tiles of %d rows", bm);
+  return with_dlt_cfg(bsrc, glu, bm / 32, [&](auto cfg) { return launch_dlt_cfg<decltype(cfg)>(p, M, G_total, s); });
+}
+
+}  // namespace moe

@@ -1,8 +1,9 @@
-// Grouped matmul: the persistent 256 x 256 kernel for bf16 activations x int8 / int4 / mxfp4 weights (prefill).
+// Grouped matmul: the persistent 256 x 256 kernel for bf16 activations x int4 / mxfp4 weights (prefill) whose block scales do
+// not fit LDS beside the stages of gmm_dlt_kernel (MXFP4 beyond K = 3072, int4 of group 128 beyond 6144, of group 32 beyond 1536).
 //
 // Both operands go global -> LDS without passing through registers (buffer_load ... lds, 1 KB per wave instruction):
 // the activations as XOR-swizzled rows of 128 bytes (64 bf16 values of K), the weights as the RAW bytes of the
-// checkpoint format (64 or 32 bytes per row and stage).  A weight becomes bf16 only in the registers of the wave that
+// checkpoint format (32 bytes per row and stage).  A weight becomes bf16 only in the registers of the wave that
 // multiplies it: each of the 8 waves owns 32 of the tile's 256 weight rows for all 256 activation rows (16 x 2 MFMA
 // tiles of 16 x 16 x 32), so every weight is widened exactly once per block, by the wave that needs it, in the shadow
 // of that wave's own MFMAs, and no weight byte is ever written to LDS by a thread.  The fragments of the next k-step are
@@ -31,20 +32,18 @@ struct DlwCfg {
   // either way) and its 16 registers push lane-constant addresses of the int4 kernel out to scratch memory INSIDE the
   // main loop, where every reload waits for all requests in flight (GPT-OSS second projection: 0.74 ms against 0.48 ms)
   static constexpr int RING = 4;
-  static constexpr bool NIBBLES = BSRC == BSRC_I4 || BSRC == BSRC_MX4;
-  static constexpr int W_ROW = NIBBLES ? BK / 2 : BK;  // raw bytes of a weight row per stage: 32 or 64
+  static constexpr int W_ROW = BK / 2;  // raw bytes of a weight row per stage
   static constexpr int A_STAGE = BM * BKB, B_STAGE = BN * W_ROW, STAGE = A_STAGE + B_STAGE;
   static constexpr int NSTAGE = 3, LDS_BYTES = NSTAGE * STAGE;
   static constexpr int A_IPW = A_STAGE / 1024 / NWAVES;  // activation requests per wave and stage: 4
-  static constexpr int B_IPW = B_STAGE / 1024 / NWAVES;  // weight requests per wave and stage: 2 (int8) or 1
-  static constexpr int B_RPI = 1024 / W_ROW;             // weight rows per request: 16 or 32
+  static constexpr int B_IPW = B_STAGE / 1024 / NWAVES;  // weight requests per wave and stage: 1
+  static constexpr int B_RPI = 1024 / W_ROW;             // weight rows per request: 32
   static constexpr int OUT_BN = GLU ? BN / 2 : BN;
-  static_assert(BSRC != BSRC_SAME && TN == 2 && TM == 16 && LDS_BYTES <= 160 * 1024, "shape");
+  static_assert((BSRC == BSRC_I4 || BSRC == BSRC_MX4) && TN == 2 && TM == 16 && LDS_BYTES <= 160 * 1024, "shape");
   // activations: chunk q of row r sits in slot q ^ swz_a(r) of the row's eight 16-byte slots
   __device__ static __forceinline__ int swz_a(int row) { return (row >> 1) & 7; }
-  // weights: slot q ^ swz_b(r) of the row's four (int8) or two (4-bit) slots, so that the 16 rows a fragment read covers
-  // spread over all banks
-  __device__ static __forceinline__ int swz_b(int row) { return NIBBLES ? (row >> 3) & 1 : (row >> 2) & 3; }
+  // weights: slot q ^ swz_b(r) of the row's two slots, so that the 16 rows a fragment read covers spread over all banks
+  __device__ static __forceinline__ int swz_b(int row) { return (row >> 3) & 1; }
 };
 
 // HALF: the tile list holds tiles of at most 128 rows (32 to 104 rows per expert on average): 8 row tiles per wave are
@@ -60,7 +59,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int N = p.N, K = p.K;
   const uint32_t row_bytes = (uint32_t)K * 2;
-  const uint32_t w_row_bytes = C::NIBBLES ? (uint32_t)K / 2 : (uint32_t)K;
+  const uint32_t w_row_bytes = (uint32_t)K / 2;
   const int num_tiles = p.header[0];
   const int nk = K / C::BK;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
@@ -130,9 +129,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
   const bool i4g32 = C::BSRC == BSRC_I4 && p.i4_group == 32;
   const uint32_t nkg = C::BSRC == BSRC_I4 ? (uint32_t)((K + p.i4_group - 1) / p.i4_group) : (uint32_t)(K / 32);
   const uint32_t s_row_bytes = C::BSRC == BSRC_I4 ? nkg * 2 : nkg;
-  if (C::NIBBLES) s_voff = (uint32_t)((C::GLU ? wave * 16 : wave * C::WN) + lane % 16) * s_row_bytes;
+  s_voff = (uint32_t)((C::GLU ? wave * 16 : wave * C::WN) + lane % 16) * s_row_bytes;
   auto set_s_sources = [&](const Tile& t) {
-    if (!C::NIBBLES) return;
 #pragma unroll
     for (int j = 0; j < C::TN; j++)
       s_desc[j] = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)(C::GLU && j == 1 ? p.rhs_up_scale : p.rhs_scale) + (size_t)t.info.group * N * s_row_bytes),
@@ -144,7 +142,6 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
   uint32_t sc_raw[C::TN] = {0, 0};
   float sc_cur[C::TN][2] = {{1.0f, 1.0f}, {1.0f, 1.0f}};  // [fragment][k-step] of the stage being widened
   auto load_scales = [&](int kt) {
-    if (!C::NIBBLES) return;
 #pragma unroll
     for (int j = 0; j < C::TN; j++) {
       const uint32_t row_off = s_voff + (C::GLU ? 0u : (uint32_t)j * 16 * s_row_bytes);
@@ -154,7 +151,6 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
     }
   };
   auto scales_to_current = [&]() {
-    if (!C::NIBBLES) return;
 #pragma unroll
     for (int j = 0; j < C::TN; j++)
 #pragma unroll
@@ -174,13 +170,11 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
     ga[i % C::RING] = *(const v4i*)(smem + buf * C::STAGE + i * 16 * C::BKB + (a_lane ^ (ks * 64)));
   };
   // raw weight fragment j, k-step ks: row frag_row(j) + lane % 16, the 8 values of K from 32 ks + 8 (lane / 16) on
-  const int b_lane = C::NIBBLES ? (lane % 16) * C::W_ROW + (lane / 16) * 4 : (lane % 16) * C::W_ROW + ((lane / 16) & 1) * 8;
+  const int b_lane = (lane % 16) * C::W_ROW + (lane / 16) * 4;
   const int b_sw = C::swz_b(lane % 16);
-  typedef typename std::conditional<C::NIBBLES, uint32_t, uint2>::type raw_t;
-  raw_t braw[C::TN];
+  uint32_t braw[C::TN];
   auto read_braw = [&](int buf, int ks, int j) {
-    const int slot = C::NIBBLES ? ks : 2 * ks + (lane / 32);  // 16-byte slot of the row that holds the lane's bytes
-    braw[j] = *(const raw_t*)(smem + buf * C::STAGE + C::A_STAGE + frag_row(j) * C::W_ROW + b_lane + ((slot ^ b_sw) << 4));
+    braw[j] = *(const uint32_t*)(smem + buf * C::STAGE + C::A_STAGE + frag_row(j) * C::W_ROW + b_lane + ((ks ^ b_sw) << 4));
   };
   // widened weight fragments: the set of the current k-step and the one being built for the next
   v4i gb[2][C::TN];
@@ -189,11 +183,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
   // piece pc (0 .. 3) of fragment j: two of its eight values -> one register of gb[set][j]
   auto widen_piece = [&](int set, int j, int pc, float sc) {
     uint32_t o;
-    if constexpr (C::BSRC == BSRC_I8) {
-      const int w = (int)(pc < 2 ? braw[j].x : braw[j].y);
-      const int sh = (pc & 1) * 16;
-      o = pack_bf16x2((float)((w << (24 - sh)) >> 24), (float)((w << (16 - sh)) >> 24));
-    } else if constexpr (C::BSRC == BSRC_MX4) {
+    if constexpr (C::BSRC == BSRC_MX4) {
       // (the byte selector is an immediate)
       o = pc == 0   ? __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(braw[j], sc, 0))
           : pc == 1 ? __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(braw[j], sc, 1))
@@ -224,7 +214,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
     constexpr int W0 = HALF ? 4 : 8, WSTEP = HALF ? 1 : 2;  // slots of the eight widening pieces: W0, W0 + WSTEP, ...
     static_assert(2 * (C::A_IPW + C::B_IPW) <= TMX * C::TN && W0 + WSTEP * 4 * C::TN <= TMX * C::TN, "slots");
     float sc[C::TN] = {1.0f, 1.0f};
-    if (RD && C::NIBBLES) {
+    if (RD) {
 #pragma unroll
       for (int j = 0; j < C::TN; j++) sc[j] = rd_ks ? sc_cur[j][1] : sc_cur[j][0];
     }
@@ -332,7 +322,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dlw_kernel(const TiledParam
     // Qwen3 second projection 0.437 -> 0.411 ms)
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
-    load_epilogue_scales<C::TM, NT_OUT, C::GLU, C::BSRC == BSRC_I8, C::MI>(esc, p, cur.info, 0, n_out0, lane_e);
+    load_epilogue_scales<C::TM, NT_OUT, C::GLU, false, C::MI>(esc, p, cur.info, 0, n_out0, lane_e);
     iteration(nk - 1, T_{});
     store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, HALF ? C::TM / 2 : C::TM>(acc, esc, p, cur.info, 0, n_out0, lane_e);
     if (!have_n) break;
@@ -363,7 +353,7 @@ int prepare_dlw() {
 #define MOE_PREP(BSRC)                                       \
   if (!st) st = prepare_dlw_cfg<DlwCfg<BSRC, false>>();      \
   if (!st) st = prepare_dlw_cfg<DlwCfg<BSRC, true>>();
-  MOE_PREP(BSRC_I8) MOE_PREP(BSRC_I4) MOE_PREP(BSRC_MX4)
+  MOE_PREP(BSRC_I4) MOE_PREP(BSRC_MX4)
 #undef MOE_PREP
   return st;
 }
@@ -399,11 +389,10 @@ int launch_dlw(int bsrc, bool glu, bool half, const TiledParams& p, int M, int G
     return fail(MOE_ERR_UNSUPPORTED, "gmm: the weight-only direct-to-LDS kernel needs K %% 64 == 0, K >= 192, scales in the default layout and 32-bit byte offsets");
 #define MOE_DLW_CASE(BSRC) \
   if (bsrc == BSRC) return glu ? launch_dlw_cfg<DlwCfg<BSRC, true>>(half, p, M, G_total, s) : launch_dlw_cfg<DlwCfg<BSRC, false>>(half, p, M, G_total, s);
-  MOE_DLW_CASE(BSRC_I8)
   MOE_DLW_CASE(BSRC_I4)
   MOE_DLW_CASE(BSRC_MX4)
 #undef MOE_DLW_CASE
-  return fail(MOE_ERR_UNSUPPORTED, "gmm: no weight-only direct-to-LDS kernel for weight format %d", bsrc);
+  return fail(MOE_ERR_UNSUPPORTED, "gmm: no 4-bit direct-to-LDS kernel for weight format %d", bsrc);
 }
 
 }  // namespace moe

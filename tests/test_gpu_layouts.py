@@ -327,6 +327,50 @@ def test_weight_only_prefill_kernel_against_the_tiled_kernel_at_size(K, fmt, glu
     assert relerr(got[rows], want, atol_rms=ELEM_ATOL_RMS_CHAINED) <= 2e-2
 
 
+# (k, n): three stages (the shortest stream), an odd number of them (the last 128-value scale group half filled), the last K
+# whose scales fit LDS beside the stages and the first that takes the older kernel; ragged n-tiles
+@pytest.mark.parametrize("fmt,k,n", [("int8", 192, 1992), ("int8", 320, 2056), ("int4", 192, 1992), ("int4", 576, 2056), ("int4", 6144, 1160), ("int4", 6208, 1160),
+                                     ("int4g32", 192, 1992), ("int4g32", 1536, 1160), ("int4g32", 1600, 1160),
+                                     ("mxfp4", 192, 1992), ("mxfp4", 320, 2056), ("mxfp4", 3072, 1160), ("mxfp4", 3136, 1160)])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("rows", [192, 256])
+def test_weight_only_stream_kernel_at_the_edges_of_its_tiles(K, fmt, k, n, glu, rows):
+  """Both tile heights with groups around whole tiles (one row, a tile less one, a tile, a tile and one, none), rows gathered
+  through an index, against the register-staged kernel on the same operands.  Both round the same products of the same bf16
+  weights once per result from f32 sums: half a bf16 step each plus the order of the sums.  (Group-128 int4 and MXFP4: a
+  group's short last tiles run on the decode kernel, whose int4 weights are not rounded; the bound of the test above.)"""
+  from maxtext_amd._lib import MOE_INT4, MOE_MXFP4
+
+  g = torch.Generator(device="cuda").manual_seed(k + n + rows)
+  gs_h = np.array([1, 191, 192, 193, 0, 60, 97, 49, 48, 130, 66, 111, 90, 128, 3, 77] if rows == 192 else
+                  [1, 255, 256, 257, 0, 511, 512, 513, 305, 304, 200, 249, 256, 303, 100, 270], np.int32)
+  e, m = len(gs_h), int(gs_h.sum()) + 7  # 7 rows in no group
+  gs = torch.from_numpy(gs_h).cuda()
+  src = torch.randperm(m, device="cuda", generator=g).to(torch.int32)
+  lhs = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+  grp = {"int4": 128, "int4g32": 32}.get(fmt)
+
+  def weight():
+    if fmt == "int8":
+      return torch.randint(-128, 128, (e, n, k), device="cuda", dtype=torch.int8, generator=g), torch.rand(e, n, device="cuda", generator=g) * 0.01 + 1e-3
+    q = torch.randint(0, 256, (e, n, k // 2), device="cuda", dtype=torch.uint8, generator=g)
+    if fmt == "mxfp4":
+      return q, torch.randint(118, 126, (e, n, k // 32), device="cuda", dtype=torch.uint8, generator=g)
+    return q, (torch.rand(e, n, (k + grp - 1) // grp, device="cuda", generator=g) * 0.01 + 1e-3).to(torch.bfloat16)
+
+  kw = {} if fmt == "int8" else dict(rhs_dtype=MOE_MXFP4, rhs_scale_block_k=32) if fmt == "mxfp4" else dict(rhs_dtype=MOE_INT4, rhs_scale_block_k=grp)
+  w, kw["rhs_scale"] = weight()
+  if glu:
+    kw["rhs_up"], kw["rhs_up_scale"] = weight()
+    kw["act"] = "silu"
+  got = K.gmm_raw(lhs, w, gs, lhs_row_idx=src, **kw)
+  ref = K.gmm_raw(lhs, w, gs, lhs_row_idx=src, kernel="tiled", **kw)
+  assert relerr(got, ref, elementwise=fmt not in ("int4", "mxfp4")) <= (8e-3 if fmt in ("int4", "mxfp4") else 1e-3)
+  assert torch.all(got[int(gs_h.sum()):] == 0)
+  direct = K.gmm_raw(lhs[src.long()].contiguous(), w, gs, **kw)
+  assert torch.equal(direct, got)
+
+
 @pytest.mark.parametrize("glu", [False, True])
 @pytest.mark.parametrize("indexed", [False, True])
 def test_fp8_prefill_stream_kernel_against_the_tiled_kernel_at_size(K, glu, indexed):

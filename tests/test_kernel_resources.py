@@ -16,7 +16,7 @@ import pytest
 
 from maxtext_amd import build
 
-STREAM_KERNELS = ["moe_gmm_dls.hip", "moe_gmm_dlw.hip", "moe_gmm_f8s.hip"]
+STREAM_KERNELS = ["moe_gmm_dls.hip", "moe_gmm_dlw.hip", "moe_gmm_dlt.hip", "moe_gmm_f8s.hip"]
 
 
 def _assembly(src, tmp):
