@@ -869,6 +869,7 @@ __device__ __forceinline__ float quant_value(float f, float sc, float inv, int r
     q = fmaf(fmaf(-est, sc, f), inv, est);
     q = fmaf(fmaf(-q, sc, f), inv, q);
     q = fabsf(est) < 1024.0f ? q : est;  // (beyond the range by far: a static scale; the residual may overflow there)
+    q = copysignf(q, f);  // (a sum of zeros is +0: -0 would lose its sign, which e4m3 keeps)
   } else {
     q = sc == 0.f ? 0.f : f / sc;
   }

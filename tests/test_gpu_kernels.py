@@ -215,10 +215,12 @@ def test_gather_rows_fp8_block_quant(K, d):
 @pytest.mark.parametrize("d", [2040, 2048, 2056, 4096, 4104, 8192, 8200])
 @pytest.mark.parametrize("block_k", [0, 128, 256, 512])
 def test_gather_rows_fp8_at_chunk_edges_and_extreme_scales(K, d, block_k):
-  """Rows just within and just past what 1, 2, 4 and 8 chunks per thread hold; magnitudes from subnormal to the largest."""
+  """Rows just within and just past what 1, 2, 4 and 8 chunks per thread hold; magnitudes from subnormal to the largest, zeros of
+  both signs."""
   g = torch.Generator().manual_seed(d + block_k)
   x = (torch.randn(24, d, generator=g) * torch.logspace(-38, 37, 24)[:, None]).to(torch.bfloat16)
   x[7] = 0
+  x[::3, ::5] = -0.0  # (the sign of a zero is part of the value)
   q, s = K.gather_rows(cuda(x), None, 1, out_dtype=torch.float8_e4m3fn, block_k=block_k)
   width = block_k or d
   pad = torch.nn.functional.pad(x, (0, -d % width))
