@@ -582,38 +582,22 @@ def gmm_raw(lhs, rhs, group_sizes, *, lhs_scale=None, rhs_scale=None, rhs_up=Non
     raise ValueError(f"unknown kernel family {kernel!r}")
   lib = _lib.load()
   g_total = group_sizes.numel()
-  wsb = lib.moe_gmm_workspace_bytes(m, g_total)
-  ws = workspace if workspace is not None else torch.empty((max(wsb, 16),), dtype=torch.uint8, device=lhs.device)
-  a = _lib.GmmArgs()
-  a.struct_size = ctypes.sizeof(_lib.GmmArgs)
-  a.lhs, a.lhs_scale = lhs.data_ptr(), (lhs_scale.data_ptr() if lhs_scale is not None else None)
-  a.rhs, a.rhs_scale = rhs.data_ptr(), (rhs_scale.data_ptr() if rhs_scale is not None else None)
-  a.rhs_up = rhs_up.data_ptr() if rhs_up is not None else None
-  a.rhs_up_scale = rhs_up_scale.data_ptr() if rhs_up_scale is not None else None
-  a.group_sizes, a.out = group_sizes.data_ptr(), out.data_ptr()
-  a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * ws.element_size()
-  a.M, a.K, a.N = m, kdim, n
-  a.num_groups_total, a.num_groups_local, a.group_offset = g_total, g_local, int(group_offset)
-  a.lhs_dtype, a.rhs_dtype = _LHS_DTYPE_CODE[lhs.dtype], rhs_dtype
-  a.lhs_scale_block_k, a.rhs_scale_block_n, a.rhs_scale_block_k = int(lhs_scale_block_k), int(rhs_scale_block_n), int(rhs_scale_block_k)
-  a.act = _lib.ACT_BY_NAME[act]
-  a.act_limit = float(act_limit)
-  a.out_dtype = _lib.MOE_BF16 if out_dtype == torch.bfloat16 else _lib.MOE_F32
-  a.lhs_row_idx = lhs_row_idx.data_ptr() if lhs_row_idx is not None else None
-  a.lhs_row_idx_div, a.lhs_rows = int(lhs_row_idx_div), lhs_rows
-  a.out_row_scale = out_row_scale.data_ptr() if out_row_scale is not None else None
+  ws = workspace if workspace is not None else gmm_workspace(m, g_total, lhs.device)
+  p = _lib.ptr
   if group_offset_dev is not None:
     _need(group_offset_dev, "group_offset_dev", torch.int32)
     if group_offset_dev.numel() != 1:
       raise ValueError("group_offset_dev must hold one value")
-    a.group_offset_dev = group_offset_dev.data_ptr()
-  a.rhs_bias = rhs_bias.data_ptr() if rhs_bias is not None else None
-  a.rhs_up_bias = rhs_up_bias.data_ptr() if rhs_up_bias is not None else None
-  a.partial_sum = partial_sum.data_ptr() if partial_sum is not None else None
-  a.partial_sum_up = partial_sum_up.data_ptr() if partial_sum_up is not None else None
-  a.flags = ((_lib.MOE_GMM_KEEP_OTHER_ROWS if keep_other_rows else 0) | (_lib.MOE_GMM_RHS_KN if rhs_kn else 0)
-             | (_lib.MOE_GMM_RHS_SCALE_KMAJOR if rhs_scale_kmajor else 0) | (_lib.MOE_GMM_RHS_SCALE_SHARED if rhs_scale_shared else 0)
-             | (_lib.MOE_GMM_SAME_GROUPS if same_groups and workspace is not None else 0))
+  flags = ((_lib.MOE_GMM_KEEP_OTHER_ROWS if keep_other_rows else 0) | (_lib.MOE_GMM_RHS_KN if rhs_kn else 0)
+           | (_lib.MOE_GMM_RHS_SCALE_KMAJOR if rhs_scale_kmajor else 0) | (_lib.MOE_GMM_RHS_SCALE_SHARED if rhs_scale_shared else 0)
+           | (_lib.MOE_GMM_SAME_GROUPS if same_groups and workspace is not None else 0))
+  # (in the structure's order: one call instead of an attribute write per field)
+  a = _lib.GmmArgs(
+      _lib.GMM_ARGS_BYTES, lhs.data_ptr(), p(lhs_scale), rhs.data_ptr(), p(rhs_scale), p(rhs_up), p(rhs_up_scale), group_sizes.data_ptr(), out.data_ptr(),
+      ws.data_ptr(), ws.numel() * ws.element_size(), m, kdim, n, g_total, g_local, int(group_offset), _LHS_DTYPE_CODE[lhs.dtype], rhs_dtype,
+      int(lhs_scale_block_k), int(rhs_scale_block_n), int(rhs_scale_block_k), _lib.ACT_BY_NAME[act], float(act_limit),
+      _lib.MOE_BF16 if out_dtype == torch.bfloat16 else _lib.MOE_F32, int(lhs_row_idx_div), lhs_rows, 0,
+      p(rhs_bias), p(rhs_up_bias), p(partial_sum), p(partial_sum_up), flags, 0, p(lhs_row_idx), p(out_row_scale), p(group_offset_dev))
   code = _lib.GMM_KERNEL_BY_NAME[kernel]
   if code or raster:
     st = lib.moe_gmm_tuned(ctypes.byref(a), code, int(raster), _lib.current_stream())
