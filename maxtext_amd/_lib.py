@@ -103,6 +103,7 @@ SIGNATURES = {
     "moe_gather_rows": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p]),
     "moe_gmm_workspace_bytes": (c_size_t, [c_int, c_int]),
+    "moe_gmm_split_workspace_bytes": (c_size_t, [c_int, c_int]),
     "moe_gmm_rhs_kn_supported": (c_int, [c_int, c_int, c_int, c_int]),
     "moe_gmm_lhs_e5m2_supported": (c_int, [c_int, c_int, c_int, c_int]),
     "moe_gmm_fp8_rhs_kn_supported": (c_int, [c_int, c_int, c_int, c_int]),

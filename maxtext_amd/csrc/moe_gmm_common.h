@@ -221,6 +221,10 @@ struct TiledParams {
   int lhs_nb, lhs_qb, rhs_nb, rhs_qb, rhs_bs_gstride;
   // weight-only int8 / int4 with K-major block scales [G, nb, N] (f32), multiplied in while the weights are widened
   int wq_kmajor;
+  // tiles of the last, partly filled round cut along K (split_of): partial sums, one slot of a tile per block, and arrival
+  // counters, or NULL
+  uint8_t* split_parts;
+  int32_t* split_counts;
   RowOpts ro;
 };
 
@@ -485,15 +489,58 @@ __device__ __forceinline__ void dma16_buffer(const v4i& rsrc, uint32_t voff, uin
 struct StreamTile {
   TileInfo info;
   int n0, id;
+  int k0, k1;  // the stages that this block runs: 0 .. all of them, or its part of a tile cut along K
 };
 struct TilePeek {  // a tile record that has been requested but not looked at yet
   TileInfo ti;
   int n0, id;
   bool valid;
 };
+// ---- tiles cut along K ----
+// A launch of 256 persistent blocks takes ceil(tiles / 256) rounds, and the tiles of a last round that is at most half full leave
+// half of the chip or more idle (second projection of the Mixtral shape at 127 rows per expert: 128 tiles in all).  Those tiles
+// are cut into 2 .. kSplitMost parts along K, one per block of the XCD that has the tile (each XCD owns a range of the tiles and
+// walks it with its 32 blocks).  A wave writes its partial sums to its block's slot, counts itself in, and the wave that comes
+// last adds the parts up and runs the epilogue: nobody waits for anybody.  The sums are added in the order of K whoever comes
+// last, so results do not change from run to run.
+// The last part is kSplitSkew stages longer than the others: its waves then mostly come last, find everything there and need
+// not write their own (15 us for a 256-row tile of every block at once): Mixtral second projection at 127 rows per expert 144 us
+// uncut, 122 in equal parts, 112 with 4 or 8 stages more, 115 with 14.  A part of fewer than kSplitStages stages costs more in
+// the joining than it gains (Mixtral first projection, 32 stages, at 60 to 212 rows 4 to 6 % slower in 3 and 4 parts, 0 to 4 %
+// faster in 2).  Mixtral shape, launches alone: int8 second projection at 512 / 2048 rows per expert 271 -> 236, 836 -> 783 us, first
+// 512 -> 487, 1583 -> 1564, bf16 second 276 -> 197 at 127 rows, 1578 -> 1477 at 2048.  Only gmm_dls_kernel cuts: on gmm_dlt_kernel
+// and gmm_f8s_kernel launches alone gained as well (GPT-OSS int4 second projection 151 -> 121, DeepSeek first 1647 -> 1610), but
+// layers run at the power limit there, and the idle blocks' share of it went to the others (GPT-OSS int4 layer at 1023 tokens
+// 358 -> 361, DeepSeek at 4099 3280 -> 3295).
+constexpr int kSplitBlocks = 256, kSplitPerXcd = kSplitBlocks / 8, kSplitWaves = 8;
+constexpr int kSplitMost = 4, kSplitStages = 12, kSplitSkew = 8;
+constexpr size_t kSplitCountBytes = (size_t)kSplitBlocks * kSplitWaves * 4, kSplitSlotBytes = 256 * 256 * 4;
+struct Split {
+  int loc;  // index in the XCD's range, or -1: the block has nothing there
+  int part, parts, rest;
+};
+// loc: the block's place in its XCD's range of tiles; nk: stages of a whole tile
+__device__ __forceinline__ Split split_of(const TiledParams& p, int xcd_tiles, int loc, int nk) {
+  Split sp{loc < xcd_tiles ? loc : -1, 0, 1, 0};
+  const int rest = xcd_tiles % kSplitPerXcd, full = xcd_tiles - rest;
+  if (p.split_parts && rest > 0 && loc >= full) {
+    const int parts = min(min(kSplitPerXcd / rest, kSplitMost), nk / kSplitStages);
+    if (parts > 1) {
+      const int j = loc - full;  // the block's own index in the XCD
+      sp = j < rest * parts ? Split{full + j % rest, j / rest, parts, rest} : Split{-1, 0, 1, 0};
+    }
+  }
+  return sp;
+}
+// tiles in the range of XCD `xcd`, and the range's first tile in the order
+__device__ __forceinline__ int xcd_range(int total, int xcd, int* first) {
+  const int q = total / 8, rem = total % 8;
+  *first = xcd * q + min(xcd, rem);
+  return q + (xcd < rem ? 1 : 0);
+}
 // The block's first id >= id0 that names an existing m-tile; its record is requested, not waited for.
 template <int OUT_BN>
-__device__ __forceinline__ TilePeek peek_tile(const TiledParams& p, int num_tiles, int id0) {
+__device__ __forceinline__ TilePeek peek_tile(const TiledParams& p, int num_tiles, int id0, int nk = 0) {
   // the order covers the tiles that exist (the count the tile map left on the device), not the host's upper bound: with
   // the bound, the ids of tiles that do not exist all fall into the last XCD's range and leave its blocks idle while the
   // other seven work through full ranges (GPT-OSS at 4096 tokens: 97 slots for 80 m-tiles, 8.7 rounds instead of 7.2)
@@ -503,12 +550,13 @@ __device__ __forceinline__ TilePeek peek_tile(const TiledParams& p, int num_tile
   pk.n0 = 0;
   pk.id = total;
   pk.ti = TileInfo{-1, 0, 0, 0};
-  const int q = total / 8, rem = total % 8;
-  const int GSM = p.tune > 0 ? p.tune : 8;
-  const int width = GSM * p.tiles_n;
-  for (int id = id0; id < total; id += gridDim.x) {
-    const int xcd = id % 8, loc = id / 8;
-    const int logical = xcd < rem ? xcd * (q + 1) + loc : rem * (q + 1) + (xcd - rem) * q + loc;
+  int first;
+  const int count = xcd_range(total, id0 % 8, &first);
+  const int loc = __builtin_amdgcn_readfirstlane(split_of(p, count, id0 / 8, nk).loc);
+  if (loc >= 0) {
+    const int GSM = p.tune > 0 ? p.tune : 8;
+    const int width = GSM * p.tiles_n;
+    const int logical = first + loc;
     const int sg = logical / width, first_m = sg * GSM;
     const int gsz = min(num_tiles - first_m, GSM);
     const int m_idx = first_m + (logical % width) % gsz;
@@ -518,16 +566,16 @@ __device__ __forceinline__ TilePeek peek_tile(const TiledParams& p, int num_tile
     const rec_t rec = *(const __attribute__((address_space(4))) rec_t*)(uintptr_t)(p.tiles + m_idx);
     pk.ti = TileInfo{rec[0], rec[1], rec[2], rec[3]};
     pk.n0 = ((logical % width) / gsz) * OUT_BN;
-    pk.id = id;
+    pk.id = id0;
     pk.valid = true;
-    break;
   }
   return pk;
 }
 // Turns a requested record into the block's next tile that needs the matmul (its fields uniform, in scalar registers);
 // tiles of rows that belong to no local group are written as zeros on the way, and the search goes on from there.
+// nk: stages of a whole tile
 template <int OUT_BN, int THREADS>
-__device__ __forceinline__ bool resolve_tile(const TiledParams& p, int num_tiles, TilePeek pk, StreamTile& t, int tid) {
+__device__ __forceinline__ bool resolve_tile(const TiledParams& p, int num_tiles, TilePeek pk, StreamTile& t, int tid, int nk = 0) {
   while (pk.valid) {
     t.info.group = __builtin_amdgcn_readfirstlane(pk.ti.group);
     t.info.row0 = __builtin_amdgcn_readfirstlane(pk.ti.row0);
@@ -535,11 +583,88 @@ __device__ __forceinline__ bool resolve_tile(const TiledParams& p, int num_tiles
     t.info.pad = 0;
     t.n0 = __builtin_amdgcn_readfirstlane(pk.n0);
     t.id = __builtin_amdgcn_readfirstlane(pk.id);
-    if (t.info.group >= 0) return true;
+    if (t.info.group >= 0) {
+      int first;
+      const Split sp = split_of(p, xcd_range(num_tiles * p.tiles_n, t.id % 8, &first), t.id / 8, nk);
+      const int cut = sp.parts > 1 ? nk - kSplitSkew : nk;
+      t.k0 = __builtin_amdgcn_readfirstlane(cut * sp.part / sp.parts);
+      t.k1 = __builtin_amdgcn_readfirstlane(sp.part + 1 == sp.parts ? nk : cut * (sp.part + 1) / sp.parts);
+      return true;
+    }
     zero_fill_tile(p.out, p.ro, t.info.row0, t.info.nrows, t.n0, OUT_BN, p.N, tid, THREADS);
-    pk = peek_tile<OUT_BN>(p, num_tiles, t.id + gridDim.x);
+    pk = peek_tile<OUT_BN>(p, num_tiles, t.id + gridDim.x, nk);
   }
   return false;
+}
+// f(0), f(1), .. f(N - 1), each number a constant
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void for_each_step(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    for_each_step<N, I + 1>(f);
+  }
+}
+// A wave's share of a tile of several parts: true in the wave that comes last, with all parts' sums in acc.  Stores and loads go
+// past the XCD's L2 (sc1): the parts' blocks usually share one, but nothing guarantees it.
+template <int TM, int TN, typename acc_t>
+__device__ __forceinline__ bool join_parts(acc_t (&acc)[TN][TM], const TiledParams& p, int num_tiles, const StreamTile& t, int nk, int wave, int tid) {
+  // (what is used here gets registers of its own here: through the main loop there are none to spare)
+  asm volatile("" : "+v"(tid));
+#pragma unroll
+  for (int j = 0; j < TN; j++)
+#pragma unroll
+    for (int i = 0; i < TM; i++) asm volatile("" : "+v"(acc[j][i]));
+  int first;
+  const Split sp = split_of(p, xcd_range(num_tiles * p.tiles_n, t.id % 8, &first), t.id / 8, nk);
+  const int peer_step = __builtin_amdgcn_readfirstlane(8 * sp.rest), peer = __builtin_amdgcn_readfirstlane((int)blockIdx.x - sp.part * 8 * sp.rest);  // the blocks: part q in peer + q * peer_step
+  constexpr int kSc1 = 16, kRowBytes = kSplitWaves * kWave * 16;
+  static_assert(sizeof(acc_t) == 16 && (size_t)TM * TN * kRowBytes <= kSplitSlotBytes, "a slot holds the tile");
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  auto slot = [&](int part) {
+    return __builtin_amdgcn_make_buffer_rsrc(p.split_parts + (size_t)(peer + part * peer_step) * kSplitSlotBytes, 0, (int)kSplitSlotBytes, 0x00020000);
+  };
+  int32_t* count = p.split_counts + peer * kSplitWaves + wave;
+  const int last = sp.parts - 1;
+  auto value = [](int32_t v) { return __builtin_amdgcn_readfirstlane(v); };
+  // the sums of parts 0 .. n - 1, in this order, then this wave's own if it is the last part's
+  auto gather = [&](int n, bool own) __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    for_each_step<TN * ((TM + 3) / 4)>([&](auto step) {  // (four tiles at a time: registers)
+      constexpr int j = decltype(step)::value / ((TM + 3) / 4), i0 = decltype(step)::value % ((TM + 3) / 4) * 4, n_i = TM - i0 < 4 ? TM - i0 : 4;
+      acc_t v[n_i];
+      for (int q = 0; q < n; q++) {
+        const auto from = slot(q);
+#pragma unroll
+        for (int i = 0; i < n_i; i++) {
+          const acc_t x = __builtin_bit_cast(acc_t, __builtin_amdgcn_raw_buffer_load_b128(from, tid * 16, (j * TM + i0 + i) * kRowBytes, kSc1));
+          v[i] = q ? v[i] + x : x;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < n_i; i++) acc[j][i0 + i] = own ? v[i] + acc[j][i0 + i] : v[i];
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  // (zero again for the next launch)
+  auto reset = [&]() { if (tid % kWave == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  if (sp.part == last && value(__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == last) {
+    reset();
+    gather(last, true);
+    return true;
+  }
+  const auto mine = slot(sp.part);
+#pragma unroll
+  for (int j = 0; j < TN; j++)
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[j][i]), mine, tid * 16, (j * TM + i) * kRowBytes, kSc1);
+  wait_vmcnt<0>();
+  int before = 0;
+  if (tid % kWave == 0) before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (value(before) != last) return false;
+  reset();
+  gather(sp.parts, false);
+  return true;
 }
 
 struct SkinnyParams {
@@ -609,6 +734,21 @@ constexpr int kMaxDevices = 64;
 
 int current_device(int* dev);
 int device_cu_count(int* cus);
+
+// Blocks of a stream kernel: one persistent block per CU (the LDS footprint allows no more); a multiple of 8 keeps "tile id mod
+// 8" equal to the XCD a block runs on.  With room for partial sums all of them, so that a last round can be cut along K.
+static inline int stream_blocks(long long tiles, TiledParams& p, int* blocks) {
+  int cus = 0;
+  if (int st = device_cu_count(&cus)) return st;
+  if (cus < kSplitBlocks || tiles < 8) p.split_parts = nullptr;  // (split_of counts on 32 blocks to an XCD)
+  if (p.split_parts) {
+    *blocks = kSplitBlocks;
+    return MOE_OK;
+  }
+  *blocks = (int)(tiles < cus ? tiles : cus);
+  if (*blocks >= 8) *blocks -= *blocks % 8;
+  return MOE_OK;
+}
 
 template <typename K>
 static int reserve_lds(K kernel, int bytes, bool (&done)[kMaxDevices]) {

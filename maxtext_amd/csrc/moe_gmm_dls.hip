@@ -87,8 +87,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
 
   using Tile = StreamTile;
   using Peek = TilePeek;
-  auto peek_from = [&](int id0) { return peek_tile<C::OUT_BN>(p, num_tiles, id0); };
-  auto resolve = [&](Peek pk, Tile& t) { return resolve_tile<C::OUT_BN, C::THREADS>(p, num_tiles, pk, t, tid); };
+  auto peek_from = [&](int id0) { return peek_tile<C::OUT_BN>(p, num_tiles, id0, nk); };
+  auto resolve = [&](Peek pk, Tile& t) { return resolve_tile<C::OUT_BN, C::THREADS>(p, num_tiles, pk, t, tid, nk); };
 
   // ---- the loading side of the stream ---------------------------------------------------------------------------
   // A stage arrives in four halves of two requests per wave (1 KB = 8 rows x 128 bytes each; the second half of a lower tile:
@@ -111,13 +111,20 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   auto set_a_sources = [&](const Tile& t) {
     if (p.ro.row_idx) {
       a_desc = buffer_desc(p.lhs, clamp_u32((size_t)p.ro.lhs_rows * row_bytes));
+      // (opaque: rows and chunks of the requests are made again for each tile; kept, they do not fit the registers of the
+      // 256-row instances and come back from scratch memory, each behind the requests in flight)
+      int lane_s = lane, wave_s = wave_v;
+      asm volatile("" : "+v"(lane_s), "+v"(wave_s));
       int rows[C::A_IPW];
 #pragma unroll
-      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + a_req_row(i, wave_v) + lane / 8, p.M - 1);
+      for (int i = 0; i < C::A_IPW; i++) rows[i] = min(t.info.row0 + a_req_row(i, wave_s) + lane_s / 8, p.M - 1);
       lhs_rows_of<C::A_IPW>(p.ro, rows);
       // (rows past the tile's end: one row past the descriptor's, i.e. zeros without a request to memory)
 #pragma unroll
-      for (int i = 0; i < C::A_IPW; i++) a_voff[i] = lane_off(a_req_row(i, wave_v), (uint32_t)(a_req_row(i, wave_v) + lane / 8 < t.info.nrows ? rows[i] : p.ro.lhs_rows));
+      for (int i = 0; i < C::A_IPW; i++) {
+        const int r = a_req_row(i, wave_s) + lane_s / 8;
+        a_voff[i] = (uint32_t)(r < t.info.nrows ? rows[i] : p.ro.lhs_rows) * row_bytes + (uint32_t)(((lane_s % 8) ^ C::swz(r)) << 4);
+      }
     } else {
       a_desc = buffer_desc(p.lhs + (size_t)t.info.row0 * row_bytes, clamp_u32((size_t)t.info.nrows * row_bytes));
     }
@@ -272,19 +279,28 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
   // ---- head of the stream: the first tile's stage 0, and stage 1 up to the half that its first phase requests ----
   set_a_sources(cur);
   set_b_sources(cur);
-  issue_a(0, 0, 0); issue_b(0, 0, 0); issue_b(0, 0, 1); issue_a(0, 0, 1);
-  issue_a(1, 1, 0); issue_b(1, 1, 0); issue_b(1, 1, 1);
+  issue_a(cur.k0, 0, 0); issue_b(cur.k0, 0, 0); issue_b(cur.k0, 0, 1); issue_a(cur.k0, 0, 1);
+  issue_a(cur.k0 + 1, 1, 0); issue_b(cur.k0 + 1, 1, 0); issue_b(cur.k0 + 1, 1, 1);
   wait_vmcnt<0>();
   asm volatile("s_barrier" ::: "memory");
 
+  auto epilogue = [&]() __attribute__((always_inline)) {
+    const int n_out0 = cur.n0 + (C::GLU ? wn * (C::WN / 2) : wn * C::WN);
+    EpilogueScales<C::TM, NT_OUT, C::GLU> esc;
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));
+    load_epilogue_scales<C::TM, NT_OUT, C::GLU, true, C::MI, 32>(esc, p, cur.info, wm * C::MI, n_out0, lane_e);
+    // the next tile's stage 0 lands ahead of the stores, so that its phases need not count them (stage 1's three halves are
+    // waited for in that stage's last phase, the stores with them)
+    wait_vmcnt<6>();
+    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, C::TM, 32>(acc, esc, p, cur.info, wm * C::MI, n_out0, lane_e);
+  };
   int cb = 0;  // buffer of the current stage
   while (true) {
     // the record of the block's next tile is requested now and looked at two stages before this tile ends
     Peek pk = peek_from(cur.id + gridDim.x);
     bool have_n = false;
-    const int n_out0 = cur.n0 + (C::GLU ? wn * (C::WN / 2) : wn * C::WN);
-    EpilogueScales<C::TM, NT_OUT, C::GLU> esc;
-    auto stream_kt = [&](int s) { return s < nk ? s : (have_n ? s - nk : nk - 1); };
+    auto stream_kt = [&](int s) { return s < cur.k1 ? s : have_n ? nxt.k0 + s - cur.k1 : cur.k1 - 1; };
     // Stage `it`, in four phases.  first: the stage's data landed before the tile began.  cross: the stream moves on to the next tile after the first phase.
     auto stage_head = [&](int it, auto first_c) __attribute__((always_inline)) {
       using WA = typename std::conditional<decltype(first_c)::value, NOWAIT, W1>::type;
@@ -320,32 +336,28 @@ __global__ __launch_bounds__(C::THREADS, 2) void gmm_dls_kernel(const TiledParam
       cb ^= 1;
     };
     if (late) asm volatile("s_barrier" ::: "memory");
-    stage_head(0, T_{});
-    stage_rest(0, T_{});
-    for (int it = 1; it < nk - 2; it++) {
+    stage_head(cur.k0, T_{});
+    stage_rest(cur.k0, T_{});
+    for (int it = cur.k0 + 1; it < cur.k1 - 2; it++) {
       stage_head(it, F_{});
       stage_rest(it, F_{});
     }
-    stage_head(nk - 2, F_{});
+    stage_head(cur.k1 - 2, F_{});
     have_n = resolve(pk, nxt);
     if (have_n) {
       set_a_sources(nxt);
       set_b_sources(nxt);
     }
-    stage_rest(nk - 2, F_{});
-    stage_head(nk - 1, F_{});
-    stage_rest(nk - 1, F_{});
+    stage_rest(cur.k1 - 2, F_{});
+    stage_head(cur.k1 - 1, F_{});
+    stage_rest(cur.k1 - 1, F_{});
     if (!late) asm volatile("s_barrier" ::: "memory");
-    int lane_e = lane;
-    asm volatile("" : "+v"(lane_e));
-    load_epilogue_scales<C::TM, NT_OUT, C::GLU, true, C::MI, 32>(esc, p, cur.info, wm * C::MI, n_out0, lane_e);
-    // the next tile's stage 0 lands ahead of the stores, so that its phases need not count them (stage 1's three halves are
-    // waited for in that stage's last phase, the stores with them)
-    wait_vmcnt<6>();
-    store_epilogue<C::TM, C::TN, NT_OUT, C::GLU, C::TM, 32>(acc, esc, p, cur.info, wm * C::MI, n_out0, lane_e);
+    if (cur.k1 - cur.k0 != nk) break;  // (a part of a tile is the last that a block has)
+    epilogue();
     if (!have_n) break;
     cur = nxt;
   }
+  if (cur.k1 - cur.k0 != nk && join_parts(acc, p, num_tiles, cur, nk, wave, tid)) epilogue();
   // nothing may still be writing LDS when the block ends
   __builtin_amdgcn_s_waitcnt(0xC07F);
   wait_vmcnt<0>();
@@ -398,12 +410,8 @@ static int launch_dls_cfg(const TiledParams& p0, int M, int G_total, hipStream_t
   const long long tiles = (long long)p.max_m_tiles * p.tiles_n;
   if (tiles > 0x7fffffffLL) return fail(MOE_ERR_UNSUPPORTED, "gmm: grid too large");
   if (p.tune <= 0) p.tune = default_super_row(M, G_total, C::BM);
-  // one persistent block per CU (the LDS footprint allows no more); a multiple of 8 keeps "tile id mod 8"
-  // equal to the XCD a block runs on
-  int num_cus = 0;
-  if (int st = device_cu_count(&num_cus)) return st;
-  long long blocks = tiles < num_cus ? tiles : num_cus;
-  if (blocks >= 8) blocks -= blocks % 8;
+  int blocks = 0;
+  if (int st = stream_blocks(tiles, p, &blocks)) return st;
   gmm_dls_kernel<C><<<(unsigned)blocks, C::THREADS, C::LDS_BYTES, s>>>(p);
   return check_launch("gmm_dls_kernel");
 }

@@ -492,7 +492,7 @@ def gmm_raw(lhs, rhs, group_sizes, *, lhs_scale=None, rhs_scale=None, rhs_up=Non
             group_offset=0, out=None, kernel=None, raster=0, rhs_bias=None, rhs_up_bias=None, partial_sum=None, partial_sum_up=None,
             keep_other_rows=False, rhs_kn=False, rhs_scale_kmajor=False, rhs_scale_shared=False, out_dtype=torch.bfloat16,
             lhs_row_idx=None, lhs_row_idx_div=1, out_row_scale=None, num_rows=None, workspace=None, same_groups=False,
-            group_offset_dev=None):
+            group_offset_dev=None, split=False):
   """Grouped matmul on native layouts: lhs [M,K], rhs [G,N,K] (INT4 / MXFP4: uint8 [G,N,K/2]).
   rhs_kn: rhs is [G,K,N] instead (bf16 x bf16 on shapes `gmm_rhs_kn_supported` accepts, fp8 x fp8 on shapes
   `gmm_fp8_rhs_kn_supported` accepts; no rhs_up).
@@ -501,7 +501,8 @@ def gmm_raw(lhs, rhs, group_sizes, *, lhs_scale=None, rhs_scale=None, rhs_up=Non
   rhs_scale_shared; bn = -1: one scale for all channels.
   lhs_row_idx [M] int32: row i of the product reads lhs row lhs_row_idx[i] // lhs_row_idx_div (lhs then has any number of
   rows); out_row_scale [M] f32 multiplies the result rows.  kernel / raster select a kernel family (moe_gmm_tuned).
-  workspace: a caller-held uint8 buffer of moe_gmm_workspace_bytes; same_groups: MOE_GMM_SAME_GROUPS (group_sizes and the
+  workspace: a caller-held uint8 buffer of moe_gmm_workspace_bytes or more (gmm_workspace); without one, split allocates it with
+  room for the sums of tiles cut along K; same_groups: MOE_GMM_SAME_GROUPS (group_sizes and the
   workspace are those of the previous call, untouched: its tile list is used again when the tile height agrees).
   group_offset_dev: int32 [1] on the device; replaces group_offset without the host ever reading it."""
   _need(lhs, "lhs", None, 2)
@@ -582,7 +583,7 @@ def gmm_raw(lhs, rhs, group_sizes, *, lhs_scale=None, rhs_scale=None, rhs_up=Non
     raise ValueError(f"unknown kernel family {kernel!r}")
   lib = _lib.load()
   g_total = group_sizes.numel()
-  ws = workspace if workspace is not None else gmm_workspace(m, g_total, lhs.device)
+  ws = workspace if workspace is not None else gmm_workspace(m, g_total, lhs.device, split=split)
   p = _lib.ptr
   if group_offset_dev is not None:
     _need(group_offset_dev, "group_offset_dev", torch.int32)
@@ -608,10 +609,10 @@ def gmm_raw(lhs, rhs, group_sizes, *, lhs_scale=None, rhs_scale=None, rhs_up=Non
 
 
 def gmm_route(m, k, n, num_groups_total, *, lhs_dtype, rhs_dtype, lhs_scale_block_k=0, rhs_scale_block_n=1, rhs_scale_block_k=0,
-              glu=False, num_groups_local=None, indexed_rows=0, rhs_kn=False, kernel=None):
+              glu=False, num_groups_local=None, indexed_rows=0, rhs_kn=False, kernel=None, split=False):
   """(kernel name, tile rows, tail rows, tail height) that `gmm_raw` runs a call of these sizes on (moe_gmm_route: the library's
   own choice, nothing is launched and no GPU is needed).  lhs_dtype / rhs_dtype: MOE_* codes.  indexed_rows > 0: lhs has that
-  many rows, read through an index.  Raises where gmm_raw would."""
+  many rows, read through an index.  split: with a workspace of gmm_workspace(split=True).  Raises where gmm_raw would."""
   lib = _lib.load()
   a = _lib.GmmArgs()
   a.struct_size = _lib.GMM_ARGS_BYTES
@@ -622,7 +623,7 @@ def gmm_route(m, k, n, num_groups_total, *, lhs_dtype, rhs_dtype, lhs_scale_bloc
   a.rhs_scale = None if rhs_dtype == _lib.MOE_BF16 else some
   if glu:
     a.rhs_up, a.rhs_up_scale, a.act = some, a.rhs_scale, _lib.MOE_ACT_SILU
-  a.workspace_bytes = lib.moe_gmm_workspace_bytes(m, num_groups_total)
+  a.workspace_bytes = _gmm_workspace_bytes(m, num_groups_total, split)
   a.M, a.K, a.N, a.num_groups_total, a.num_groups_local = m, k, n, num_groups_total, num_groups_local or num_groups_total
   a.lhs_dtype, a.rhs_dtype = lhs_dtype, rhs_dtype
   a.lhs_scale_block_k, a.rhs_scale_block_n, a.rhs_scale_block_k = lhs_scale_block_k, rhs_scale_block_n, rhs_scale_block_k
@@ -634,9 +635,17 @@ def gmm_route(m, k, n, num_groups_total, *, lhs_dtype, rhs_dtype, lhs_scale_bloc
   return info.kernel.decode() if info.kernel else None, info.tile_rows, info.tail_rows, info.tail_height
 
 
-def gmm_workspace(m, num_groups_total, device):
-  """A tile-list buffer for moe_gmm calls on m rows and num_groups_total groups (uint8)."""
-  return torch.empty((max(_lib.load().moe_gmm_workspace_bytes(int(m), int(num_groups_total)), 16),), dtype=torch.uint8, device=device)
+def gmm_workspace(m, num_groups_total, device, split=False):
+  """A tile-list buffer for moe_gmm calls on m rows and num_groups_total groups (uint8).  split: with room for the partial sums of
+  tiles that the prefill kernels cut along K (64 MiB; not for calls smaller than any of those kernels takes)."""
+  return torch.empty((_gmm_workspace_bytes(int(m), int(num_groups_total), split),), dtype=torch.uint8, device=device)
+
+
+def _gmm_workspace_bytes(m, num_groups_total, split):
+  lib = _lib.load()
+  # (15 rows per group on average: the lowest that a prefill kernel takes)
+  size = lib.moe_gmm_split_workspace_bytes if split and m >= 15 * num_groups_total else lib.moe_gmm_workspace_bytes
+  return max(size(m, num_groups_total), 16)
 
 
 def gmm_lhs_e5m2_supported(m, k, n, num_groups_total):

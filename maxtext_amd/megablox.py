@@ -262,7 +262,7 @@ def gmm(
     return out if preferred_element_type == torch.bfloat16 else out.to(preferred_element_type)
 
   common = dict(group_offset=offset, group_offset_dev=offset_dev, out_dtype=preferred_element_type, lhs_row_idx=lhs_row_idx,
-                lhs_row_idx_div=lhs_row_idx_div, out_row_scale=out_row_scale, workspace=workspace, same_groups=same_groups)
+                lhs_row_idx_div=lhs_row_idx_div, out_row_scale=out_row_scale, workspace=workspace, same_groups=same_groups, split=True)
   if rhs_bias is not None:
     common["rhs_bias"] = rhs_bias.float().contiguous()  # [G, N] (rhs_bias [G, 1, N] of the v2 kernel, :573)
   if partial_sum is not None:  # [m, n], added to the product before the activation (ops.py:77)
@@ -490,16 +490,16 @@ class _GmmFn(torch.autograd.Function):
       if as_fp8:
         # e5m2 x e4m3 on the fp8 MFMA; the rows' scales are the activations' epilogue scales
         dlhs = kernels.gmm_raw(d, rq if as_kn else w_t, group_sizes, lhs_scale=s_row, rhs_scale=one, rhs_scale_block_n=_lib_per_tensor(),
-                               rhs_scale_shared=True, group_offset=ctx.offset, rhs_kn=as_kn)
+                               rhs_scale_shared=True, group_offset=ctx.offset, rhs_kn=as_kn, split=True)
       else:
         # the row scales go back on in the product's epilogue (rounded bf16 result times scale, rounded again: what the
         # reference's two steps give)
         w_b = w_t if w_t.dtype == torch.int8 else w_t.to(torch.bfloat16)
         if w_b.dtype == torch.int8:
           dlhs = kernels.gmm_raw(d, w_b, group_sizes, rhs_scale=one, rhs_scale_block_n=_lib_per_tensor(), rhs_scale_shared=True,
-                                 group_offset=ctx.offset, out_row_scale=s_row)
+                                 group_offset=ctx.offset, out_row_scale=s_row, split=True)
         else:
-          dlhs = kernels.gmm_raw(d, w_b, group_sizes, group_offset=ctx.offset, out_row_scale=s_row)
+          dlhs = kernels.gmm_raw(d, w_b, group_sizes, group_offset=ctx.offset, out_row_scale=s_row, split=True)
       dlhs = _GmmFn._rows_to_tokens(ctx, dlhs, row_idx, row_inv)
     if marks:
       marks[1].record()

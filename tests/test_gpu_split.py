@@ -1,0 +1,83 @@
+"""Tiles cut along K: the persistent prefill kernels with a workspace that holds partial sums against the same calls without one.
+
+The parts' sums are added in another order than one block adds them, in 32 bits: int8 x int8 results are the same bits, the others
+differ by f32 rounding ahead of the one rounding to bf16, i.e. by at most one bf16 step (2^-8 to 2^-7 of the value) and, where a sum
+cancels, by a small share of the result's magnitude.
+"""
+
+import pytest
+import torch
+
+from routes import FORMATS, route
+
+pytestmark = pytest.mark.gpu
+
+# (formats, k, n, group sizes, glu): the rests of 256-tile rounds that the tiles come to, and the parts they are cut into
+CASES = [
+    # 8 tiles of rows x 16: 128 tiles, two parts of each; 25 stages of 8-bit operands, 50 of bf16 ones
+    (("int8", "fp8", "bf16", "e5m2"), 3200, 4096, [90, 60, 128, 33, 150, 1, 100, 70], False),
+    # 9 x 32 tiles: one round and 4 tiles to each XCD in four parts, both projections; the last 128 channels are a short tile
+    (("int8", "fp8"), 6144, 4032, [100, 80, 60, 120, 90, 0, 77, 140, 65, 51], True),
+    # 13 x 10 = 130 tiles: 16 to six XCDs, cut, and 17 to two, not cut; N ends inside a tile
+    (("int8", "bf16"), 3072, 2312, [100] * 13, False),
+]
+
+
+def _operands(fmt, m, k, n, e, glu, gen):
+  lhs_t, rhs_t = FORMATS[fmt][:2]
+  kw = {}
+  x = torch.randn((m, k), generator=gen, device="cuda")
+  if lhs_t == "int8":
+    lhs, kw["lhs_scale"] = (x * 40).clamp(-127, 127).to(torch.int8), torch.rand((m,), generator=gen, device="cuda") + 0.5
+  elif lhs_t in ("fp8", "e5m2"):
+    lhs = x.to(torch.float8_e4m3fn if lhs_t == "fp8" else torch.float8_e5m2)
+    kw["lhs_scale"] = torch.rand((m,), generator=gen, device="cuda") + 0.5
+  else:
+    lhs = x.to(torch.bfloat16)
+
+  def weight():
+    if rhs_t == "int8":
+      return torch.randint(-127, 128, (e, n, k), generator=gen, device="cuda", dtype=torch.int8), torch.rand((e, n), generator=gen, device="cuda") * 1e-2
+    w = torch.randn((e, n, k), generator=gen, device="cuda")
+    if rhs_t == "bf16":
+      return w.to(torch.bfloat16), None
+    return w.to(torch.float8_e4m3fn), torch.rand((e, n), generator=gen, device="cuda") * 1e-2 + 1e-3
+
+  rhs, kw["rhs_scale"] = weight()
+  if glu:
+    (kw["rhs_up"], kw["rhs_up_scale"]), kw["act"] = weight(), "silu"
+  return lhs, rhs, kw
+
+
+@pytest.mark.parametrize("fmt,k,n,sizes,glu", [(f, *c[1:]) for c in CASES for f in c[0]])
+def test_tiles_cut_along_k_against_whole_ones(fmt, k, n, sizes, glu):
+  from maxtext_amd import kernels as K
+
+  gen = torch.Generator(device="cuda").manual_seed(k + n)
+  if fmt == "e5m2":
+    sizes = [s + 70 for s in sizes]  # (the gradient operand runs from 128 rows per group on)
+  e, m = len(sizes), sum(sizes) + 5
+  assert route(fmt, m, k, n, e, glu=glu, split=True)[0] == "gmm_dls_kernel"
+  lhs, rhs, kw = _operands(fmt, m, k, n, e, glu, gen)
+  gs = torch.tensor(sizes, dtype=torch.int32, device="cuda")
+  idx = torch.randperm(m, generator=gen, device="cuda").to(torch.int32)
+  scale = torch.rand((m,), generator=gen, device="cuda")
+  ws = K.gmm_workspace(m, e, "cuda", split=True)
+  for extra in ({}, {"lhs_row_idx": idx}, {"out_dtype": torch.float32, "out_row_scale": scale}):
+    if fmt == "e5m2" and "lhs_row_idx" in extra:
+      continue
+    want = K.gmm_raw(lhs, rhs, gs, **kw, **extra)
+    # the same workspace again and again: every launch leaves its counters as it found them, and the sums do not depend on who
+    # comes last
+    runs = [K.gmm_raw(lhs, rhs, gs, workspace=ws, same_groups=i > 0, **kw, **extra) for i in range(4)]
+    assert all(torch.equal(runs[0], r) for r in runs[1:])
+    got, want = runs[0].float(), want.float()
+    assert bool((want[-5:] == 0).all()) and bool((got[-5:] == 0).all())
+    if fmt == "int8":
+      assert torch.equal(got, want)
+    else:
+      # one step of bf16, and what the order of k f32 additions can make: each rounds by 2^-24 of a partial sum, which is some
+      # times the results' rms at most (four, with the activation of two products)
+      rms = float(want[:-5].double().pow(2).mean().sqrt())
+      slack = 4 * k * 2.0**-24 * rms
+      assert bool(((got - want).abs() <= 2.0**-7 * want.abs() + slack).all()), float((got - want).abs().max())
