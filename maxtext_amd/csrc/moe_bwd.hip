@@ -47,13 +47,15 @@ struct E5m2Scale {
   float s, inv;
   bool exact;
 };
-__device__ __forceinline__ E5m2Scale e5m2_prepare(float amax) {
+__device__ __forceinline__ E5m2Scale e5m2_of_scale(float scale) {
   E5m2Scale r;
-  r.s = e5m2_scale(amax);
+  r.s = scale;
   r.exact = !(r.s > 0.f && r.s < INFINITY);
   r.inv = 1.0f / r.s;
   return r;
 }
+
+__device__ __forceinline__ E5m2Scale e5m2_prepare(float amax) { return e5m2_of_scale(e5m2_scale(amax)); }
 
 // float8_e5m2 bytes of x0 / s0 and x1 / s1 (bits 0-7 and 8-15), equal to e5m2_byte(to_e5m2_grid(x, s)) bit for bit at a
 // fraction of its instructions: the quotient is formed as x * (1 / s), which lies within 2 ulps of x / s, and rounded by
@@ -92,22 +94,6 @@ __device__ __forceinline__ void round_bf16_pair(float a, float b, float& ra, flo
   const uint32_t p = pack_bf16x2(a, b);
   ra = __uint_as_float(p << 16);
   rb = __uint_as_float(p & 0xffff0000u);
-}
-
-// 8 results of one lane: bf16 (16 bytes at `out` + 16 * idx) or, BYTES, float8_e5m2 (8 bytes at `out` + 8 * idx)
-template <bool BYTES>
-__device__ __forceinline__ void store8(void* out, size_t idx, const float (&o)[8]) {
-  if (BYTES) {
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      lo |= e5m2_byte(o[e]) << (8 * e);
-      hi |= e5m2_byte(o[4 + e]) << (8 * e);
-    }
-    ((uint2*)out)[idx] = make_uint2(lo, hi);
-  } else {
-    ((uint4*)out)[idx] = make_uint4(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7]));
-  }
 }
 
 // expert of row m as the reference's backward sees it: the number of group ends <= m, taken relative to the first
@@ -159,15 +145,28 @@ __device__ __forceinline__ void block_group_ends(const int* __restrict__ group_s
   __syncthreads();
 }
 
-// One block per row: d = bf16(dout * bf16(factor)), factor = rhs_scale[group(row), n] (BY_CHANNEL) or lhs_scale[row];
-// ROW_QUANT: the row's absmax, then the e5m2 values and the row's scale.
-template <bool BY_CHANNEL, bool ROW_QUANT, bool BYTES = false>
+// One block per row: d = bf16(dout * bf16(factor)), factor = rhs_scale[group(row), n] (BY_CHANNEL) or lhs_scale[row]; ROW_QUANT: the
+// row's absmax, then the e5m2 values and the row's scale.  d is held as the bf16 values it is between the two, CH 16-byte chunks to a
+// thread, the least of 2, 4 and 8 that covers the row.
+// Bound by HBM and by the vector work on a value: 16384 x 14336 into e5m2 bytes 222 -> 195 us, 5998 x 14336 74 -> 71, 5998 x 4096 33 ->
+// 26 (d as floats, eight chunks for every row before).  Two or four rows to a block, which share the channels' factors, run at half the
+// waves: 121 us at 5998 x 14336.
+template <bool BY_CHANNEL, bool ROW_QUANT, bool BYTES, int CH>
 __global__ __launch_bounds__(kBwdThreads) void bwd_scale_rows_kernel(const uint4* dout, int N, const float* factor, const int* group_sizes,
                                                                      int G_total, int G_local, int group_offset, void* out,
-                                                                     float* scale_out, int factor_stride = 1) {
+                                                                     float* scale_out, int factor_stride) {
+  typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+  typedef float v4fu __attribute__((ext_vector_type(4), aligned(4)));  // (the factors come with a float's alignment)
   __shared__ int ends[BY_CHANNEL ? kBwdMaxGroups : 1];
   __shared__ uint32_t wmax[kBwdThreads / kWave];
   const int m = blockIdx.x, tid = threadIdx.x;
+  const int nvec = N / 8;
+  uint4 d[CH];
+#pragma unroll
+  for (int c = 0; c < CH; c++) {
+    const int i = c * kBwdThreads + tid;
+    d[c] = i < nvec ? dout[(size_t)m * nvec + i] : make_uint4(0, 0, 0, 0);
+  }
   const float* f = factor;
   float row_f = 1.0f;
   if (BY_CHANNEL) {
@@ -176,78 +175,110 @@ __global__ __launch_bounds__(kBwdThreads) void bwd_scale_rows_kernel(const uint4
   } else {
     row_f = round_bf16_fn(factor[(size_t)m * factor_stride]);  // (stride 0: one factor for the tensor)
   }
-  const int nvec = N / 8;
-  float v[kBwdMaxChunks][8];
-  uint32_t amax_bits = 0u;  // max of the bit patterns of |d|: orders like the values, and a NaN's pattern beats every number's
+  v2us m2 = {0, 0};  // max of the bit patterns of |d|: orders like the values, and a NaN's pattern beats every number's
 #pragma unroll
-  for (int c = 0; c < kBwdMaxChunks; c++) {
+  for (int c = 0; c < CH; c++) {
     const int i = c * kBwdThreads + tid;
     if (i < nvec) {
-      const uint4 x = dout[(size_t)m * nvec + i];
-      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+      float fc[8] = {row_f, row_f, row_f, row_f, row_f, row_f, row_f, row_f};
+      if (BY_CHANNEL) {
+        const v4fu lo = *(const v4fu*)(f + (size_t)i * 8), hi = *(const v4fu*)(f + (size_t)i * 8 + 4);
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const float x0 = __uint_as_float(w[e / 2] << 16), x1 = __uint_as_float(w[e / 2] & 0xffff0000u);
-        float f0 = row_f, f1 = row_f;
-        if (BY_CHANNEL) round_bf16_pair(f[i * 8 + e], f[i * 8 + e + 1], f0, f1);
-        round_bf16_pair(x0 * f0, x1 * f1, v[c][e], v[c][e + 1]);
-        amax_bits = max(amax_bits, max(__float_as_uint(v[c][e]) & 0x7fffffffu, __float_as_uint(v[c][e + 1]) & 0x7fffffffu));
+        for (int e = 0; e < 4; e += 2) {
+          round_bf16_pair(lo[e], lo[e + 1], fc[e], fc[e + 1]);
+          round_bf16_pair(hi[e], hi[e + 1], fc[4 + e], fc[4 + e + 1]);
+        }
       }
+      uint32_t w[4] = {d[c].x, d[c].y, d[c].z, d[c].w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        w[e] = pack_bf16x2(__uint_as_float(w[e] << 16) * fc[2 * e], __uint_as_float(w[e] & 0xffff0000u) * fc[2 * e + 1]);
+        if (ROW_QUANT) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(v2us, w[e] & 0x7fff7fffu));
+      }
+      d[c] = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
   E5m2Scale sc = {1.0f, 1.0f, false};
   if (ROW_QUANT) {
+    uint32_t amax = (uint32_t)max(m2[0], m2[1]) << 16;
 #pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) amax_bits = max(amax_bits, (uint32_t)__shfl_xor((int)amax_bits, o, kWave));
-    if (tid % kWave == 0) wmax[tid / kWave] = amax_bits;
+    for (int o = kWave / 2; o > 0; o >>= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o, kWave));
+    if (tid % kWave == 0) wmax[tid / kWave] = amax;
     __syncthreads();
-    const float amax = __uint_as_float(max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
-    sc = e5m2_prepare(amax);
+    sc = e5m2_prepare(__uint_as_float(max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]))));
     if (tid == 0) scale_out[m] = sc.s;
   }
 #pragma unroll
-  for (int c = 0; c < kBwdMaxChunks; c++) {
+  for (int c = 0; c < CH; c++) {
     const int i = c * kBwdThreads + tid;
     if (i < nvec) {
       if (ROW_QUANT) {
+        const uint32_t w[4] = {d[c].x, d[c].y, d[c].z, d[c].w};
         uint32_t pk[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) pk[e] = e5m2_bytes2(v[c][2 * e], v[c][2 * e + 1], sc, sc);
+        for (int e = 0; e < 4; e++) pk[e] = e5m2_bytes2(__uint_as_float(w[e] << 16), __uint_as_float(w[e] & 0xffff0000u), sc, sc);
         store8_e5m2<BYTES>(out, (size_t)m * nvec + i, pk);
       } else {
-        store8<false>(out, (size_t)m * nvec + i, v[c]);
+        ((uint4*)out)[(size_t)m * nvec + i] = d[c];
       }
     }
   }
 }
 
-// Column maxima of |d|, d = bf16(dout * bf16(lhs_scale[m])): a block walks a band of rows, a lane owns 8 columns; the
-// bands meet in an atomic max on the bit patterns (non-negative floats order like integers; a NaN's pattern is larger
-// than every number's and so survives, as it does in the reference's amax).
-constexpr int kColBand = 64;
-__global__ __launch_bounds__(kBwdThreads) void bwd_col_absmax_kernel(const uint4* dout, int M, int N, const float* lhs_scale, int scale_stride,
-                                                                     uint32_t* colmax) {
-  const int nvec = N / 8;
-  const int i = blockIdx.x * kBwdThreads + threadIdx.x;
-  if (i >= nvec) return;
-  const int m0 = blockIdx.y * kColBand, m1 = min(m0 + kColBand, M);
-  uint32_t mx[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-#pragma unroll 8
-  for (int m = m0; m < m1; m++) {
-    const uint4 x = dout[(size_t)m * nvec + i];
-    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-    const float fm = round_bf16_fn(lhs_scale[(size_t)m * scale_stride]);
+template <bool BY_CHANNEL, bool ROW_QUANT, bool BYTES>
+static void launch_scale_rows(const uint4* dout, int M, int N, const float* factor, const int* group_sizes, int G_total, int G_local, int group_offset,
+                              void* out, float* scale_out, int factor_stride, hipStream_t s) {
+  const auto go = [&](auto ch) {
+    bwd_scale_rows_kernel<BY_CHANNEL, ROW_QUANT, BYTES, decltype(ch)::value><<<M, kBwdThreads, 0, s>>>(dout, N, factor, group_sizes, G_total, G_local,
+                                                                                                       group_offset, out, scale_out, factor_stride);
+  };
+  const int ch = cdiv(N / 8, kBwdThreads);
+  if (ch <= 2) go(std::integral_constant<int, 2>{});
+  else if (ch <= 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, kBwdMaxChunks>{});
+}
+
+// Column maxima of |d|, d = bf16(dout * bf16(lhs_scale[m])): a block walks a band of rows, its waves kColRows of them each, a lane
+// owns 8 columns.  The waves meet in LDS, the bands in an atomic max on the bit patterns (non-negative floats order like integers; a
+// NaN's pattern is larger than every number's and so survives, as it does in the reference's amax).
+constexpr int kColWaves = 4, kColRows = 16, kColBand = kColWaves * kColRows;
+__global__ __launch_bounds__(kColWaves * kWave) void bwd_col_absmax_kernel(const uint4* dout, int M, int N, const float* lhs_scale, int scale_stride,
+                                                                           uint32_t* colmax) {
+  typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+  __shared__ uint4 s_max[kColWaves - 1][kWave];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int nvec = N / 8, i = blockIdx.x * kWave + lane;
+  const int m0 = blockIdx.y * kColBand + wave * kColRows;
+  v2us mx[4] = {};  // (of the rounded values' 16 bits)
+  uint4 x[kColRows];
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      float d0, d1;
-      round_bf16_pair(__uint_as_float(w[e / 2] << 16) * fm, __uint_as_float(w[e / 2] & 0xffff0000u) * fm, d0, d1);
-      // (the bit patterns of |d| order like the values, and a NaN's pattern beats every number's)
-      mx[e] = max(mx[e], __float_as_uint(d0) & 0x7fffffffu);
-      mx[e + 1] = max(mx[e + 1], __float_as_uint(d1) & 0x7fffffffu);
+  for (int j = 0; j < kColRows; j++) x[j] = i < nvec && m0 + j < M ? dout[(size_t)(m0 + j) * nvec + i] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int j = 0; j < kColRows; j++) {
+    const float fm = round_bf16_fn(lhs_scale[(size_t)min(m0 + j, M - 1) * scale_stride]);
+    const uint32_t w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const uint32_t d = pack_bf16x2(__uint_as_float(w[e] << 16) * fm, __uint_as_float(w[e] & 0xffff0000u) * fm);
+      mx[e] = __builtin_elementwise_max(mx[e], __builtin_bit_cast(v2us, m0 + j < M ? d & 0x7fff7fffu : 0u));
     }
   }
+  auto bits = [&](int e) { return __builtin_bit_cast(uint32_t, mx[e]); };
+  if (wave > 0) s_max[wave - 1][lane] = make_uint4(bits(0), bits(1), bits(2), bits(3));
+  __syncthreads();
+  if (wave > 0 || i >= nvec) return;
 #pragma unroll
-  for (int e = 0; e < 8; e++) atomicMax(colmax + i * 8 + e, mx[e] > 0x7f800000u ? 0x7fc00000u : mx[e]);
+  for (int v = 0; v < kColWaves - 1; v++) {
+    const uint4 o = s_max[v][lane];
+    const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) mx[e] = __builtin_elementwise_max(mx[e], __builtin_bit_cast(v2us, w[e]));
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const uint32_t m = (uint32_t)mx[e / 2][e % 2] << 16;
+    atomicMax(colmax + i * 8 + e, m > 0x7f800000u ? 0x7fc00000u : m);
+  }
 }
 
 __global__ void bwd_clear_kernel(uint32_t* p, int n) {
@@ -255,30 +286,44 @@ __global__ void bwd_clear_kernel(uint32_t* p, int n) {
   if (i < n) p[i] = 0u;
 }
 
-// d on the e5m2 grid of its column's scale; `colmax` still holds the maxima
+// d on the e5m2 grid of its column's scale.  A wave has kColRows rows: with 64 the chain of a wave's instructions took 70 us whatever
+// the size.  Maxima and values together: 777 x 512 75 -> 27 us, 5998 x 4096 100 -> 53, 5998 x 14336 137 -> 104.
 template <bool BYTES>
-__global__ __launch_bounds__(kBwdThreads) void bwd_col_quant_kernel(const uint4* dout, int M, int N, const float* lhs_scale, int scale_stride,
-                                                                    const float* colmax, void* out) {
+__global__ __launch_bounds__(kWave) void bwd_col_quant_kernel(const uint4* dout, int M, int N, const float* lhs_scale, int scale_stride,
+                                                              const float* col_scale, void* out) {
   const int nvec = N / 8;
-  const int i = blockIdx.x * kBwdThreads + threadIdx.x;
+  const int strips = (nvec + kWave - 1) / kWave;  // (one grid dimension: more rows than the second one counts)
+  const int i = blockIdx.x % strips * kWave + threadIdx.x;
   if (i >= nvec) return;
-  const int m0 = blockIdx.y * kColBand, m1 = min(m0 + kColBand, M);
+  const int m0 = blockIdx.x / strips * kColRows, m1 = min(m0 + kColRows, M);
   E5m2Scale s[8];
 #pragma unroll
-  for (int e = 0; e < 8; e++) s[e] = e5m2_prepare(colmax[i * 8 + e]);
-#pragma unroll 4
-  for (int m = m0; m < m1; m++) {
-    const uint4 x = dout[(size_t)m * nvec + i];
-    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-    const float fm = round_bf16_fn(lhs_scale[(size_t)m * scale_stride]);
-    uint32_t pk[4];
+  for (int e = 0; e < 8; e++) s[e] = e5m2_of_scale(col_scale[i * 8 + e]);
+  // (eight rows' loads ahead of their stores: a store, which might be to what the next load reads, keeps the compiler from moving
+  // that load up, and each row then waits for memory by itself)
+  constexpr int AHEAD = 8;
+  for (int mb = m0; mb < m1; mb += AHEAD) {
+    uint4 x[AHEAD];
+    float fm[AHEAD];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      float d0, d1;
-      round_bf16_pair(__uint_as_float(w[e] << 16) * fm, __uint_as_float(w[e] & 0xffff0000u) * fm, d0, d1);
-      pk[e] = e5m2_bytes2(d0, d1, s[2 * e], s[2 * e + 1]);
+    for (int j = 0; j < AHEAD; j++) {
+      const int m = min(mb + j, m1 - 1);
+      x[j] = dout[(size_t)m * nvec + i];
+      fm[j] = round_bf16_fn(lhs_scale[(size_t)m * scale_stride]);
     }
-    store8_e5m2<BYTES>(out, (size_t)m * nvec + i, pk);
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) {
+      if (mb + j >= m1) break;
+      const uint32_t w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+      uint32_t pk[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float d0, d1;
+        round_bf16_pair(__uint_as_float(w[e] << 16) * fm[j], __uint_as_float(w[e] & 0xffff0000u) * fm[j], d0, d1);
+        pk[e] = e5m2_bytes2(d0, d1, s[2 * e], s[2 * e + 1]);
+      }
+      store8_e5m2<BYTES>(out, (size_t)(mb + j) * nvec + i, pk);
+    }
   }
 }
 
@@ -353,30 +398,31 @@ int moe_bwd_scale_grad(const void* dout, int M, int N, int mode, int quantize, c
     if (!group_sizes || num_groups_total <= 0 || num_groups_total > kBwdMaxGroups || num_groups_local <= 0 || group_offset < 0)
       return fail(MOE_ERR_INVALID_ARG, "bwd_scale_grad: bad groups (at most %d)", kBwdMaxGroups);
     if (bytes)
-      bwd_scale_rows_kernel<true, true, true><<<M, kBwdThreads, 0, s>>>(x, N, factor, group_sizes, num_groups_total, num_groups_local, group_offset, out, scale_out);
+      launch_scale_rows<true, true, true>(x, M, N, factor, group_sizes, num_groups_total, num_groups_local, group_offset, out, scale_out, 1, s);
     else if (quantize)
-      bwd_scale_rows_kernel<true, true><<<M, kBwdThreads, 0, s>>>(x, N, factor, group_sizes, num_groups_total, num_groups_local, group_offset, out, scale_out);
+      launch_scale_rows<true, true, false>(x, M, N, factor, group_sizes, num_groups_total, num_groups_local, group_offset, out, scale_out, 1, s);
     else
-      bwd_scale_rows_kernel<true, false><<<M, kBwdThreads, 0, s>>>(x, N, factor, group_sizes, num_groups_total, num_groups_local, group_offset, out, scale_out);
+      launch_scale_rows<true, false, false>(x, M, N, factor, group_sizes, num_groups_total, num_groups_local, group_offset, out, scale_out, 1, s);
     return check_launch("bwd_scale_rows_kernel");
   }
   // per tensor: one factor for every row, and the columns' maxima merged into one before they are used
   const bool tensor = mode == MOE_BWD_PER_TENSOR;
   const int fstride = tensor ? 0 : 1;
   if (!quantize) {
-    bwd_scale_rows_kernel<false, false><<<M, kBwdThreads, 0, s>>>(x, N, factor, nullptr, 0, 0, 0, out, scale_out, fstride);
+    launch_scale_rows<false, false, false>(x, M, N, factor, nullptr, 0, 0, 0, out, scale_out, fstride, s);
     return check_launch("bwd_scale_rows_kernel");
   }
-  // per column: clear the maxima, take them, quantise with them, turn them into the scales
+  // per column: clear the maxima, take them, turn them into the scales, quantise with these
   const int nvec = N / 8;
-  const dim3 grid(cdiv(nvec, kBwdThreads), cdiv(M, kColBand));
-  if (grid.y > 65535) return fail(MOE_ERR_UNSUPPORTED, "bwd_scale_grad: too many rows (%d)", M);
+  const dim3 bands(cdiv(nvec, kWave), cdiv(M, kColBand));
+  const int rows = cdiv(nvec, kWave) * cdiv(M, kColRows);
+  if (bands.y > 65535) return fail(MOE_ERR_UNSUPPORTED, "bwd_scale_grad: too many rows (%d)", M);
   bwd_clear_kernel<<<cdiv(N, 256), 256, 0, s>>>((uint32_t*)scale_out, N);
-  bwd_col_absmax_kernel<<<grid, kBwdThreads, 0, s>>>(x, M, N, factor, fstride, (uint32_t*)scale_out);
+  bwd_col_absmax_kernel<<<bands, kColWaves * kWave, 0, s>>>(x, M, N, factor, fstride, (uint32_t*)scale_out);
   if (tensor) bwd_col_merge_kernel<<<1, kBwdThreads, 0, s>>>((uint32_t*)scale_out, N);
-  if (bytes) bwd_col_quant_kernel<true><<<grid, kBwdThreads, 0, s>>>(x, M, N, factor, fstride, scale_out, out);
-  else bwd_col_quant_kernel<false><<<grid, kBwdThreads, 0, s>>>(x, M, N, factor, fstride, scale_out, out);
   bwd_col_scale_kernel<<<cdiv(N, 256), 256, 0, s>>>(scale_out, N);
+  if (bytes) bwd_col_quant_kernel<true><<<rows, kWave, 0, s>>>(x, M, N, factor, fstride, scale_out, out);
+  else bwd_col_quant_kernel<false><<<rows, kWave, 0, s>>>(x, M, N, factor, fstride, scale_out, out);
   return check_launch("bwd_col_quant_kernel");
 }
 

@@ -128,4 +128,34 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// f / sc as the dynamic quantisers round it: to the nearest integer in [-127, 127] (INT8) or, in f32, into [-448, 448] for the
+// e4m3 cast; a zero scale gives 0.  inv = 1 / sc rounded once (0 for sc == 0).
+template <bool INT8>
+__device__ __forceinline__ float quotient_on_range(float f, float sc, float inv) {
+  const float qmax = INT8 ? 127.0f : 448.0f;
+  if (INT8) {
+    // rint(f / sc) without dividing: f * (1 / sc) is off the rounded quotient by at most 1.2e-7 of its value, 2.4e-5
+    // for |q| < 200, so unless it lies within 1e-4 of k + 1/2 both round to the same integer; the few values that do lie
+    // there (and those beyond 200, NaN included) take the division.  sc == 0 has inv == 0 and gives 0.
+    float q = f * inv;
+    if (fabsf(__builtin_amdgcn_fractf(q) - 0.5f) < 1e-4f || !(fabsf(q) < 200.0f)) q = sc == 0.f ? 0.f : f / sc;
+    return fminf(fmaxf(rintf(q), -qmax), qmax);
+  }
+  // The correctly rounded quotient in five operations instead of a division's dozen: inv is the rounded reciprocal, the
+  // first correction brings the estimate within an ulp, and from there one exact residual and one fma round correctly
+  // (Markstein's theorem).  Nothing in it may overflow, or lose bits below the normal range that e4m3 could see; scales
+  // outside [2^-80, 2^80] (0 and infinity among them) divide.
+  float q;
+  if (sc >= 0x1p-80f && sc <= 0x1p80f) {
+    const float est = f * inv;
+    q = fmaf(fmaf(-est, sc, f), inv, est);
+    q = fmaf(fmaf(-q, sc, f), inv, q);
+    q = fabsf(est) < 1024.0f ? q : est;  // (beyond the range by far: a static scale; the residual may overflow there)
+    q = copysignf(q, f);  // (a sum of zeros is +0: -0 would lose its sign, which e4m3 keeps)
+  } else {
+    q = sc == 0.f ? 0.f : f / sc;
+  }
+  return fminf(fmaxf(q, -qmax), qmax);
+}
+
 }  // namespace moe

@@ -3,18 +3,17 @@
 // shared by the experts and by K) or manual_quantize (layers/quantizations.py:961-991: one static scale for the tensor).
 //
 // Weights are [G, N, K] with K contiguous, so a channel's values are G rows of K.  Dynamic scales per channel are made
-// and applied by one block per channel that sweeps its rows twice, the second time out of the caches (bf16 in once, 1 byte
-// out: 3 bytes per value from HBM); a scale over more than a million values (per tensor, or hundreds of experts sharing
-// long rows) takes two launches (5 bytes per value): every block reduces one row to its absmax and merges it into the
-// scale's maximum with an atomic max on the bit pattern, the second pass divides by absmax / qmax and rounds.  A static
-// scale needs the second pass only.
+// and applied by one block per channel: up to 128 thousand values (256 KB) stay in the block's registers between the absmax and
+// the rounding, more (to a million) are swept twice, the second time out of the caches (bf16 in once, 1 byte out: 3 bytes per
+// value from HBM); a scale over more than that (per tensor, or hundreds of experts sharing long rows) takes two launches (5 bytes
+// per value): every block reduces one row to its absmax and merges it into the scale's maximum with an atomic max on the bit
+// pattern, the second pass divides by absmax / qmax and rounds.  A static scale needs the second pass only.
 
 #include "moe_common.h"
 
 namespace moe {
 
 constexpr int kQThreads = 256;
-constexpr int kQMaxChunks = 8;  // 8 bf16 per lane and chunk: rows of up to 16384 values
 
 __device__ __forceinline__ void unpack_bf16x8(const uint4& u, float (&f)[8]) {
   const uint32_t w[4] = {u.x, u.y, u.z, u.w};
@@ -43,6 +42,23 @@ __global__ __launch_bounds__(kQThreads) void rhs_absmax_kernel(const uint4* __re
   if (tid == 0) atomicMax(maxima + scale_slot(row, N, shared), max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
 }
 
+// eight quantised values as bytes
+template <int MODE>
+__device__ __forceinline__ uint2 pack_q8(const float (&f)[8]) {
+  if (MODE == 0) {
+    uint32_t b[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) b[e] = (uint32_t)((int)f[e]) & 0xffu;
+    return make_uint2(b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24), b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24));
+  }
+  int l = 0, h = 0;
+  l = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], l, false);
+  l = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], l, true);
+  h = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], h, false);
+  h = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], h, true);
+  return make_uint2((uint32_t)l, (uint32_t)h);
+}
+
 // MODE 0: int8, 1: float8_e4m3fn.  STATIC: q = clip(bf16(w / bf16(scale)), +-bf16(qmax)) cast as `.astype` does (int8
 // truncates, fp8 rounds to nearest even), manual_quantize's arithmetic for bf16 weights.  Otherwise scale = absmax / qmax
 // and q = rint(w / scale) (int8) or the nearest-even cast of w / scale (fp8), in f32; a zero scale gives zeros.
@@ -55,6 +71,7 @@ __global__ __launch_bounds__(kQThreads) void rhs_quant_kernel(const uint4* __res
   float sc;
   if (STATIC) sc = round_bf16_fn(*static_scale);
   else sc = maxima[scale_slot(row, N, shared)] / qmax;
+  const float inv = STATIC || sc == 0.f ? 0.f : 1.0f / sc;
   for (int i = tid; i < nvec; i += kQThreads) {
     float f[8];
     unpack_bf16x8(w[(size_t)row * nvec + i], f);
@@ -65,87 +82,126 @@ __global__ __launch_bounds__(kQThreads) void rhs_quant_kernel(const uint4* __res
         y = fminf(fmaxf(round_bf16_fn(f[e] / sc), -qmax), qmax);  // (127 and 448 are bf16 values)
         if (MODE == 0) y = truncf(y);
       } else {
-        y = sc == 0.f ? 0.f : f[e] / sc;
-        y = fminf(fmaxf(MODE == 0 ? rintf(y) : y, -qmax), qmax);
+        y = quotient_on_range<MODE == 0>(f[e], sc, inv);
       }
       f[e] = y;
     }
-    uint32_t lo, hi;
-    if (MODE == 0) {
-      uint32_t b[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) b[e] = (uint32_t)((int)f[e]) & 0xffu;
-      lo = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-      hi = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
-    } else {
-      int l = 0, h = 0;
-      l = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], l, false);
-      l = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], l, true);
-      h = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], h, false);
-      h = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], h, true);
-      lo = (uint32_t)l;
-      hi = (uint32_t)h;
-    }
-    q[(size_t)row * nvec + i] = make_uint2(lo, hi);
+    q[(size_t)row * nvec + i] = pack_q8<MODE>(f);
   }
 }
 
-// Dynamic scales per channel in one launch: a block owns one scale (a channel's G rows of K when the experts share it,
-// one row otherwise), sweeps its rows once for the absmax and a second time, while they still sit in the caches (64 to
-// 230 KB per block on the Mixtral shapes), to quantise them: the weights come from HBM once instead of twice.  Same
-// arithmetic as the two kernels above.
+// Dynamic scales per channel in one launch: a block owns one scale (a channel's G rows of K when the experts share it, one row
+// otherwise) and its weights come from HBM once.  CH > 0: they stay in registers, CH 16-byte chunks to a thread; CH == 0: a second
+// sweep of the block, out of the caches.  Same arithmetic as the two kernels above.  Bound by HBM once the values fit the
+// registers and are divided by a reciprocal and exact residuals: Mixtral shape, 8 x 14336 x 4096 in e4m3 357 -> 264 us (5.3 TB/s, a large copy's rate), 8 x
+// 4096 x 14336 470 -> 294 (two sweeps and a division before).
+template <int MODE, int THREADS, int CH>
+__global__ __launch_bounds__(THREADS) void rhs_quant_slot_kernel(const uint4* __restrict__ w, int G, int N, int K, int shared, uint2* __restrict__ q,
+                                                                 float* __restrict__ scale) {
+  constexpr int NW = THREADS / kWave;
+  __shared__ uint32_t wmax[2][NW];
+  typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+  const int tid = threadIdx.x, slots = shared ? N : G * N;
+  const int nvec = K / 8, total = (shared ? G : 1) * nvec;  // chunks of a row, of the block
+  const size_t row_step = (size_t)(shared ? N : 0) * nvec;
+  // chunk i of a slot: row i / nvec, i % nvec in it; both advance by THREADS without a division
+  struct Cursor { int i, col; size_t row; };
+  const int step_rows = THREADS / nvec, step_cols = THREADS % nvec;
+  auto begin = [&](int t) { return Cursor{t, t % nvec, (size_t)(t / nvec) * row_step}; };
+  auto next = [&](Cursor& c) {
+    c.i += THREADS;
+    c.col += step_cols;
+    c.row += (size_t)step_rows * row_step;
+    if (c.col >= nvec) {
+      c.col -= nvec;
+      c.row += row_step;
+    }
+  };
+  // (bit patterns of |bf16| order like the values, and a NaN's pattern beats every number's)
+  v2us m2;
+  auto take = [&](const uint4& x) {
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(v2us, v[e] & 0x7fff7fffu));
+  };
+  auto put = [&](const uint4& x, size_t at, float sc, float inv) {
+    float f[8];
+    unpack_bf16x8(x, f);
+#pragma unroll
+    for (int e = 0; e < 8; e++) f[e] = quotient_on_range<MODE == 0>(f[e], sc, inv);
+    q[at] = pack_q8<MODE>(f);
+  };
+  uint4 regs[CH > 0 ? CH : 1];
+  if constexpr (CH > 0) {
+    Cursor c = begin(tid);
+    const size_t base = (size_t)blockIdx.x * nvec;
+#pragma unroll
+    for (int j = 0; j < CH; j++, next(c)) regs[j] = c.i < total ? w[base + c.row + c.col] : make_uint4(0, 0, 0, 0);
+  }
+  int turn = 0;
+  for (int slot = blockIdx.x; slot < slots; slot += gridDim.x, turn ^= 1) {
+    const size_t base = (size_t)slot * nvec;
+    m2 = v2us{0, 0};
+    if constexpr (CH > 0) {
+#pragma unroll
+      for (int j = 0; j < CH; j++) take(regs[j]);
+    } else {
+      for (Cursor c = begin(tid); c.i < total; next(c)) take(w[base + c.row + c.col]);
+    }
+    uint32_t m = (uint32_t)max(m2[0], m2[1]) << 16;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, kWave));
+    if (tid % kWave == 0) wmax[turn][tid / kWave] = m;
+    __syncthreads();  // (one to a slot: the next one's maxima go to the other half)
+#pragma unroll
+    for (int i = 0; i < NW; i++) m = max(m, wmax[turn][i]);
+    const float sc = __uint_as_float(m) / (MODE == 0 ? 127.0f : 448.0f), inv = sc == 0.f ? 0.f : 1.0f / sc;
+    if (tid == 0) scale[slot] = sc;
+    int again = tid;  // (opaque: the chunks' places are made again, kept they would take the registers of the values)
+    asm volatile("" : "+v"(again));
+    Cursor c = begin(again);
+    if constexpr (CH > 0) {
+      // the block's next slot is requested while this one is rounded
+      const bool more = slot + (int)gridDim.x < slots;
+      const size_t base_n = (size_t)(slot + (int)gridDim.x) * nvec;
+#pragma unroll
+      for (int j = 0; j < CH; j++, next(c)) {
+        const uint4 x = regs[j];
+        const bool have = c.i < total;
+        if (have && more) regs[j] = w[base_n + c.row + c.col];
+        if (have) put(x, base + c.row + c.col, sc, inv);
+      }
+    } else {
+      for (; c.i < total; next(c)) put(w[base + c.row + c.col], base + c.row + c.col, sc, inv);
+    }
+  }
+}
+
 template <int MODE>
-__global__ __launch_bounds__(kQThreads) void rhs_quant_slot_kernel(const uint4* __restrict__ w, int G, int N, int K, int shared, uint2* __restrict__ q,
-                                                                    float* __restrict__ scale) {
-  __shared__ uint32_t wmax[kQThreads / kWave];
-  const int slot = blockIdx.x, tid = threadIdx.x;
-  const int nvec = K / 8, nrows = shared ? G : 1;
-  const float qmax = MODE == 0 ? 127.0f : 448.0f;
-  uint32_t m = 0u;
-  for (int r = 0; r < nrows; r++) {
-    const uint4* row = w + ((size_t)(shared ? r * N + slot : slot)) * nvec;
-    for (int i = tid; i < nvec; i += kQThreads) {
-      float f[8];
-      unpack_bf16x8(row[i], f);
-#pragma unroll
-      for (int e = 0; e < 8; e++) m = max(m, __float_as_uint(fabsf(f[e])));
-    }
-  }
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, kWave));
-  if (tid % kWave == 0) wmax[tid / kWave] = m;
-  __syncthreads();
-  const float sc = __uint_as_float(max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]))) / qmax;
-  if (tid == 0) scale[slot] = sc;
-  for (int r = 0; r < nrows; r++) {
-    const size_t base = ((size_t)(shared ? r * N + slot : slot)) * nvec;
-    for (int i = tid; i < nvec; i += kQThreads) {
-      float f[8];
-      unpack_bf16x8(w[base + i], f);
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const float y = sc == 0.f ? 0.f : f[e] / sc;
-        f[e] = fminf(fmaxf(MODE == 0 ? rintf(y) : y, -qmax), qmax);
-      }
-      uint32_t lo, hi;
-      if (MODE == 0) {
-        uint32_t b[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) b[e] = (uint32_t)((int)f[e]) & 0xffu;
-        lo = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
-        hi = b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24);
-      } else {
-        int l = 0, h = 0;
-        l = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], l, false);
-        l = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], l, true);
-        h = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], h, false);
-        h = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], h, true);
-        lo = (uint32_t)l;
-        hi = (uint32_t)h;
-      }
-      q[base + i] = make_uint2(lo, hi);
-    }
-  }
+static void launch_rhs_quant_slot(const uint4* w, int G, int N, int K, int shared, uint2* q, float* scale, int slots, hipStream_t s) {
+  const auto go = [&](auto threads, auto ch) {
+    constexpr int THREADS = decltype(threads)::value, CH = decltype(ch)::value;
+    // a block that fills its CU walks slots, requesting the next one's values while it rounds (8 x 4096 x 14336: 293 us, 368 with a
+    // block for each slot); smaller blocks overlap one another (8 x 14336 x 4096: a block for each slot 263, walking 300)
+    const int blocks = CH == 16 && slots > 256 ? 256 : slots;
+    rhs_quant_slot_kernel<MODE, THREADS, CH><<<blocks, THREADS, 0, s>>>(w, G, N, K, shared, q, scale);
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C2 = std::integral_constant<int, 2>;
+  using C4 = std::integral_constant<int, 4>;
+  using C8 = std::integral_constant<int, 8>;
+  using C16 = std::integral_constant<int, 16>;
+  using T256 = std::integral_constant<int, 256>;
+  using T512 = std::integral_constant<int, 512>;
+  using T1024 = std::integral_constant<int, 1024>;
+  const long long chunks = (long long)(shared ? G : 1) * (K / 8);
+  if (chunks <= 256 * 2) go(T256{}, C2{});
+  else if (chunks <= 256 * 4) go(T256{}, C4{});
+  else if (chunks <= 256 * 8) go(T256{}, C8{});
+  else if (chunks <= 512 * 8) go(T512{}, C8{});
+  else if (chunks <= 1024 * 8) go(T1024{}, C8{});
+  else if (chunks <= 1024 * 16) go(T1024{}, C16{});
+  else go(T256{}, C0{});
 }
 
 __global__ void rhs_clear_kernel(uint32_t* p, int n) {
@@ -182,11 +238,11 @@ extern "C" int moe_quantize_rhs(const void* w, int G, int N, int K, int out_dtyp
   }
   if (shared < 0 || shared > 2) return fail(MOE_ERR_INVALID_ARG, "quantize_rhs: shared must be 0 (per expert), 1 (shared by the experts) or 2 (per tensor)");
   const int ns = shared == 2 ? 1 : shared ? N : rows;
-  // a scale whose values fit the caches between two sweeps of one block (2 MB: 128 experts of 8192) is made and applied in
-  // one launch
+  // a scale whose values fit a block's registers, or the caches between two sweeps of it (2 MB: 128 experts of 8192), is made and
+  // applied in one launch
   if (shared != 2 && (long long)(shared ? G : 1) * K <= (1LL << 20)) {
-    if (out_dtype == MOE_INT8) rhs_quant_slot_kernel<0><<<ns, kQThreads, 0, s>>>(x, G, N, K, shared, (uint2*)q, scale);
-    else rhs_quant_slot_kernel<1><<<ns, kQThreads, 0, s>>>(x, G, N, K, shared, (uint2*)q, scale);
+    if (out_dtype == MOE_INT8) launch_rhs_quant_slot<0>(x, G, N, K, shared, (uint2*)q, scale, ns, s);
+    else launch_rhs_quant_slot<1>(x, G, N, K, shared, (uint2*)q, scale, ns, s);
     return check_launch("rhs_quant_slot_kernel");
   }
   rhs_clear_kernel<<<cdiv(ns, 256), 256, 0, s>>>((uint32_t*)scale, ns);

@@ -851,29 +851,7 @@ __device__ __forceinline__ float quant_value(float f, float sc, float inv, int r
     (void)is_static;
     return MODE == GQ_INT8 ? truncf(y) : y;
   }
-  if (MODE == GQ_INT8) {
-    // rint(f / sc) without dividing: f * (1 / sc) is off the rounded quotient by at most 1.2e-7 of its value, 2.4e-5
-    // for |q| < 200, so unless it lies within 1e-4 of k + 1/2 both round to the same integer; the few values that do lie
-    // there (and those beyond 200, NaN included) take the division.  sc == 0 has inv == 0 and gives 0.
-    float q = f * inv;
-    if (fabsf(__builtin_amdgcn_fractf(q) - 0.5f) < 1e-4f || !(fabsf(q) < 200.0f)) q = sc == 0.f ? 0.f : f / sc;
-    return fminf(fmaxf(rintf(q), -qmax), qmax);
-  }
-  // The correctly rounded quotient in five operations instead of a division's dozen: inv is the rounded reciprocal, the
-  // first correction brings the estimate within an ulp, and from there one exact residual and one fma round correctly
-  // (Markstein's theorem).  Nothing in it may overflow, or lose bits below the normal range that e4m3 could see; scales
-  // outside [2^-80, 2^80] (0 and infinity among them) divide.
-  float q;
-  if (sc >= 0x1p-80f && sc <= 0x1p80f) {
-    const float est = f * inv;
-    q = fmaf(fmaf(-est, sc, f), inv, est);
-    q = fmaf(fmaf(-q, sc, f), inv, q);
-    q = fabsf(est) < 1024.0f ? q : est;  // (beyond the range by far: a static scale; the residual may overflow there)
-    q = copysignf(q, f);  // (a sum of zeros is +0: -0 would lose its sign, which e4m3 keeps)
-  } else {
-    q = sc == 0.f ? 0.f : f / sc;
-  }
-  return fminf(fmaxf(q, -qmax), qmax);
+  return quotient_on_range<MODE == GQ_INT8>(f, sc, inv);
 }
 
 // Largest of the lane's value and those of the lanes that share its K block (16, 32 or 64 consecutive lanes).

@@ -279,6 +279,54 @@ def test_quantize_rhs_bit_exact(K, qdt, shared, G, N, Kd):
   assert float(s.cpu().reshape(-1, N)[0, 5]) == 0.0 and torch.all(q[:, 5].float() == 0)
 
 
+@pytest.mark.parametrize("qdt", [torch.int8, E4M3], ids=["int8", "fp8"])
+@pytest.mark.parametrize("G,N,Kd", [(1, 5, 4096), (1, 5, 4104), (2, 3, 4096), (2, 3, 4104), (4, 3, 4104), (8, 3, 4096), (8, 3, 4104), (8, 3, 8200),
+                                    (8, 300, 16384), (9, 3, 14568)])
+def test_quantize_rhs_at_the_edges_of_its_chunk_counts(K, qdt, G, N, Kd):
+  """Channels of just as many 16-byte chunks as one variant's registers hold, and of the next few more (512, 1024, 2048, 4096, 8192 and
+  16384), blocks that walk several channels, and channels past the registers: values and scales bit for bit, infinities, a
+  channel of subnormal weights and one of negative zeros among them."""
+  g = torch.Generator().manual_seed(G + Kd)
+  w = (torch.randn(G, N, Kd, generator=g) * 0.05).to(torch.bfloat16)
+  w[0, 1, -1] = 3.0  # the largest value in a row's last chunk
+  w[:, 2] *= 1e-38
+  w[-1, 2] = -0.0
+  if N > 4:
+    w[0, 3, 5] = float("inf")
+    w[:, 4] *= 1e30
+  qmax = 127.0 if qdt == torch.int8 else 448.0
+  wf = w.float()
+  sc = wf.abs().amax(dim=(0, 2), keepdim=True) / qmax
+  y = torch.where(sc == 0, torch.zeros_like(wf), wf / sc)
+  want = torch.round(y).clamp(-qmax, qmax).nan_to_num(0).to(qdt) if qdt == torch.int8 else y.clamp(-qmax, qmax).to(qdt)
+  q, s = K.quantize_rhs(cuda(w), qdt, shared=True)
+  assert torch.equal(s.cpu().reshape(-1), sc.reshape(-1))
+  finite = torch.isfinite(y)  # (infinity over infinity has no value to agree on)
+  assert torch.equal(torch.where(finite, q.cpu().float(), 0.0), torch.where(finite, want.float(), 0.0))
+  if qdt == E4M3:  # the sign of zeros
+    assert torch.equal(torch.signbit(q.cpu().float()) & finite, torch.signbit(want.float()) & finite)
+
+
+@pytest.mark.parametrize("n", [8, 4096, 4104, 8192, 8200, 16384])
+@pytest.mark.parametrize("m", [1, 17, 65])
+def test_bwd_scale_grad_at_the_edges_of_its_chunk_counts(K, m, n):
+  """Rows of just as many chunks as a variant's registers hold and of one more, columns that end inside a band of rows: e5m2 bytes and
+  scales of both directions bit for bit."""
+  g = torch.Generator().manual_seed(m * n)
+  dout = (torch.randn(m, n, generator=g) * torch.rand(m, 1, generator=g) * 8).to(torch.bfloat16)
+  dout[m // 2, n - 1] = -60.0
+  gs = np.array([m // 3, m - m // 3], np.int32)
+  rs, ls = torch.rand(2, n, generator=g) * 0.02 + 1e-4, torch.rand(m, generator=g) * 0.05 + 1e-4
+  group = torch.from_numpy(np.repeat(np.arange(2), gs))
+  for mode, factor, scaled, dim, kw in (("dlhs", rs, dout * rs.to(torch.bfloat16)[group], 1, dict(group_sizes=cuda(gs), num_groups_local=2)),
+                                        ("drhs", ls, dout * ls.to(torch.bfloat16)[:, None], 0, {})):
+    want, want_s = O.quantize_e5m2(scaled, dim=dim)
+    got, s = K.bwd_scale_grad(cuda(dout), cuda(factor), mode=mode, quantize=True, as_fp8=True, **kw)
+    assert torch.equal(s.cpu(), want_s.reshape(-1)) and torch.equal(got.float().cpu(), want)
+    plain, none = K.bwd_scale_grad(cuda(dout), cuda(factor), mode=mode, quantize=False, **kw)
+    assert none is None and torch.equal(plain.cpu(), scaled)
+
+
 @pytest.mark.parametrize("qdt,cal", [(torch.int8, "fixed,-4,4"), (E4M3, "fixed,-224,224"), (E4M3, "fixed,3")])
 def test_quantize_rhs_static_equals_manual_quantize(K, qdt, cal):
   """The static per-tensor rule against the oracle's restatement of manual_quantize (layers/quantizations.py:961-991),
