@@ -437,6 +437,49 @@ MOE_API int moe_gmm(const moe_gmm_args* args, void* stream);
 MOE_API size_t moe_gmm_static_ws_capacity(void);
 MOE_API int moe_gmm_static_ws(const moe_gmm_args* args, void* stream);
 
+/* A whole expert layer for inference through one call: moe_gate_route, the sort, the activation quantisers, both grouped
+ * matmuls and the combine, in that order, on buffers of the caller's one workspace.  Replaces RoutedMoE.__call__ (moe.py:3143)
+ * and, with shared_experts > 0, RoutedAndSharedMoE.__call__ (moe.py:3338) for layers without biases, auxiliary outputs or
+ * gradients: the result is that of the single calls, bit for bit.
+ *
+ *   x            [T, d] bf16; gate_x [T, d] bf16, what the router reads, or NULL for x
+ *   gate_terms .. topk_routing_group   as moe_gate_route
+ *   shared_experts   experts E .. E + shared_experts - 1 of the stacked weights, which every token takes with weight 1
+ *   wi_0, wi_1   [E + shared_experts, f, d], wo [E + shared_experts, d, f], of rhs_dtype with scales as moe_gmm takes them
+ *                (block sizes and MOE_GMM_RHS_SCALE_* flags of each)
+ *   act_dtype    MOE_BF16, or MOE_INT8 / MOE_FP8_E4M3: the activations of both products are quantised by MOE_QUANT_RINT_DIV with
+ *                a scale per row (act_block_k 0) or per row and act_block_k values
+ *   out          [T, d] bf16
+ *   workspace    moe_layer_workspace_bytes(args) bytes, 256-byte aligned (0: the arguments are refused, moe_last_error says why)
+ */
+typedef struct moe_layer_args {
+  size_t struct_size; /* sizeof(moe_layer_args), checked */
+  const void* x;
+  const void* gate_x;
+  const void* gate_terms;
+  const float* gate_bias;
+  const void* wi_0;
+  const void* wi_0_scale;
+  const void* wi_1;
+  const void* wi_1_scale;
+  const void* wo;
+  const void* wo_scale;
+  void* out;
+  int32_t T, d, f, E, k, shared_experts;
+  int32_t num_gate_terms, score_func, gate_round_bf16;
+  int32_t route_mode, norm_topk_prob, weights_round_bf16;
+  float routed_scaling_factor;
+  int32_t n_routing_groups, topk_routing_group;
+  int32_t rhs_dtype;
+  int32_t wi_scale_block_n, wi_scale_block_k, wi_flags;
+  int32_t wo_scale_block_n, wo_scale_block_k, wo_flags;
+  int32_t act_dtype, act_block_k;
+  int32_t act; /* moe_act */
+  float act_limit;
+} moe_layer_args;
+MOE_API size_t moe_layer_workspace_bytes(const moe_layer_args* args);
+MOE_API int moe_layer(const moe_layer_args* args, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Per-device set-up, for the device that is current: the CU count, the address of the static workspace and the raised
  * LDS limit of every kernel.  Optional: each entry point does its share on first use.  No counterpart in the reference. */
 MOE_API int moe_init(void);

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 # MOE_MI355X_LIB points the loader at another build of the same library (a tuning variant, an installed copy)
@@ -103,6 +104,8 @@ SIGNATURES = {
     "moe_gather_rows": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p]),
     "moe_gmm_workspace_bytes": (c_size_t, [c_int, c_int]),
+    "moe_layer_workspace_bytes": (c_size_t, [ctypes.c_char_p]),
+    "moe_layer": (c_int, [ctypes.c_char_p, c_void_p, c_size_t, c_void_p]),
     "moe_gmm_split_workspace_bytes": (c_size_t, [c_int, c_int]),
     "moe_gmm_rhs_kn_supported": (c_int, [c_int, c_int, c_int, c_int]),
     "moe_gmm_lhs_e5m2_supported": (c_int, [c_int, c_int, c_int, c_int]),
@@ -136,6 +139,9 @@ SIGNATURES = {
     "moe_ring_ragged_indices_dev": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
     "moe_all_to_all_params_dev": (c_int, [c_void_p, c_int, c_void_p, c_int, ctypes.c_longlong, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
 }
+
+# moe_layer_args, packed by struct: its 38 fields one by one in a ctypes structure take three times as long
+LAYER_ARGS = struct.Struct("@N11P12if12if")
 
 _lib = None
 

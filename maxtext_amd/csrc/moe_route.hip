@@ -100,12 +100,13 @@ struct GateEpilogue {
 
 // One token per wave: token t_raw of T (a wave past the end repeats the last token and writes nothing; every wave of the
 // block must make the call, there is a block barrier inside).  s_row_w / s_pre_w: this wave's 64 * VPL floats of LDS.
-// VPL: scores per lane, at least E / 64.
+// VPL: scores per lane, at least E / 64.  shared: always-on experts E .. E + shared - 1 behind the k selected ones of a token's row,
+// with weight 1.
 template <bool GATE, int VPL>
 __device__ __forceinline__ void route_token(
     const float* __restrict__ logits, const float* __restrict__ pre_bias, int T, int E, int k,
     int mode, int norm, int round_bf16, float scaling, int n_groups, int topk_groups,
-    float* __restrict__ w_out, int32_t* __restrict__ idx_out, const GateEpilogue& g, int t_raw, int lane, float* s_row_w, float* s_pre_w) {
+    float* __restrict__ w_out, int32_t* __restrict__ idx_out, int shared, const GateEpilogue& g, int t_raw, int lane, float* s_row_w, float* s_pre_w) {
   const bool active = t_raw < T;
   const int t = active ? t_raw : T - 1;
   const float* row = logits + (size_t)t * E;
@@ -248,9 +249,9 @@ __device__ __forceinline__ void route_token(
       if (round_bf16) w = round_bf16_fn(w);
     }
   }
-  if (active && lane < k) {
-    w_out[(size_t)t * k + lane] = w;
-    idx_out[(size_t)t * k + lane] = myi;
+  if (active && lane < k + shared) {
+    w_out[(size_t)t * (k + shared) + lane] = lane < k ? w : 1.0f;
+    idx_out[(size_t)t * (k + shared) + lane] = lane < k ? myi : E + lane - k;
   }
 }
 
@@ -258,11 +259,11 @@ template <bool GATE, int VPL>
 __global__ __launch_bounds__(kRouteWaves* kWave) void route_topk_kernel(
     const float* __restrict__ logits, const float* __restrict__ pre_bias, int T, int E, int k,
     int mode, int norm, int round_bf16, float scaling, int n_groups, int topk_groups,
-    float* __restrict__ w_out, int32_t* __restrict__ idx_out, const GateEpilogue g) {
+    float* __restrict__ w_out, int32_t* __restrict__ idx_out, int shared, const GateEpilogue g) {
   __shared__ float s_row[kRouteWaves][VPL * kWave];
   __shared__ float s_pre[GATE ? kRouteWaves : 1][GATE ? VPL * kWave : 1];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  route_token<GATE, VPL>(logits, pre_bias, T, E, k, mode, norm, round_bf16, scaling, n_groups, topk_groups, w_out, idx_out, g,
+  route_token<GATE, VPL>(logits, pre_bias, T, E, k, mode, norm, round_bf16, scaling, n_groups, topk_groups, w_out, idx_out, shared, g,
                          blockIdx.x * kRouteWaves + wave, lane, s_row[wave], s_pre[GATE ? wave : 0]);
 }
 
@@ -760,18 +761,21 @@ struct RouteArgs {
   int n_groups, topk_groups;
   float* w_out;
   int32_t* idx_out;
+  int shared;
 };
 
-template <int NW, int VPL>
+// GATE: from the gate product's partial sums (one launch less again)
+template <int NW, int VPL, bool GATE = false>
 __global__ __launch_bounds__(NW* kWave) void route_sort_small_kernel(
-    const RouteArgs r, int roll, int ebits, int32_t* __restrict__ group_sizes, int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm,
+    const RouteArgs r, const GateEpilogue g, int roll, int ebits, int32_t* __restrict__ group_sizes, int32_t* __restrict__ perm, int32_t* __restrict__ inv_perm,
     int32_t* __restrict__ sorted_experts, const SortMapArgs mp) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   // (one token per wave, all at once: r.T <= NW, no routing groups)
-  route_token<false, VPL>(r.logits, r.pre_bias, r.T, r.E, r.k, r.mode, r.norm, r.round_bf16, r.scaling, 0, 0, r.w_out, r.idx_out, GateEpilogue{}, wave, lane,
-                     nullptr, nullptr);
+  __shared__ float s_pre[GATE ? NW : 1][GATE ? VPL * kWave : 1];
+  route_token<GATE, VPL>(r.logits, r.pre_bias, r.T, r.E, r.k, r.mode, r.norm, r.round_bf16, r.scaling, 0, 0, r.w_out, r.idx_out, r.shared, g, wave, lane,
+                         nullptr, s_pre[GATE ? wave : 0]);
   __syncthreads();  // the indices, written above by this block, are read back from memory
-  sort_small_block<NW>(r.idx_out, r.T * r.k, r.E, roll, nullptr, ebits, group_sizes, perm, inv_perm, sorted_experts, mp);
+  sort_small_block<NW>(r.idx_out, r.T * (r.k + r.shared), r.E + r.shared, roll, nullptr, ebits, group_sizes, perm, inv_perm, sorted_experts, mp);
 }
 
 __global__ void invert_perm_kernel(const int32_t* __restrict__ perm, int M,
@@ -1251,10 +1255,16 @@ int moe_route_topk(const float* gate_logits, const float* pre_bias_logits, int T
   dispatch_vpl(E, [&](auto vpl) {
     route_topk_kernel<false, decltype(vpl)::value><<<cdiv(T, kRouteWaves), kRouteWaves * kWave, 0, (hipStream_t)stream>>>(
         gate_logits, pre_bias_logits, T, E, k, mode, norm_topk_prob, weights_round_bf16,
-        routed_scaling_factor, ng, topk_routing_group, topk_weights, topk_idx, GateEpilogue{});
+        routed_scaling_factor, ng, topk_routing_group, topk_weights, topk_idx, 0, GateEpilogue{});
   });
   return check_launch("route_topk_kernel");
 }
+
+// What moe_layer hands the routing for the smallest steps, where the sort runs behind it in the same launch.
+struct GateSort {
+  int32_t *group_sizes, *perm, *inv_perm;
+  void* gmm_workspace;
+};
 
 // How the gate product is cut.  Below 129 tiles of 32 tokens x 32 experts the chip is filled by splitting K (at least 8
 // chunks of 64, 2 per wave, in a block).  From there on, with more than 32 experts, the wide kernel: with up to 32 the
@@ -1285,11 +1295,11 @@ size_t moe_gate_route_workspace_bytes(int T, int d, int E) {
   return (size_t)std::max(gate_plan(T, d, E, 1).ks, gate_plan(T, d, E, 3).ks) * T * E * sizeof(float) + 16;
 }
 
-int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, const float* gate_bias, int T, int d,
+static int gate_route_impl(const void* x, const void* gate_kernel_terms, int num_terms, const float* gate_bias, int T, int d,
                    int E, int k, int score_func, int gate_round_bf16, int mode, int norm_topk_prob,
                    int weights_round_bf16, float routed_scaling_factor, int n_routing_groups, int topk_routing_group,
                    float* topk_weights, int32_t* topk_idx, float* gate_logits_out, float* pre_bias_logits_out,
-                   void* workspace, size_t workspace_bytes, void* stream) {
+                   void* workspace, size_t workspace_bytes, int shared, const GateSort* sort, bool* sorted, void* stream) {
   if (!x || !gate_kernel_terms || !topk_weights || !topk_idx || !workspace) return fail(MOE_ERR_INVALID_ARG, "gate_route: NULL pointer");
   if (T < 0 || d <= 0 || E <= 0 || k <= 0) return fail(MOE_ERR_INVALID_ARG, "gate_route: bad sizes T=%d d=%d E=%d k=%d", T, d, E, k);
   if (num_terms != 1 && num_terms != 3) return fail(MOE_ERR_INVALID_ARG, "gate_route: num_terms must be 1 or 3");
@@ -1327,12 +1337,41 @@ int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, 
   GateEpilogue ge;
   ge.partials = (const float*)workspace; ge.bias = gate_bias; ge.logits_out = gate_logits_out; ge.pre_bias_out = pre_bias_logits_out;
   ge.num_partials = ks; ge.score_func = score_func; ge.round_bf16 = gate_round_bf16;
+  // the smallest decode steps: a wave per token and the sort behind them in one block (route_sort_small_kernel)
+  if (sort && ng == 0 && T <= 4 * kSortWaves && (long long)T * (k + shared) <= kSortChunk && E + shared <= kSortMaxE) {
+    int ebits = 0;
+    while ((1 << ebits) < E + shared) ebits++;
+    const SortMapArgs mp = {(TileInfo*)((uint8_t*)sort->gmm_workspace + 16), (int32_t*)sort->gmm_workspace, E + shared, 0, 16, 1};
+    const RouteArgs r = {nullptr, nullptr, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, 0, 0, topk_weights, topk_idx, shared};
+    dispatch_vpl(E, [&](auto vpl) {
+      constexpr int V = decltype(vpl)::value;
+      if (T <= kSortWaves)
+        route_sort_small_kernel<kSortWaves, V, true><<<1, kSortWaves * kWave, 0, s>>>(r, ge, 0, ebits, sort->group_sizes, sort->perm, sort->inv_perm, nullptr, mp);
+      else
+        route_sort_small_kernel<4 * kSortWaves, V, true><<<1, 4 * kSortWaves * kWave, 0, s>>>(r, ge, 0, ebits, sort->group_sizes, sort->perm, sort->inv_perm,
+                                                                                              nullptr, mp);
+    });
+    if (int st = check_launch("route_sort_small_kernel")) return st;
+    note_tile_map_built(sort->gmm_workspace, sort->group_sizes, T * (k + shared), E + shared, 0, E + shared, 16, 1);
+    *sorted = true;
+    return MOE_OK;
+  }
   dispatch_vpl(E, [&](auto vpl) {
     route_topk_kernel<true, decltype(vpl)::value><<<cdiv(T, kRouteWaves), kRouteWaves * kWave, 0, s>>>(
         nullptr, nullptr, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, ng, topk_routing_group,
-        topk_weights, topk_idx, ge);
+        topk_weights, topk_idx, shared, ge);
   });
   return check_launch("gate_route");
+}
+
+int moe_gate_route(const void* x, const void* gate_kernel_terms, int num_terms, const float* gate_bias, int T, int d,
+                   int E, int k, int score_func, int gate_round_bf16, int mode, int norm_topk_prob,
+                   int weights_round_bf16, float routed_scaling_factor, int n_routing_groups, int topk_routing_group,
+                   float* topk_weights, int32_t* topk_idx, float* gate_logits_out, float* pre_bias_logits_out,
+                   void* workspace, size_t workspace_bytes, void* stream) {
+  return gate_route_impl(x, gate_kernel_terms, num_terms, gate_bias, T, d, E, k, score_func, gate_round_bf16, mode, norm_topk_prob, weights_round_bf16,
+                         routed_scaling_factor, n_routing_groups, topk_routing_group, topk_weights, topk_idx, gate_logits_out, pre_bias_logits_out, workspace,
+                         workspace_bytes, 0, nullptr, nullptr, stream);
 }
 
 size_t moe_sort_workspace_bytes(int T, int k, int E) {
@@ -1440,14 +1479,14 @@ int moe_route_sort_mapped(const float* gate_logits, const float* pre_bias_logits
   while ((1 << ebits) < E) ebits++;
   const int zero_fill = keep_other_rows ? 0 : 1;
   const SortMapArgs mp = {(TileInfo*)((uint8_t*)gmm_workspace + 16), (int32_t*)gmm_workspace, num_groups_local, group_offset, tile_rows, zero_fill};
-  const RouteArgs r = {gate_logits, pre_bias_logits, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, 0, 0, topk_weights, topk_idx};
+  const RouteArgs r = {gate_logits, pre_bias_logits, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, 0, 0, topk_weights, topk_idx, 0};
   dispatch_vpl(E, [&](auto vpl) {
     constexpr int V = decltype(vpl)::value;
     const hipStream_t st = (hipStream_t)stream;
     if (T <= kSortWaves)
-      route_sort_small_kernel<kSortWaves, V><<<1, kSortWaves * kWave, 0, st>>>(r, roll_to_expert_id, ebits, group_sizes, perm, inv_perm, sorted_experts, mp);
+      route_sort_small_kernel<kSortWaves, V><<<1, kSortWaves * kWave, 0, st>>>(r, GateEpilogue{}, roll_to_expert_id, ebits, group_sizes, perm, inv_perm, sorted_experts, mp);
     else
-      route_sort_small_kernel<4 * kSortWaves, V><<<1, 4 * kSortWaves * kWave, 0, st>>>(r, roll_to_expert_id, ebits, group_sizes, perm, inv_perm,
+      route_sort_small_kernel<4 * kSortWaves, V><<<1, 4 * kSortWaves * kWave, 0, st>>>(r, GateEpilogue{}, roll_to_expert_id, ebits, group_sizes, perm, inv_perm,
                                                                                         sorted_experts, mp);
   });
   if (int st = check_launch("route_sort_small_kernel")) return st;
@@ -1575,6 +1614,147 @@ int moe_transpose_rhs(const void* rhs_gkn, int G, int K, int N, int elem_bytes, 
   else
     return fail(MOE_ERR_UNSUPPORTED, "transpose: elem_bytes %d", elem_bytes);
   return check_launch("transpose_kernel");
+}
+
+// ---- one expert layer, router included, as one call ----
+// Host work only: the launches are those of the entry points above, called one after the other on buffers cut out of one
+// workspace.  From Python the calls and their tensors took longer than a decode step's kernels (GPT-OSS shape, one token: 83 us for
+// 42 us of kernels).
+namespace {
+struct LayerPlan {
+  int M, K2, Et;          // routed rows, selections per token and experts with the shared ones
+  bool mapped;            // the sort leaves the tile list of the streaming kernels
+  size_t weights, idx, perm, inv, groups, gate_ws, sort_ws, gmm_ws, gmm_bytes, xq, xs, inter, iq, is, y, total;
+};
+}  // namespace
+
+static int layer_plan(const moe_layer_args* a, LayerPlan* p) {
+  if (!a) return fail(MOE_ERR_INVALID_ARG, "layer: NULL args");
+  if (a->struct_size != sizeof(moe_layer_args)) return fail(MOE_ERR_INVALID_ARG, "layer: struct_size %zu != %zu", a->struct_size, sizeof(moe_layer_args));
+  if (a->T <= 0 || a->d <= 0 || a->f <= 0 || a->E <= 0 || a->k <= 0 || a->shared_experts < 0) return fail(MOE_ERR_INVALID_ARG, "layer: bad sizes");
+  if (a->k + a->shared_experts > 16) return fail(MOE_ERR_UNSUPPORTED, "layer: at most 16 selections per token, shared ones included");
+  const long long rows = (long long)a->T * (a->k + a->shared_experts);
+  if (rows > INT_MAX / 2) return fail(MOE_ERR_UNSUPPORTED, "layer: too many rows");
+  if (a->act_dtype != MOE_BF16 && a->act_dtype != MOE_INT8 && a->act_dtype != MOE_FP8_E4M3) return fail(MOE_ERR_INVALID_ARG, "layer: bad act_dtype %d", a->act_dtype);
+  if (a->act_block_k < 0) return fail(MOE_ERR_INVALID_ARG, "layer: bad act_block_k");
+  p->M = (int)rows;
+  p->K2 = a->k + a->shared_experts;
+  p->Et = a->E + a->shared_experts;
+  // (the sort's one-launch limit, and the rows per expert up to which moe_gmm takes 16-row tiles)
+  p->mapped = rows <= std::min(4096LL, 16LL * p->Et);
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  const bool quant = a->act_dtype != MOE_BF16;
+  const size_t M = p->M, T = a->T, d = a->d, f = a->f;
+  auto scales = [&](size_t r, size_t n) { return r * (a->act_block_k ? (n + a->act_block_k - 1) / a->act_block_k : 1) * 4; };
+  p->weights = take(M * 4);
+  p->idx = take(M * 4);
+  p->perm = take(M * 4);
+  p->inv = take(M * 4);
+  p->groups = take((size_t)p->Et * 4);
+  p->gate_ws = take(moe_gate_route_workspace_bytes(a->T, a->d, a->E));
+  p->sort_ws = take(std::max(moe_sort_workspace_bytes(a->T, p->K2, p->Et), (size_t)16));
+  // (15 rows per group on average: the lowest that a prefill kernel takes)
+  p->gmm_bytes = p->M >= 15LL * p->Et ? moe_gmm_split_workspace_bytes(p->M, p->Et) : moe_gmm_workspace_bytes(p->M, p->Et);
+  p->gmm_ws = take(p->gmm_bytes);
+  p->xq = p->xs = p->iq = p->is = 0;
+  if (quant) {
+    p->xq = take(T * d);
+    p->xs = take(scales(T, d));
+    p->iq = take(M * f);
+    p->is = take(scales(M, f));
+    // the second product's rows take the place of the activations that were quantised for it
+    p->inter = p->y = take(std::max(M * f, M * d) * 2);
+  } else {
+    p->inter = take(M * f * 2);
+    p->y = take(M * d * 2);
+  }
+  p->total = at;
+  return MOE_OK;
+}
+
+size_t moe_layer_workspace_bytes(const moe_layer_args* a) {
+  LayerPlan p;
+  return layer_plan(a, &p) == MOE_OK ? p.total : 0;
+}
+
+int moe_layer(const moe_layer_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  LayerPlan p;
+  if (int st = layer_plan(a, &p)) return st;
+  if (!a->x || !a->gate_terms || !a->wi_0 || !a->wi_1 || !a->wo || !a->out || !workspace) return fail(MOE_ERR_INVALID_ARG, "layer: NULL pointer");
+  if (workspace_bytes < p.total) return fail(MOE_ERR_WORKSPACE, "layer: workspace too small");
+  if ((uintptr_t)workspace & 255) return fail(MOE_ERR_UNSUPPORTED, "layer: the workspace must be 256-byte aligned");
+  uint8_t* ws = (uint8_t*)workspace;
+  float* weights = (float*)(ws + p.weights);
+  int32_t *idx = (int32_t*)(ws + p.idx), *perm = (int32_t*)(ws + p.perm), *inv = (int32_t*)(ws + p.inv), *groups = (int32_t*)(ws + p.groups);
+  void* gmm_ws = ws + p.gmm_ws;
+  const int T = a->T, d = a->d, f = a->f;
+  const bool quant = a->act_dtype != MOE_BF16;
+  const GateSort gs = {groups, perm, inv, gmm_ws};
+  bool sorted = false;
+  if (int st = gate_route_impl(a->gate_x ? a->gate_x : a->x, a->gate_terms, a->num_gate_terms, a->gate_bias, T, d, a->E, a->k, a->score_func, a->gate_round_bf16,
+                               a->route_mode, a->norm_topk_prob, a->weights_round_bf16, a->routed_scaling_factor, a->n_routing_groups, a->topk_routing_group,
+                               weights, idx, nullptr, nullptr, ws + p.gate_ws, moe_gate_route_workspace_bytes(T, d, a->E), a->shared_experts,
+                               p.mapped ? &gs : nullptr, &sorted, stream))
+    return st;
+  if (!sorted) {
+    const size_t sort_bytes = std::max(moe_sort_workspace_bytes(T, p.K2, p.Et), (size_t)16);
+    const int st = p.mapped ? moe_sort_by_expert_mapped(idx, T, p.K2, p.Et, 0, perm, inv, groups, nullptr, ws + p.sort_ws, sort_bytes, 16, p.Et, 0, 0, gmm_ws,
+                                                        p.gmm_bytes, stream)
+                            : moe_sort_by_expert_rolled(idx, T, p.K2, p.Et, 0, perm, inv, groups, nullptr, ws + p.sort_ws, sort_bytes, stream);
+    if (st) return st;
+  }
+  moe_gmm_args g = {};
+  g.struct_size = sizeof(g);
+  g.group_sizes = groups;
+  g.workspace = gmm_ws;
+  g.workspace_bytes = p.gmm_bytes;
+  g.M = p.M;
+  g.num_groups_total = g.num_groups_local = p.Et;
+  g.lhs_dtype = a->act_dtype;
+  g.rhs_dtype = a->rhs_dtype;
+  g.lhs_scale_block_k = quant ? a->act_block_k : 0;
+  g.act_limit = a->act_limit;
+  g.out_dtype = MOE_BF16;
+  g.lhs_rows = T;
+  g.lhs = a->x;
+  if (quant) {
+    if (int st = moe_gather_rows(a->x, nullptr, 1, T, T, d, a->act_dtype, a->act_block_k, MOE_QUANT_RINT_DIV, nullptr, nullptr, nullptr, ws + p.xq,
+                                 (float*)(ws + p.xs), stream))
+      return st;
+    g.lhs = ws + p.xq;
+    g.lhs_scale = (const float*)(ws + p.xs);
+  }
+  g.rhs = a->wi_0; g.rhs_scale = a->wi_0_scale; g.rhs_up = a->wi_1; g.rhs_up_scale = a->wi_1_scale;
+  g.out = ws + p.inter;
+  g.K = d; g.N = f;
+  g.rhs_scale_block_n = a->wi_scale_block_n; g.rhs_scale_block_k = a->wi_scale_block_k;
+  g.act = a->act;
+  g.lhs_row_idx = perm; g.lhs_row_idx_div = p.K2;
+  g.flags = a->wi_flags | (p.mapped ? MOE_GMM_SAME_GROUPS : 0);
+  if (int st = moe_gmm(&g, stream)) return st;
+  g.lhs = ws + p.inter;
+  g.lhs_scale = nullptr;
+  if (quant) {
+    if (int st = moe_gather_rows(ws + p.inter, nullptr, 1, p.M, p.M, f, a->act_dtype, a->act_block_k, MOE_QUANT_RINT_DIV, nullptr, nullptr, nullptr, ws + p.iq,
+                                 (float*)(ws + p.is), stream))
+      return st;
+    g.lhs = ws + p.iq;
+    g.lhs_scale = (const float*)(ws + p.is);
+  }
+  g.rhs = a->wo; g.rhs_scale = a->wo_scale; g.rhs_up = nullptr; g.rhs_up_scale = nullptr;
+  g.out = ws + p.y;
+  g.K = f; g.N = d;
+  g.rhs_scale_block_n = a->wo_scale_block_n; g.rhs_scale_block_k = a->wo_scale_block_k;
+  g.act = MOE_ACT_NONE;
+  g.lhs_row_idx = nullptr; g.lhs_row_idx_div = 1; g.lhs_rows = p.M;
+  g.flags = a->wo_flags | MOE_GMM_SAME_GROUPS;
+  if (int st = moe_gmm(&g, stream)) return st;
+  return moe_unpermute_combine(ws + p.y, nullptr, inv, weights, nullptr, T, p.K2, d, a->out, nullptr, 0, stream);
 }
 
 }  // extern "C"

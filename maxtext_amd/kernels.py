@@ -648,6 +648,28 @@ def _gmm_workspace_bytes(m, num_groups_total, split):
   return max(size(m, num_groups_total), 16)
 
 
+def layer(x, gate_terms, wi_0, wi_1, wo, *, num_experts, k, gate_x=None, gate_bias=None, shared_experts=0, score_func="", gate_round_bf16=False,
+          mode="softmax_topk", norm_topk_prob=False, weights_round_bf16=True, routed_scaling_factor=1.0, n_routing_groups=-1, topk_routing_group=-1,
+          wi_0_scale=None, wi_1_scale=None, wo_scale=None, rhs_dtype=_lib.MOE_BF16, wi_layout=(1, 0, 0), wo_layout=(1, 0, 0),
+          act_dtype=_lib.MOE_BF16, act_block_k=0, act="silu", act_limit=7.0):
+  """A whole expert layer without gradients through one library call (moe_layer): x [T, d] bf16 -> [T, d] bf16.
+  Operands as include/moe_mi355x.h has them; the caller has checked shapes, types and contiguity (`RoutedMoE` does).
+  wi_layout / wo_layout: (scale block_n, scale block_k, MOE_GMM_RHS_SCALE_* flags) of the weights' scales."""
+  t, d = x.shape
+  lib = _lib.load()
+  p = _lib.ptr
+  out = torch.empty_like(x)
+  args = _lib.LAYER_ARGS.pack(
+      _lib.LAYER_ARGS.size, x.data_ptr(), p(gate_x) or 0, gate_terms.data_ptr(), p(gate_bias) or 0, wi_0.data_ptr(), p(wi_0_scale) or 0, wi_1.data_ptr(),
+      p(wi_1_scale) or 0, wo.data_ptr(), p(wo_scale) or 0, out.data_ptr(), t, d, wi_0.shape[1], num_experts, k, shared_experts, gate_terms.shape[0],
+      _SCORE_FUNC_CODE[score_func], bool(gate_round_bf16), _lib.ROUTE_BY_NAME[mode], bool(norm_topk_prob), bool(weights_round_bf16), routed_scaling_factor,
+      n_routing_groups, topk_routing_group, rhs_dtype, *wi_layout, *wo_layout, act_dtype, act_block_k, _lib.ACT_BY_NAME[act], act_limit)
+  nbytes = lib.moe_layer_workspace_bytes(args)
+  ws = torch.empty((nbytes,), dtype=torch.uint8, device=x.device)
+  _lib.check(lib.moe_layer(args, ws.data_ptr(), nbytes, _lib.current_stream()), "moe_layer")
+  return out
+
+
 def gmm_lhs_e5m2_supported(m, k, n, num_groups_total):
   """True when `gmm_raw` takes float8_e5m2 activations (against e4m3 weights) for this shape."""
   return bool(_lib.load().moe_gmm_lhs_e5m2_supported(int(m), int(k), int(n), int(num_groups_total)))

@@ -13,7 +13,7 @@ from typing import Optional
 
 import torch
 
-from maxtext_amd import kernels, megablox
+from maxtext_amd import _lib, kernels, megablox
 from maxtext_amd.quantizations import QArray
 
 
@@ -171,22 +171,62 @@ class RoutedMoE:
     cfg = self.config
     if cfg.routed_score_func not in ("", "sigmoid", "sqrtsoftplus"):
       raise NotImplementedError(cfg.routed_score_func)
-    if self._gate_terms is None or self._gate_terms.device != inputs_2d.device:
+    x = inputs_2d.to(torch.bfloat16).contiguous()
+    r = kernels.gate_route(x, self._terms_on(inputs_2d.device), self._bias_f32(), return_logits=return_logits, **self._gate_args())
+    if cfg.is_deepseek:
+      return r
+    return (self._scale_per_expert(r[0], r[1]),) + tuple(r[1:])
+
+  def _terms_on(self, device):
+    if self._gate_terms is None or self._gate_terms.device != device:
       from maxtext_amd.quantizations import split_gate_kernel
 
-      self._gate_terms = split_gate_kernel(self.gate_kernel, 3 if cfg.float32_gate_logits else 1).to(inputs_2d.device)
-    bias = None if self.gate_bias is None else self.gate_bias.float().contiguous()
-    common = dict(k=self.num_experts_per_tok, score_func=cfg.routed_score_func, gate_round_bf16=not cfg.float32_gate_logits,
-                  return_logits=return_logits)
-    x = inputs_2d.to(torch.bfloat16).contiguous()
+      self._gate_terms = split_gate_kernel(self.gate_kernel, 3 if self.config.float32_gate_logits else 1).to(device)
+    return self._gate_terms
+
+  def _bias_f32(self):
+    return None if self.gate_bias is None else self.gate_bias.float().contiguous()
+
+  def _gate_args(self):
+    """Score function and weight rule of the router, as moe_gate_route takes them."""
+    cfg = self.config
+    common = dict(k=self.num_experts_per_tok, score_func=cfg.routed_score_func, gate_round_bf16=not cfg.float32_gate_logits)
     if cfg.is_deepseek:
-      return kernels.gate_route(x, self._gate_terms, bias, mode="deepseek",
-                                norm_topk_prob=cfg.routed_score_func in ("sigmoid", "sqrtsoftplus"),
-                                routed_scaling_factor=cfg.routed_scaling_factor, n_routing_groups=cfg.n_routing_groups,
-                                topk_routing_group=cfg.topk_routing_group, **common)
-    r = kernels.gate_route(x, self._gate_terms, bias, mode=cfg.route_mode, norm_topk_prob=cfg.norm_topk_prob,
-                           weights_round_bf16=cfg.route_mode != "topk_raw", **common)
-    return (self._scale_per_expert(r[0], r[1]),) + tuple(r[1:])
+      return dict(common, mode="deepseek", norm_topk_prob=cfg.routed_score_func in ("sigmoid", "sqrtsoftplus"),
+                  routed_scaling_factor=cfg.routed_scaling_factor, n_routing_groups=cfg.n_routing_groups, topk_routing_group=cfg.topk_routing_group)
+    mode = cfg.route_mode
+    return dict(common, mode=mode, norm_topk_prob=cfg.norm_topk_prob, weights_round_bf16=mode != "topk_raw")
+
+  # -- the whole layer through one library call ------------------------------------------------
+  def _layer(self, inputs, routing_inputs, shared_experts=0):
+    """The layer's output by moe_layer, or None where it does not apply: gradients, auxiliary outputs, routing the call does not
+    know, operands that the single calls would convert or refuse.  Bit for bit what the single calls give."""
+    cfg = self.config
+    if (self.tid2eid is not None or self.per_expert_scale is not None or self.profile_events is not None or cfg.load_balance_loss_weight > 0.0
+        or (cfg.routed_bias and cfg.routed_bias_update_rate > 0.0) or not cfg.float32_weight_sum or cfg.decoder_block == "llama4"):
+      return None
+    d = inputs.shape[-1]
+    if inputs.dtype != torch.bfloat16 or not inputs.is_cuda or inputs.numel() == 0 or routing_inputs.shape != inputs.shape or routing_inputs.device != inputs.device:
+      return None
+    w = _native_weights(self.wi_0, self.wi_1, self.wo, self.num_experts + shared_experts, d, inputs.device)
+    if w is None:
+      return None
+    if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in (inputs, routing_inputs, self.gate_kernel, self.gate_bias, *w["tensors"])):
+      return None
+    quant = {None: (_lib.MOE_BF16, 0), "int8": (_lib.MOE_INT8, 0), "fp8": (_lib.MOE_FP8_E4M3, 128), "fp8_row": (_lib.MOE_FP8_E4M3, 0)}.get(cfg.act_quant)
+    if quant is None:
+      return None
+    terms, bias = self._terms_on(inputs.device), self._bias_f32()
+    if terms.shape[1:] != (self.num_experts, d) or (bias is not None and (bias.numel() != self.num_experts or bias.device != inputs.device)):
+      return None
+    x = inputs.reshape(-1, d).contiguous()
+    gx = None if routing_inputs is inputs else routing_inputs.reshape(-1, d).contiguous()
+    wi_0, s0, wi_1, s1, wo, so = w["tensors"]
+    out = kernels.layer(x, terms, wi_0, wi_1, wo, num_experts=self.num_experts, gate_x=gx, gate_bias=bias,
+                        shared_experts=shared_experts, wi_0_scale=s0, wi_1_scale=s1, wo_scale=so, rhs_dtype=w["dtype"], wi_layout=w["wi"], wo_layout=w["wo"],
+                        act_dtype=quant[0], act_block_k=quant[1], act=cfg.activation,
+                        act_limit=cfg.mlp_activations_limit if cfg.mlp_activations_limit > 0 else 7.0, **self._gate_args())
+    return out.reshape(inputs.shape)
 
   def _scale_per_expert(self, w, idx):
     if self.per_expert_scale is None:
@@ -494,6 +534,9 @@ class RoutedMoE:
         isinstance(t, torch.Tensor) and t.requires_grad for t in (routing_inputs, self.gate_kernel, self.gate_bias))
     fused_router = self.tid2eid is None and self.config.routed_score_func in ("", "sigmoid", "sqrtsoftplus")
     if fused_router and not needs_grad and routing_inputs.dtype == torch.bfloat16 and routing_inputs.shape[-1] % 64 == 0 and self.num_experts % 4 == 0:
+      out = self._layer(inputs, routing_inputs)
+      if out is not None:
+        return out, None, None
       want_logits = self.config.load_balance_loss_weight > 0.0  # the auxiliary loss needs the full distribution
       r = self.gate_and_route(routing_inputs.reshape(b * s, -1), return_logits=want_logits)
       logits = r[2].reshape(b, s, -1) if want_logits else None
@@ -502,6 +545,43 @@ class RoutedMoE:
     gate_logits = gate_logits.reshape(b, s, -1)
     pre_bias = None if pre_bias is None else pre_bias.reshape(b, s, -1)
     return self.sparse_matmul(inputs, gate_logits, pre_bias, self.wi_0, self.wi_1, self.wo, input_ids=input_ids)
+
+
+_WEIGHT_CODES = {"int8": (_lib.MOE_INT8, torch.int8, 1), "fp8": (_lib.MOE_FP8_E4M3, torch.float8_e4m3fn, 1), "int4": (_lib.MOE_INT4, torch.uint8, 2),
+                 "int4g32": (_lib.MOE_INT4, torch.uint8, 2), "mxfp4": (_lib.MOE_MXFP4, torch.uint8, 2)}
+
+
+def _native_weights(wi_0, wi_1, wo, groups, d, device):
+  """The expert weights as moe_layer takes them (values and scales, type code, scale layouts), or None unless they are just that:
+  contiguous [G, N, K] on the device, of one type, scales of the size and type their layout implies."""
+  if all(isinstance(w, QArray) for w in (wi_0, wi_1, wo)):
+    if not (wi_0.qtype == wi_1.qtype == wo.qtype) or wi_0.qtype not in _WEIGHT_CODES:
+      return None
+    code, dtype, per_byte = _WEIGHT_CODES[wi_0.qtype]
+    values, scales = (wi_0.qvalue, wi_1.qvalue, wo.qvalue), (wi_0.scale, wi_1.scale, wo.scale)
+    layouts = [megablox._rhs_layout(w) for w in (wi_0, wi_1, wo)]
+    if layouts[0] != layouts[1]:
+      return None
+  elif all(isinstance(w, torch.Tensor) for w in (wi_0, wi_1, wo)):
+    code, dtype, per_byte = _lib.MOE_BF16, torch.bfloat16, 1
+    values, scales, layouts = (wi_0, wi_1, wo), (None, None, None), None
+  else:
+    return None
+  if any(v.dtype != dtype or v.dim() != 3 or v.device != device or not v.is_contiguous() for v in values):
+    return None
+  f = values[0].shape[1]
+  if d % per_byte or f % per_byte or any(v.shape != want for v, want in zip(values, ((groups, f, d // per_byte), (groups, f, d // per_byte), (groups, d, f // per_byte)))):
+    return None
+  triples = [(1, 0, 0)] * 3
+  if layouts is not None:
+    for i, (s, lay, n, k) in enumerate(zip(scales, layouts, (f, f, d), (d, d, f))):
+      bn, bk, kmajor, shared = lay["rhs_scale_block_n"], lay["rhs_scale_block_k"], lay["rhs_scale_kmajor"], lay["rhs_scale_shared"]
+      want = torch.bfloat16 if code == _lib.MOE_INT4 and not kmajor else torch.uint8 if code == _lib.MOE_MXFP4 else torch.float32
+      count = (1 if shared else groups) * (1 if bn == _lib.MOE_SCALE_PER_TENSOR else -(-n // bn)) * (1 if bk == 0 else -(-k // bk))
+      if s.dtype != want or s.numel() != count or s.device != device or not s.is_contiguous():
+        return None
+      triples[i] = (bn, bk, (_lib.MOE_GMM_RHS_SCALE_KMAJOR if kmajor else 0) | (_lib.MOE_GMM_RHS_SCALE_SHARED if shared else 0))
+  return {"tensors": (values[0], scales[0], values[1], scales[1], values[2], scales[2]), "dtype": code, "wi": triples[0], "wo": triples[2]}
 
 
 def _quantize_tokens(x2d, act_quant):
@@ -569,6 +649,9 @@ class RoutedAndSharedMoE:
     routing_inputs = inputs if gate_inputs is None else gate_inputs
     fused = r.tid2eid is None and routing_inputs.dtype == torch.bfloat16 and routing_inputs.shape[-1] % 64 == 0 and cfg_ok(self.config)
     if fused:
+      out = r._layer(inputs, routing_inputs, self.config.shared_experts)
+      if out is not None:
+        return out, None, None
       want_logits = self.config.load_balance_loss_weight > 0.0  # the auxiliary loss needs the full distribution
       g = r.gate_and_route(routing_inputs.reshape(b * s, -1), return_logits=want_logits)
       logits = g[2].reshape(b, s, -1) if want_logits else None
