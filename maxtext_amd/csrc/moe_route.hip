@@ -630,11 +630,11 @@ __device__ __forceinline__ void sort_small_block(
   constexpr int NT = NW * kWave;
   roll = resolve_roll(roll, roll_dev, E);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  if (M <= kWave && E <= kWave) {
-    // The smallest decode steps (at most 64 routed rows over at most 64 experts): one wave holds an entry and an expert per
-    // lane and sorts without a block barrier or a trip through memory: equal keys found by ballots, their count left in LDS
-    // by the first of them, the experts' first rows by a scan over the lanes.  The tile list is then built from the counts in LDS.
-    __shared__ int t_cnt[kWave], t_off[kWave];
+  if (M <= kWave) {
+    // The smallest decode steps (at most 64 routed rows): one wave holds an entry per lane and sorts without a block barrier or a
+    // trip through memory: equal keys found by ballots, their count left in LDS by the first of them, the experts' first rows by a
+    // scan over the lanes, each of which has `per` experts.  The tile list is then built from the counts in LDS.
+    __shared__ int t_cnt[kSortMaxE], t_off[kSortMaxE];
     if (wave == 0) {
       const bool valid = lane < M;
       const int e = valid ? sort_key(flat[lane], E, roll) : 0;
@@ -645,20 +645,26 @@ __device__ __forceinline__ void sort_small_block(
         mask &= bit ? bal : ~bal;
       }
       const int rank = __popcll(mask & ((1ull << lane) - 1ull)), cnt = __popcll(mask);
-      t_cnt[lane] = 0;
+      for (int i = lane; i < E; i += kWave) t_cnt[i] = 0;
       __builtin_amdgcn_wave_barrier();
       if (valid && rank == 0) t_cnt[e] = cnt;
       __builtin_amdgcn_wave_barrier();
-      const int c = lane < E ? t_cnt[lane] : 0;
+      const int per = (E + kWave - 1) / kWave, first = lane * per;
+      int c = 0;
+      for (int i = first; i < min(first + per, E); i++) c += t_cnt[i];
       int incl = c;
 #pragma unroll
       for (int o = 1; o < kWave; o <<= 1) {
         const int t = __shfl_up(incl, o);
         if (lane >= o) incl += t;
       }
-      t_off[lane] = incl - c;
-      if (lane < E) group_sizes[lane] = c;
+      int at = incl - c;
+      for (int i = first; i < min(first + per, E); i++) {
+        t_off[i] = at;
+        at += t_cnt[i];
+      }
       __builtin_amdgcn_wave_barrier();
+      for (int i = lane; i < E; i += kWave) group_sizes[i] = t_cnt[i];
       if (valid) {
         const int dest = t_off[e] + rank;
         perm[dest] = lane;

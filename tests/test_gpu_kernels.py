@@ -2196,6 +2196,28 @@ def test_sort_leaves_the_tile_list_for_the_matmuls(K, t, e, k):
   assert torch.equal(y2, y)
 
 
+@pytest.mark.parametrize("t,e,k,roll", [(1, 65, 4, 0), (8, 128, 8, 0), (2, 512, 16, 500), (7, 257, 9, 0), (8, 256, 8, 31), (9, 128, 8, 0), (64, 130, 1, 7)])
+def test_sort_of_at_most_64_rows_over_many_experts(K, t, e, k, roll):
+  """One wave sorts up to 64 rows over any number of experts, several to a lane: permutation, its inverse, group sizes, sorted ids and
+  the tile list (by the matmul on it), up to the last expert."""
+  rng = np.random.default_rng(e + k)
+  sel = np.stack([rng.permutation(e)[:k] for _ in range(t)]).astype(np.int32)
+  sel[0, 0] = e - 1 if e - 1 not in sel[0, 1:] else sel[0, 0]
+  keys = (sel.reshape(-1) - roll) % e
+  want = np.argsort(keys, kind="stable")
+  perm, inv, gs, se = K.sort_by_expert(cuda(sel), e, roll_to_expert_id=roll)
+  np.testing.assert_array_equal(perm.cpu().numpy(), want)
+  np.testing.assert_array_equal(inv.cpu().numpy(), np.argsort(want))
+  np.testing.assert_array_equal(gs.cpu().numpy(), np.bincount(keys, minlength=e))
+  np.testing.assert_array_equal(se.cpu().numpy(), keys[want])
+  ws = K.gmm_workspace(t * k, e, "cuda")
+  perm, inv, gs, se = K.sort_by_expert(cuda(sel), e, roll_to_expert_id=roll, gmm_workspace=ws)
+  g = torch.Generator(device="cuda").manual_seed(t)
+  x = torch.randn((t * k, 128), generator=g, device="cuda").to(torch.bfloat16)
+  w, sc = torch.randint(-127, 128, (e, 256, 128), generator=g, device="cuda", dtype=torch.int8), torch.rand((e, 256), generator=g, device="cuda") * 0.01
+  assert torch.equal(K.gmm_raw(x, w, gs, rhs_scale=sc, workspace=ws, same_groups=True), K.gmm_raw(x, w, gs.clone(), rhs_scale=sc))
+
+
 @pytest.mark.parametrize("t,e,k,mode", [(1, 32, 4, "softmax_topk"), (16, 32, 4, "softmax_topk"), (3, 128, 5, "topk_raw"), (13, 256, 8, "deepseek"),
                                         (4, 8, 2, "softmax_all"), (5, 8, 2, "softmax_all"), (17, 32, 4, "softmax_topk"), (300, 32, 4, "softmax_topk")])
 def test_route_and_sort_in_one_call(K, t, e, k, mode):
