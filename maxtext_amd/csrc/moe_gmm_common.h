@@ -230,7 +230,7 @@ struct TiledParams {
 
 __device__ __forceinline__ uint32_t i8x2_to_bf16x2(int lo, int hi) {
   // |value| <= 128 is exact in bf16, so truncating the f32 is the conversion
-  return (__float_as_uint((float)lo) >> 16) | (__float_as_uint((float)hi) & 0xffff0000u);
+  return __builtin_amdgcn_perm(__float_as_uint((float)hi), __float_as_uint((float)lo), 0x07060302u);
 }
 
 // Bias of 4 consecutive output channels of one group (zeros without a bias).
@@ -807,5 +807,8 @@ int launch_fp8_skinny(bool few_rows, const SkinnyParams& p, bool glu, int max_ti
 // moe_gmm_wq.hip: fmt is one of WQ_*; one_tile: 16-row tiles (else 32)
 enum { WQ_I8 = 0, WQ_I4 = 1, WQ_MX4 = 2, WQ_I4G32 = 3 };  // weight formats of the streaming kernel (int4: group 128 / 32)
 int launch_wq(int fmt, bool one_tile, const WqSkinnyParams& q, bool glu, int max_tiles, int tune, hipStream_t s);
+bool wq_i8_persistent(const WqSkinnyParams& p, int num_groups_local, bool glu);
+int launch_wq_i8(int rows, const WqSkinnyParams& q, bool glu, int num_groups_local, hipStream_t s);
+int prepare_wq();
 
 }  // namespace moe

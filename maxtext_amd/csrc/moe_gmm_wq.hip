@@ -1,6 +1,6 @@
 // Grouped matmul: the streaming kernel for bf16 activations x int8 / int4 / mxfp4 weights (decode).
 
-#include "moe_gmm_common.h"
+#include "moe_gmm_wqs_run.h"
 
 namespace moe {
 
@@ -429,6 +429,13 @@ __global__ __launch_bounds__(256) void gmm_wq_skinny_kernel(const WqSkinnyParams
 }
 
 
+// The persistent form for int8: the weights travel through LDS (moe_gmm_wqs_run.h), NSEG segments of 512 bytes to a row.
+template <int NSEG, bool GLU, int ROWS>
+__global__ __launch_bounds__(kWqsThreads) void gmm_wq_skinny_kernel(const WqSkinnyParams p, int num_groups) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  wqs_run<WQ_I8, NSEG, GLU, ROWS>(p, num_groups, smem);
+}
+
 // ---------------------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------------------
@@ -479,6 +486,65 @@ int launch_wq(int fmt, bool one_tile, const WqSkinnyParams& q, bool glu, int mx,
   MOE_WQ_CASE(WQ_I4G32)
 #undef MOE_WQ_CASE
   return fail(MOE_ERR_INVALID_ARG, "gmm: unknown streaming weight format %d", fmt);
+}
+
+// ---- the persistent form for int8 ----
+
+// K up to 3072 (six k-blocks of activations to a wave), at least four channel groups to a tile, whole channels' scales in a row on
+// 16-byte boundaries, tensors within 32-bit offsets (an item's last rows may lie up to 63 rows past N)
+bool wq_i8_persistent(const WqSkinnyParams& p, int num_groups, bool glu) {
+  return p.K % 32 == 0 && p.K <= kWqsMaxKBlocks * 128 && p.N % 8 == 0 && cdiv(p.N, glu ? 32 : 64) >= 4 && p.ch_nstride == 1 && p.ch_gstride == p.N &&
+         (long long)num_groups * p.N * p.K + 65LL * p.K + 1024 < (1LL << 32);
+}
+
+template <int NSEG, bool GLU, int ROWS>
+static int reserve_wq_i8() {
+  auto kernel = static_cast<void (*)(const WqSkinnyParams, int)>(gmm_wq_skinny_kernel<NSEG, GLU, ROWS>);
+  return reserve_lds(kernel, kWqsLds, lds_flags<std::integral_constant<int, 7600 + ROWS * 100 + NSEG * 2 + (GLU ? 1 : 0)>>());
+}
+
+template <int NSEG, bool GLU, int ROWS>
+static int launch_wq_i8_one(const WqSkinnyParams& p, int num_groups, int blocks, hipStream_t s) {
+  if (int st = reserve_wq_i8<NSEG, GLU, ROWS>()) return st;
+  gmm_wq_skinny_kernel<NSEG, GLU, ROWS><<<blocks, kWqsThreads, kWqsLds, s>>>(p, num_groups);
+  return check_launch("gmm_wq_skinny_kernel");
+}
+
+template <int NSEG>
+static int launch_wq_i8_seg(int rows, const WqSkinnyParams& p, bool glu, int num_groups, int blocks, hipStream_t s) {
+  if (rows == 32) return glu ? launch_wq_i8_one<NSEG, true, 32>(p, num_groups, blocks, s) : launch_wq_i8_one<NSEG, false, 32>(p, num_groups, blocks, s);
+  return glu ? launch_wq_i8_one<NSEG, true, 16>(p, num_groups, blocks, s) : launch_wq_i8_one<NSEG, false, 16>(p, num_groups, blocks, s);
+}
+
+int launch_wq_i8(int rows, const WqSkinnyParams& p, bool glu, int num_groups, hipStream_t s) {
+  int cus = 0;
+  if (int st = device_cu_count(&cus)) return st;
+  switch (cdiv(p.K, 512)) {
+    case 1: return launch_wq_i8_seg<1>(rows, p, glu, num_groups, cus, s);
+    case 2: return launch_wq_i8_seg<2>(rows, p, glu, num_groups, cus, s);
+    case 3: return launch_wq_i8_seg<3>(rows, p, glu, num_groups, cus, s);
+    case 4: return launch_wq_i8_seg<4>(rows, p, glu, num_groups, cus, s);
+    case 5: return launch_wq_i8_seg<5>(rows, p, glu, num_groups, cus, s);
+    case 6: return launch_wq_i8_seg<6>(rows, p, glu, num_groups, cus, s);
+  }
+  return fail(MOE_ERR_UNSUPPORTED, "gmm: K = %d is past the LDS-streamed decode kernel", p.K);
+}
+
+template <int NSEG>
+static int prepare_wq_seg() {
+  if (int st = reserve_wq_i8<NSEG, true, 16>()) return st;
+  if (int st = reserve_wq_i8<NSEG, false, 16>()) return st;
+  if (int st = reserve_wq_i8<NSEG, true, 32>()) return st;
+  return reserve_wq_i8<NSEG, false, 32>();
+}
+
+int prepare_wq() {
+  if (int st = prepare_wq_seg<1>()) return st;
+  if (int st = prepare_wq_seg<2>()) return st;
+  if (int st = prepare_wq_seg<3>()) return st;
+  if (int st = prepare_wq_seg<4>()) return st;
+  if (int st = prepare_wq_seg<5>()) return st;
+  return prepare_wq_seg<6>();
 }
 
 }  // namespace moe

@@ -875,6 +875,76 @@ def test_int4_rows_past_whole_128_or_256_rows_multiply_f32_weights_on_any_tile_h
   assert relerr(got, ref, elementwise=False) <= 8e-3
 
 
+# int8 weights at up to 16 rows per expert, streamed through LDS: one to six segments of 512 values to a row, with and without a
+# partial last one; channel counts that end inside a group of 32 or 64; tiles of one row, whole tiles, experts with none or several
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("k,n", [(32, 200), (512, 264), (544, 1000), (1536, 256), (2048, 776), (2592, 312), (3072, 328)])
+def test_gmm_int8_weights_streamed_through_lds(K, k, n, glu):
+  gs_h = np.array([1, 0, 16, 3, 17, 0, 40, 2, 0, 1], np.int32)
+  e, m = len(gs_h), int(gs_h.sum())
+  g = torch.Generator(device="cuda").manual_seed(k + n)
+  lhs = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+  weight = lambda: (torch.randint(-128, 128, (e, n, k), device="cuda", dtype=torch.int8, generator=g),
+                    torch.rand(e, n, device="cuda", generator=g) * 0.01 + 1e-3, torch.randn(e, n, device="cuda", generator=g))
+  w, scale, bias = weight()
+  kw = dict(rhs_scale=scale, rhs_bias=bias)
+  if glu:
+    kw["rhs_up"], kw["rhs_up_scale"], kw["rhs_up_bias"] = weight()
+    kw["act"] = "silu"
+  from routes import route
+
+  assert route("int8w", m, k, n, e, glu=glu)[:2] == ("gmm_wq_skinny_kernel", 32)
+  got = K.gmm_raw(lhs, w, cuda(gs_h), **kw)
+  if glu:
+    # the register-staged kernel: the same products, added in another order, and one rounding of the result each
+    assert relerr(got, K.gmm_raw(lhs, w, cuda(gs_h), kernel="stream", **kw), elementwise=False) <= 2.0**-8
+    return
+  start = 0
+  for i, r in enumerate(gs_h):
+    x, wd = lhs[start:start + r].double(), w[i].double() * scale[i].double()[:, None]
+    want = x @ wd.T.contiguous() + bias[i].double()
+    # sums of K products in f32 in any order, scale, bias, one rounding to bf16
+    bound = want.abs() * 2.0**-8 + (x.abs() @ wd.abs().T.contiguous() + bias[i].double().abs()) * (k + 4) * 2.0**-24
+    assert ((got[start:start + r].double() - want).abs() <= bound).all()
+    start += r
+
+
+# the persistent decode kernels: a row's result does not depend on whether its tile had 16 or 32 rows (empty experts lower the average
+# that picks the height), also where a tile ends after its first 16 rows
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("fmt,k,n", [("int8w", 1056, 264), ("int8w", 3072, 328), ("int4", 256, 1000), ("int4", 2880, 328), ("mxfp4", 1056, 784),
+                                     ("mxfp4", 3072, 264)])
+def test_persistent_decode_kernels_give_one_result_on_both_tile_heights(K, fmt, k, n, glu):
+  from maxtext_amd._lib import MOE_INT4, MOE_MXFP4
+  from routes import route
+
+  gs_h = np.array([1, 0, 16, 3, 17, 31, 40, 32, 33, 64], np.int32)
+  e, m = len(gs_h), int(gs_h.sum())
+  g = torch.Generator(device="cuda").manual_seed(k + n)
+  lhs = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+  rand = lambda *s: torch.rand(*s, device="cuda", generator=g)
+  packed = lambda: torch.randint(0, 256, (e, n, k // 2), device="cuda", dtype=torch.uint8, generator=g)
+  weight = {"int8w": lambda: (torch.randint(-128, 128, (e, n, k), device="cuda", dtype=torch.int8, generator=g), rand(e, n) * 0.01 + 1e-3),
+            "int4": lambda: (packed(), (rand(e, n, (k + 127) // 128) * 0.01 + 1e-3).to(torch.bfloat16)),
+            "mxfp4": lambda: (packed(), torch.randint(118, 124, (e, n, k // 32), device="cuda", dtype=torch.uint8, generator=g))}[fmt]
+  kw = {"int8w": {}, "int4": dict(rhs_dtype=MOE_INT4, rhs_scale_block_k=128), "mxfp4": dict(rhs_dtype=MOE_MXFP4, rhs_scale_block_k=32)}[fmt]
+  w, kw["rhs_scale"] = weight()
+  kw["rhs_bias"] = torch.randn(e, n, device="cuda", generator=g)
+  if glu:
+    kw["rhs_up"], kw["rhs_up_scale"] = weight()
+    kw["rhs_up_bias"], kw["act"] = torch.randn(e, n, device="cuda", generator=g), "silu"
+  more = 64 - e  # (groups without rows)
+  assert route(fmt, m, k, n, 64, glu=glu)[1] == 16 and route(fmt, m, k, n, 15, glu=glu)[1] == 32
+  grown = lambda t, x: torch.cat([t, t[:1].expand(x, *t.shape[1:])]).contiguous()
+  out = []
+  for x in (5, more):
+    kx = {a: grown(b, x) if torch.is_tensor(b) else b for a, b in kw.items()}
+    out.append(K.gmm_raw(lhs, grown(w, x), cuda(np.concatenate([gs_h, np.zeros(x, np.int32)])), **kx))
+  assert torch.equal(out[0], out[1])
+  ref = K.gmm_raw(lhs, w, cuda(gs_h), kernel="tiled", **kw)
+  assert relerr(out[0], ref, elementwise=False) <= 8e-3
+
+
 FP8_SHAPES = [
     (40, 256, 128, [7, 0, 12, 1, 20]),
     (256, 1024, 384, [8] * 32),
