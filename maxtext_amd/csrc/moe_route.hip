@@ -1270,6 +1270,7 @@ int moe_route_topk(const float* gate_logits, const float* pre_bias_logits, int T
 struct GateSort {
   int32_t *group_sizes, *perm, *inv_perm;
   void* gmm_workspace;
+  int tile_rows;
 };
 
 // How the gate product is cut.  Below 129 tiles of 32 tokens x 32 experts the chip is filled by splitting K (at least 8
@@ -1347,7 +1348,7 @@ static int gate_route_impl(const void* x, const void* gate_kernel_terms, int num
   if (sort && ng == 0 && T <= 4 * kSortWaves && (long long)T * (k + shared) <= kSortChunk && E + shared <= kSortMaxE) {
     int ebits = 0;
     while ((1 << ebits) < E + shared) ebits++;
-    const SortMapArgs mp = {(TileInfo*)((uint8_t*)sort->gmm_workspace + 16), (int32_t*)sort->gmm_workspace, E + shared, 0, 16, 1};
+    const SortMapArgs mp = {(TileInfo*)((uint8_t*)sort->gmm_workspace + 16), (int32_t*)sort->gmm_workspace, E + shared, 0, sort->tile_rows, 1};
     const RouteArgs r = {nullptr, nullptr, T, E, k, mode, norm_topk_prob, weights_round_bf16, routed_scaling_factor, 0, 0, topk_weights, topk_idx, shared};
     dispatch_vpl(E, [&](auto vpl) {
       constexpr int V = decltype(vpl)::value;
@@ -1358,7 +1359,7 @@ static int gate_route_impl(const void* x, const void* gate_kernel_terms, int num
                                                                                               nullptr, mp);
     });
     if (int st = check_launch("route_sort_small_kernel")) return st;
-    note_tile_map_built(sort->gmm_workspace, sort->group_sizes, T * (k + shared), E + shared, 0, E + shared, 16, 1);
+    note_tile_map_built(sort->gmm_workspace, sort->group_sizes, T * (k + shared), E + shared, 0, E + shared, sort->tile_rows, 1);
     *sorted = true;
     return MOE_OK;
   }
@@ -1629,7 +1630,6 @@ int moe_transpose_rhs(const void* rhs_gkn, int G, int K, int N, int elem_bytes, 
 namespace {
 struct LayerPlan {
   int M, K2, Et;          // routed rows, selections per token and experts with the shared ones
-  bool mapped;            // the sort leaves the tile list of the streaming kernels
   size_t weights, idx, perm, inv, groups, gate_ws, sort_ws, gmm_ws, gmm_bytes, xq, xs, inter, iq, is, y, total;
 };
 }  // namespace
@@ -1646,8 +1646,6 @@ static int layer_plan(const moe_layer_args* a, LayerPlan* p) {
   p->M = (int)rows;
   p->K2 = a->k + a->shared_experts;
   p->Et = a->E + a->shared_experts;
-  // (the sort's one-launch limit, and the rows per expert up to which moe_gmm takes 16-row tiles)
-  p->mapped = rows <= std::min(4096LL, 16LL * p->Et);
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t here = at;
@@ -1700,20 +1698,6 @@ int moe_layer(const moe_layer_args* a, void* workspace, size_t workspace_bytes, 
   void* gmm_ws = ws + p.gmm_ws;
   const int T = a->T, d = a->d, f = a->f;
   const bool quant = a->act_dtype != MOE_BF16;
-  const GateSort gs = {groups, perm, inv, gmm_ws};
-  bool sorted = false;
-  if (int st = gate_route_impl(a->gate_x ? a->gate_x : a->x, a->gate_terms, a->num_gate_terms, a->gate_bias, T, d, a->E, a->k, a->score_func, a->gate_round_bf16,
-                               a->route_mode, a->norm_topk_prob, a->weights_round_bf16, a->routed_scaling_factor, a->n_routing_groups, a->topk_routing_group,
-                               weights, idx, nullptr, nullptr, ws + p.gate_ws, moe_gate_route_workspace_bytes(T, d, a->E), a->shared_experts,
-                               p.mapped ? &gs : nullptr, &sorted, stream))
-    return st;
-  if (!sorted) {
-    const size_t sort_bytes = std::max(moe_sort_workspace_bytes(T, p.K2, p.Et), (size_t)16);
-    const int st = p.mapped ? moe_sort_by_expert_mapped(idx, T, p.K2, p.Et, 0, perm, inv, groups, nullptr, ws + p.sort_ws, sort_bytes, 16, p.Et, 0, 0, gmm_ws,
-                                                        p.gmm_bytes, stream)
-                            : moe_sort_by_expert_rolled(idx, T, p.K2, p.Et, 0, perm, inv, groups, nullptr, ws + p.sort_ws, sort_bytes, stream);
-    if (st) return st;
-  }
   moe_gmm_args g = {};
   g.struct_size = sizeof(g);
   g.group_sizes = groups;
@@ -1727,21 +1711,43 @@ int moe_layer(const moe_layer_args* a, void* workspace, size_t workspace_bytes, 
   g.act_limit = a->act_limit;
   g.out_dtype = MOE_BF16;
   g.lhs_rows = T;
-  g.lhs = a->x;
-  if (quant) {
-    if (int st = moe_gather_rows(a->x, nullptr, 1, T, T, d, a->act_dtype, a->act_block_k, MOE_QUANT_RINT_DIV, nullptr, nullptr, nullptr, ws + p.xq,
-                                 (float*)(ws + p.xs), stream))
-      return st;
-    g.lhs = ws + p.xq;
-    g.lhs_scale = (const float*)(ws + p.xs);
-  }
+  g.lhs = quant ? (const void*)(ws + p.xq) : a->x;
+  g.lhs_scale = quant ? (const float*)(ws + p.xs) : nullptr;
   g.rhs = a->wi_0; g.rhs_scale = a->wi_0_scale; g.rhs_up = a->wi_1; g.rhs_up_scale = a->wi_1_scale;
   g.out = ws + p.inter;
   g.K = d; g.N = f;
   g.rhs_scale_block_n = a->wi_scale_block_n; g.rhs_scale_block_k = a->wi_scale_block_k;
   g.act = a->act;
   g.lhs_row_idx = perm; g.lhs_row_idx_div = p.K2;
-  g.flags = a->wi_flags | (p.mapped ? MOE_GMM_SAME_GROUPS : 0);
+  g.flags = a->wi_flags;
+  // Up to the 4096 rows of its one launch the sort leaves the first product's tile list (a launch of its own is 4.7 us).  Not for the
+  // 160 rows and more of the kernel that may cut a last round along K: the sort does not clear its counters.
+  moe_gmm_route_info first = {};
+  if (int st = moe_gmm_route(&g, MOE_GMM_KERNEL_AUTO, &first)) return st;
+  const bool mapped = p.M <= 4096 && first.tile_rows > 0 && first.tile_rows <= 128 && first.tail_rows == 0;
+  if (mapped) {
+    g.flags |= MOE_GMM_SAME_GROUPS;
+    g.workspace_bytes = moe_gmm_workspace_bytes(p.M, p.Et);
+  }
+  const GateSort gs = {groups, perm, inv, gmm_ws, first.tile_rows};
+  bool sorted = false;
+  if (int st = gate_route_impl(a->gate_x ? a->gate_x : a->x, a->gate_terms, a->num_gate_terms, a->gate_bias, T, d, a->E, a->k, a->score_func, a->gate_round_bf16,
+                               a->route_mode, a->norm_topk_prob, a->weights_round_bf16, a->routed_scaling_factor, a->n_routing_groups, a->topk_routing_group,
+                               weights, idx, nullptr, nullptr, ws + p.gate_ws, moe_gate_route_workspace_bytes(T, d, a->E), a->shared_experts,
+                               mapped ? &gs : nullptr, &sorted, stream))
+    return st;
+  if (!sorted) {
+    const size_t sort_bytes = std::max(moe_sort_workspace_bytes(T, p.K2, p.Et), (size_t)16);
+    const int st = mapped ? moe_sort_by_expert_mapped(idx, T, p.K2, p.Et, 0, perm, inv, groups, nullptr, ws + p.sort_ws, sort_bytes, first.tile_rows, p.Et,
+                                                      0, 0, gmm_ws, p.gmm_bytes, stream)
+                          : moe_sort_by_expert_rolled(idx, T, p.K2, p.Et, 0, perm, inv, groups, nullptr, ws + p.sort_ws, sort_bytes, stream);
+    if (st) return st;
+  }
+  if (quant) {
+    if (int st = moe_gather_rows(a->x, nullptr, 1, T, T, d, a->act_dtype, a->act_block_k, MOE_QUANT_RINT_DIV, nullptr, nullptr, nullptr, ws + p.xq,
+                                 (float*)(ws + p.xs), stream))
+      return st;
+  }
   if (int st = moe_gmm(&g, stream)) return st;
   g.lhs = ws + p.inter;
   g.lhs_scale = nullptr;
@@ -1759,6 +1765,11 @@ int moe_layer(const moe_layer_args* a, void* workspace, size_t workspace_bytes, 
   g.act = MOE_ACT_NONE;
   g.lhs_row_idx = nullptr; g.lhs_row_idx_div = 1; g.lhs_rows = p.M;
   g.flags = a->wo_flags | MOE_GMM_SAME_GROUPS;
+  if (mapped) {
+    moe_gmm_route_info second = {};
+    if (int st = moe_gmm_route(&g, MOE_GMM_KERNEL_AUTO, &second)) return st;
+    if (second.tile_rows > 128 || second.tail_rows) g.workspace_bytes = p.gmm_bytes;
+  }
   if (int st = moe_gmm(&g, stream)) return st;
   return moe_unpermute_combine(ws + p.y, nullptr, inv, weights, nullptr, T, p.K2, d, a->out, nullptr, 0, stream);
 }

@@ -44,9 +44,9 @@ def _both(block, *args, **kw):
 
 
 @pytest.mark.parametrize("name", ["c2", "c2f8", "c3", "c4", "c5", "c5mx"])
-# (one block routes and sorts up to 4 and up to 16 tokens; 65 rows and more: the sort's larger variants; past 16 rows per expert no
-# tile list is handed on; the largest run on the prefill kernels)
-@pytest.mark.parametrize("tokens", [1, 4, 5, 16, 17, 130, 700, 2100])
+# (one block routes and sorts up to 4 and up to 16 tokens; 65 rows and more: the sort's larger variants, with tile lists of 16 to 128
+# rows; past 4096 rows and on the prefill kernels no tile list is handed on)
+@pytest.mark.parametrize("tokens", [1, 4, 5, 16, 17, 60, 130, 300, 700, 2100])
 def test_layer_call_equals_the_single_calls(name, tokens):
   block, x, _ = _block(name, tokens)
   got, want = _both(block, x)
