@@ -879,8 +879,9 @@ def test_int4_rows_past_whole_128_or_256_rows_multiply_f32_weights_on_any_tile_h
 # partial last one; channel counts that end inside a group of 32 or 64; tiles of one row, whole tiles, experts with none or several
 @pytest.mark.parametrize("glu", [False, True])
 @pytest.mark.parametrize("k,n", [(32, 200), (512, 264), (544, 1000), (1536, 256), (2048, 776), (2592, 312), (3072, 328)])
-def test_gmm_int8_weights_streamed_through_lds(K, k, n, glu):
-  gs_h = np.array([1, 0, 16, 3, 17, 0, 40, 2, 0, 1], np.int32)
+@pytest.mark.parametrize("most", [40, 110])
+def test_gmm_int8_weights_streamed_through_lds(K, k, n, glu, most):
+  gs_h = np.array([1, 0, 16, 3, 17, 0, most, 2, 0, 1], np.int32)
   e, m = len(gs_h), int(gs_h.sum())
   g = torch.Generator(device="cuda").manual_seed(k + n)
   lhs = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
@@ -893,7 +894,7 @@ def test_gmm_int8_weights_streamed_through_lds(K, k, n, glu):
     kw["act"] = "silu"
   from routes import route
 
-  assert route("int8w", m, k, n, e, glu=glu)[:2] == ("gmm_wq_skinny_kernel", 32)
+  assert route("int8w", m, k, n, e, glu=glu)[:2] == ("gmm_wq_skinny_kernel", 32 if m > 14 * e else 16)
   got = K.gmm_raw(lhs, w, cuda(gs_h), **kw)
   if glu:
     # the register-staged kernel: the same products, added in another order, and one rounding of the result each
@@ -933,11 +934,11 @@ def test_persistent_decode_kernels_give_one_result_on_both_tile_heights(K, fmt, 
   if glu:
     kw["rhs_up"], kw["rhs_up_scale"] = weight()
     kw["rhs_up_bias"], kw["act"] = torch.randn(e, n, device="cuda", generator=g), "silu"
-  more = 64 - e  # (groups without rows)
-  assert route(fmt, m, k, n, 64, glu=glu)[1] == 16 and route(fmt, m, k, n, 15, glu=glu)[1] == 32
+  few, many = (5 if fmt == "int8w" else 4), 64 - e  # (groups without rows)
+  assert route(fmt, m, k, n, 64, glu=glu)[1] == 16 and route(fmt, m, k, n, e + few, glu=glu)[1] == 32
   grown = lambda t, x: torch.cat([t, t[:1].expand(x, *t.shape[1:])]).contiguous()
   out = []
-  for x in (5, more):
+  for x in (few, many):
     kx = {a: grown(b, x) if torch.is_tensor(b) else b for a, b in kw.items()}
     out.append(K.gmm_raw(lhs, grown(w, x), cuda(np.concatenate([gs_h, np.zeros(x, np.int32)])), **kx))
   assert torch.equal(out[0], out[1])
