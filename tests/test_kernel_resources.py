@@ -100,6 +100,19 @@ def test_lds_streamed_decode_kernel_uses_no_scratch_and_waits_only_where_written
 
 
 @pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")), reason="needs hipcc")
+def test_persistent_decode_kernels_on_32_rows_and_int8_use_no_scratch(tmp_path):
+  """The same body on tiles of up to 32 rows and on int8 weights: every instance fits its registers."""
+  # 2 formats x 3 segment counts x with / without the second projection; 6 segment counts x the same x 2 tile heights
+  found = {"moe_gmm_wqs32.hip": (r"_ZN3moe14gmm_wqs_kernel\w+", 12), "moe_gmm_wq.hip": (r"_ZN3moe20gmm_wq_skinny_kernelILi\dELb[01]ELi\d\dEE\w+", 24)}
+  with ThreadPoolExecutor(max_workers=2) as pool:
+    texts = list(pool.map(lambda src: _assembly(src, str(tmp_path)), found))
+  for (name, count), asm in zip(found.values(), texts):
+    sizes = re.findall(r"\.name:\s+(" + name + r")\n\s+\.private_segment_fixed_size:\s+(\d+)", asm)
+    assert len(sizes) == count, sizes
+    assert all(int(b) == 0 for _, b in sizes), sizes
+
+
+@pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")), reason="needs hipcc")
 def test_lds_streamed_fp8_decode_kernel_uses_no_scratch_and_waits_only_where_written(tmp_path):
   """The persistent fp8 decode kernel follows the same rules: up to 112 registers of activations stay resident per lane, so
   every instantiation must fit its registers, and between the barriers of its item loop the only waits on the
